@@ -1,0 +1,86 @@
+"""The matrix-core decode at head_dim 64: chunk, wave and split edges, partial
+row groups, unmapped tokens, and query magnitudes outside the fp16 range,
+against the fp64 oracle.
+
+Bound: the kernel's fp32 sums and hi/lo operands are exact to ~2^-20 of a row,
+far below fp16's half ulp, so an output differs from the correctly rounded
+exact result by at most one fp16 ulp of its row's largest element (both sides
+of a rounding boundary)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from turborag_amd.synthetic import as_u16, kv_tokens_major, permuted_slots
+
+pytestmark = pytest.mark.gpu
+D, B = 64, 16
+
+
+def _row_ulps(got16: np.ndarray, ref: np.ndarray) -> float:
+    g = got16.reshape(-1, D).astype(np.float64)
+    r = ref.reshape(-1, D)
+    m = np.abs(r).max(axis=1).astype(np.float16)
+    ulp = np.nextafter(m, np.float16(np.inf)).astype(np.float64) - m.astype(np.float64)
+    return float((np.abs(g - r.astype(np.float16).astype(np.float64)).max(axis=1) / ulp).max())
+
+
+def _check(tq, oracle, cuda, scheme, q, k, v, slots, all_slots):
+    Q, H, N = q.shape[0], q.shape[1], k.shape[0]
+    cfg = tq.default_config()
+    cfg.num_kv_heads, cfg.head_dim = H, D
+    prod = scheme == "turbo_prod"
+    lay = tq.make_layout_for(cfg) if prod else tq.make_mse_layout_for(cfg)
+    pages = int(all_slots.max()) // B + 1
+    pack = oracle.prod_pack if prod else oracle.mse_pack
+    pool = pack(as_u16(k), as_u16(v), all_slots.numpy(), pages, B)
+    f64 = oracle.prod_attention_f64 if prod else oracle.mse_attention_f64
+    ref = f64(as_u16(q), pool, slots.numpy(), B)
+    out = torch.full((Q, H, D), 7.0, dtype=torch.float16, device=cuda)
+    fn = tq.fused_attn_output if prod else tq.mse_fused_attn_output
+    fn(q.to(cuda), torch.from_numpy(pool).to(cuda), slots.to(cuda), out, lay, cfg, Q, N)
+    torch.cuda.synchronize()
+    u = _row_ulps(out.cpu().numpy(), ref)
+    print(f"    {u:.2f} row-max ulps", flush=True)
+    assert u <= 1.0
+
+
+@pytest.mark.parametrize("scheme", ["turbo_prod", "turbo_mse"])
+@pytest.mark.parametrize("Q,H,N", [(1, 1, 1), (1, 2, 31), (7, 2, 32), (8, 3, 33), (9, 2, 256),
+                                   (17, 1, 257), (7, 2, 6001), (8, 8, 2049)])
+def test_edges(tq, oracle, cuda, scheme, Q, H, N):
+    print(f"[decode64 {scheme}] Q={Q} H={H} N={N}", flush=True)
+    k, v = kv_tokens_major(N, H, D, seed=N)
+    slots = permuted_slots(N, B, seed=N + 1)
+    _check(tq, oracle, cuda, scheme, kv_tokens_major(Q, H, D, seed=N + 2)[0], k, v, slots, slots)
+
+
+@pytest.mark.parametrize("scheme", ["turbo_prod", "turbo_mse"])
+def test_unmapped_tokens(tq, oracle, cuda, scheme):
+    N, H = 700, 2
+    print(f"[decode64 holes {scheme}]", flush=True)
+    k, v = kv_tokens_major(N, H, D, seed=5)
+    slots = permuted_slots(N, B, seed=6)
+    holes = slots.clone()
+    holes[::7] = -1
+    holes[256:600] = -1  # one whole split and most of the next
+    _check(tq, oracle, cuda, scheme, kv_tokens_major(3, H, D, seed=7)[0], k, v, holes, slots)
+
+
+@pytest.mark.parametrize("scheme", ["turbo_prod", "turbo_mse"])
+@pytest.mark.parametrize("q_scale,k_scale", [(2.0 ** 14, 2.0 ** -13), (2.0 ** -11, 2.0 ** 10)])
+def test_query_magnitudes(tq, oracle, cuda, scheme, q_scale, k_scale):
+    """Rotated queries past fp16's largest value, and queries and keys whose
+    product is ordinary but whose own sizes are far from 1: the logits, and so
+    the outputs, are those of scale 1.  (|k| < 50 before its scale, outlier
+    channels included, so the scaled keys stay finite in fp16.)"""
+    N, H, Q = 500, 2, 8
+    print(f"[decode64 magnitude {scheme}] {q_scale:g} {k_scale:g}", flush=True)
+    k, v = kv_tokens_major(N, H, D, seed=8)
+    q = (kv_tokens_major(Q, H, D, seed=9)[0].float().clamp(-3.9, 3.9) * q_scale)
+    d = torch.arange(D)
+    for h in range(H):  # a row whose rotation is one spike of 8 x its entries
+        q[0, h] = (1 - 2 * ((d + h) % 2)).float() * q_scale
+    _check(tq, oracle, cuda, scheme, q.half(), (k.float() * k_scale).half(), v,
+           permuted_slots(N, B, seed=10), permuted_slots(N, B, seed=10))

@@ -88,8 +88,8 @@ struct PagedTokens {
 // ---------------------------------------------------------------------------
 // Split-K partial: one wave per (split, row = q*H + h).
 // ws[(split * rows + row) * (D + 2) + ...] = acc[0..D), m, l.
-// Any head_dim and page geometry (the matrix-core kernels take D = 128 with
-// aligned pages).
+// Any head_dim and page geometry (the matrix-core kernels take D = 64 and 128
+// with aligned pages).
 // ---------------------------------------------------------------------------
 template <int D, bool PROD, class Tok>
 __global__ __launch_bounds__(64) void attn_partial_kernel(
@@ -435,6 +435,19 @@ struct TableWords {
     static constexpr int kR1Stores = PROD ? 8 : 4;
     uint32_t r0[4], r1[kR1Stores];
 };
+// The lo parts of aV*V4 as pairs: store k < 4 of wave w holds row
+// 32w + 8k + lane / 8 (turbo_mse's S rows; turbo_prod's V lo rows).
+__device__ __forceinline__ void lo_table_words(int w, int lane, uint32_t (&r)[4]) {
+    const int g8 = lane >> 3;
+    const uint32_t sel8 = lut4_sel(g8 & 3);
+    const bool hi8 = (g8 & 4) != 0;
+    uint32_t llo[2];
+#pragma unroll
+    for (int hh = 0; hh < 2; ++hh)
+        llo[hh] = hi8 ? lut4(kF16.v4lo, 2 * hh + 1, sel8) : lut4(kF16.v4lo, 2 * hh, sel8);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) r[k] = llo[k & 1] | (kF16.v4lo[2 * w + (k >> 1)] << 16);
+}
 template <bool PROD>
 __device__ __forceinline__ TableWords<PROD> decode_table_words(int w, int lane) {
     TableWords<PROD> tw;
@@ -458,20 +471,20 @@ __device__ __forceinline__ TableWords<PROD> decode_table_words(int w, int lane) 
                 r1[k] = vq ? vpair : kpair;
             }
         } else {
-            uint32_t llo[2], vlo[2];
+            uint32_t vlo[2];
 #pragma unroll
-            for (int hh = 0; hh < 2; ++hh) {
-                llo[hh] = hi8 ? lut4(kF16.v4lo, 2 * hh + 1, sel8) : lut4(kF16.v4lo, 2 * hh, sel8);
+            for (int hh = 0; hh < 2; ++hh)
                 vlo[hh] = hi8 ? lut4(kF16.v4, 2 * hh + 1, sel8) : lut4(kF16.v4, 2 * hh, sel8);
-            }
+            lo_table_words(w, lane, r0);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                r0[k] = llo[k & 1] | (kF16.v4lo[2 * w + (k >> 1)] << 16);
-                r1[k] = vlo[k & 1] | (kF16.v4[2 * w + (k >> 1)] << 16);
-            }
+            for (int k = 0; k < 4; ++k) r1[k] = vlo[k & 1] | (kF16.v4[2 * w + (k >> 1)] << 16);
         }
     }
     return tw;
+}
+// Exponent e with x * 2^-e in [0.5, 1); 0 for a zero or non-finite x.
+__device__ __forceinline__ int scale_exp(float x) {
+    return __builtin_isfinite(x) ? __builtin_amdgcn_frexp_expf(x) : 0;
 }
 template <bool PROD>
 __device__ __forceinline__ void store_decode_tables(uint32_t* lut, int kv_words, int w, int lane,
@@ -2179,7 +2192,7 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(
 // ===========================================================================
 // Decode over slot-mapped tokens: the reference's fused attention entries
 // (src/cuda/tq_turbo_prod_kernels.cu:439-571, 650-671;
-// src/cuda/tq_turbo_mse_kernels.cu:302-417, 459-479) for D = 128 and
+// src/cuda/tq_turbo_mse_kernels.cu:302-417, 459-479) for D = 64, 128 and
 // turbo_prod / turbo_mse pages.
 //
 // Flash-decoding split-K on a (split, kv head, row group) grid, 8 waves of
@@ -2208,16 +2221,20 @@ using namespace mfma;
 
 // LDS layout of the tables (entries as decode_table_words describes) (32 copies of each entry, copy c at 4c; lane l
 // reads copy l % 32, so a half-wave's random lookups hit distinct banks):
-//   S table: byte 256b + 4c (the rows' upper halves unused: the table ends
-//   below kOffK);
+//   S table: byte 256b + 4c;
 //   K table: byte kOffK + 256b + 4c (turbo_mse's V lookups read it too);
-//   turbo_prod's V table: kOffK + 256b + 128 + 4c.
+//   turbo_prod's V table: kOffK + 256b + 128 + 4c;
+//   turbo_prod's V lo table (head_dim 64): 256b + 128 + 4c, c < kLoCopies (the
+//   S rows' upper halves; the last four copies of the last row would lie past
+//   kOffK, so lanes 28 .. 31 of a half-wave read copies 0 .. 3).
 // A K lookup reads its S and K entries from one address register with
 // offsets 0 and kOffK: no two-address LDS read reaches that pair (ds_read2
 // spans up to 1020 bytes, ds_read2st64 multiples of 256), so each result
 // goes straight into its MFMA operand registers.
 constexpr int kOffK = 65520;
 constexpr int kLutWords = (kOffK + 256 * 256) / 4;
+constexpr int kLoCopies = 28;
+static_assert(256 * 255 + 128 + 4 * kLoCopies <= kOffK, "the V lo rows end below the K table");
 
 // LDS address of copy (lane & 31) of entry `byte b of word` in a table of
 // 256-byte entries at `base` (base = table + copy offset): v_perm puts the
@@ -2245,12 +2262,23 @@ __device__ __forceinline__ uint32_t hilo_pair(float a0, float b0, float a1, floa
 }
 
 constexpr int kWaves = 8, kChunk = 32, kPass = kWaves * kChunk;
-// Partial of (split, row): o[128] at po[(pid * 8 + r) * 128], (m, l) at
+// Partial of (split, row): o[D] at po[(pid * 8 + r) * D], (m, l) at
 // pml[(item * 8 + r) * S + split] with pid = item * S + split and item =
 // row group * H + kv head.
-constexpr size_t kPartBytes = kRows * (128 * sizeof(float) + 2 * sizeof(float));
+constexpr size_t part_bytes(int D) { return kRows * (D + 2) * sizeof(float); }
 
-template <int SCH>
+// D = 128, or D = 64: half the dims per token (two QK k-steps instead of
+// four, four PV tiles instead of eight), 8-byte K and 2-byte V loads per
+// lane.  D = 64 also carries what keeps it as exact as fp32 arithmetic: V's
+// fp16 lo parts (a second PV product in its own accumulators; the table's
+// hi parts alone are 5e-5 off in the mean, a quarter of the output's own
+// fp16 rounding), and a power of two per query row that holds the row's fp16
+// parts in range whatever its magnitude.  Bound by its dependent loads and
+// the setup, as D = 128: 7 rows x 2 heads x 6,001 tokens (turbo_mse) take 6.0
+// (split) + 2.9 us (combine); the generic one-wave-per-row kernels, whose
+// cross-lane sum per token and serial merge over 147 splits this replaces,
+// took 22.7 + 70.2 us.
+template <int SCH, int D>
 __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     const uint16_t* __restrict__ query, const uint8_t* __restrict__ pool,
     const int32_t* __restrict__ slots, float* __restrict__ po, float2* __restrict__ pml,
@@ -2258,15 +2286,21 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     PageGeom g) {
     constexpr bool PROD = SCH == kSchProd;
     static_assert(SCH == kSchProd || SCH == kSchMse, "turbo_prod or turbo_mse pages");
+    static_assert(D == 128 || D == 64, "head_dim 64 or 128");
+    constexpr int kS = D / 32;       // QK k-steps; lane group gq holds dims [D/4 gq, D/4 gq + D/4)
+    constexpr int kNT = D / 16;      // PV tiles: lane i holds dims kNT i .. + kNT - 1
+    constexpr int kL = D / 2;        // lanes of a row held two values per lane
+    constexpr bool VLO = D == 64, QSCALE = D == 64;
     // The decode tables (layout above); after the chunk loop the space holds
     // the waves' results for the merge.
     __shared__ __attribute__((aligned(256))) uint32_t lut[kLutWords];
-    __shared__ uint4 bqs[4][64];  // QK B operand of k-step s for lane l
+    __shared__ uint4 bqs[kS][64];  // QK B operand of k-step s for lane l
     __shared__ uint64_t tko[kWaves][kChunk], tvo[kWaves][kChunk];
     __shared__ float4 tsc[kWaves][kChunk];  // per token: K scale, residual scale, vs / aV, bias
     __shared__ float mm[kWaves][kRows], ml[kWaves][kRows];
-    float(*mo)[kRows][128] = reinterpret_cast<float(*)[kRows][128]>(&lut[0]);
-    static_assert(sizeof(float) * kWaves * kRows * 128 <= sizeof(lut), "merge space");
+    __shared__ float rsc[kRows];  // QSCALE: the rows' power of two
+    float(*mo)[kRows][D] = reinterpret_cast<float(*)[kRows][D]>(&lut[0]);
+    static_assert(sizeof(float) * kWaves * kRows * D <= sizeof(lut), "merge space");
 
     int split, h, rg;
     if (gridDim.x == (unsigned)num_splits) {
@@ -2282,6 +2316,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int i = lane & 15, gq = lane >> 4;
+    const int jl = lane & (kL - 1);  // this lane's pair of a row (D = 64: lanes l and l + 32 alike)
     const int t_begin = split * tokens_per_split;
     const int t_end = min(num_kv_tokens, t_begin + tokens_per_split);
     // logit scale per unit ks (log2(e) / alpha folded at compile time: no run-time division)
@@ -2293,7 +2328,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     //    first chunk's slots, then the decode-table words.
     const int qrow = rg * kRows + w;
     const uint32_t qraw = *reinterpret_cast<const uint32_t*>(
-        query + ((size_t)min(qrow, num_queries - 1) * g.H + h) * 128 + 2 * lane);
+        query + ((size_t)min(qrow, num_queries - 1) * g.H + h) * D + 2 * jl);
     int t0 = t_begin + w * kChunk;
     auto load_slot = [&](int t) -> int {
         return slots[max(min(t + (lane & (kChunk - 1)), t_end - 1), 0)];
@@ -2304,8 +2339,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     //    Tokens past the range or with a negative slot read the first bytes
     //    of the query instead (always valid memory) and get bias -inf.
     struct Chunk {
-        uint4 kw[2];     // K: tile tau, token 16 tau + i, bytes [16 gq, 16 gq + 16)
-        uint32_t vw[8];  // V: k-index 8 gq + e (token below), dword i
+        uint32_t kw[2][kS];  // K: tile tau, token 16 tau + i, bytes [4 kS gq, 4 kS gq + 4 kS)
+        uint32_t vw[8];  // V: k-index 8 gq + e (token below), bytes [D/32 i, D/32 i + D/32)
         uint16_t ks, re, vs;
         bool valid;
     };
@@ -2326,12 +2361,22 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-        for (int tau = 0; tau < 2; ++tau) c.kw[tau] = ld_u4_nt(pool + (tko[w][16 * tau + i] + 16 * gq));
+        for (int tau = 0; tau < 2; ++tau) {
+            const uint8_t* kp = pool + (tko[w][16 * tau + i] + 4 * kS * gq);
+            if constexpr (D == 128) {
+                const uint4 x = ld_u4_nt(kp);
+                c.kw[tau][0] = x.x, c.kw[tau][1] = x.y, c.kw[tau][2] = x.z, c.kw[tau][3] = x.w;
+            } else {
+                const uint2 x = ld_u2_nt(kp);
+                c.kw[tau][0] = x.x, c.kw[tau][1] = x.y;
+            }
+        }
         // k-index 8 gq + e is token 4 gq + e (e < 4) or 16 + 4 gq + (e - 4)
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             const int tok = e < 4 ? 4 * gq + e : 16 + 4 * gq + (e - 4);
-            c.vw[e] = ld_u32_nt(pool + (tvo[w][tok] + 4 * i));
+            const uint8_t* vp = pool + (tvo[w][tok] + D / 32 * i);
+            c.vw[e] = D == 128 ? ld_u32_nt(vp) : (uint32_t)ld_u16_nt(vp);
         }
     };
     Chunk cur;
@@ -2342,29 +2387,49 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     // The tables' words, computed in registers while the codes are in flight
     // (no memory traffic; each 16-byte store writes four copies).
     const TableWords<PROD> tw = decode_table_words<PROD>(w, lane);
+    uint32_t vlo[4];
+    if constexpr (VLO && PROD) lo_table_words(w, lane, vlo);
     // 3. This wave's query row: qrot = WHT(q * s) * inv, stored as fp16 hi
     //    and lo parts into the B operand (column 2w: hi, 2w + 1: lo; lane l
-    //    holds d = 2l, 2l + 1: k-group l / 16, k-step (l / 4) % 4, halves
+    //    holds d = 2l, 2l + 1: k-group l / (4 kS), k-step (l / 4) % kS, halves
     //    2(l % 4), + 1 of the half8).
     {
         const float sh = (h & 1) ? -1.0f : 1.0f;
         float q0 = h2f(qraw & 0xffff) * sh, q1 = h2f(qraw >> 16) * (-sh);
-        wht_pair<64>(q0, q1, lane);
+        wht_pair<kL>(q0, q1, lane);
         const bool live = qrow < num_queries;
         q0 = live ? q0 * inv : 0.0f;
         q1 = live ? q1 * inv : 0.0f;
+        if constexpr (QSCALE) {
+            // the row's largest |q| scaled into [0.5, 1) (a zero or non-finite
+            // row is left as it is); its logits are multiplied back
+            const int ex = scale_exp(max_lanes<kL>(fmaxf(fabsf(q0), fabsf(q1))));
+            q0 = __builtin_amdgcn_ldexpf(q0, -ex);
+            q1 = __builtin_amdgcn_ldexpf(q1, -ex);
+            if (lane == 0) rsc[w] = __builtin_amdgcn_ldexpf(1.0f, ex);
+        }
         const uint32_t hi = pack_h2(q0, q1);
         const uint32_t lo = lo_pair(q0, q1, hi);
-        uint32_t* b = reinterpret_cast<uint32_t*>(&bqs[(lane >> 2) & 3][16 * (lane >> 4) + 2 * w]);
-        b[lane & 3] = hi;
-        b[4 + (lane & 3)] = lo;  // the next lane's (column 2w + 1) half8
+        uint32_t* b = reinterpret_cast<uint32_t*>(
+            &bqs[(jl >> 2) & (kS - 1)][16 * (jl / (4 * kS)) + 2 * w]);
+        b[jl & 3] = hi;  // (D = 64: both halves of the wave write the same words)
+        b[4 + (jl & 3)] = lo;  // the next lane's (column 2w + 1) half8
     }
     // 4. The decode tables.
     store_decode_tables<PROD>(lut, kOffK / 4, w, lane, tw);
-    lds_barrier();
-    half8 bq[4];
+    if constexpr (VLO && PROD) {
+        if ((lane & 7) < kLoCopies / 4) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) bq[s] = __builtin_bit_cast(half8, bqs[s][lane]);
+            for (int k = 0; k < 4; ++k)
+                *reinterpret_cast<u32x4*>(
+                    &lut[(32 * w + 8 * k + (lane >> 3)) * 64 + 32 + 4 * (lane & 7)]) =
+                    (u32x4){vlo[k], vlo[k], vlo[k], vlo[k]};
+        }
+    }
+    lds_barrier();
+    half8 bq[kS];
+#pragma unroll
+    for (int s = 0; s < kS; ++s) bq[s] = __builtin_bit_cast(half8, bqs[s][lane]);
 
     // Lookup bases: copy lane % 32 of entry 0 of the S table (the K table
     // is kOffK above it; turbo_mse's V lookups read it that way), and of
@@ -2374,13 +2439,24 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         PROD ? (uint32_t)reinterpret_cast<uintptr_t>((lds_u32*)&lut[kOffK / 4 + 32 + (lane & 31)])
              : basek;
     constexpr uint32_t offv = PROD ? 0u : (uint32_t)kOffK;
+    // VLO: base of the V lo lookups, whose hi pair is kOffK above (turbo_prod:
+    // its copies of the S rows' upper halves; turbo_mse: the S table)
+    const uint32_t basel =
+        PROD ? (uint32_t)reinterpret_cast<uintptr_t>(
+                   (lds_u32*)&lut[32 + ((lane & 31) < kLoCopies ? lane & 31 : (lane & 31) - kLoCopies)])
+             : basek;
+    const float qsc = QSCALE ? rsc[i >> 1] : 1.0f;
     const bool lo_col = (i & 1) != 0;
     const uint32_t lomask = lo_col ? 0xFFFFFFFFu : 0u;
 
     float m_run = kInitMax, l_run = 0.0f;
-    f32x4 acc[8];
+    f32x4 acc[kNT], acl[VLO ? kNT : 1];  // PV sums; VLO: of V's lo parts (x 2^kLoShift)
 #pragma unroll
-    for (int v = 0; v < 8; ++v) acc[v] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    for (int v = 0; v < kNT; ++v) acc[v] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    if constexpr (VLO) {
+#pragma unroll
+        for (int v = 0; v < kNT; ++v) acl[v] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
     bool first = true;
 
     while (t0 < t_end) {  // wave-uniform
@@ -2406,16 +2482,15 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
 #pragma unroll
             for (int e = 0; e < 4; ++e) scv[tau][e] = tsc[w][16 * tau + 4 * gq + e];
         // QK: every K lookup of the chunk issued before the first MFMA.
-        half8 ka[2][4], kb[2][4];
+        half8 ka[2][kS], kb[2][kS];
 #pragma unroll
         for (int tau = 0; tau < 2; ++tau) {
-            const uint32_t wd[4] = {cur.kw[tau].x, cur.kw[tau].y, cur.kw[tau].z, cur.kw[tau].w};
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
+            for (int s = 0; s < kS; ++s) {
                 uint32_t e0[4], e1[4];  // K entries, S entries
 #pragma unroll
                 for (int b = 0; b < 4; ++b) {
-                    const uint32_t a = lut_addr(wd[s], b, basek);
+                    const uint32_t a = lut_addr(cur.kw[tau][s], b, basek);
                     e0[b] = *reinterpret_cast<const lds_u32*>(a + kOffK);
                     e1[b] = *reinterpret_cast<const lds_u32*>(a);
                 }
@@ -2430,22 +2505,43 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
             cb[tau] = (f32x4){0.f, 0.f, 0.f, 0.f};
             cs[tau] = cb[tau];
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
+            for (int s = 0; s < kS; ++s) {
                 cb[tau] = mma(ka[tau][s], bq[s], cb[tau]);
                 cs[tau] = mma(kb[tau][s], bq[s], cs[tau]);  // prod: residual signs; mse: lo parts
             }
         }
         // V lookups (B operands of PV), in flight during the softmax.
-        uint32_t bv[8][4];  // [N-tile v = d - 8i][token pair]
+        uint32_t bv[kNT][4];  // [N-tile v = d - kNT i][token pair]
+        uint32_t bl[VLO ? kNT : 1][4];
+        if constexpr (D == 128) {
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const uint32_t we = cur.vw[2 * q], wo = cur.vw[2 * q + 1];
-            const uint32_t lob = (we & 0x0F0F0F0Fu) | ((wo & 0x0F0F0F0Fu) << 4);
-            const uint32_t hib = ((we >> 4) & 0x0F0F0F0Fu) | (wo & 0xF0F0F0F0u);
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t we = cur.vw[2 * q], wo = cur.vw[2 * q + 1];
+                const uint32_t lob = (we & 0x0F0F0F0Fu) | ((wo & 0x0F0F0F0Fu) << 4);
+                const uint32_t hib = ((we >> 4) & 0x0F0F0F0Fu) | (wo & 0xF0F0F0F0u);
 #pragma unroll
-            for (int b = 0; b < 4; ++b) {
-                bv[2 * b][q] = *reinterpret_cast<const lds_u32*>(lut_addr(lob, b, basev) + offv);
-                bv[2 * b + 1][q] = *reinterpret_cast<const lds_u32*>(lut_addr(hib, b, basev) + offv);
+                for (int b = 0; b < 4; ++b) {
+                    bv[2 * b][q] = *reinterpret_cast<const lds_u32*>(lut_addr(lob, b, basev) + offv);
+                    bv[2 * b + 1][q] = *reinterpret_cast<const lds_u32*>(lut_addr(hib, b, basev) + offv);
+                }
+            }
+        } else {
+            // two token pairs per word (a lane's row part is two bytes)
+#pragma unroll
+            for (int p = 0; p < 2; ++p) {
+                const uint32_t we = cur.vw[4 * p] | (cur.vw[4 * p + 2] << 16);
+                const uint32_t wo = cur.vw[4 * p + 1] | (cur.vw[4 * p + 3] << 16);
+                const uint32_t lob = (we & 0x0F0F0F0Fu) | ((wo & 0x0F0F0F0Fu) << 4);
+                const uint32_t hib = ((we >> 4) & 0x0F0F0F0Fu) | (wo & 0xF0F0F0F0u);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) {
+                    const int v = 2 * (b & 1), q = 2 * p + (b >> 1);
+                    const uint32_t a0 = lut_addr(lob, b, basel), a1 = lut_addr(hib, b, basel);
+                    bv[v][q] = *reinterpret_cast<const lds_u32*>(a0 + kOffK);
+                    bl[v][q] = *reinterpret_cast<const lds_u32*>(a0);
+                    bv[v + 1][q] = *reinterpret_cast<const lds_u32*>(a1 + kOffK);
+                    bl[v + 1][q] = *reinterpret_cast<const lds_u32*>(a1);
+                }
             }
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -2459,7 +2555,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
                 const float4 sc = scv[tau][e];
                 const float sb = cb[tau][e] + quad_xor<1>(cb[tau][e]);
                 const float sr = cs[tau][e] + quad_xor<1>(cs[tau][e]);
-                lg[tau][e] = fmaf(sb, sc.x, fmaf(sr, sc.y, sc.w));
+                lg[tau][e] = QSCALE ? fmaf(fmaf(sb, sc.x, sr * sc.y), qsc, sc.w)
+                                    : fmaf(sb, sc.x, fmaf(sr, sc.y, sc.w));
                 mloc = fmaxf(mloc, lg[tau][e]);
             }
         mloc = lane_xor_reduce<16>(mloc, [](float x, float y) { return fmaxf(x, y); });
@@ -2482,11 +2579,17 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
             // acc lane (d, g) holds columns 4g .. 4g + 3 = rows 2g, 2g + 1
             const float a0 = __shfl(alpha, 4 * gq), a1 = __shfl(alpha, 4 * gq + 2);
 #pragma unroll
-            for (int v = 0; v < 8; ++v) {
+            for (int v = 0; v < kNT; ++v) {
                 acc[v][0] *= a0;
                 acc[v][1] *= a0;
                 acc[v][2] *= a1;
                 acc[v][3] *= a1;
+                if constexpr (VLO) {
+                    acl[v][0] *= a0;
+                    acl[v][1] *= a0;
+                    acl[v][2] *= a1;
+                    acl[v][3] *= a1;
+                }
             }
         }
         // PV: P' = p * vs / aV as this column's fp16 part; k-index 8 gq + e is
@@ -2496,8 +2599,13 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
                                hilo_pair(lg[1][0], scv[1][0].z, lg[1][1], scv[1][1].z, lomask),
                                hilo_pair(lg[1][2], scv[1][2].z, lg[1][3], scv[1][3].z, lomask));
 #pragma unroll
-        for (int v = 0; v < 8; ++v)
+        for (int v = 0; v < kNT; ++v)
             acc[v] = mma(ap, as_h8(bv[v][0], bv[v][1], bv[v][2], bv[v][3]), acc[v]);
+        if constexpr (VLO) {
+#pragma unroll
+            for (int v = 0; v < kNT; ++v)
+                acl[v] = mma(ap, as_h8(bl[v][0], bl[v][1], bl[v][2], bl[v][3]), acl[v]);
+        }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         cur = nxt;
@@ -2518,9 +2626,14 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     }
     lds_barrier();  // every wave is done with the tables mo overwrites
 #pragma unroll
-    for (int v = 0; v < 8; ++v) {
-        mo[w][2 * gq][8 * i + v] = acc[v][0] + acc[v][1];
-        mo[w][2 * gq + 1][8 * i + v] = acc[v][2] + acc[v][3];
+    for (int v = 0; v < kNT; ++v) {
+        float x0 = acc[v][0] + acc[v][1], x1 = acc[v][2] + acc[v][3];
+        if constexpr (VLO) {
+            x0 = fmaf(acl[v][0] + acl[v][1], kLoScale, x0);
+            x1 = fmaf(acl[v][2] + acl[v][3], kLoScale, x1);
+        }
+        mo[w][2 * gq][kNT * i + v] = x0;
+        mo[w][2 * gq + 1][kNT * i + v] = x1;
     }
     lds_barrier();
     const int r = w;  // this wave's row of the group
@@ -2532,16 +2645,18 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
 #pragma unroll
     for (int u = 0; u < kWaves; ++u) {
         const float wt = __builtin_amdgcn_exp2f(mm[u][r] - M);  // (argument <= 0)
-        const float2 ov = *reinterpret_cast<const float2*>(&mo[u][r][2 * lane]);
+        const float2 ov = *reinterpret_cast<const float2*>(&mo[u][r][2 * jl]);
         L += ml[u][r] * wt;
         o0 += ov.x * wt;
         o1 += ov.y * wt;
     }
-    wht_pair<64>(o0, o1, lane);
+    wht_pair<kL>(o0, o1, lane);
     const float s0 = (h & 1) ? -inv : inv;
     const size_t item = (size_t)rg * g.H + h;
     const size_t pid = item * num_splits + split;
-    *reinterpret_cast<float2*>(po + (pid * kRows + r) * 128 + 2 * lane) = make_float2(o0 * s0, o1 * -s0);
+    if (D == 128 || lane < kL)
+        *reinterpret_cast<float2*>(po + (pid * kRows + r) * D + 2 * jl) =
+            make_float2(o0 * s0, o1 * -s0);
     if (lane == 0) pml[(item * kRows + r) * num_splits + split] = make_float2(M, L);
 }
 
@@ -2553,22 +2668,24 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
 // barrier).  The 4 slices of one 128-byte line of the partials run on one
 // XCD (block b on XCD b % 8), so three of them find the line in that XCD's
 // L2.
+template <int D>
 __global__ __launch_bounds__(64) void attn_decode_combine_kernel(
     const float* __restrict__ po, const float2* __restrict__ pml, uint16_t* __restrict__ output,
     int H, int rows, int S) {
     using namespace mfma;
     const int b = blockIdx.x;
     const int xcd = b & 7, m = b >> 3;
+    constexpr int kLines = D / 32;     // 128-byte lines of a partial row
     const int p = (m >> 2) * 8 + xcd;  // (row, line) pair
-    const int row = p >> 2;
+    const int row = p / kLines;
     if (row >= rows) return;
     const int t = threadIdx.x, dd = t & 7, grp = t >> 3;
-    const int d = 32 * (p & 3) + 8 * (m & 3) + dd;
+    const int d = 32 * (p % kLines) + 8 * (m & 3) + dd;
     const int q = row / H, h = row - q * H;
     const int rg = q / kRows, r = q % kRows;
     const size_t item = (size_t)rg * H + h;
     const float2* mlr = pml + (item * kRows + r) * S;
-    const float* orow = po + (item * S * kRows + r) * 128 + d;  // split s: + s * kRows * 128
+    const float* orow = po + (item * S * kRows + r) * D + d;  // split s: + s * kRows * D
     constexpr int kB = 16;
     float M = kInitMax, L = 0.f, A = 0.f;
     for (int base = grp; base < S; base += 8 * kB) {
@@ -2580,7 +2697,7 @@ __global__ __launch_bounds__(64) void attn_decode_combine_kernel(
             const float2 v = mlr[sc];
             pm[k] = s < S ? v.x : kInitMax;
             pl[k] = v.y;
-            pv[k] = orow[(size_t)sc * kRows * 128];
+            pv[k] = orow[(size_t)sc * kRows * D];
         }
         float mb = M;
 #pragma unroll
@@ -2608,7 +2725,7 @@ __global__ __launch_bounds__(64) void attn_decode_combine_kernel(
     merge(lane_xor<8>(M), lane_xor<8>(L), lane_xor<8>(A));
     merge(lane_xor<16>(M), lane_xor<16>(L), lane_xor<16>(A));
     merge(lane_xor<32>(M), lane_xor<32>(L), lane_xor<32>(A));
-    if (t < 8) output[(size_t)row * 128 + d] = f2h(L > 0.f ? A / L : A);
+    if (t < 8) output[(size_t)row * D + d] = f2h(L > 0.f ? A / L : A);
 }
 
 }  // namespace dec
@@ -2644,6 +2761,12 @@ bool mfma_attention_ok(const PageGeom& g, const void* pool) {
     const auto al = [](uint64_t v, uint64_t a) { return (v & (a - 1)) == 0; };
     return g.D == 128 && g.code_stride == 64 && al(g.page_size, 16) && al(g.kc_off, 16) &&
            al(g.vc_off, 4) && al(reinterpret_cast<uintptr_t>(pool), 16);
+}
+// head_dim 64 on the matrix cores: 8-byte K and 2-byte V loads.
+bool mfma_attention64_ok(const PageGeom& g, const void* pool) {
+    const auto al = [](uint64_t v, uint64_t a) { return (v & (a - 1)) == 0; };
+    return g.D == 64 && g.code_stride == 32 && al(g.page_size, 8) && al(g.kc_off, 8) &&
+           al(g.vc_off, 2) && al(reinterpret_cast<uintptr_t>(pool), 8);
 }
 
 }  // namespace
@@ -2709,44 +2832,57 @@ void launch_mfma_attention(const uint16_t* query, const uint8_t* pool, const int
     check_launch(combine_name);
 }
 
-// The slot-mapped decode (turbo_prod, turbo_mse; D = 128): split + combine.
-template <int SCH>
-void launch_decode_attention(const uint16_t* query, const uint8_t* pool, const int32_t* slots,
-                             uint16_t* output, const PageGeom& g, int num_queries,
-                             int num_kv_tokens, float inv, hipStream_t stream,
-                             const char* split_name, const char* combine_name,
-                             const Scratch& scratch) {
+// The slot-mapped decode (turbo_prod, turbo_mse; D = 64, 128): split + combine.
+struct DecodeSplit {
+    int rows, row_groups, heads, splits, tps;
+    long long combine_blocks;
+    size_t blocks, ws_bytes;
+};
+DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens) {
     using namespace mfma;
-    const int rows = num_queries * g.H;
-    const int row_groups = (num_queries + kRows - 1) / kRows;
-    const int heads = g.H * row_groups;
+    DecodeSplit d{};
+    d.rows = num_queries * g.H;
+    d.row_groups = (num_queries + kRows - 1) / kRows;
+    d.heads = g.H * d.row_groups;
     // One 256-token split per workgroup, or longer splits once there are
     // more than ~2 workgroups per CU.
     const int max_splits = std::max(1, (num_kv_tokens + kSplitMinTokens - 1) / kSplitMinTokens);
-    const int want = std::max(1, (kSplitBlocksPerCU * num_cus() + heads - 1) / heads);
-    int splits = std::min(std::min(max_splits, want), 1024);
-    const int tps = num_kv_tokens > 0 ? (num_kv_tokens + splits - 1) / splits : 0;
-    if (tps > 0) splits = (num_kv_tokens + tps - 1) / tps;
-    // The combine: 32 blocks per pair of output rows (8-element slices).
-    const long long combine_blocks = ((long long)rows + 1) / 2 * 32;
-    if (combine_blocks > INT32_MAX) throw Error(std::string(combine_name) + ": too many query rows");
-    const size_t blocks = (size_t)splits * heads;
-    char* ws = static_cast<char*>(scratch.get(stream, blocks * dec::kPartBytes, split_name));
+    const int want = std::max(1, (kSplitBlocksPerCU * num_cus() + d.heads - 1) / d.heads);
+    d.splits = std::min(std::min(max_splits, want), 1024);
+    d.tps = num_kv_tokens > 0 ? (num_kv_tokens + d.splits - 1) / d.splits : 0;
+    if (d.tps > 0) d.splits = (num_kv_tokens + d.tps - 1) / d.tps;
+    // The combine: 32 blocks per 8 (row, 128-byte line) pairs.
+    d.combine_blocks = ((long long)d.rows * (g.D / 32) + 7) / 8 * 32;
+    d.blocks = (size_t)d.splits * d.heads;
+    d.ws_bytes = d.blocks * dec::part_bytes(g.D);
+    return d;
+}
+template <int SCH, int D>
+void launch_decode_attention(const uint16_t* query, const uint8_t* pool, const int32_t* slots,
+                             uint16_t* output, const PageGeom& g, const DecodeSplit& d,
+                             int num_queries, int num_kv_tokens, float inv, hipStream_t stream,
+                             const char* split_name, const char* combine_name,
+                             const Scratch& scratch) {
+    using namespace mfma;
+    if (d.combine_blocks > INT32_MAX)
+        throw Error(std::string(combine_name) + ": too many query rows");
+    char* ws = static_cast<char*>(scratch.get(stream, d.ws_bytes, split_name));
     float* po = reinterpret_cast<float*>(ws);
-    float2* pml = reinterpret_cast<float2*>(ws + blocks * kRows * 128 * sizeof(float));
+    float2* pml = reinterpret_cast<float2*>(ws + d.blocks * kRows * D * sizeof(float));
     if (num_kv_tokens > 0) {
         constexpr int kMaxGridYZ = 65535;
-        const dim3 grid = row_groups <= kMaxGridYZ && g.H <= kMaxGridYZ
-                              ? dim3(splits, g.H, row_groups)
-                              : dim3((unsigned)blocks);
-        hipLaunchKernelGGL((dec::attn_decode_split_kernel<SCH>), grid, dim3(64 * dec::kWaves), 0,
-                           stream, query, pool, slots, po, pml, inv, num_queries, num_kv_tokens,
-                           tps, splits, g);
+        const dim3 grid = d.row_groups <= kMaxGridYZ && g.H <= kMaxGridYZ
+                              ? dim3(d.splits, g.H, d.row_groups)
+                              : dim3((unsigned)d.blocks);
+        hipLaunchKernelGGL((dec::attn_decode_split_kernel<SCH, D>), grid, dim3(64 * dec::kWaves),
+                           0, stream, query, pool, slots, po, pml, inv, num_queries,
+                           num_kv_tokens, d.tps, d.splits, g);
         check_launch(split_name);
     }
     // (no partials for an empty context: the combine writes zeros)
-    hipLaunchKernelGGL(dec::attn_decode_combine_kernel, dim3((unsigned)combine_blocks), dim3(64),
-                       0, stream, po, pml, output, g.H, rows, num_kv_tokens > 0 ? splits : 0);
+    hipLaunchKernelGGL(dec::attn_decode_combine_kernel<D>, dim3((unsigned)d.combine_blocks),
+                       dim3(64), 0, stream, po, pml, output, g.H, d.rows,
+                       num_kv_tokens > 0 ? d.splits : 0);
     check_launch(combine_name);
 }
 
@@ -2796,21 +2932,38 @@ void launch_attention(Scheme s, const uint16_t* query, const uint8_t* pool, cons
     const int rows = num_queries * g.H;
     if (rows <= 0) return;
     const float inv = inv_sqrt_d(g.D);
-    if (mfma_attention_ok(g, pool)) {
-        if (s == Scheme::Prod)
-            launch_decode_attention<mfma::kSchProd>(query, pool, slots, output, g, num_queries,
-                                                    num_kv_tokens, inv, stream,
-                                                    "turbo_prod_fused_attn_split",
-                                                    "turbo_prod_fused_attn_combine", scratch);
-        else
-            launch_decode_attention<mfma::kSchMse>(query, pool, slots, output, g, num_queries,
-                                                   num_kv_tokens, inv, stream,
-                                                   "turbo_mse_fused_attn_split",
-                                                   "turbo_mse_fused_attn_combine", scratch);
-        return;
+    const bool prod = s == Scheme::Prod;
+    const char* split_name = prod ? "turbo_prod_fused_attn_split" : "turbo_mse_fused_attn_split";
+    const char* combine_name =
+        prod ? "turbo_prod_fused_attn_combine" : "turbo_mse_fused_attn_combine";
+    const bool d64 = mfma_attention64_ok(g, pool);
+    if (d64 || mfma_attention_ok(g, pool)) {
+        const DecodeSplit d = decode_split(g, num_queries, num_kv_tokens);
+        // head_dim 64: where a caller's scratch is too small for the padded
+        // row groups' partials, or there are too many rows for the combine's
+        // grid, the generic decode below takes the call if it can.
+        const bool fits = !d64 || ((!scratch.ptr || d.ws_bytes <= scratch.cap) &&
+                                   d.combine_blocks <= INT32_MAX && d.blocks <= INT32_MAX);
+        const auto go = [&](auto sch) {
+            constexpr int kSch = decltype(sch)::value;
+            if (d64)
+                launch_decode_attention<kSch, 64>(query, pool, slots, output, g, d, num_queries,
+                                                  num_kv_tokens, inv, stream, split_name,
+                                                  combine_name, scratch);
+            else
+                launch_decode_attention<kSch, 128>(query, pool, slots, output, g, d, num_queries,
+                                                   num_kv_tokens, inv, stream, split_name,
+                                                   combine_name, scratch);
+        };
+        if (fits) {
+            if (prod)
+                go(std::integral_constant<int, mfma::kSchProd>{});
+            else
+                go(std::integral_constant<int, mfma::kSchMse>{});
+            return;
+        }
     }
     const GenericSplit sp = generic_split(rows, num_kv_tokens, g.D);
-    const bool prod = s == Scheme::Prod;
     float* ws = static_cast<float*>(scratch.get(
         stream, sp.ws_bytes, prod ? "turbo_prod_fused_attn_partial" : "turbo_mse_fused_attn_partial"));
     launch_generic_attention(s, query, pool, SlotTokens{slots, num_kv_tokens}, output, g, rows, sp,

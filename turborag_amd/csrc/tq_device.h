@@ -450,6 +450,11 @@ __device__ __forceinline__ uint16_t ld_u16_nt(const uint8_t* p) {
 __device__ __forceinline__ uint32_t ld_u32_nt(const uint8_t* p) {
     return __builtin_nontemporal_load(reinterpret_cast<const uint32_t*>(p));
 }
+__device__ __forceinline__ uint2 ld_u2_nt(const uint8_t* p) {
+    typedef uint32_t v2u __attribute__((ext_vector_type(2)));
+    const v2u x = __builtin_nontemporal_load(reinterpret_cast<const v2u*>(p));
+    return make_uint2(x[0], x[1]);
+}
 __device__ __forceinline__ uint4 ld_u4_nt(const uint8_t* p) {
     typedef uint32_t v4u __attribute__((ext_vector_type(4)));
     const v4u x = __builtin_nontemporal_load(reinterpret_cast<const v4u*>(p));
