@@ -84,3 +84,33 @@ def test_query_magnitudes(tq, oracle, cuda, scheme, q_scale, k_scale):
         q[0, h] = (1 - 2 * ((d + h) % 2)).float() * q_scale
     _check(tq, oracle, cuda, scheme, q.half(), (k.float() * k_scale).half(), v,
            permuted_slots(N, B, seed=10), permuted_slots(N, B, seed=10))
+
+
+@pytest.mark.parametrize("scheme,H,lens,widths", [
+    ("turbo_prod", 2, [3000, 700, 256, 1, 1500], [8, 3, 5, 1, 2]),  # units of 4, 3, 2 and 1 positions
+    ("turbo_mse", 2, [3000, 700, 256, 1, 1500], [8, 3, 5, 1, 2]),
+    ("turbo_prod", 1, [31, 33, 255], [1, 4, 6]),
+    ("turbo_mse", 8, [2049, 17], [3, 1]),
+])
+def test_paged(tq, oracle, cuda, scheme, H, lens, widths):
+    """The batched paged decode: every row over its causal token range."""
+    from turborag_amd.batched import PagedBatch
+    print(f"[decode64 paged {scheme}] H={H} lens={lens} widths={widths}", flush=True)
+    b = PagedBatch(tq, scheme, lens, widths, kv_heads=H, q_heads=8 * H, head_dim=D, seed=640,
+                   device=cuda)
+    b.append_new_tokens(seed=641)
+    query, row_seq, row_len = b.decode_rows(seed=642)
+    out = torch.full_like(query, 7.0)
+    b.attention(query, row_seq, row_len, b.block_tables(), out)
+    torch.cuda.synchronize()
+    pool, q = b.pool.cpu().numpy(), as_u16(query)
+    f64 = oracle.prod_attention_f64 if scheme == "turbo_prod" else oracle.mse_attention_f64
+    refs, r = [], 0
+    for s, (L, w) in enumerate(zip(lens, widths)):
+        for j in range(w):
+            refs.append(f64(q[r:r + 8].copy(), pool, b.slots_of(s, L + j + 1), B))
+            r += 8
+    u = _row_ulps(out.cpu().numpy(), np.concatenate(refs))
+    print(f"    {u:.2f} row-max ulps", flush=True)
+    b.close()
+    assert u <= 1.0

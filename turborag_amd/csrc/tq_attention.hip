@@ -235,10 +235,11 @@ __global__ __launch_bounds__(256) void prod_logits_kernel(
 }
 
 // ===========================================================================
-// Matrix-core path: D = 128, up to 8 query rows per kv head per workgroup.
+// Matrix-core path: D = 64 and 128, query rows in groups of 8.
 //
-// Per kv head h and row group (8 query rows), a workgroup of 4 waves owns a
-// range of tokens; each wave takes 64-token chunks.
+// Per kv head h and row group (8 query rows; up to four groups in
+// unit::attn_unit_split_kernel), a workgroup of 8 waves owns a range of
+// tokens; each wave takes 32-token chunks.
 //   QK: S^T[token][col] = sum_d K[token][d] * Q^T[d][col] with
 //       v_mfma_f32_16x16x32_f16.  A = K, decoded from nibbles to fp16 through
 //       256-entry LDS tables indexed by code byte; B = the rotated query split
@@ -278,11 +279,9 @@ constexpr int kLoShift = 10;
 constexpr float kLoScale = 1.0f / (float)(1 << kLoShift);
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr int kRows = 8;     // query rows per workgroup (16 MFMA columns, hi/lo)
-// Page schemes of the split kernel: turbo_mse, turbo_prod, and the
-// reference's unexported QJL-1b page (K = +-1 signs times one fp16 scale per
-// (token, head); src/cuda/tq_qjl_kernels.cu).
-constexpr int kSchMse = 0, kSchProd = 1, kSchQjl = 2;
-constexpr int kPartStride = 128 + 4;  // floats per partial row: o[128], m, l, pad (16-B rows)
+// Page schemes of the split kernels.
+constexpr int kSchMse = 0, kSchProd = 1;
+constexpr int kPartStride = 128 + 4;  // QJL: floats per partial row: o[128], m, l, pad (16-B rows)
 
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
     return __builtin_bit_cast(uint32_t, (half2v){(_Float16)a, (_Float16)b});
@@ -734,79 +733,393 @@ __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
 }
 }  // namespace lgt
 
-// CH = tokens per wave iteration (32: two QK tiles, one PV step; 64: four and
-// two); NW = waves per workgroup; NP = row groups per workgroup.
-// NP = 1: the 16 MFMA columns are the group's 8 query rows as fp16 hi and lo
-// parts (columns 2r, 2r + 1), summed after each product.
-// NP = 2 or 4 (paged rows): the new tokens (row groups) of one sequence in a
-// unit share every decoded K/V chunk; each tile of 16 columns is (position,
-// row) = (i / 8, i % 8) of two positions, and the hi and lo parts are stacked
-// along the reduction instead (QK: the same decoded K against the hi and the
-// lo query; PV: the hi and the lo P against the same decoded V), so each
-// lane's column is one query row and its softmax runs once.  A unit of one
-// position uses the one-group column layout in its tile.  PAGED: the grid is
-// one workgroup per work segment of the step's plan (paged_plan_kernel).
-// SCH = page scheme (kSch*).  QJL: the A operand of QK is the +-1 sign
-// matrix, read as fp16 octets from an LDS table indexed by sign byte; the
-// logit is ks * <qrot, signs> (no 1/sqrt(D) beyond the rotation's, :254);
-// the rotation's sign flip has no head term.
-template <int SCH, int CH, int NW, bool PAGED, int NP = 1>
-__global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
+// ---------------------------------------------------------------------------
+// Decode over the reference's unexported QJL-1b pages (src/cuda/
+// tq_qjl_kernels.cu), D = 128: 8 waves of 32-token chunks per (split, kv head,
+// row group) workgroup; the 16 MFMA columns are the group's 8 query rows as
+// fp16 hi and lo parts (columns 2r, 2r + 1), summed after each product.  The A
+// operand of QK is the +-1 sign matrix, read as fp16 octets from an LDS table
+// indexed by sign byte; the logit is ks * <qrot, signs> (no 1/sqrt(D) beyond
+// the rotation's, :254); the rotation's sign flip has no head term.
+// ---------------------------------------------------------------------------
+namespace qjl {
+using namespace mfma;
+constexpr int kWaves = 8, kChunk = 32, kPass = kWaves * kChunk;
+
+__global__ __launch_bounds__(64 * kWaves) void attn_qjl_split_kernel(
     const uint16_t* __restrict__ query, const uint8_t* __restrict__ pool,
     const int32_t* __restrict__ slots, float* __restrict__ ws, float inv, int num_queries,
-    int num_kv_tokens, int tokens_per_split, int num_splits, PageGeom g, mfma::PagedRows pr) {
-    using namespace mfma;
-    constexpr int kChunk = CH, kWaves = NW;
-    constexpr int kTiles = CH / 16, kSteps = CH / 32;
-    static_assert(CH == 32 || CH == 64, "chunk of 32 or 64 tokens");
-    static_assert(NW == 4 || NW == 8, "4 or 8 waves");
-    static_assert(NP == 1 || ((NP == 2 || NP == 4) && PAGED), "2 or 4 positions: paged rows");
-    constexpr bool PROD = SCH == kSchProd, QJL = SCH == kSchQjl;
-    static_assert(!QJL || (!PAGED && NP == 1), "QJL: slot-mapped rows, one position");
-    constexpr int kR = kRows * NP;  // query rows of the workgroup
-    // NP >= 2: NT tiles of 16 MFMA columns, (position 2t + i / 8, row i % 8)
-    constexpr int NT = NP >= 2 ? NP / 2 : 1;
-    constexpr int kMoRows = NP >= 2 ? 16 : kR;  // rows merged per pass (one tile)
-    // Decode tables indexed by a code byte (low nibble = even d), fp16 pairs,
-    // 32 copies each: copy c of entry e at byte 256e + 4c of its table and lane
-    // l reads copy l % 32, so a half-wave's 32 random lookups hit 32 distinct
-    // banks.
-    //  - NP = 1 (the QJL-1b decode; the layout the one-group loop reads for
-    //    any scheme): one region of K|V rows, table 0 in bytes 0..127 of each
-    //    row (QJL: the sign octets; prod: aK*K3; mse: the lo parts of aV*V4)
-    //    and table 1 = V (aV*V4) in bytes 128..255.
-    //  - NP >= 2 (turbo_prod, turbo_mse): the layout of decode_table_words,
-    //    S rows at byte 0 and K|V rows at byte kOffKV.  One address then reads
-    //    a code byte's S pair (offset 0) and its K pair (offset kOffKV, which
-    //    no two-address LDS read merges with 0), each straight into its MFMA
-    //    operand, and a V lookup's address is that of the byte's S row + 128
-    //    (turbo_prod's V copies; turbo_mse reads its K copies, + 0).
-    // After the token loop the tables' space holds the per-wave results for
-    // the merge (NP = 1: the K|V rows; NP >= 2: one tile in each half).
-    constexpr bool STAB = NP >= 2;
-    constexpr int kOffKV = STAB ? 65520 : 0;
-    constexpr int kTabWords = STAB ? 32768 : 256 * 64;
-    __shared__ __attribute__((aligned(256))) uint32_t lut[kTabWords];
-    __shared__ float qs_sep[STAB ? 1 : kR][128];  // NP = 1: the rotated queries
-    __shared__ uint4 bqs[NP][4][64];  // QK B operand (fp16 hi/lo q) of k-step s for lane l
+    int num_kv_tokens, int tokens_per_split, int num_splits, PageGeom g) {
+    // One region of 256-byte rows per code byte: in bytes 0..127 of row e the 8
+    // copies of the fp16 sign octet of sign byte e, in 128..255 the 32 copies of
+    // V's fp16 pair aV*V4 (low nibble = even d); lane l reads copy l % 8 or
+    // l % 32.  After the token loop the space holds the waves' results.
+    __shared__ __attribute__((aligned(256))) uint32_t lut[256 * 64];
+    __shared__ float qs[kRows][128];  // the rotated queries
+    __shared__ uint4 bqs[4][64];      // QK B operand (fp16 hi/lo q) of k-step s for lane l
     __shared__ uint64_t tko[kWaves][kChunk], tvo[kWaves][kChunk];
-    __shared__ float4 tsc[kWaves][kChunk];  // per token: K scale a, residual scale b, vs, bias
+    __shared__ float4 tsc[kWaves][kChunk];  // per token: (unused), K scale, vs, bias
+    __shared__ float mm[kWaves][kRows], ml[kWaves][kRows];
+    __shared__ uint32_t vstage[256];  // the staged V entries
+    static_assert(sizeof(float) * kWaves * kRows * 128 <= sizeof(lut), "merge space");
+    float(*mo)[kRows][128] = reinterpret_cast<float(*)[kRows][128]>(&lut[0]);
+
+    // Grid (split, kv head, row group), or one dimension of splits x heads when
+    // there are more row groups than a grid dimension holds (the first form
+    // needs no divisions before the first loads).
+    int split, h, rg;
+    if (gridDim.x == (unsigned)num_splits) {
+        split = blockIdx.x;
+        h = blockIdx.y;
+        rg = blockIdx.z;
+    } else {
+        split = blockIdx.x % num_splits;
+        const int hr = blockIdx.x / num_splits;
+        h = hr % g.H;
+        rg = hr / g.H;
+    }
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar)
+    const int i = lane & 15, gq = lane >> 4;
+    const int t_begin = split * tokens_per_split;
+    const int t_end = min(num_kv_tokens, t_begin + tokens_per_split);
+    const size_t pid = ((size_t)rg * g.H + h) * num_splits + split;
+    // This wave's query row, loaded before anything waits.
+    const int qi = min(rg * kRows + w, num_queries - 1);
+    const uint32_t qraw =
+        *reinterpret_cast<const uint32_t*>(query + ((size_t)qi * g.H + h) * 128 + 2 * lane);
+
+    // A chunk's codes and per-token scales, loaded ahead of its compute.
+    struct Chunk {
+        uint32_t kw[2];  // K: tile tau, token 16*tau + i, sign bytes 4gq .. 4gq + 3 (k-steps 0 .. 3)
+        uint32_t vw[8];  // V: k-index 8gq + e (token below), dword i
+        uint16_t ks, vs;  // this lane's token's fp16 scales (raw: still in flight)
+        bool valid;
+    };
+    // Slot of this lane's token in the chunk at t0 (lanes past the range re-read
+    // the last token of the range).
+    auto load_slot = [&](int t0) -> int {
+        return slots[max(min(t0 + (lane & (kChunk - 1)), t_end - 1), 0)];
+    };
+    // slot -> cell offsets (exchanged through LDS) -> scale and code loads,
+    // issued for every lane.  Tokens past the range or with a negative slot read
+    // the first bytes of the query instead (always valid memory: the offset of
+    // the query from the pool) and get bias -inf.  The loads stay in flight
+    // until the chunk is computed.  Each pool byte is read once per row group:
+    // non-temporal loads keep the L2 for the slots and queries.
+    const uint64_t dummy_off =
+        (uint64_t)(reinterpret_cast<uintptr_t>(query) - reinterpret_cast<uintptr_t>(pool));
+    auto fetch = [&](int t0, int slot, Chunk& c) {
+        c.valid = t0 + (lane & (kChunk - 1)) < t_end && slot >= 0;
+        int page, tib;
+        split_slot(c.valid ? slot : 0, g, page, tib);
+        const uint64_t cell = (uint64_t)(tib * g.H + h);
+        const uint64_t pb = (uint64_t)page * g.page_size;
+        // Byte offsets from pool (integer selects: no branches around loads).
+        const uint64_t so = pb + cell * g.scale_stride;
+        c.ks = ld_u16_nt(pool + (c.valid ? so + g.ks_off : dummy_off));
+        c.vs = ld_u16_nt(pool + (c.valid ? so + g.vs_off : dummy_off + 2));
+        // (lanes l and l + 32 hold the same token; K rows are 16 sign bytes)
+        tko[w][lane & (kChunk - 1)] = c.valid ? pb + g.kc_off + cell * 16u : dummy_off;
+        tvo[w][lane & (kChunk - 1)] = c.valid ? pb + g.vc_off + cell * g.code_stride : dummy_off;
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll
+        for (int tau = 0; tau < 2; ++tau)
+            c.kw[tau] = ld_u32_nt(pool + (tko[w][16 * tau + i] + 4 * gq));
+        // (the K words first: the QK waits for them while the V words may still
+        // be in flight)
+        __builtin_amdgcn_sched_barrier(0);
+        // k-index 8gq + e is token 4gq + e (e < 4) or 16 + 4gq + (e - 4).
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            const int tok = e < 4 ? 4 * gq + e : 16 + 4 * gq + (e - 4);
+            c.vw[e] = ld_u32_nt(pool + (tvo[w][tok] + 4 * i));
+        }
+    };
+
+    // Issue order matters (the vector-memory counter is in order): the query row
+    // (above), then the first chunk's slots; the tables are built while they are
+    // in flight.
+    int t0 = t_begin + w * kChunk;
+    const int slot0 = load_slot(t0);
+    if (w < 4)  // V's entries staged one per thread, replicated after the first barrier
+        vstage[tid] = pack_h2(kAlphaV * pick(kV4, tid & 15), kAlphaV * pick(kV4, tid >> 4));
+    float q0 = h2f(qraw & 0xffff), q1 = -h2f(qraw >> 16);
+    Chunk cur;
+    fetch(t0, slot0, cur);  // in flight during the setup below (empty waves: all invalid)
+    {  // this wave's rotated query row: qrot = WHT(q * s) * inv
+        wht_pair<64>(q0, q1, lane);
+        const bool live = rg * kRows + w < num_queries;
+        qs[w][2 * lane] = live ? q0 * inv : 0.0f;
+        qs[w][2 * lane + 1] = live ? q1 * inv : 0.0f;
+    }
+    lds_barrier();  // staged entries and rotated queries visible
+    // Every wave writes its rows of both tables with conflict-free 1 KB stores.
+#pragma unroll
+    for (int k = 0; k < 256 / kWaves; k += 4) {
+        const int e = w * (256 / kWaves) + k + (lane >> 4);
+        uint4 v4;
+        if (lane & 8) {
+            const uint32_t v = vstage[e];
+            v4 = make_uint4(v, v, v, v);
+        } else {
+            uint32_t wd[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                wd[q] = ((e >> (2 * q)) & 1 ? 0x3C00u : 0xBC00u) |
+                        ((e >> (2 * q + 1)) & 1 ? 0x3C000000u : 0xBC000000u);
+            v4 = make_uint4(wd[0], wd[1], wd[2], wd[3]);
+        }
+        *reinterpret_cast<uint4*>(&lut[64 * e + 4 * (lane & 15)]) = v4;
+    }
+    // B operand of QK: column i = row i/2, hi (i even) or lo (i odd) part; k-index
+    // 8*gq + e of step s is d = 32*gq + 8*s + e.
+    const bool lo_col = (i & 1) != 0;
+    if (w < 4) {
+        half8 b;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) b[e] = hi_lo(qs[i >> 1][32 * gq + 8 * w + e], lo_col);
+        bqs[w][lane] = __builtin_bit_cast(uint4, b);
+    }
+    lds_barrier();
+    half8 bq[4];
+#pragma unroll
+    for (int s = 0; s < 4; ++s) bq[s] = __builtin_bit_cast(half8, bqs[s][lane]);
+    // A lookup puts the code byte into byte 1 of its table's address (entry
+    // stride 256 B) with one v_perm; byte 1 of the base is re-added.
+    const uint32_t lutv = (uint32_t)reinterpret_cast<uintptr_t>((lds_u32*)&lut[32 + (lane & 31)]);
+    const uint32_t lutq = (uint32_t)reinterpret_cast<uintptr_t>((lds_u32*)&lut[4 * (lane & 7)]);
+    auto at = [](uint32_t word, int b, uint32_t base) -> uint32_t {
+        return __builtin_amdgcn_perm(word, base, 0x03020000u | ((4u + b) << 8)) + (base & 0xFF00u);
+    };
+    typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
+
+    float m_run = kInitMax, l_run = 0.0f;
+    f32x4 acc[8];
+#pragma unroll
+    for (int v = 0; v < 8; ++v) acc[v] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    bool first = true;
+    int slot_nx = load_slot(t0 + kPass);
+    while (t0 < t_end) {  // wave-uniform
+        {
+            const float ks = h2f(cur.ks), vs = h2f(cur.vs);
+            tsc[w][lane & (kChunk - 1)] = cur.valid ? make_float4(0.0f, ks * kLog2e, vs, 0.0f)
+                                                    : make_float4(0.f, 0.f, 0.f, -INFINITY);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        Chunk nxt;
+        const int t1 = t0 + kPass;
+        if (t1 < t_end) {  // codes of the next chunk, slots of the one after
+            fetch(t1, slot_nx, nxt);
+            slot_nx = load_slot(t1 + kPass);
+        }
+        // The scale rows of this lane's tokens, read before any lookup (LDS reads
+        // complete in order: a read issued after the V lookups would wait for
+        // all of them).
+        float4 scv[2][4];
+#pragma unroll
+        for (int tau = 0; tau < 2; ++tau)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) scv[tau][e] = tsc[w][16 * tau + 4 * gq + e];
+        // QK: every lookup of the chunk's sign octets before the first MFMA.
+        half8 ka[2][4];
+#pragma unroll
+        for (int tau = 0; tau < 2; ++tau)
+#pragma unroll
+            for (int s = 0; s < 4; ++s)
+                ka[tau][s] = __builtin_bit_cast(
+                    half8, *reinterpret_cast<const lds_u32x4*>(at(cur.kw[tau], s, lutq)));
+        __builtin_amdgcn_sched_barrier(0);
+        f32x4 cs[2];
+#pragma unroll
+        for (int tau = 0; tau < 2; ++tau) {
+            cs[tau] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int s = 0; s < 4; ++s) cs[tau] = mma(ka[tau][s], bq[s], cs[tau]);
+        }
+        // The V lookups (B operands of PV) go out now: the softmax below runs
+        // while they are in flight.
+        uint32_t bv[8][4];  // [N-tile v = d - 8i][token pair]
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t we = cur.vw[2 * q], wo = cur.vw[2 * q + 1];
+            const uint32_t lob = (we & 0x0F0F0F0Fu) | ((wo & 0x0F0F0F0Fu) << 4);
+            const uint32_t hib = ((we >> 4) & 0x0F0F0F0Fu) | (wo & 0xF0F0F0F0u);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                bv[2 * b][q] = *reinterpret_cast<const lds_u32*>(at(lob, b, lutv));
+                bv[2 * b + 1][q] = *reinterpret_cast<const lds_u32*>(at(hib, b, lutv));
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        // Logits (base 2) of tokens 16*tau + 4*gq + e; hi + lo columns summed.
+        float lg[2][4];
+        float mloc = -INFINITY;
+#pragma unroll
+        for (int tau = 0; tau < 2; ++tau)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float4 sc = scv[tau][e];
+                lg[tau][e] = fmaf(cs[tau][e] + quad_xor<1>(cs[tau][e]), sc.y, sc.w);
+                mloc = fmaxf(mloc, lg[tau][e]);
+            }
+        mloc = lane_xor_reduce<16>(mloc, [](float x, float y) { return fmaxf(x, y); });
+        mloc = lane_xor_reduce<32>(mloc, [](float x, float y) { return fmaxf(x, y); });
+        // v_exp_f32 without denormal handling: arguments are <= 0 and a weight
+        // below 2^-126 of the running maximum is negligible.
+        const float m_new = fmaxf(m_run, mloc);
+        const float alpha = first ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
+        m_run = m_new;
+        float lsum = 0.0f;
+#pragma unroll
+        for (int tau = 0; tau < 2; ++tau)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                lg[tau][e] = __builtin_amdgcn_exp2f(lg[tau][e] - m_new);
+                lsum += lg[tau][e];
+            }
+        l_run = l_run * alpha + lsum;
+        if (!first && __any(alpha != 1.0f)) {
+            // acc lane (d, gq) holds columns 4gq..4gq+3 = rows 2gq, 2gq+1.
+            const float a0 = __shfl(alpha, 4 * gq), a1 = __shfl(alpha, 4 * gq + 2);
+#pragma unroll
+            for (int v = 0; v < 8; ++v) {
+                acc[v][0] *= a0;
+                acc[v][1] *= a0;
+                acc[v][2] *= a1;
+                acc[v][3] *= a1;
+            }
+        }
+        half8 ap;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) ap[e] = hi_lo(lg[e >> 2][e & 3] * scv[e >> 2][e & 3].z, lo_col);
+#pragma unroll
+        for (int v = 0; v < 8; ++v)
+            acc[v] = mma(ap, as_h8(bv[v][0], bv[v][1], bv[v][2], bv[v][3]), acc[v]);
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        cur = nxt;
+        t0 = t1;
+        first = false;
+    }
+
+    // Wave results: l summed over the g lanes of each column; o rows from the hi
+    // + lo columns, the V codebook scale divided out.  Then the waves are merged
+    // per row, the inverse WHT and sign flip applied, and the partial written.
+    {
+        float l_tot = lane_xor_reduce<16>(l_run, [](float x, float y) { return x + y; });
+        l_tot = lane_xor_reduce<32>(l_tot, [](float x, float y) { return x + y; });
+        if (gq == 0 && !lo_col) {
+            mm[w][i >> 1] = m_run;
+            ml[w][i >> 1] = l_tot;
+        }
+    }
+    const float iav = 1.0f / kAlphaV;
+    __syncthreads();  // every wave is done with the tables mo overwrites
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+        mo[w][2 * gq][8 * i + v] = (acc[v][0] + acc[v][1]) * iav;
+        mo[w][2 * gq + 1][8 * i + v] = (acc[v][2] + acc[v][3]) * iav;
+    }
+    __syncthreads();
+    const int r = w;  // this wave's row of the group
+    float M = mm[0][r];
+#pragma unroll
+    for (int u = 1; u < kWaves; ++u) M = fmaxf(M, mm[u][r]);
+    float L = 0.f, o0 = 0.f, o1 = 0.f;
+#pragma unroll
+    for (int u = 0; u < kWaves; ++u) {
+        const float wt = __builtin_amdgcn_exp2f(mm[u][r] - M);  // (argument <= 0)
+        L += ml[u][r] * wt;
+        o0 += mo[u][r][2 * lane] * wt;
+        o1 += mo[u][r][2 * lane + 1] * wt;
+    }
+    wht_pair<64>(o0, o1, lane);
+    float* part = ws + (pid * kRows + r) * kPartStride;
+    part[2 * lane] = o0 * inv;
+    part[2 * lane + 1] = o1 * -inv;
+    if (lane == 0) {
+        part[128] = M;
+        part[129] = L;
+    }
+}
+}  // namespace qjl
+
+// ---------------------------------------------------------------------------
+// Decode of units of up to four row groups (kNP positions of 8 query rows)
+// that share every decoded K/V chunk: the new tokens of one paged sequence
+// (PAGED), or consecutive row groups over one slot map (many query rows, a
+// question's tokens over a cached document).
+// Each tile of 16 MFMA columns is (position, row) = (i / 8, i % 8) of two
+// positions, and the fp16 hi and lo parts of the query and of P are stacked
+// along the reductions (QK: the same decoded K against the hi and the lo
+// query; PV: the hi and the lo P against the same decoded V), so each lane's
+// column is one query row and its softmax runs once.  A unit of one position
+// holds its rows' hi parts in columns 0-7 and lo parts in 8-15 instead: half
+// the MFMAs.
+// Eight waves of 32-token chunks per workgroup, one workgroup per CU (the
+// decode tables).  PAGED: the grid is one workgroup per work segment of the
+// step's plan (paged_plan_kernel).  Slot-mapped: grid (split, kv head, unit).
+// D = 64: half the k-steps and PV tiles per token, V's fp16 lo parts and a
+// power of two per query row, as dec::attn_decode_split_kernel.
+// Issue-bound at many passes per workgroup (D = 128, 32 sequences of 1K-32K
+// tokens: 94 us), bound by the setup and the merge at few.  A D = 64 step of
+// 8 sequences (500-4,000 tokens, 2 new tokens, 2 heads) with its append takes
+// 26.8 us, against 212.6 on the generic kernels it ran on before.
+// ---------------------------------------------------------------------------
+namespace unit {
+using namespace mfma;
+constexpr int kNP = 4;                // positions (row groups) per unit
+constexpr int kNT = kNP / 2;          // tiles of 16 MFMA columns
+constexpr int kWaves = 8, kChunk = 32, kPass = kWaves * kChunk;
+constexpr int kTiles = kChunk / 16;   // QK tiles of a chunk
+constexpr int kR = kRows * kNP;       // query rows of the workgroup
+constexpr int kMoRows = 16;           // rows merged per tile
+// Decode tables in the layout of decode_table_words: S rows at byte 0 and K|V
+// rows at byte kOffKV.  One address reads a code byte's S pair (offset 0) and
+// its K pair (offset kOffKV, which no two-address LDS read merges with 0),
+// each straight into its MFMA operand; a V lookup's address is that of the
+// byte's S row + 128 (turbo_prod's V copies; turbo_mse reads its K copies,
+// + 0).  turbo_prod's V lo parts (D = 64) are copies of the S rows' upper
+// halves, kLoCopies of them.  After the token loop the space holds the waves'
+// results for the merge, one tile in each half.
+constexpr int kOffKV = 65520;
+constexpr int kTabWords = 32768;
+constexpr int kLoCopies = 28;
+static_assert(kOffKV + 256 * 256 <= 4 * kTabWords, "K|V rows");
+static_assert(256 * 255 + 128 + 4 * kLoCopies <= kOffKV, "the V lo rows end below the K table");
+static_assert(kRows % kWaves == 0 && kWaves == 8, "eight waves, one row per wave and position");
+constexpr int part_stride(int D) { return D + 4; }  // paged partial row: o[D], m, l, pad
+
+template <int SCH, int D, bool PAGED>
+__global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
+    const uint16_t* __restrict__ query, const uint8_t* __restrict__ pool,
+    const int32_t* __restrict__ slots, float* __restrict__ ws, float2* __restrict__ pml, float inv,
+    int num_queries, int num_kv_tokens, int tokens_per_split, int num_splits, PageGeom g,
+    PagedRows pr) {
+    constexpr bool PROD = SCH == kSchProd;
+    static_assert(SCH == kSchProd || SCH == kSchMse, "turbo_prod or turbo_mse pages");
+    static_assert(D == 128 || D == 64, "head_dim 64 or 128");
+    constexpr int kS = D / 32;   // QK k-steps; lane group gq holds dims [D/4 gq, D/4 gq + D/4)
+    constexpr int kND = D / 16;  // PV tiles: lane i holds dims kND i .. + kND - 1
+    constexpr int kL = D / 2;    // lanes of a row held two values per lane
+    constexpr bool VLO = D == 64, QSCALE = D == 64;
+    static_assert(kNT * sizeof(float) * kWaves * kMoRows * D <= 4 * kTabWords, "merge spaces");
+    __shared__ __attribute__((aligned(256))) uint32_t lut[kTabWords];
+    __shared__ uint4 bqs[kNP][kS][64];  // QK B operand (fp16 hi/lo q) of k-step s for lane l
+    __shared__ uint64_t tko[kWaves][kChunk], tvo[kWaves][kChunk];
+    __shared__ float4 tsc[kWaves][kChunk];  // per token: K scale a, residual scale b, vs / 2, bias
     __shared__ float mm[kWaves][kR], ml[kWaves][kR];
-    __shared__ uint32_t kstage[256], vstage[256];  // NP = 1: the staged table entries
-    static_assert(kOffKV + 256 * 256 <= (int)sizeof(lut), "K|V rows");
-    static_assert(kOffKV + sizeof(float) * kWaves * kMoRows * 128 <= sizeof(lut), "merge space");
-    float(*mo)[kMoRows][128] = reinterpret_cast<float(*)[kMoRows][128]>(&lut[kOffKV / 4]);
-    // K|V row e (its 64 words: 32 K copies, then 32 V copies)
-    auto kv_row = [&](int e) -> uint32_t* { return &lut[kOffKV / 4 + 64 * e]; };
-    // Rotated query element (r, d) (NP = 1; NP >= 2 writes the B operands
-    // directly)
-    auto qs_at = [&](int r, int d) -> float& { return qs_sep[STAB ? 0 : r][d]; };
+    __shared__ float rsc[QSCALE ? kR : 1];  // the rows' power of two
 
     // logit scale per unit ks (log2(e) / alpha folded at compile time: no run-time division)
     const float ck = inv * (PROD ? kLog2e / kAlphaK : kLog2e / kAlphaV);
     const float cr = inv * kLog2e;                                 // residual: ks * re
     // One work item: kv head h, row groups rg .. rg + npos - 1, tokens
-    // [t_begin, t_cap) (paged: and below each row's length), partial slot pid.
+    // [t_begin, t_cap) (paged: and below each row's length), partial slot pid
+    // (slot-mapped: split pid).
     // (tid is a parameter so that a caller looping over items can keep the
     // per-thread values derived from it from being hoisted out of the loop
     // and held across the token loop.)
@@ -815,29 +1128,25 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
         const int lane = tid & 63;
         const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar)
         const int i = lane & 15, gq = lane >> 4;
-        // Paged rows: the group's sequence and per-row kv lengths (causal limit);
-        // rowlen is that of this lane's MFMA column row.  A piece past every row's
-        // length has no partial (the combine does not read it).
+        const int jl = lane & (kL - 1);  // this lane's pair of a row (D = 64: lanes l, l + 32 alike)
+        // Paged rows: the unit's sequence and per-row kv lengths (causal limit).
+        // A piece past every row's length has no partial (the combine does not
+        // read it).  Per position: the group's longest row; per tile: this
+        // lane's column row length; the shortest live row.
         int kv_end = num_kv_tokens, seq = 0;
-        // per position: this lane's column row length, the group's longest and
-        // shortest row
-        int rowlen[NP] = {}, gend[NP] = {}, gmin[NP] = {};
-        // NP >= 2: this lane's column row length per tile and the shortest live row
-        int rl_col[NT] = {}, gmin_live = 0x7fffffff;
+        int gend[kNP] = {}, rl_col[kNT] = {}, gmin_live = 0x7fffffff;
         // This wave's query rows (row r of the workgroup is row r % 8 of group
         // rg + r / 8: rows rg * 8 + r), loaded before anything waits: paged rows
         // issue them right after the row lengths and the sequence, so the
         // length processing waits only for those (the vector-memory counter is
         // in order) while the queries are in flight.
-        constexpr int kQPerWave = kR / kWaves;
-        static_assert(kR % kWaves == 0, "rows per wave");
-        uint32_t qraw[kQPerWave];
+        uint32_t qraw[kNP];
         auto load_queries = [&]() {
 #pragma unroll
-            for (int k = 0; k < kQPerWave; ++k) {
+            for (int k = 0; k < kNP; ++k) {
                 const int qi = min(rg * kRows + w + k * kWaves, num_queries - 1);
-                qraw[k] = *reinterpret_cast<const uint32_t*>(query + ((size_t)qi * g.H + h) * 128 +
-                                                              2 * lane);
+                qraw[k] = *reinterpret_cast<const uint32_t*>(query + ((size_t)qi * g.H + h) * D +
+                                                              2 * jl);
             }
         };
         if constexpr (!PAGED) load_queries();
@@ -846,30 +1155,29 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
             // Every row length and the sequence are loaded unconditionally (rows
             // past the end re-read the last row), so the loads go out together:
             // a load under a condition sits in a branch whose join waits for it.
-            int lraw[NP];
+            int lraw[kNP];
 #pragma unroll
-            for (int p = 0; p < NP; ++p)
+            for (int p = 0; p < kNP; ++p)
                 lraw[p] = pr.row_kv_len[min((rg + p) * kRows + (lane & 7), num_queries - 1)];
             const int seq_raw = pr.row_seq[rg * kRows];
             load_queries();
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int p = 0; p < NP; ++p) {
+            for (int p = 0; p < kNP; ++p) {
                 const int rr = (rg + p) * kRows + (lane & 7);
                 const int lv = p < npos && rr < num_queries ? lraw[p] : 0;
-                rowlen[p] = __shfl(lv, i >> 1);
                 const int lc = __shfl(lv, i & 7);
                 // (one position: both halves of the tile hold its rows, hi and lo)
-                if (NP >= 2 && (npos == 1 ? p == 0 : (i >> 3) == (p & 1))) rl_col[p >> 1] = lc;
+                if (npos == 1 ? p == 0 : (i >> 3) == (p & 1)) rl_col[p >> 1] = lc;
                 int m = max(lv, __shfl_xor(lv, 1)), n = min(lv, __shfl_xor(lv, 1));
                 m = max(m, __shfl_xor(m, 2));
                 n = min(n, __shfl_xor(n, 2));
                 m = max(m, __shfl_xor(m, 4));
                 n = min(n, __shfl_xor(n, 4));
                 gend[p] = __builtin_amdgcn_readfirstlane(m);
-                gmin[p] = __builtin_amdgcn_readfirstlane(n);
+                const int gmin = __builtin_amdgcn_readfirstlane(n);
                 kv_end = max(kv_end, gend[p]);
-                if (p < npos) gmin_live = min(gmin_live, gmin[p]);
+                if (p < npos) gmin_live = min(gmin_live, gmin);
             }
             seq = __builtin_amdgcn_readfirstlane(seq_raw);
             // (a piece always starts below its unit's kv end: the walk calls
@@ -877,12 +1185,12 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
             // past every row would run no chunk and write no partial)
         }
         const int t_end = min(kv_end, t_cap);
-        const int ntile = (npos + 1) >> 1;  // NP >= 2: tiles of 16 columns in use
+        const int ntile = (npos + 1) >> 1;  // tiles of 16 columns in use
 
         // A chunk's codes and per-token scales, loaded ahead of its compute.
         struct Chunk {
-            uint4 kw[kTiles];        // K: tile tau, token 16*tau + i, bytes [16gq, 16gq + 16)
-            uint32_t vw[kSteps][8];  // V: step p, k-index 8gq + e (token below), dword i
+            uint32_t kw[kTiles][kS];  // K: tile tau, token 16*tau + i, bytes [4 kS gq, 4 kS gq + 4 kS)
+            uint32_t vw[8];       // V: k-index 8gq + e (token below), bytes [D/32 i, D/32 i + D/32)
             uint16_t ks, re, vs;  // this lane's token's fp16 scales (raw: still in flight)
             bool valid;
         };
@@ -892,7 +1200,7 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
         // work runs in between; arithmetic on the loaded value here would make
         // the in-order vector-memory counter wait, right after the next chunk's
         // code loads are issued, for all of them (129-130 -> 125-127.5 us per
-        // config-5 step).
+        // 32-sequence step).
         auto chunk_token = [&](int t0) -> int {
             return max(min(t0 + (lane & (kChunk - 1)), t_end - 1), 0);
         };
@@ -905,43 +1213,26 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                 return slots[t];
             }
         };
-        // slot -> cell offsets (exchanged through LDS) -> scale and code loads,
-        // issued for every lane.  Slot-mapped rows: tokens past the range or
-        // with a negative slot read the first bytes of the query instead (always
-        // valid memory: the offset of the query from the pool) and get bias
-        // -inf.  The loads stay in flight until the chunk is computed.
-        const uint64_t dummy_off =
-            (uint64_t)(reinterpret_cast<uintptr_t>(query) - reinterpret_cast<uintptr_t>(pool));
-        // Slot-mapped rows read each pool byte once: non-temporal loads keep
-        // the L2 for the slots and queries (10.3 -> 10.0 us per 32K layer).
-        // Paged rows keep plain loads: the workgroups of the two kv heads of
-        // a work segment read each 128-byte code line together, one through
-        // the other's L2 copy.
+        // Token -> cell addresses (exchanged through LDS) -> scale and code
+        // loads, issued for every lane; they stay in flight until the chunk is
+        // computed.  Plain loads (not non-temporal): the workgroups of the two
+        // kv heads of a work segment read each 128-byte code line together, one
+        // through the other's L2 copy, and the units over one slot map read the
+        // same cells.
         typedef __attribute__((address_space(1))) const uint8_t gbyte;
+        typedef __attribute__((address_space(1))) const uint16_t ghalf;
         typedef __attribute__((address_space(1))) const uint32_t gword;
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        typedef __attribute__((address_space(1))) const u32x2 gpair;
         typedef __attribute__((address_space(1))) const u32x4 gquad;
-        auto ld16 = [](const uint8_t* p) -> uint16_t { return PAGED ? ld_u16(p) : ld_u16_nt(p); };
-        auto ld32 = [](gbyte* p) -> uint32_t {
-            if constexpr (PAGED) return *reinterpret_cast<gword*>(p);
-            return ld_u32_nt((const uint8_t*)p);
-        };
-        auto ld128 = [](gbyte* p) -> uint4 {
-            if constexpr (PAGED) return __builtin_bit_cast(uint4, *reinterpret_cast<gquad*>(p));
-            return ld_u4_nt((const uint8_t*)p);
-        };
-        // The code rows' addresses go through LDS: paged rows as global
-        // addresses, slot-mapped rows as offsets from pool.
-        auto code_row = [&](uint64_t v) -> gbyte* {
-            return PAGED ? reinterpret_cast<gbyte*>(v) : (gbyte*)(pool + v);
-        };
         auto fetch = [&](int t0, int loaded, Chunk& c) {
+            c.valid = t0 + (lane & (kChunk - 1)) < t_end && loaded >= 0;
             if constexpr (PAGED) {
                 // loaded: the token's page table entry.  A cell's bytes are its
                 // page's address plus 32-bit offsets within the page (integer
                 // selects: no branches around loads).  Masked lanes (past the
                 // range, or an unmapped page) address the workspace's spare page
                 // instead: always valid memory, its bytes unused (bias -inf).
-                c.valid = t0 + (lane & (kChunk - 1)) < t_end && loaded >= 0;
                 const int t = chunk_token(t0);
                 const int tib = g.bs_shift >= 0 ? t & (g.block_size - 1) : t % g.block_size;
                 const uint32_t cell = (uint32_t)(tib * g.H + h);
@@ -949,56 +1240,57 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                     c.valid ? pool + (uint64_t)(uint32_t)loaded * (uint32_t)g.page_size
                             : pr.spare_page;
                 const uint32_t so = cell * (uint32_t)g.scale_stride;
-                c.ks = ld16(pg + (so + (uint32_t)g.ks_off));
-                c.vs = ld16(pg + (so + (uint32_t)g.vs_off));
-                c.re = PROD ? ld16(pg + (so + (uint32_t)g.kres_off)) : (uint16_t)0;
+                c.ks = ld_u16(pg + (so + (uint32_t)g.ks_off));
+                c.vs = ld_u16(pg + (so + (uint32_t)g.vs_off));
+                c.re = PROD ? ld_u16(pg + (so + (uint32_t)g.kres_off)) : (uint16_t)0;
                 const uint32_t co = cell * (uint32_t)g.code_stride;
                 tko[w][lane & (kChunk - 1)] = reinterpret_cast<uint64_t>(pg + (co + (uint32_t)g.kc_off));
                 tvo[w][lane & (kChunk - 1)] = reinterpret_cast<uint64_t>(pg + (co + (uint32_t)g.vc_off));
             } else {
-                const int slot = loaded;
-                c.valid = t0 + (lane & (kChunk - 1)) < t_end && slot >= 0;
+                // loaded: the token's slot.  Masked lanes (past the range, or a
+                // negative slot) read the first bytes of the query instead.
                 int page, tib;
-                split_slot(c.valid ? slot : 0, g, page, tib);
+                split_slot(c.valid ? loaded : 0, g, page, tib);
                 const uint64_t cell = (uint64_t)(tib * g.H + h);
-                const uint64_t pb = (uint64_t)page * g.page_size;
-                // Byte offsets from pool (integer selects: no branches around loads).
-                // (distinct dummy bytes per field, so the three loads stay separate)
-                const uint64_t so = pb + cell * g.scale_stride;
-                c.ks = ld16(pool + (c.valid ? so + g.ks_off : dummy_off));
-                c.vs = ld16(pool + (c.valid ? so + g.vs_off : dummy_off + 2));
-                c.re = PROD ? ld16(pool + (c.valid ? so + g.kres_off : dummy_off + 4)) : (uint16_t)0;
-                // (with 32-token chunks lanes l and l + 32 hold the same token)
-                // K row: code_stride bytes, or QJL's D/8 = 16 sign bytes
-                const uint64_t kstride = QJL ? 16u : (uint64_t)g.code_stride;
-                tko[w][lane & (kChunk - 1)] = c.valid ? pb + g.kc_off + cell * kstride : dummy_off;
+                const uint8_t* pg = pool + (uint64_t)page * g.page_size;
+                const uint8_t* dummy = reinterpret_cast<const uint8_t*>(query);
+                const uint64_t so = cell * g.scale_stride, co = cell * g.code_stride;
+                c.ks = ld_u16(c.valid ? pg + (so + g.ks_off) : dummy);
+                c.vs = ld_u16(c.valid ? pg + (so + g.vs_off) : dummy + 2);
+                c.re = PROD ? ld_u16(c.valid ? pg + (so + g.kres_off) : dummy + 4) : (uint16_t)0;
+                tko[w][lane & (kChunk - 1)] =
+                    reinterpret_cast<uint64_t>(c.valid ? pg + (co + g.kc_off) : dummy);
                 tvo[w][lane & (kChunk - 1)] =
-                    c.valid ? pb + g.vc_off + cell * g.code_stride : dummy_off;
+                    reinterpret_cast<uint64_t>(c.valid ? pg + (co + g.vc_off) : dummy);
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
             for (int tau = 0; tau < kTiles; ++tau) {
-                if constexpr (QJL)  // sign bytes 4gq .. 4gq + 3: k-steps 0 .. 3
-                    c.kw[tau] = make_uint4(
-                        *reinterpret_cast<gword*>(code_row(tko[w][16 * tau + i]) + 4 * gq),
-                        0u,
-                        0u, 0u);
-                else
-                    c.kw[tau] = ld128(code_row(tko[w][16 * tau + i]) + 16 * gq);
+                gbyte* kp = reinterpret_cast<gbyte*>(tko[w][16 * tau + i]) + 4 * kS * gq;
+                if constexpr (D == 128) {
+                    const u32x4 x = *reinterpret_cast<gquad*>(kp);
+#pragma unroll
+                    for (int s = 0; s < kS; ++s) c.kw[tau][s] = x[s];
+                } else {
+                    const u32x2 x = *reinterpret_cast<gpair*>(kp);
+#pragma unroll
+                    for (int s = 0; s < kS; ++s) c.kw[tau][s] = x[s];
+                }
             }
             // (the K words first: the QK waits for them while the V words may
             // still be in flight)
             __builtin_amdgcn_sched_barrier(0);
-            // k-step p covers tiles 2p, 2p+1; k-index 8gq + e is token
-            // 32p + 4gq + e (e < 4) or 32p + 16 + 4gq + (e - 4).
+            // k-index 8gq + e is token 4gq + e (e < 4) or 16 + 4gq + (e - 4).
 #pragma unroll
-            for (int p = 0; p < kSteps; ++p)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    const int tok = 32 * p + (e < 4 ? 4 * gq + e : 16 + 4 * gq + (e - 4));
-                    c.vw[p][e] = ld32(code_row(tvo[w][tok]) + 4 * i);
-                }
+            for (int e = 0; e < 8; ++e) {
+                const int tok = e < 4 ? 4 * gq + e : 16 + 4 * gq + (e - 4);
+                gbyte* vp = reinterpret_cast<gbyte*>(tvo[w][tok]) + D / 32 * i;
+                if constexpr (D == 128)
+                    c.vw[e] = *reinterpret_cast<gword*>(vp);
+                else
+                    c.vw[e] = *reinterpret_cast<ghalf*>(vp);
+            }
         };
 
         // Issue order matters (the vector-memory counter is in order): the
@@ -1006,148 +1298,71 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
         // are built while they are in flight.
         int t0 = t_begin + w * kChunk;
         const int slot0 = load_slot(t0);
-
-        // NP = 1: decode tables staged one entry per thread (waves 0-3), then
-        // replicated after the first barrier.
-        if (!STAB && w < 4) {
-            const int lo = tid & 15, hi = tid >> 4;
-            const float vlo = pick(kV4, lo), vhi = pick(kV4, hi);
-            const uint32_t vv = pack_h2(kAlphaV * vlo, kAlphaV * vhi);
-            // prod: aK * K3; mse: the lo parts of aV * V4 (its hi parts are the V table)
-            const uint32_t kv =
-                PROD ? pack_h2(kAlphaK * pick(kK3, lo & 7), kAlphaK * pick(kK3, hi & 7))
-                     : pack_h2(lo_part(kAlphaV * vlo), lo_part(kAlphaV * vhi));
-            kstage[tid] = kv;
-            vstage[tid] = vv;
-        }
         // Query halves to fp32 (times the sign flip) before the code loads are
         // issued, so waiting for them never waits for the codes.
-        float qf[kQPerWave][2];
+        float qf[kNP][2];
         {
-            const float sh = (!QJL && (h & 1)) ? -1.0f : 1.0f;
+            const float sh = (h & 1) ? -1.0f : 1.0f;
 #pragma unroll
-            for (int k = 0; k < kQPerWave; ++k) {
+            for (int k = 0; k < kNP; ++k) {
                 qf[k][0] = h2f(qraw[k] & 0xffff) * sh;
                 qf[k][1] = h2f(qraw[k] >> 16) * (-sh);
             }
         }
         Chunk cur;
         fetch(t0, slot0, cur);  // in flight during the setup below (empty waves: all invalid)
-
-        const bool lo_col = (i & 1) != 0;  // NP = 1: column i holds row i / 2's hi (even) or lo part
-        if constexpr (STAB) {
-            static_assert(kWaves == 8 && kRows == 8, "eight waves, one row per wave and position");
-            __builtin_amdgcn_sched_barrier(0);  // the first chunk's loads go out before the setup
-            // The decode tables from registers, and each wave's rotated rows
-            // (position k: row w of group rg + k) as fp16 hi and lo parts
-            // straight into the QK B operand: one barrier for the setup.  Lane l
-            // holds d = 2l, 2l + 1: k-group l / 16, k-step (l / 4) % 4, halves
-            // 2(l % 4), + 1 of the half8.  Two or more positions: tile k / 2,
-            // column 8(k % 2) + w, hi in operand 2(k / 2), lo in 2(k / 2) + 1;
-            // one position: tile 0, hi in column w, lo in column w + 8.
+        __builtin_amdgcn_sched_barrier(0);  // the first chunk's loads go out before the setup
+        // The decode tables from registers, and each wave's rotated rows
+        // (position k: row w of group rg + k) as fp16 hi and lo parts straight
+        // into the QK B operand: one barrier for the setup.  Lane l holds d = 2l,
+        // 2l + 1: k-group l / (4 kS), k-step (l / 4) % kS, halves 2(l % 4), + 1 of
+        // the half8.  Two or more positions: tile k / 2, column 8(k % 2) + w, hi
+        // in operand 2(k / 2), lo in 2(k / 2) + 1; one position: tile 0, hi in
+        // column w, lo in column w + 8.
+        {
             const TableWords<PROD> tw = decode_table_words<PROD>(w, lane);
-            const int s_l = (lane >> 2) & 3, g_l = lane >> 4;
+            const int s_l = (jl >> 2) & (kS - 1), g_l = jl / (4 * kS);
 #pragma unroll
-            for (int k = 0; k < kQPerWave; ++k) {
+            for (int k = 0; k < kNP; ++k) {
                 if (k >= 2 * ntile || (npos == 1 && k > 0)) continue;  // never read (wave-uniform)
                 float q0 = qf[k][0], q1 = qf[k][1];
-                wht_pair<64>(q0, q1, lane);
+                wht_pair<kL>(q0, q1, lane);
                 const bool live = k < npos && rg * kRows + w + k * kWaves < num_queries;
                 q0 = live ? q0 * inv : 0.0f;
                 q1 = live ? q1 * inv : 0.0f;
+                if constexpr (QSCALE) {
+                    const int ex = scale_exp(max_lanes<kL>(fmaxf(fabsf(q0), fabsf(q1))));
+                    q0 = __builtin_amdgcn_ldexpf(q0, -ex);
+                    q1 = __builtin_amdgcn_ldexpf(q1, -ex);
+                    if (lane == 0) rsc[k * kRows + w] = __builtin_amdgcn_ldexpf(1.0f, ex);
+                }
                 const uint32_t hi = pack_h2(q0, q1);
                 const uint32_t lo = lo_pair(q0, q1, hi);
                 const int col_hi = npos == 1 ? w : 8 * (k & 1) + w;
                 const int col_lo = npos == 1 ? w + 8 : col_hi;
                 const int op_hi = npos == 1 ? 0 : 2 * (k >> 1);
                 const int op_lo = npos == 1 ? 0 : op_hi + 1;
-                reinterpret_cast<uint32_t*>(&bqs[op_hi][s_l][16 * g_l + col_hi])[lane & 3] = hi;
-                reinterpret_cast<uint32_t*>(&bqs[op_lo][s_l][16 * g_l + col_lo])[lane & 3] = lo;
+                reinterpret_cast<uint32_t*>(&bqs[op_hi][s_l][16 * g_l + col_hi])[jl & 3] = hi;
+                reinterpret_cast<uint32_t*>(&bqs[op_lo][s_l][16 * g_l + col_lo])[jl & 3] = lo;
             }
             store_decode_tables<PROD>(lut, kOffKV / 4, w, lane, tw);
-        } else {
-        // Rotated query rows of this group (wave w: rows w, w + NW, ...):
-        // qrot = WHT(q * s) * inv.
+            if constexpr (VLO && PROD) {
+                uint32_t vlo[4];
+                lo_table_words(w, lane, vlo);
+                if ((lane & 7) < kLoCopies / 4) {
 #pragma unroll
-        for (int k = 0; k < kQPerWave; ++k) {
-            const int r = w + k * kWaves;
-            if (NP >= 2 && r / kRows >= 2 * ntile) continue;  // an unused tile (wave-uniform)
-            float q0 = qf[k][0], q1 = qf[k][1];
-            wht_pair<64>(q0, q1, lane);
-            const bool live = r / kRows < npos && rg * kRows + r < num_queries;
-            qs_at(r, 2 * lane) = live ? q0 * inv : 0.0f;
-            qs_at(r, 2 * lane + 1) = live ? q1 * inv : 0.0f;
-        }
-        lds_barrier();  // staged table rows and rotated queries visible
-
-        // Every wave replicates staged rows with conflict-free 1 KB stores.
-        {
-            constexpr int kRowsPerWave = 256 / kWaves;
-            // (all staged words read before the first store: one LDS round trip)
-            uint32_t stv[kRowsPerWave / 4];
-            if constexpr (!QJL) {
-#pragma unroll
-                for (int k = 0; k < kRowsPerWave; k += 4) {
-                    const int e = w * kRowsPerWave + k + (lane >> 4);
-                    stv[k / 4] = (lane & 8) ? vstage[e] : kstage[e];  // words 32..63: V
-                }
-            }
-#pragma unroll
-            for (int k = 0; k < kRowsPerWave; k += 4) {
-                const int e = w * kRowsPerWave + k + (lane >> 4);
-                if constexpr (QJL) {  // K half: 8 copies of the fp16 +-1 octet of sign byte e
-                    uint4 v4;
-                    if (lane & 8) {
-                        const uint32_t v = vstage[e];
-                        v4 = make_uint4(v, v, v, v);
-                    } else {
-                        uint32_t wd[4];
-#pragma unroll
-                        for (int q = 0; q < 4; ++q)
-                            wd[q] = ((e >> (2 * q)) & 1 ? 0x3C00u : 0xBC00u) |
-                                    ((e >> (2 * q + 1)) & 1 ? 0x3C000000u : 0xBC000000u);
-                        v4 = make_uint4(wd[0], wd[1], wd[2], wd[3]);
-                    }
-                    *reinterpret_cast<uint4*>(kv_row(e) + 4 * (lane & 15)) = v4;
-                } else {
-                    const uint32_t v = stv[k / 4];
-                    *reinterpret_cast<uint4*>(kv_row(e) + 4 * (lane & 15)) = make_uint4(v, v, v, v);
+                    for (int k = 0; k < 4; ++k)
+                        *reinterpret_cast<u32x4*>(
+                            &lut[(32 * w + 8 * k + (lane >> 3)) * 64 + 32 + 4 * (lane & 7)]) =
+                            (u32x4){vlo[k], vlo[k], vlo[k], vlo[k]};
                 }
             }
         }
-        // B operand of QK, built once per workgroup: column i = row i/2, hi (i
-        // even) or lo (i odd) part; k-index 8*gq + e of step s is d = 32*gq + 8*s + e.
-        for (int ps = w; ps < 4 * NP; ps += kWaves) {
-            const int p = ps >> 2, s = ps & 3;
-            half8 b;
-#pragma unroll
-            for (int e = 0; e < 8; ++e)
-                b[e] = hi_lo(qs_at(p * kRows + (i >> 1), 32 * gq + 8 * s + e), lo_col);
-            bqs[p][s][lane] = __builtin_bit_cast(uint4, b);
-        }
-        }  // !STAB
         lds_barrier();
-        // NP = 1: the B operands in registers; NP >= 2 reads them from LDS per
-        // k-step (64 registers fewer in the two-tile loop).
-        half8 bq[1][4];
-        if constexpr (NP == 1) {
-#pragma unroll
-            for (int s = 0; s < 4; ++s) bq[0][s] = __builtin_bit_cast(half8, bqs[0][s][lane]);
-        }
-        // Byte address of this lane's copy of entry 0 of each table; a lookup
-        // puts the code byte into byte 1 (entry stride 256 B) with one v_perm.
-        const uint32_t lutk = (uint32_t)reinterpret_cast<uintptr_t>((lds_u32*)(kv_row(0) + (lane & 31)));
-        const uint32_t lutv = lutk + 128u;
-        const uint32_t lut_hi = lutk & 0xFF00u;  // byte 1 of the base, re-added after the perm
-        auto lookup = [&](uint32_t word, int b, int table) -> uint32_t {
-            const uint32_t base = table ? lutv : lutk;
-            const uint32_t a =
-                __builtin_amdgcn_perm(word, base, 0x03020000u | ((4u + b) << 8)) + lut_hi;
-            return *reinterpret_cast<const lds_u32*>(a);
-        };
-        // STAB: the S-row address of byte b of word (this lane's copy; its K pair
-        // at + kOffKV), and that of a V code byte (S row + 128: its V pair at
-        // + kOffKV).
+        // The S-row address of byte b of word (this lane's copy; its K pair at
+        // + kOffKV), and that of a V code byte (S row + 128: its V pair at
+        // + kOffKV): the code byte goes into byte 1 (entry stride 256 B) with one
+        // v_perm, byte 1 of the base is re-added.
         const uint32_t luts = (uint32_t)reinterpret_cast<uintptr_t>((lds_u32*)&lut[lane & 31]);
         const uint32_t luts_hi = luts & 0xFF00u;
         auto s_addr = [&](uint32_t word, int b, uint32_t off) -> uint32_t {
@@ -1156,243 +1371,42 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
         auto lds_at = [](uint32_t a, int off) -> uint32_t {
             return *reinterpret_cast<const lds_u32*>(a + off);
         };
-        // QJL: the fp16 +-1 octet of sign byte b of word (copy lane % 8).
-        const uint32_t lutq =
-            (uint32_t)reinterpret_cast<uintptr_t>((lds_u32*)(kv_row(0) + 4 * (lane & 7)));
-        auto signs = [&](uint32_t word, int b) -> half8 {
-            const uint32_t a =
-                __builtin_amdgcn_perm(word, lutq, 0x03020000u | ((4u + b) << 8)) + (lutq & 0xFF00u);
-            typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
-            return __builtin_bit_cast(half8, *reinterpret_cast<const lds_u32x4*>(a));
-        };
+        // V lookups' offset from the S row; with VLO the lanes past the lo
+        // copies read their copy kLoCopies below.
+        const uint32_t voff = !PROD ? 0u
+                              : VLO && (lane & 31) >= kLoCopies ? 128u - 4u * kLoCopies
+                                                                : 128u;
 
-        float m_run[NP], l_run[NP];
-        f32x4 acc[NP][8];
-#pragma unroll
-        for (int p = 0; p < NP; ++p) {
-            m_run[p] = kInitMax;
-            l_run[p] = 0.0f;
-#pragma unroll
-            for (int v = 0; v < 8; ++v) acc[p][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
-        }
-        bool first = true;
-        int slot_nx = load_slot(t0 + kWaves * kChunk);
-
-        // The chunk loop of the one-group layout (NP = 1).
-        auto chunk_loop = [&](auto npa) {
-            constexpr int NPA = decltype(npa)::value;
-            while (t0 < t_end) {  // wave-uniform
-                const uint4* kw = cur.kw;
-                const uint32_t(*vw)[8] = cur.vw;
-                {
-                    const float ks = h2f(cur.ks), vs = h2f(cur.vs), re = PROD ? h2f(cur.re) : 0.0f;
-                    const float4 sc = QJL    ? make_float4(0.0f, ks * kLog2e, vs, 0.0f)
-                                      : PROD ? make_float4(ks * ck, ks * re * cr, vs, 0.0f)
-                                             : make_float4(ks * ck, ks * ck * kLoScale, vs, 0.0f);
-                    tsc[w][lane & (kChunk - 1)] =
-                        cur.valid ? sc : make_float4(0.f, 0.f, 0.f, -INFINITY);
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                Chunk nxt;
-                const int t1 = t0 + kWaves * kChunk;
-                if (t1 < t_end) {  // codes of the next chunk, slots of the one after
-                    fetch(t1, slot_nx, nxt);
-                    slot_nx = load_slot(t1 + kWaves * kChunk);
-                }
-
-                // The scale rows of this lane's tokens, read before any lookup
-                // (LDS reads complete in order: a read issued after the V
-                // lookups would wait for all of them).
-                float4 scv[kTiles][4];
-#pragma unroll
-                for (int tau = 0; tau < kTiles; ++tau)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) scv[tau][e] = tsc[w][16 * tau + 4 * gq + e];
-                // QK: every table lookup of the chunk's K codes is issued before
-                // the first MFMA, so their LDS latencies overlap.  prod: aK*K3
-                // (table 0); mse: aV*V4 hi parts (table 1) and lo parts (table 0)
-                // in kl; QJL: the sign octets.
-                half8 ka[kTiles][4], kl[kTiles][4];
-#pragma unroll
-                for (int tau = 0; tau < kTiles; ++tau) {
-                    const uint32_t wd[4] = {kw[tau].x, kw[tau].y, kw[tau].z, kw[tau].w};
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        if constexpr (QJL) {  // sign byte s of the lane's word
-                            ka[tau][s] = signs(wd[0], s);
-                        } else {
-                            const int kt = PROD ? 0 : 1;
-                            ka[tau][s] = as_h8(lookup(wd[s], 0, kt), lookup(wd[s], 1, kt),
-                                               lookup(wd[s], 2, kt), lookup(wd[s], 3, kt));
-                            if constexpr (!PROD)
-                                kl[tau][s] = as_h8(lookup(wd[s], 0, 0), lookup(wd[s], 1, 0),
-                                                   lookup(wd[s], 2, 0), lookup(wd[s], 3, 0));
-                        }
-                    }
-                }
-                __builtin_amdgcn_sched_barrier(0);
-                f32x4 cb[NPA][kTiles], cs[NPA][kTiles];
-#pragma unroll
-                for (int tau = 0; tau < kTiles; ++tau) {
-#pragma unroll
-                    for (int p = 0; p < NPA; ++p) {
-                        cb[p][tau] = (f32x4){0.f, 0.f, 0.f, 0.f};
-                        cs[p][tau] = cb[p][tau];
-                    }
-                    const uint32_t wd[4] = {kw[tau].x, kw[tau].y, kw[tau].z, kw[tau].w};
-#pragma unroll
-                    for (int s = 0; s < 4; ++s) {
-                        if constexpr (QJL) {
-#pragma unroll
-                            for (int p = 0; p < NPA; ++p)
-                                cs[p][tau] = mma(ka[tau][s], bq[p][s], cs[p][tau]);
-                            continue;
-                        }
-#pragma unroll
-                        for (int p = 0; p < NPA; ++p)
-                            cb[p][tau] = mma(ka[tau][s], bq[p][s], cb[p][tau]);
-                        if constexpr (!PROD) {  // mse: the lo parts into cs
-#pragma unroll
-                            for (int p = 0; p < NPA; ++p)
-                                cs[p][tau] = mma(kl[tau][s], bq[p][s], cs[p][tau]);
-                        } else {
-                            // Residual signs (nibble bit 3: 1 -> +1) as fp16 pairs in
-                            // registers: high bytes 0x3C / 0xBC, low bytes 0.
-                            // even d, odd d
-                            const uint32_t he = ((wd[s] << 4) & 0x80808080u) ^ 0xBCBCBCBCu;
-                            const uint32_t ho = (wd[s] & 0x80808080u) ^ 0xBCBCBCBCu;
-                            const half8 sa = as_h8(__builtin_amdgcn_perm(ho, he, 0x040C000Cu),
-                                                   __builtin_amdgcn_perm(ho, he, 0x050C010Cu),
-                                                   __builtin_amdgcn_perm(ho, he, 0x060C020Cu),
-                                                   __builtin_amdgcn_perm(ho, he, 0x070C030Cu));
-#pragma unroll
-                            for (int p = 0; p < NPA; ++p)
-                                cs[p][tau] = mma(sa, bq[p][s], cs[p][tau]);
-                        }
-                    }
-                }
-                // The V lookups (B operands of PV) go out now: the softmax below
-                // runs while they are in flight.
-                uint32_t bv[kSteps][8][4];  // [step][N-tile v = d - 8i][token pair]
-#pragma unroll
-                for (int st = 0; st < kSteps; ++st)
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint32_t we = vw[st][2 * q], wo = vw[st][2 * q + 1];
-                        const uint32_t lob = (we & 0x0F0F0F0Fu) | ((wo & 0x0F0F0F0Fu) << 4);
-                        const uint32_t hib = ((we >> 4) & 0x0F0F0F0Fu) | (wo & 0xF0F0F0F0u);
-#pragma unroll
-                        for (int b = 0; b < 4; ++b) {
-                            bv[st][2 * b][q] = lookup(lob, b, 1);
-                            bv[st][2 * b + 1][q] = lookup(hib, b, 1);
-                        }
-                    }
-                __builtin_amdgcn_sched_barrier(0);
-                // Logits (base 2) of tokens 16*tau + 4*gq + e; hi + lo columns summed.
-                float lg[NPA][kTiles][4];
-#pragma unroll
-                for (int p = 0; p < NPA; ++p) {
-                    // rows shorter than the chunk's end need the causal mask
-                    const bool masked = PAGED && t0 + kChunk > gmin[p];
-                    float mloc = -INFINITY;
-#pragma unroll
-                    for (int tau = 0; tau < kTiles; ++tau)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float4 sc = scv[tau][e];
-                            if constexpr (QJL) {
-                                const float sr = cs[p][tau][e] + quad_xor<1>(cs[p][tau][e]);
-                                lg[p][tau][e] = fmaf(sr, sc.y, sc.w);
-                            } else {
-                                const float sb = cb[p][tau][e] + quad_xor<1>(cb[p][tau][e]);
-                                const float sr = cs[p][tau][e] + quad_xor<1>(cs[p][tau][e]);
-                                lg[p][tau][e] = fmaf(sb, sc.x, fmaf(sr, sc.y, sc.w));
-                            }
-                            if (masked)  // causal limit of this column's row
-                                if (t0 + 16 * tau + 4 * gq + e >= rowlen[p])
-                                    lg[p][tau][e] = -INFINITY;
-                            mloc = fmaxf(mloc, lg[p][tau][e]);
-                        }
-                    mloc = lane_xor_reduce<16>(mloc, [](float x, float y) { return fmaxf(x, y); });
-                    mloc = lane_xor_reduce<32>(mloc, [](float x, float y) { return fmaxf(x, y); });
-                    // v_exp_f32 without denormal handling: arguments are <= 0 and a
-                    // weight below 2^-126 of the running maximum is negligible.
-                    const float m_new = fmaxf(m_run[p], mloc);
-                    const float alpha = first ? 0.0f : __builtin_amdgcn_exp2f(m_run[p] - m_new);
-                    m_run[p] = m_new;
-                    float lsum = 0.0f;
-#pragma unroll
-                    for (int tau = 0; tau < kTiles; ++tau)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            lg[p][tau][e] = __builtin_amdgcn_exp2f(lg[p][tau][e] - m_new);
-                            lsum += lg[p][tau][e];
-                        }
-                    l_run[p] = l_run[p] * alpha + lsum;
-                    if (!first && __any(alpha != 1.0f)) {
-                        // acc lane (d, gq) holds columns 4gq..4gq+3 = rows 2gq, 2gq+1.
-                        const float a0 = __shfl(alpha, 4 * gq), a1 = __shfl(alpha, 4 * gq + 2);
-#pragma unroll
-                        for (int v = 0; v < 8; ++v) {
-                            acc[p][v][0] *= a0;
-                            acc[p][v][1] *= a0;
-                            acc[p][v][2] *= a1;
-                            acc[p][v][3] *= a1;
-                        }
-                    }
-                }
-                // PV: one decoded B operand per N-tile, an MFMA per position
-#pragma unroll
-                for (int st = 0; st < kSteps; ++st) {
-                    half8 ap[NPA];
-#pragma unroll
-                    for (int p = 0; p < NPA; ++p)
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) {
-                            const int tau = 2 * st + (e >> 2), ee = e & 3;
-                            ap[p][e] = hi_lo(lg[p][tau][ee] * scv[tau][ee].z, lo_col);
-                        }
-#pragma unroll
-                    for (int v = 0; v < 8; ++v) {
-                        const half8 bvv =
-                            as_h8(bv[st][v][0], bv[st][v][1], bv[st][v][2], bv[st][v][3]);
-#pragma unroll
-                        for (int p = 0; p < NPA; ++p)
-                            acc[p][v] = mma(ap[p], bvv, acc[p][v]);
-                    }
-                }
-                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                cur = nxt;
-                t0 = t1;
-                first = false;
-            }
-        };
-        // NP >= 2: one softmax state per lane and tile (its column's row), hi and
-        // lo stacked along the reductions.  A unit with fewer positions runs the
+        int slot_nx = load_slot(t0 + kPass);
+        // One softmax state per lane and tile (its column's row), hi and lo
+        // stacked along the reductions.  A unit with fewer positions runs the
         // loop over the tiles it needs; a tile's unused columns compute on zero
         // queries and are dropped.
-        float m_col[NT], l_col[NT];
-        f32x4 acc_col[NT][8];
+        float m_col[kNT], l_col[kNT];
+        f32x4 acc_col[kNT][kND], acl_col[VLO ? kNT : 1][VLO ? kND : 1];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
+        for (int t = 0; t < kNT; ++t) {
             m_col[t] = kInitMax;
             l_col[t] = 0.0f;
 #pragma unroll
-            for (int v = 0; v < 8; ++v) acc_col[t][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            for (int v = 0; v < kND; ++v) {
+                acc_col[t][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                if constexpr (VLO) acl_col[t][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            }
         }
+        float qsc[kNT];
+#pragma unroll
+        for (int t = 0; t < kNT; ++t)
+            qsc[t] = QSCALE && t < ntile ? rsc[npos == 1 ? i & 7 : 16 * t + i] : 1.0f;
         // COLS (a unit of one position): one tile whose columns are the
-        // position's rows as hi (columns 0-7) and lo (8-15) parts, as in the
-        // one-group kernel: one MFMA per product instead of two, and the two
-        // halves of a column pair summed (logits; outputs at the merge).
+        // position's rows as hi (columns 0-7) and lo (8-15) parts: one MFMA per
+        // product instead of two, and the two halves of a column pair summed
+        // (logits; outputs at the merge).
         auto stacked_loop = [&](auto nta, auto cols) {
             constexpr int NTA = decltype(nta)::value;
             constexpr bool COLS = decltype(cols)::value;
             static_assert(!COLS || NTA == 1, "one tile");
             while (t0 < t_end) {  // wave-uniform
-                const uint4* kw = cur.kw;
-                const uint32_t(*vw)[8] = cur.vw;
                 {
                     const float ks = h2f(cur.ks), vs = h2f(cur.vs), re = PROD ? h2f(cur.re) : 0.0f;
                     tsc[w][lane & (kChunk - 1)] =
@@ -1402,7 +1416,7 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                 }
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-                const int t1 = t0 + kWaves * kChunk;
+                const int t1 = t0 + kPass;
                 // QK: each decoded A operand against every tile's hi and lo query
                 f32x4 cb[NTA][kTiles], cs[NTA][kTiles];
 #pragma unroll
@@ -1424,16 +1438,12 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                         o.bk[pp] = __builtin_bit_cast(half8, bqs[pp][s][lane]);
 #pragma unroll
                     for (int tau = 0; tau < kTiles; ++tau) {
-                        const uint32_t wd = s == 0   ? kw[tau].x
-                                            : s == 1 ? kw[tau].y
-                                            : s == 2 ? kw[tau].z
-                                                     : kw[tau].w;
                         // one address per byte: its K pair (prod aK*K3, mse the hi
                         // parts) and its S pair (prod the residual signs, mse the lo
                         // parts)
                         uint32_t ad[4];
 #pragma unroll
-                        for (int b = 0; b < 4; ++b) ad[b] = s_addr(wd, b, 0);
+                        for (int b = 0; b < 4; ++b) ad[b] = s_addr(cur.kw[tau][s], b, 0);
                         o.a[tau] = as_h8(lds_at(ad[0], kOffKV), lds_at(ad[1], kOffKV),
                                          lds_at(ad[2], kOffKV), lds_at(ad[3], kOffKV));
                         o.al[tau] = as_h8(lds_at(ad[0], 0), lds_at(ad[1], 0), lds_at(ad[2], 0),
@@ -1444,8 +1454,8 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                 float4 scq[kTiles][4];  // the logits' per-token scales, read during the last k-step
                 load_ops(0, ops[0]);
 #pragma unroll
-                for (int s = 0; s < 4; ++s) {
-                    if (s < 3) {
+                for (int s = 0; s < kS; ++s) {
+                    if (s < kS - 1) {
                         load_ops(s + 1, ops[(s + 1) & 1]);
                     } else {
 #pragma unroll
@@ -1475,7 +1485,6 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                const bool masked = t0 + kChunk > gmin_live;
                 // Logits (base 2) of tokens 16*tau + 4*gq + e for this lane's column.
                 float lg[NTA][kTiles][4];
 #pragma unroll
@@ -1490,25 +1499,46 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                                 b += lane_xor<8>(b);
                                 r += lane_xor<8>(r);
                             }
-                            lg[t][tau][e] = fmaf(b, sc.x, fmaf(r, sc.y, sc.w));
+                            lg[t][tau][e] = QSCALE ? fmaf(fmaf(b, sc.x, r * sc.y), qsc[t], sc.w)
+                                                   : fmaf(b, sc.x, fmaf(r, sc.y, sc.w));
                         }
                 // The V lookups (B operands of PV) go out before the softmax,
                 // whose VALU work hides their LDS latency.
-                uint32_t bv[kSteps][8][4];  // [step][N-tile v = d - 8i][token pair]
-#pragma unroll
-                for (int st = 0; st < kSteps; ++st)
+                uint32_t bv[kND][4], bl[VLO ? kND : 1][4];  // [N-tile v = d - kND i][token pair]
+                if constexpr (D == 128) {
 #pragma unroll
                     for (int q = 0; q < 4; ++q) {
-                        const uint32_t we = vw[st][2 * q], wo = vw[st][2 * q + 1];
+                        const uint32_t we = cur.vw[2 * q], wo = cur.vw[2 * q + 1];
                         const uint32_t lob = (we & 0x0F0F0F0Fu) | ((wo & 0x0F0F0F0Fu) << 4);
                         const uint32_t hib = ((we >> 4) & 0x0F0F0F0Fu) | (wo & 0xF0F0F0F0u);
 #pragma unroll
                         for (int b = 0; b < 4; ++b) {
                             // (turbo_prod: the V copies; turbo_mse: its K copies hold aV*V4)
-                            bv[st][2 * b][q] = lds_at(s_addr(lob, b, PROD ? 128u : 0u), kOffKV);
-                            bv[st][2 * b + 1][q] = lds_at(s_addr(hib, b, PROD ? 128u : 0u), kOffKV);
+                            bv[2 * b][q] = lds_at(s_addr(lob, b, PROD ? 128u : 0u), kOffKV);
+                            bv[2 * b + 1][q] = lds_at(s_addr(hib, b, PROD ? 128u : 0u), kOffKV);
                         }
                     }
+                } else {
+                    // two token pairs per word (a lane's row part is two bytes)
+#pragma unroll
+                    for (int p = 0; p < 2; ++p) {
+                        const uint32_t we = cur.vw[4 * p] | (cur.vw[4 * p + 2] << 16);
+                        const uint32_t wo = cur.vw[4 * p + 1] | (cur.vw[4 * p + 3] << 16);
+                        const uint32_t lob = (we & 0x0F0F0F0Fu) | ((wo & 0x0F0F0F0Fu) << 4);
+                        const uint32_t hib = ((we >> 4) & 0x0F0F0F0Fu) | (wo & 0xF0F0F0F0u);
+#pragma unroll
+                        for (int b = 0; b < 4; ++b) {
+                            const int v = 2 * (b & 1), q = 2 * p + (b >> 1);
+                            const uint32_t a0 = s_addr(lob, b, voff), a1 = s_addr(hib, b, voff);
+                            bv[v][q] = lds_at(a0, kOffKV);
+                            bv[v + 1][q] = lds_at(a1, kOffKV);
+                            if constexpr (VLO) {
+                                bl[v][q] = lds_at(a0, 0);
+                                bl[v + 1][q] = lds_at(a1, 0);
+                            }
+                        }
+                    }
+                }
                 __builtin_amdgcn_sched_barrier(0);
                 // This chunk's codes are consumed: the next chunk's codes and the
                 // slots of the one after are fetched into cur's registers, in
@@ -1518,10 +1548,11 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                 // buffer behind the first k-step).
                 if (t1 < t_end) {
                     fetch(t1, slot_nx, cur);
-                    slot_nx = load_slot(t1 + kWaves * kChunk);
+                    slot_nx = load_slot(t1 + kPass);
                 }
-                if (masked) {  // a row of the unit ends in this chunk (wave-uniform)
-                    asm volatile("" ::: "memory");  // a branch: no selects on every chunk
+                if (PAGED && t0 + kChunk > gmin_live) {  // a row of the unit ends in this chunk
+                    // (wave-uniform; a branch: no selects on every chunk)
+                    asm volatile("" ::: "memory");
 #pragma unroll
                     for (int t = 0; t < NTA; ++t)
 #pragma unroll
@@ -1561,9 +1592,12 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
 #pragma unroll
                         for (int e = 0; e < 4; ++e) a[e] = __shfl(alpha, 4 * gq + e);
 #pragma unroll
-                        for (int v = 0; v < 8; ++v)
+                        for (int v = 0; v < kND; ++v)
 #pragma unroll
-                            for (int e = 0; e < 4; ++e) acc_col[t][v][e] *= a[e];
+                            for (int e = 0; e < 4; ++e) {
+                                acc_col[t][v][e] *= a[e];
+                                if constexpr (VLO) acl_col[t][v][e] *= a[e];
+                            }
                     }
                 }
 #pragma unroll
@@ -1584,95 +1618,82 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
                     l_col[t] += lsum;
                 }
                 // PV: every tile's hi and lo P against each decoded B operand
+                half8 ah[NTA], al[NTA];
 #pragma unroll
-                for (int st = 0; st < kSteps; ++st) {
-                    half8 ah[NTA], al[NTA];
+                for (int t = 0; t < NTA; ++t) {
+                    uint32_t hw[4], lw[4];
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const int tau = e >> 2, ee = e & 3;
+                        const float x0 = lg[t][tau][ee] * tsc[w][16 * tau + 4 * gq + ee].z;
+                        const float x1 = lg[t][tau][ee + 1] * tsc[w][16 * tau + 4 * gq + ee + 1].z;
+                        hw[e >> 1] = pack_h2(x0, x1);
+                        lw[e >> 1] = lo_pair(x0, x1, hw[e >> 1]);
+                    }
+                    if constexpr (COLS) {  // column i < 8: hi; i >= 8: lo
+                        const bool lo = (i >> 3) != 0;
+                        ah[t] = as_h8(lo ? lw[0] : hw[0], lo ? lw[1] : hw[1], lo ? lw[2] : hw[2],
+                                      lo ? lw[3] : hw[3]);
+                    } else {
+                        ah[t] = as_h8(hw[0], hw[1], hw[2], hw[3]);
+                        al[t] = as_h8(lw[0], lw[1], lw[2], lw[3]);
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < kND; ++v) {
+                    const half8 bvv = as_h8(bv[v][0], bv[v][1], bv[v][2], bv[v][3]);
 #pragma unroll
                     for (int t = 0; t < NTA; ++t) {
-                        uint32_t hw[4], lw[4];
-#pragma unroll
-                        for (int e = 0; e < 8; e += 2) {
-                            const int tau = 2 * st + (e >> 2), ee = e & 3;
-                            const float x0 = lg[t][tau][ee] * tsc[w][16 * tau + 4 * gq + ee].z;
-                            const float x1 =
-                                lg[t][tau][ee + 1] * tsc[w][16 * tau + 4 * gq + ee + 1].z;
-                            hw[e >> 1] = pack_h2(x0, x1);
-                            lw[e >> 1] = lo_pair(x0, x1, hw[e >> 1]);
-                        }
-                        if constexpr (COLS) {  // column i < 8: hi; i >= 8: lo
-                            const bool lo = (i >> 3) != 0;
-                            ah[t] = as_h8(lo ? lw[0] : hw[0], lo ? lw[1] : hw[1], lo ? lw[2] : hw[2],
-                                          lo ? lw[3] : hw[3]);
-                        } else {
-                            ah[t] = as_h8(hw[0], hw[1], hw[2], hw[3]);
-                            al[t] = as_h8(lw[0], lw[1], lw[2], lw[3]);
-                        }
+                        acc_col[t][v] = mma(ah[t], bvv, acc_col[t][v]);
+                        if (!COLS) acc_col[t][v] = mma(al[t], bvv, acc_col[t][v]);
                     }
+                }
+                if constexpr (VLO) {  // (the lo P against V's lo parts: ~2^-22 of the sum, left out)
 #pragma unroll
-                    for (int v = 0; v < 8; ++v) {
-                        const half8 bvv =
-                            as_h8(bv[st][v][0], bv[st][v][1], bv[st][v][2], bv[st][v][3]);
+                    for (int v = 0; v < kND; ++v) {
+                        const half8 blv = as_h8(bl[v][0], bl[v][1], bl[v][2], bl[v][3]);
 #pragma unroll
-                        for (int t = 0; t < NTA; ++t) {
-                            acc_col[t][v] = mma(ah[t], bvv, acc_col[t][v]);
-                            if (!COLS) acc_col[t][v] = mma(al[t], bvv, acc_col[t][v]);
-                        }
+                        for (int t = 0; t < NTA; ++t) acl_col[t][v] = mma(ah[t], blv, acl_col[t][v]);
                     }
                 }
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
                 t0 = t1;
-                first = false;
             }
         };
-        if constexpr (NP >= 2) {
-            if (NT == 2 && ntile == 2)
-                stacked_loop(std::integral_constant<int, NT>{}, std::false_type{});
-            else if (npos == 1)
-                stacked_loop(std::integral_constant<int, 1>{}, std::true_type{});
-            else
-                stacked_loop(std::integral_constant<int, 1>{}, std::false_type{});
-        } else {
-            chunk_loop(std::integral_constant<int, 1>{});
-        }
+        if (ntile == 2)
+            stacked_loop(std::integral_constant<int, 2>{}, std::false_type{});
+        else if (npos == 1)
+            stacked_loop(std::integral_constant<int, 1>{}, std::true_type{});
+        else
+            stacked_loop(std::integral_constant<int, 1>{}, std::false_type{});
 
-        // Wave results: l summed over the g lanes of each column; o rows (NP = 1:
-        // from the hi + lo columns), the V codebook scale divided out.  Then the
-        // waves are merged per row, the inverse WHT and sign flip applied, and the
-        // partial written to the workspace (NP >= 2: one tile of 16 rows per pass
-        // through the merge space).  A position whose rows all end before this
-        // piece has no partial (its combine reads only the pieces below its
-        // longest row).
-        if constexpr (NP >= 2) {
+        // Wave results: l summed over the g lanes of each column; o rows with
+        // the V codebook scale divided out.  Then the waves are merged per row,
+        // the inverse WHT and sign flip applied, and the partial written.  A
+        // position whose rows all end before this piece has no partial (its
+        // combine reads only the pieces below its longest row).
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                float l_tot = lane_xor_reduce<16>(l_col[t], [](float x, float y) { return x + y; });
-                l_tot = lane_xor_reduce<32>(l_tot, [](float x, float y) { return x + y; });
-                if (gq == 0) {
-                    mm[w][16 * t + i] = m_col[t];
-                    ml[w][16 * t + i] = l_tot;
-                }
-            }
-        } else {
-#pragma unroll
-            for (int p = 0; p < NP; ++p) {
-                float l_tot = lane_xor_reduce<16>(l_run[p], [](float x, float y) { return x + y; });
-                l_tot = lane_xor_reduce<32>(l_tot, [](float x, float y) { return x + y; });
-                if (gq == 0 && !lo_col) {
-                    mm[w][p * kRows + (i >> 1)] = m_run[p];
-                    ml[w][p * kRows + (i >> 1)] = l_tot;
-                }
+        for (int t = 0; t < kNT; ++t) {
+            float l_tot = lane_xor_reduce<16>(l_col[t], [](float x, float y) { return x + y; });
+            l_tot = lane_xor_reduce<32>(l_tot, [](float x, float y) { return x + y; });
+            if (gq == 0) {
+                mm[w][16 * t + i] = m_col[t];
+                ml[w][16 * t + i] = l_tot;
             }
         }
         const float iav = 1.0f / kAlphaV;
-        const float s0 = (!QJL && (h & 1)) ? -inv : inv;
+        const float s0 = (h & 1) ? -inv : inv;
         // Row rr of tile t from the merge space mt (the 8 waves' o rows): the
         // waves' (m, l, o) merged, the inverse WHT and sign flip, the partial.
-        auto merge_row = [&](int t, int rr, float(*mt)[kMoRows][128]) {
+        auto merge_row = [&](int t, int rr, float(*mt)[kMoRows][D]) {
             const int r = kMoRows * t + rr;  // row of the workgroup
             const int p = r / kRows;
             bool keep = p < npos;
-            if constexpr (PAGED) keep = keep && t_begin < gend[p];
+            if constexpr (PAGED)
+                keep = keep && t_begin < gend[p];
+            else
+                keep = keep && rg * kRows + r < num_queries;
             if (!keep) return;  // wave-uniform
             float M = mm[0][r];
 #pragma unroll
@@ -1682,67 +1703,60 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
             for (int u = 0; u < kWaves; ++u) {
                 const float wt = __builtin_amdgcn_exp2f(mm[u][r] - M);  // (argument <= 0)
                 L += ml[u][r] * wt;
-                o0 += mt[u][rr][2 * lane] * wt;
-                o1 += mt[u][rr][2 * lane + 1] * wt;
+                o0 += mt[u][rr][2 * jl] * wt;
+                o1 += mt[u][rr][2 * jl + 1] * wt;
             }
-            if (NP >= 2 && npos == 1) {  // one position: + its lo columns 8-15
+            if (npos == 1) {  // one position: + its lo columns 8-15
 #pragma unroll
                 for (int u = 0; u < kWaves; ++u) {
                     const float wt = __builtin_amdgcn_exp2f(mm[u][r] - M);  // (argument <= 0)
-                    o0 += mt[u][rr + kRows][2 * lane] * wt;
-                    o1 += mt[u][rr + kRows][2 * lane + 1] * wt;
+                    o0 += mt[u][rr + kRows][2 * jl] * wt;
+                    o1 += mt[u][rr + kRows][2 * jl + 1] * wt;
                 }
             }
-            wht_pair<64>(o0, o1, lane);
-            float* part = ws + ((pid * NP + p) * kRows + r % kRows) * kPartStride;
-            part[2 * lane] = o0 * s0;
-            part[2 * lane + 1] = o1 * -s0;
-            if (lane == 0) {
-                part[128] = M;
-                part[129] = L;
+            wht_pair<kL>(o0, o1, lane);
+            if constexpr (PAGED) {
+                float* part = ws + ((pid * kNP + p) * kRows + r % kRows) * part_stride(D);
+                if (D == 128 || lane < kL) {
+                    part[2 * jl] = o0 * s0;
+                    part[2 * jl + 1] = o1 * -s0;
+                }
+                if (lane == 0) {
+                    part[D] = M;
+                    part[D + 1] = L;
+                }
+            } else {  // the layout of dec's partials (attn_decode_combine_kernel)
+                const size_t it = (size_t)(rg + p) * g.H + h;
+                const size_t row = (it * num_splits + pid) * kRows + r % kRows;
+                if (D == 128 || lane < kL)
+                    *reinterpret_cast<float2*>(ws + row * D + 2 * jl) = make_float2(o0 * s0, o1 * -s0);
+                if (lane == 0) pml[(it * kRows + r % kRows) * num_splits + pid] = make_float2(M, L);
             }
         };
-        if constexpr (NP >= 2) {
-            // Both tiles at once: tile t's merge space at table word 16384 t
-            // (the tables are no longer read), three barriers per piece instead
-            // of four, and each wave's four rows merged without a barrier
-            // between them.
-            static_assert(NT * sizeof(float) * kWaves * kMoRows * 128 <= sizeof(lut), "merge spaces");
-            auto mot = [&](int t) { return reinterpret_cast<float(*)[kMoRows][128]>(&lut[16384 * t]); };
-            __syncthreads();  // every wave is done with the tables
+        // Both tiles at once: tile t's merge space at table word 16384 t (the
+        // tables are no longer read), three barriers per piece instead of four,
+        // and each wave's four rows merged without a barrier between them.
+        auto mot = [&](int t) { return reinterpret_cast<float(*)[kMoRows][D]>(&lut[16384 * t]); };
+        __syncthreads();  // every wave is done with the tables
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                if (t >= ntile) break;  // wave- and workgroup-uniform
+        for (int t = 0; t < kNT; ++t) {
+            if (t >= ntile) break;  // wave- and workgroup-uniform
 #pragma unroll
-                for (int v = 0; v < 8; ++v)
+            for (int v = 0; v < kND; ++v)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)  // (x2: the PV operand was P * vs / 2)
-                        mot(t)[w][4 * gq + e][8 * i + v] = acc_col[t][v][e] * (2.0f * iav);
-            }
-            __syncthreads();
-#pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int k = 0; k < kMoRows / kWaves; ++k) merge_row(t, w + k * kWaves, mot(t));
-            // the next piece's setup writes its rotated queries into the S rows,
-            // which hold tile 0's merge space
-            __syncthreads();
-        } else {
-#pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                __syncthreads();  // every wave is done with the tables (or the last pass) mo overwrites
-#pragma unroll
-                for (int p = 0; p < NP; ++p)
-#pragma unroll
-                    for (int v = 0; v < 8; ++v) {
-                        mo[w][p * kRows + 2 * gq][8 * i + v] = (acc[p][v][0] + acc[p][v][1]) * iav;
-                        mo[w][p * kRows + 2 * gq + 1][8 * i + v] =
-                            (acc[p][v][2] + acc[p][v][3]) * iav;
-                    }
-                __syncthreads();
-                for (int rr = w; rr < kMoRows; rr += kWaves) merge_row(t, rr, mo);
-            }
+                for (int e = 0; e < 4; ++e) {  // (x2: the PV operand was P * vs / 2)
+                    float x = acc_col[t][v][e];
+                    if constexpr (VLO) x = fmaf(acl_col[t][v][e], kLoScale, x);
+                    mot(t)[w][4 * gq + e][kND * i + v] = x * (2.0f * iav);
+                }
         }
+        __syncthreads();
+#pragma unroll
+        for (int t = 0; t < kNT; ++t)
+#pragma unroll
+            for (int k = 0; k < kMoRows / kWaves; ++k) merge_row(t, w + k * kWaves, mot(t));
+        // the next piece's setup writes its decode tables over the merge spaces
+        if constexpr (PAGED) __syncthreads();
     };  // item
 
     if constexpr (PAGED) {
@@ -1754,7 +1768,6 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
         // of a token share its cache lines (cell tib * H + h), and the second
         // reader finds them in that XCD's L2.  The segments of one XCD are
         // consecutive, so the units of a sequence mostly share it too.
-        constexpr int kPass = kChunk * kWaves;
         const int Gh = (int)gridDim.x / g.H;
         const int hh = (int)blockIdx.x / Gh;
         const int bl = (int)blockIdx.x - hh * Gh;
@@ -1798,25 +1811,26 @@ __global__ __launch_bounds__(64 * NW) void attn_mfma_split_kernel(
             }
         }
     } else {
-        // Grid (split, kv head, row group), or one dimension of splits x heads
-        // when there are more row groups than a grid dimension holds (the
-        // first form needs no divisions before the first loads).
-        int split, h, rg;
+        // Grid (split, kv head, unit), or one dimension of splits x heads x
+        // units when there are more units than a grid dimension holds.
+        const int groups = (num_queries + kRows - 1) / kRows;
+        int split, h, un;
         if (gridDim.x == (unsigned)num_splits) {
             split = blockIdx.x;
             h = blockIdx.y;
-            rg = blockIdx.z;
+            un = blockIdx.z;
         } else {
             split = blockIdx.x % num_splits;
             const int hr = blockIdx.x / num_splits;
             h = hr % g.H;
-            rg = hr / g.H;
+            un = hr / g.H;
         }
         const int t_begin = split * tokens_per_split;
-        item(threadIdx.x, h, rg, 1, t_begin, t_begin + tokens_per_split,
-             ((size_t)rg * g.H + h) * num_splits + split);
+        item(threadIdx.x, h, un * kNP, min(kNP, groups - un * kNP), t_begin,
+             t_begin + tokens_per_split, (size_t)split);
     }
 }
+}  // namespace unit
 // Sum of the split partials of one output row (q, h): o = sum_s 2^(m_s - M)
 // o_s / sum_s 2^(m_s - M) l_s.  Block = (row, 32-element slice of d), 256
 // threads = 8 groups x 32 d.  Group g takes splits g, g + 8, ...: it loads up
@@ -1958,13 +1972,16 @@ __global__ __launch_bounds__(256) void attn_mfma_combine_items_kernel(
 // unit u; its item's passes were cut at segment bounds into pieces, one
 // partial per segment they start in (slot item + segment, position p), and
 // a piece starting at or past the group's longest row wrote none.
-__global__ __launch_bounds__(256) void attn_paged_combine_kernel(
+template <int D>
+__global__ __launch_bounds__(2 * D) void attn_paged_combine_kernel(
     const float* __restrict__ ws, uint16_t* __restrict__ output, int H, int num_queries,
-    int num_segments, int positions, int pass, mfma::PagedRows pr) {
+    int num_segments, mfma::PagedRows pr) {
     using namespace mfma;
+    constexpr int positions = unit::kNP, pass = unit::kPass;
+    constexpr int kT = D / 4;     // threads per row
     const int item = blockIdx.x;  // h + H * rg
     const int h = item % H, rg = item / H;
-    const int t = threadIdx.x, r = t >> 5, d0 = 4 * (t & 31);
+    const int t = threadIdx.x, r = t / kT, d0 = 4 * (t % kT);
     const PagedUnit un = pr.group_unit[rg];
     const int u = un.index;
     const int total = pr.plan[1], G = num_segments;
@@ -2006,8 +2023,8 @@ __global__ __launch_bounds__(256) void attn_paged_combine_kernel(
             item_passes(S, un.n, un.w, sg.bound(gs), sg.bound(gs + 1), x0, x1);
             okv[k] = b + k <= g_hi && x0 < x1 && x0 * pass < kv;
             const float* pp =
-                ws + ((((unit0 + gs) * H + h) * positions + p) * kRows + r) * kPartStride;
-            mlr[k] = *reinterpret_cast<const float2*>(pp + 128);
+                ws + ((((unit0 + gs) * H + h) * positions + p) * kRows + r) * unit::part_stride(D);
+            mlr[k] = *reinterpret_cast<const float2*>(pp + D);
             po[k] = *reinterpret_cast<const float4*>(pp + d0);
         }
         __builtin_amdgcn_sched_barrier(0);
@@ -2042,7 +2059,7 @@ __global__ __launch_bounds__(256) void attn_paged_combine_kernel(
     const int q = rg * kRows + r;
     if (q >= num_queries) return;
     const auto fin = [&](float o) { return (uint32_t)f2h(L > 0.f ? o / L : o); };
-    *reinterpret_cast<uint2*>(output + ((size_t)q * H + h) * 128 + d0) =
+    *reinterpret_cast<uint2*>(output + ((size_t)q * H + h) * D + d0) =
         make_uint2(fin(acc.x) | (fin(acc.y) << 16), fin(acc.z) | (fin(acc.w) << 16));
 }
 
@@ -2072,7 +2089,7 @@ __device__ int block_scan_1024(int v, int ident, int* s_tot, Op op) {
 }
 
 // Paged steps: the work positions a unit's setup counts for (a two-tile pass
-// weighs 4), before its first pass (config 5, 32 sequences: 139 us per step
+// weighs 4), before its first pass (32 sequences of 1K-32K tokens: 139 us per step
 // with 0, 135 with 4, 131-133 with 8, 12 or 16).
 #ifndef TQ_PAGED_PIECE_COST
 #define TQ_PAGED_PIECE_COST 8
@@ -2730,31 +2747,19 @@ __global__ __launch_bounds__(64) void attn_decode_combine_kernel(
 
 }  // namespace dec
 
-// New-token positions (row groups of one sequence) per paged workgroup.
-#ifndef TQ_PAGED_POSITIONS
-#define TQ_PAGED_POSITIONS 4
-#endif
-constexpr int kPagedPositions = TQ_PAGED_POSITIONS;
 // Paged steps: work segments (workgroups) per CU.
 #ifndef TQ_PAGED_SEGMENTS_PER_CU
 #define TQ_PAGED_SEGMENTS_PER_CU 1
 #endif
 constexpr int kPagedSegmentsPerCU = TQ_PAGED_SEGMENTS_PER_CU;
 
-// Split kernel shape: tokens per wave iteration and waves per workgroup.
-#ifndef TQ_SPLIT_CHUNK
-#define TQ_SPLIT_CHUNK 32
-#endif
-#ifndef TQ_SPLIT_WAVES
-#define TQ_SPLIT_WAVES 8
-#endif
+// Slot-mapped decode: the least tokens of a split, and its workgroups per CU.
 #ifndef TQ_SPLIT_MIN_TOKENS
 #define TQ_SPLIT_MIN_TOKENS 256
 #endif
 #ifndef TQ_SPLIT_BLOCKS_PER_CU
 #define TQ_SPLIT_BLOCKS_PER_CU 2
 #endif
-constexpr int kSplitChunk = TQ_SPLIT_CHUNK, kSplitWaves = TQ_SPLIT_WAVES;
 constexpr int kSplitMinTokens = TQ_SPLIT_MIN_TOKENS, kSplitBlocksPerCU = TQ_SPLIT_BLOCKS_PER_CU;
 
 bool mfma_attention_ok(const PageGeom& g, const void* pool) {
@@ -2784,12 +2789,12 @@ bool mfma_attention64_ok(const PageGeom& g, const void* pool) {
     }
 
 namespace {
-// The MFMA split-K attention over slot-mapped tokens: split + combine launches.
-template <int SCH>
-void launch_mfma_attention(const uint16_t* query, const uint8_t* pool, const int32_t* slots,
-                           uint16_t* output, const PageGeom& g, int num_queries,
-                           int num_kv_tokens, float inv, hipStream_t stream, const char* split_name,
-                           const char* combine_name, const Scratch& scratch = Scratch{}) {
+// The MFMA split-K decode of QJL-1b pages: split + combine launches.
+void launch_qjl_mfma(const uint16_t* query, const uint8_t* pool, const int32_t* slots,
+                     uint16_t* output, const PageGeom& g, int num_queries, int num_kv_tokens,
+                     float inv, hipStream_t stream) {
+    const char* split_name = "qjl_fused_attn_split";
+    const char* combine_name = "qjl_fused_attn_combine";
     using namespace mfma;
     const int rows = num_queries * g.H;
     const int row_groups = (num_queries + kRows - 1) / kRows;
@@ -2803,9 +2808,7 @@ void launch_mfma_attention(const uint16_t* query, const uint8_t* pool, const int
     if (tps > 0) splits = (num_kv_tokens + tps - 1) / tps;
     const size_t blocks = (size_t)splits * heads;
     float* ws = static_cast<float*>(
-        scratch.get(stream, blocks * kRows * kPartStride * sizeof(float), split_name));
-    constexpr int kCH = kSplitChunk, kNW = kSplitWaves;
-    const PagedRows none{};
+        workspace(stream, blocks * kRows * kPartStride * sizeof(float)));
     constexpr int kMaxGridYZ = 65535;
     const dim3 combine_grid = num_queries <= kMaxGridYZ && g.H <= kMaxGridYZ
                                   ? dim3(4, g.H, num_queries)
@@ -2819,9 +2822,8 @@ void launch_mfma_attention(const uint16_t* query, const uint8_t* pool, const int
     const dim3 grid = row_groups <= kMaxGridYZ && g.H <= kMaxGridYZ
                           ? dim3(splits, g.H, row_groups)
                           : dim3((unsigned)blocks);
-    hipLaunchKernelGGL((attn_mfma_split_kernel<SCH, kCH, kNW, false>), grid, dim3(64 * kNW), 0,
-                       stream, query, pool, slots, ws, inv, num_queries, num_kv_tokens, tps, splits,
-                       g, none);
+    hipLaunchKernelGGL(qjl::attn_qjl_split_kernel, grid, dim3(64 * qjl::kWaves), 0, stream, query,
+                       pool, slots, ws, inv, num_queries, num_kv_tokens, tps, splits, g);
     check_launch(split_name);
     if (splits <= kItemCombineMaxSplits)
         hipLaunchKernelGGL(attn_mfma_combine_items_kernel, dim3(heads), dim3(256), 0, stream,
@@ -2924,6 +2926,53 @@ void launch_generic_attention(Scheme s, const uint16_t* query, const uint8_t* po
                                           stream, ws, output, g, rows, sp.splits, inv));
     check_launch((std::string(name) + "_combine").c_str());
 }
+
+// A paged step on the matrix cores (head_dim 64, 128): the plan, one split
+// workgroup per work segment, and a merge per row group and kv head.
+template <int SCH, int D>
+void launch_paged_units(const uint16_t* query, const uint8_t* pool, const int32_t* block_tables,
+                        int max_blocks, const int32_t* row_seq, const int32_t* row_kv_len,
+                        uint16_t* output, const PageGeom& g, int num_rows, int max_kv_len,
+                        uint64_t extent, hipStream_t stream) {
+    using namespace mfma;
+    constexpr bool prod = SCH == kSchProd;
+    const int row_groups = (num_rows + kRows - 1) / kRows;
+    const int heads = g.H * row_groups;
+    // The plan gives every kv head the same work (each unit's passes over
+    // its kv length), split into Gh equal segments per head, one workgroup
+    // each: G = H * Gh workgroups, Gh a multiple of 8 (the kernel's XCD
+    // mapping).
+    const int Gh = 8 * ((kPagedSegmentsPerCU * num_cus() + 8 * g.H - 1) / (8 * g.H));
+    const int G = Gh * g.H;
+    // Workspace: the partials (slot (unit + segment) * H + head: fewer than
+    // (row_groups + Gh) * H = heads + G slots of kNP positions), then the
+    // plan: the units and a sentinel, each row group's unit, the unit count
+    // and total work.
+    const size_t part_bytes =
+        ((size_t)heads + G) * unit::kNP * kRows * unit::part_stride(D) * sizeof(float);
+    const size_t unit_bytes = (2 * (size_t)row_groups + 1) * sizeof(PagedUnit);
+    const size_t spare_at = (part_bytes + unit_bytes + 4 * sizeof(int32_t) + 255) & ~(size_t)255;
+    char* wsb = static_cast<char*>(workspace(stream, spare_at + extent));
+    float* ws = reinterpret_cast<float*>(wsb);
+    PagedUnit* units = reinterpret_cast<PagedUnit*>(wsb + part_bytes);
+    PagedUnit* group_unit = units + row_groups + 1;
+    int32_t* plan = reinterpret_cast<int32_t*>(wsb + part_bytes + unit_bytes);
+    const PagedRows pr{block_tables, row_seq,    row_kv_len, max_blocks, units, group_unit, plan,
+                       reinterpret_cast<const uint8_t*>(wsb + spare_at)};
+    hipLaunchKernelGGL(paged_plan_kernel<unit::kNP>, dim3(1), dim3(1024), 0, stream, row_seq,
+                       row_kv_len, num_rows, row_groups, unit::kPass, max_kv_len, units,
+                       group_unit, plan);
+    check_launch(prod ? "turbo_prod_paged_attn_plan" : "turbo_mse_paged_attn_plan");
+    if (max_kv_len > 0) {
+        hipLaunchKernelGGL((unit::attn_unit_split_kernel<SCH, D, true>), dim3(G),
+                           dim3(64 * unit::kWaves), 0, stream, query, pool, nullptr, ws, nullptr,
+                           inv_sqrt_d(D), num_rows, max_kv_len, 0, 0, g, pr);
+        check_launch(prod ? "turbo_prod_paged_attn_split" : "turbo_mse_paged_attn_split");
+    }
+    hipLaunchKernelGGL(attn_paged_combine_kernel<D>, dim3(heads), dim3(2 * D), 0, stream, ws,
+                       output, g.H, num_rows, Gh, pr);
+    check_launch(prod ? "turbo_prod_paged_attn_combine" : "turbo_mse_paged_attn_combine");
+}
 }  // namespace
 
 void launch_attention(Scheme s, const uint16_t* query, const uint8_t* pool, const int32_t* slots,
@@ -2984,9 +3033,19 @@ void launch_paged_attention(Scheme s, const uint16_t* query, const uint8_t* pool
     const uint64_t extent =
         std::max({g.page_size, std::max({g.ks_off, g.vs_off, g.kres_off}) + cells * g.scale_stride,
                   std::max(g.kc_off, g.vc_off) + cells * g.code_stride});
-    if (!mfma_attention_ok(g, pool) || extent > 0xFFFFFFFFu) {
-        // Other head_dims and unaligned pages: the generic split-K decode, its
-        // rows reading their tokens through the block table.
+    // The plan counts each kv head's work in int32: at most
+    // 4 * ceil(max_kv_len / kPass) + kPieceCost per row group (every head has
+    // the same).
+    const int row_groups = (num_rows + mfma::kRows - 1) / mfma::kRows;
+    const bool countable =
+        (long long)row_groups *
+            (4LL * ((std::max(max_kv_len, 0) + unit::kPass - 1) / unit::kPass) + kPieceCost) <=
+        INT32_MAX;
+    const bool d64 = mfma_attention64_ok(g, pool) && countable;
+    if (!(d64 || mfma_attention_ok(g, pool)) || extent > 0xFFFFFFFFu) {
+        // Other head_dims and unaligned pages (and head_dim 64 past the plan's
+        // count): the generic split-K decode, its rows reading their tokens
+        // through the block table.
         const GenericSplit sp = generic_split(rows, std::max(max_kv_len, 0), g.D);
         float* ws = static_cast<float*>(workspace(stream, sp.ws_bytes));
         launch_generic_attention(
@@ -2996,58 +3055,23 @@ void launch_paged_attention(Scheme s, const uint16_t* query, const uint8_t* pool
             prod ? "turbo_prod_paged_attn" : "turbo_mse_paged_attn");
         return;
     }
+    if (!countable) throw Error("paged attention: too many rows for this max_kv_len");
     using namespace mfma;
-    const float inv = inv_sqrt_d(g.D);
-    const int row_groups = (num_rows + kRows - 1) / kRows;
-    const int heads = g.H * row_groups;
-    // The plan gives every kv head the same work (each unit's passes over
-    // its kv length), split into Gh equal segments per head, one workgroup
-    // each: G = H * Gh workgroups, Gh a multiple of 8 (the kernel's XCD
-    // mapping).
-    constexpr int kPass = kSplitChunk * kSplitWaves;
-    const int Gh = 8 * ((kPagedSegmentsPerCU * num_cus() + 8 * g.H - 1) / (8 * g.H));
-    const int G = Gh * g.H;
-    // The plan counts each kv head's work in int32: at most
-    // 4 * ceil(max_kv_len / kPass) + kPieceCost per row group (every head has
-    // the same).
-    if ((long long)row_groups *
-            (4LL * ((std::max(max_kv_len, 0) + kPass - 1) / kPass) + kPieceCost) >
-        INT32_MAX)
-        throw Error("paged attention: too many rows for this max_kv_len");
-    // Workspace: the partials (slot (unit + segment) * H + head: fewer than
-    // (row_groups + Gh) * H = heads + G slots of kPagedPositions positions),
-    // then the plan: the units and a
-    // sentinel, each row group's unit, the unit count and total work.
-    const size_t part_bytes =
-        ((size_t)heads + G) * kPagedPositions * kRows * kPartStride * sizeof(float);
-    const size_t unit_bytes = (2 * (size_t)row_groups + 1) * sizeof(PagedUnit);
-    const size_t spare_at = (part_bytes + unit_bytes + 4 * sizeof(int32_t) + 255) & ~(size_t)255;
-    char* wsb = static_cast<char*>(workspace(stream, spare_at + extent));
-    float* ws = reinterpret_cast<float*>(wsb);
-    PagedUnit* units = reinterpret_cast<PagedUnit*>(wsb + part_bytes);
-    PagedUnit* group_unit = units + row_groups + 1;
-    int32_t* plan = reinterpret_cast<int32_t*>(wsb + part_bytes + unit_bytes);
-    const PagedRows pr{block_tables, row_seq,    row_kv_len, max_blocks, units, group_unit, plan,
-                       reinterpret_cast<const uint8_t*>(wsb + spare_at)};
-    constexpr int kCH = kSplitChunk, kNW = kSplitWaves;
-    hipLaunchKernelGGL(paged_plan_kernel<kPagedPositions>, dim3(1), dim3(1024), 0, stream, row_seq,
-                       row_kv_len, num_rows, row_groups, kPass, std::max(max_kv_len, 0), units,
-                       group_unit, plan);
-    check_launch(prod ? "turbo_prod_paged_attn_plan" : "turbo_mse_paged_attn_plan");
-    if (max_kv_len > 0) {
-        if (prod)
-            hipLaunchKernelGGL((attn_mfma_split_kernel<kSchProd, kCH, kNW, true, kPagedPositions>),
-                               dim3(G), dim3(64 * kNW), 0, stream, query, pool, nullptr, ws, inv,
-                               num_rows, max_kv_len, 0, 0, g, pr);
+    const auto go = [&](auto sch, auto dim) {
+        launch_paged_units<decltype(sch)::value, decltype(dim)::value>(
+            query, pool, block_tables, max_blocks, row_seq, row_kv_len, output, g, num_rows,
+            std::max(max_kv_len, 0), extent, stream);
+    };
+    const auto by_dim = [&](auto sch) {
+        if (d64)
+            go(sch, std::integral_constant<int, 64>{});
         else
-            hipLaunchKernelGGL((attn_mfma_split_kernel<kSchMse, kCH, kNW, true, kPagedPositions>),
-                               dim3(G), dim3(64 * kNW), 0, stream, query, pool, nullptr, ws, inv,
-                               num_rows, max_kv_len, 0, 0, g, pr);
-        check_launch(prod ? "turbo_prod_paged_attn_split" : "turbo_mse_paged_attn_split");
-    }
-    hipLaunchKernelGGL(attn_paged_combine_kernel, dim3(heads), dim3(256), 0, stream, ws, output,
-                       g.H, num_rows, Gh, kPagedPositions, kPass, pr);
-    check_launch(prod ? "turbo_prod_paged_attn_combine" : "turbo_mse_paged_attn_combine");
+            go(sch, std::integral_constant<int, 128>{});
+    };
+    if (prod)
+        by_dim(std::integral_constant<int, kSchProd>{});
+    else
+        by_dim(std::integral_constant<int, kSchMse>{});
 }
 
 bool launch_qjl_mfma_attention(const uint16_t* query, const uint8_t* pool, const int32_t* slots,
@@ -3071,9 +3095,8 @@ bool launch_qjl_mfma_attention(const uint16_t* query, const uint8_t* pool, const
     g.block_size = q.block_size;
     g.bs_shift = (q.block_size & (q.block_size - 1)) == 0 ? __builtin_ctz(q.block_size) : -1;
     g.h_shift = (q.H & (q.H - 1)) == 0 ? __builtin_ctz(q.H) : -1;
-    launch_mfma_attention<mfma::kSchQjl>(query, pool, slots, output, g, num_queries,
-                                         num_kv_tokens, inv_sqrt_d(q.D), stream,
-                                         "qjl_fused_attn_split", "qjl_fused_attn_combine");
+    launch_qjl_mfma(query, pool, slots, output, g, num_queries, num_kv_tokens, inv_sqrt_d(q.D),
+                    stream);
     return true;
 }
 
