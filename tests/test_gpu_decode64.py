@@ -48,7 +48,8 @@ def _check(tq, oracle, cuda, scheme, q, k, v, slots, all_slots):
 
 @pytest.mark.parametrize("scheme", ["turbo_prod", "turbo_mse"])
 @pytest.mark.parametrize("Q,H,N", [(1, 1, 1), (1, 2, 31), (7, 2, 32), (8, 3, 33), (9, 2, 256),
-                                   (17, 1, 257), (7, 2, 6001), (8, 8, 2049)])
+                                   (17, 1, 257), (7, 2, 6001), (8, 8, 2049),
+                                   (16, 128, 1500)])  # logits up to ~60: K's lo parts matter
 def test_edges(tq, oracle, cuda, scheme, Q, H, N):
     print(f"[decode64 {scheme}] Q={Q} H={H} N={N}", flush=True)
     k, v = kv_tokens_major(N, H, D, seed=N)

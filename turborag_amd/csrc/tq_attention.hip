@@ -381,13 +381,17 @@ constexpr uint32_t f16_pair(float a, float b) {
 constexpr float lo_part_c(float x) { return (x - (float)(_Float16)x) * (float)(1 << kLoShift); }
 
 // fp16 bits of the codebook values the decode tables hold: aK*K3[j],
-// aV*V4[j], and the lo parts (x - fp16(x)) * 2^kLoShift of aV*V4[j].
+// aV*V4[j], the lo parts (x - fp16(x)) * 2^kLoShift of aV*V4[j], and those of
+// aK*K3[j] unscaled (fp16 subnormals, whose step is 1e-7 of a level).
 struct Fp16Tables {
-    uint32_t k3[8], v4[16], v4lo[16];
+    uint32_t k3[8], k3lo[8], v4[16], v4lo[16];
 };
 constexpr Fp16Tables make_fp16_tables() {
     Fp16Tables t{};
-    for (int j = 0; j < 8; ++j) t.k3[j] = f16_bits(kAlphaK * dev::kK3[j]);
+    for (int j = 0; j < 8; ++j) {
+        t.k3[j] = f16_bits(kAlphaK * dev::kK3[j]);
+        t.k3lo[j] = f16_bits(kAlphaK * dev::kK3[j] - (float)(_Float16)(kAlphaK * dev::kK3[j]));
+    }
     for (int j = 0; j < 16; ++j) {
         t.v4[j] = f16_bits(kAlphaV * dev::kV4[j]);
         t.v4lo[j] = f16_bits(lo_part_c(kAlphaV * dev::kV4[j]));
@@ -417,8 +421,8 @@ __device__ __forceinline__ uint32_t lut4(const uint32_t (&t)[N], int m, uint32_t
 //   K: turbo_prod (aK*K3[b & 7], aK*K3[(b >> 4) & 7]); turbo_mse the hi
 //      parts fp16(aV*V4[b & 15]), fp16(aV*V4[b >> 4]) (its V lookups read them
 //      too);
-//   S: turbo_prod the residual signs (nibble bit 3 set: +1.0, else -1.0);
-//      turbo_mse the lo parts of aV*V4;
+//   S: turbo_prod the residual signs (nibble bit 3 set: +1.0, else -1.0), or
+//      with KLO the lo parts of aK*K3; turbo_mse the lo parts of aV*V4;
 //   V (turbo_prod): (aV*V4[b & 15], aV*V4[b >> 4]).
 // Wave w of 8 writes rows 32w .. 32w + 31 of each table from registers (no
 // memory traffic): with those rows one nibble of every entry is uniform
@@ -447,7 +451,7 @@ __device__ __forceinline__ void lo_table_words(int w, int lane, uint32_t (&r)[4]
 #pragma unroll
     for (int k = 0; k < 4; ++k) r[k] = llo[k & 1] | (kF16.v4lo[2 * w + (k >> 1)] << 16);
 }
-template <bool PROD>
+template <bool PROD, bool KLO = false>
 __device__ __forceinline__ TableWords<PROD> decode_table_words(int w, int lane) {
     TableWords<PROD> tw;
     uint32_t(&r0)[4] = tw.r0;
@@ -457,9 +461,15 @@ __device__ __forceinline__ TableWords<PROD> decode_table_words(int w, int lane) 
         const uint32_t sel4 = lut4_sel(g4), sel8 = lut4_sel(g8 & 3);
         const bool hi8 = (g8 & 4) != 0;
         if constexpr (PROD) {
-            const uint32_t sh = (w & 4) ? 0x3C000000u : 0xBC000000u;  // row bit 7 = w bit 2
+            if constexpr (KLO) {
+                const uint32_t lo = hi8 ? lut4(kF16.k3lo, 1, sel8) : lut4(kF16.k3lo, 0, sel8);
 #pragma unroll
-            for (int k = 0; k < 4; ++k) r0[k] = ((k & 1) ? 0x3C00u : 0xBC00u) | sh;  // row bit 3
+                for (int k = 0; k < 4; ++k) r0[k] = lo | (kF16.k3lo[(2 * w + (k >> 1)) & 7] << 16);
+            } else {
+                const uint32_t sh = (w & 4) ? 0x3C000000u : 0xBC000000u;  // row bit 7 = w bit 2
+#pragma unroll
+                for (int k = 0; k < 4; ++k) r0[k] = ((k & 1) ? 0x3C00u : 0xBC00u) | sh;  // row bit 3
+            }
             const bool vq = (lane & 8) != 0;
 #pragma unroll
             for (int k = 0; k < 8; ++k) {
@@ -480,6 +490,14 @@ __device__ __forceinline__ TableWords<PROD> decode_table_words(int w, int lane) 
         }
     }
     return tw;
+}
+// The residual signs of a turbo_prod code dword's 8 nibbles (bit 3 set: +1.0,
+// else -1.0) as fp16, in registers.
+__device__ __forceinline__ half8 sign_octet(uint32_t wd) {
+    const uint32_t he = ((wd << 4) & 0x80808080u) ^ 0xBCBCBCBCu;  // even dims' high bytes
+    const uint32_t ho = (wd & 0x80808080u) ^ 0xBCBCBCBCu;         // odd dims'
+    return as_h8(__builtin_amdgcn_perm(ho, he, 0x040C000Cu), __builtin_amdgcn_perm(ho, he, 0x050C010Cu),
+                 __builtin_amdgcn_perm(ho, he, 0x060C020Cu), __builtin_amdgcn_perm(ho, he, 0x070C030Cu));
 }
 // Exponent e with x * 2^-e in [0.5, 1); 0 for a zero or non-finite x.
 __device__ __forceinline__ int scale_exp(float x) {
@@ -1062,8 +1080,9 @@ __global__ __launch_bounds__(64 * kWaves) void attn_qjl_split_kernel(
 // Eight waves of 32-token chunks per workgroup, one workgroup per CU (the
 // decode tables).  PAGED: the grid is one workgroup per work segment of the
 // step's plan (paged_plan_kernel).  Slot-mapped: grid (split, kv head, unit).
-// D = 64: half the k-steps and PV tiles per token, V's fp16 lo parts and a
-// power of two per query row, as dec::attn_decode_split_kernel.
+// D = 64: half the k-steps and PV tiles per token, the fp16 lo parts of V and
+// turbo_prod's K and a power of two per query row, as
+// dec::attn_decode_split_kernel.
 // Issue-bound at many passes per workgroup (D = 128, 32 sequences of 1K-32K
 // tokens: 94 us), bound by the setup and the merge at few.  A D = 64 step of
 // 8 sequences (500-4,000 tokens, 2 new tokens, 2 heads) with its append takes
@@ -1105,7 +1124,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
     constexpr int kS = D / 32;   // QK k-steps; lane group gq holds dims [D/4 gq, D/4 gq + D/4)
     constexpr int kND = D / 16;  // PV tiles: lane i holds dims kND i .. + kND - 1
     constexpr int kL = D / 2;    // lanes of a row held two values per lane
-    constexpr bool VLO = D == 64, QSCALE = D == 64;
+    constexpr bool VLO = D == 64, QSCALE = D == 64, KLO = D == 64 && PROD;
     static_assert(kNT * sizeof(float) * kWaves * kMoRows * D <= 4 * kTabWords, "merge spaces");
     __shared__ __attribute__((aligned(256))) uint32_t lut[kTabWords];
     __shared__ uint4 bqs[kNP][kS][64];  // QK B operand (fp16 hi/lo q) of k-step s for lane l
@@ -1320,7 +1339,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         // in operand 2(k / 2), lo in 2(k / 2) + 1; one position: tile 0, hi in
         // column w, lo in column w + 8.
         {
-            const TableWords<PROD> tw = decode_table_words<PROD>(w, lane);
+            const TableWords<PROD> tw = decode_table_words<PROD, KLO>(w, lane);
             const int s_l = (jl >> 2) & (kS - 1), g_l = jl / (4 * kS);
 #pragma unroll
             for (int k = 0; k < kNP; ++k) {
@@ -1475,12 +1494,19 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                         // prod: the +-1 residual signs against the hi and lo query;
                         // mse: the codebook's lo parts (into cs) against the hi query
                         // only: the product of the two lo parts, each below 2^-11
-                        // of its value, is ~2^-22 of the logit
+                        // of its value, is ~2^-22 of the logit (KLO: so K's lo parts,
+                        // into cb)
+                        half8 sg = o.al[tau];
+                        if constexpr (KLO) {
+#pragma unroll
+                            for (int t = 0; t < NTA; ++t)
+                                cb[t][tau] = mma(o.al[tau], o.bk[2 * t], cb[t][tau]);
+                            sg = sign_octet(cur.kw[tau][s]);
+                        }
 #pragma unroll
                         for (int t = 0; t < NTA; ++t) {
-                            cs[t][tau] = mma(o.al[tau], o.bk[2 * t], cs[t][tau]);
-                            if (!COLS && PROD)
-                                cs[t][tau] = mma(o.al[tau], o.bk[2 * t + 1], cs[t][tau]);
+                            cs[t][tau] = mma(sg, o.bk[2 * t], cs[t][tau]);
+                            if (!COLS && PROD) cs[t][tau] = mma(sg, o.bk[2 * t + 1], cs[t][tau]);
                         }
                     }
                     __builtin_amdgcn_sched_barrier(0);
@@ -2286,11 +2312,14 @@ constexpr size_t part_bytes(int D) { return kRows * (D + 2) * sizeof(float); }
 
 // D = 128, or D = 64: half the dims per token (two QK k-steps instead of
 // four, four PV tiles instead of eight), 8-byte K and 2-byte V loads per
-// lane.  D = 64 also carries what keeps it as exact as fp32 arithmetic: V's
-// fp16 lo parts (a second PV product in its own accumulators; the table's
-// hi parts alone are 5e-5 off in the mean, a quarter of the output's own
-// fp16 rounding), and a power of two per query row that holds the row's fp16
-// parts in range whatever its magnitude.  Bound by its dependent loads and
+// lane.  D = 64 also carries what keeps it as exact as fp32 arithmetic: the
+// fp16 lo parts of V (a second PV product in its own accumulators; the
+// table's hi parts alone are 5e-5 off in the mean, a quarter of the output's
+// own fp16 rounding) and of turbo_prod's K (in the S table, a third QK
+// product; the signs are built in registers: logits of magnitude 60, outlier
+// channels shared by q and k, are 6e-4 off without it), and a power of two
+// per query row that holds the row's fp16 parts in range whatever its
+// magnitude.  Bound by its dependent loads and
 // the setup, as D = 128: 7 rows x 2 heads x 6,001 tokens (turbo_mse) take 6.0
 // (split) + 2.9 us (combine); the generic one-wave-per-row kernels, whose
 // cross-lane sum per token and serial merge over 147 splits this replaces,
@@ -2307,7 +2336,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     constexpr int kS = D / 32;       // QK k-steps; lane group gq holds dims [D/4 gq, D/4 gq + D/4)
     constexpr int kNT = D / 16;      // PV tiles: lane i holds dims kNT i .. + kNT - 1
     constexpr int kL = D / 2;        // lanes of a row held two values per lane
-    constexpr bool VLO = D == 64, QSCALE = D == 64;
+    constexpr bool VLO = D == 64, QSCALE = D == 64, KLO = D == 64 && PROD;
     // The decode tables (layout above); after the chunk loop the space holds
     // the waves' results for the merge.
     __shared__ __attribute__((aligned(256))) uint32_t lut[kLutWords];
@@ -2403,7 +2432,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
 
     // The tables' words, computed in registers while the codes are in flight
     // (no memory traffic; each 16-byte store writes four copies).
-    const TableWords<PROD> tw = decode_table_words<PROD>(w, lane);
+    const TableWords<PROD> tw = decode_table_words<PROD, KLO>(w, lane);
     uint32_t vlo[4];
     if constexpr (VLO && PROD) lo_table_words(w, lane, vlo);
     // 3. This wave's query row: qrot = WHT(q * s) * inv, stored as fp16 hi
@@ -2524,7 +2553,12 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
 #pragma unroll
             for (int s = 0; s < kS; ++s) {
                 cb[tau] = mma(ka[tau][s], bq[s], cb[tau]);
-                cs[tau] = mma(kb[tau][s], bq[s], cs[tau]);  // prod: residual signs; mse: lo parts
+                if constexpr (KLO) {
+                    cb[tau] = mma(kb[tau][s], bq[s], cb[tau]);
+                    cs[tau] = mma(sign_octet(cur.kw[tau][s]), bq[s], cs[tau]);
+                } else {
+                    cs[tau] = mma(kb[tau][s], bq[s], cs[tau]);  // prod: residual signs; mse: lo parts
+                }
             }
         }
         // V lookups (B operands of PV), in flight during the softmax.
