@@ -2713,13 +2713,15 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
 
 // Sum of the split partials of one output row (q, h): o = sum_s 2^(m_s - M)
 // o_s / sum_s 2^(m_s - M) l_s.  One wave per (row, 8-element slice of d):
-// lane = 8 split groups x 8 elements; group j takes splits j, j + 8, ..., 16
+// lane = 8 split groups x 8 elements; group j takes splits j, j + 8, ..., kB
 // at a time (every load of a batch in flight together), merges them with a
 // running maximum, then the groups are merged across lanes (no LDS, no
-// barrier).  The 4 slices of one 128-byte line of the partials run on one
+// barrier).  kB is the smallest of 2, 4 and 16 that takes S splits in one
+// batch: loads past S re-read a split, so a batch of 16 at few splits is
+// mostly repeats.  The 4 slices of one 128-byte line of the partials run on one
 // XCD (block b on XCD b % 8), so three of them find the line in that XCD's
 // L2.
-template <int D>
+template <int D, int kB>
 __global__ __launch_bounds__(64) void attn_decode_combine_kernel(
     const float* __restrict__ po, const float2* __restrict__ pml, uint16_t* __restrict__ output,
     int H, int rows, int S) {
@@ -2737,7 +2739,6 @@ __global__ __launch_bounds__(64) void attn_decode_combine_kernel(
     const size_t item = (size_t)rg * H + h;
     const float2* mlr = pml + (item * kRows + r) * S;
     const float* orow = po + (item * S * kRows + r) * D + d;  // split s: + s * kRows * D
-    constexpr int kB = 16;
     float M = kInitMax, L = 0.f, A = 0.f;
     for (int base = grp; base < S; base += 8 * kB) {
         float pm[kB], pl[kB], pv[kB];
@@ -2868,29 +2869,79 @@ void launch_qjl_mfma(const uint16_t* query, const uint8_t* pool, const int32_t* 
     check_launch(combine_name);
 }
 
-// The slot-mapped decode (turbo_prod, turbo_mse; D = 64, 128): split + combine.
+// The slot-mapped decode (turbo_prod, turbo_mse; D = 64, 128): split + combine,
+// with one row group per workgroup (dec::) or units of up to four that share
+// the decoded chunks (unit::).
 struct DecodeSplit {
-    int rows, row_groups, heads, splits, tps;
+    int rows, row_groups, heads, items, splits, tps;
+    bool units;
     long long combine_blocks;
-    size_t blocks, ws_bytes;
+    size_t blocks, ws_bytes, limit_bytes;  // limit_bytes: what a fixed scratch is held to
 };
-DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens) {
+// Cost of a split kernel's workgroup: a setup and merge, and a pass of 256
+// tokens, in 0.1 us (measured at D = 128, turbo_prod, 2 heads, 250 to 32,768
+// tokens, kernel trace: one group 5.9 us at one pass, 10.4 at two, 14.8 at
+// four, 22.5 at eight; a unit of two groups 8.3 at one, of four 12.0 at one,
+// 16.0 at two, 32.5 at seven).
+struct SplitCost {
+    int setup, pass;
+};
+constexpr SplitCost kGroupCost{51, 20}, kPairCost{70, 20}, kUnitCost{90, 33};
+// The split count and its cost: one workgroup runs on a CU at a time, so of
+// the counts that fill one to four rounds of the CUs the cheapest is taken
+// (the fewest splits among equals: the merge reads every split's partials).
+struct SplitChoice {
+    int splits;
+    long long cost;
+};
+SplitChoice choose_splits(int items, int passes, SplitCost c, int most) {
+    const int cus = num_cus();
+    SplitChoice best{1, -1};
+    for (int r = 1; r <= 4; ++r) {
+        int s = std::min({std::max(1, (int)((long long)r * cus / items)), passes, most});
+        const int per = (passes + s - 1) / s;
+        s = (passes + per - 1) / per;
+        const long long rounds = ((long long)items * s + cus - 1) / cus;
+        const long long cost = rounds * (c.setup + (long long)c.pass * per);
+        if (best.cost < 0 || cost < best.cost || (cost == best.cost && s < best.splits))
+            best = {s, cost};
+    }
+    return best;
+}
+// cap: a fixed scratch's bytes, or 0.
+DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens, size_t cap) {
     using namespace mfma;
     DecodeSplit d{};
     d.rows = num_queries * g.H;
     d.row_groups = (num_queries + kRows - 1) / kRows;
     d.heads = g.H * d.row_groups;
-    // One 256-token split per workgroup, or longer splits once there are
-    // more than ~2 workgroups per CU.
-    const int max_splits = std::max(1, (num_kv_tokens + kSplitMinTokens - 1) / kSplitMinTokens);
-    const int want = std::max(1, (kSplitBlocksPerCU * num_cus() + d.heads - 1) / d.heads);
-    d.splits = std::min(std::min(max_splits, want), 1024);
-    d.tps = num_kv_tokens > 0 ? (num_kv_tokens + d.splits - 1) / d.splits : 0;
-    if (d.tps > 0) d.splits = (num_kv_tokens + d.tps - 1) / d.tps;
     // The combine: 32 blocks per 8 (row, 128-byte line) pairs.
     d.combine_blocks = ((long long)d.rows * (g.D / 32) + 7) / 8 * 32;
-    d.blocks = (size_t)d.splits * d.heads;
-    d.ws_bytes = d.blocks * dec::part_bytes(g.D);
+    const size_t per_split = (size_t)d.heads * dec::part_bytes(g.D);
+    const int passes = std::max(1, (num_kv_tokens + kSplitMinTokens - 1) / kSplitMinTokens);
+    if (cap) {
+        // The partials a fixed scratch has to hold for a call to be taken: one
+        // 256-token split per workgroup, or longer splits once there are more
+        // than ~2 workgroups per CU and row group.  The launch itself takes no
+        // more splits than fit.
+        const int want = std::max(1, (kSplitBlocksPerCU * num_cus() + d.heads - 1) / d.heads);
+        int splits = std::min(std::min(passes, want), 1024);
+        const int tps = num_kv_tokens > 0 ? (num_kv_tokens + splits - 1) / splits : 0;
+        if (tps > 0) splits = (num_kv_tokens + tps - 1) / tps;
+        d.limit_bytes = splits * per_split;
+    }
+    const int most = cap ? (int)std::min<size_t>(1024, std::max<size_t>(1, cap / per_split)) : 1024;
+    const int units = g.H * ((d.row_groups + unit::kNP - 1) / unit::kNP);
+    const SplitChoice one = choose_splits(d.heads, passes, kGroupCost, most);
+    const SplitChoice un =
+        choose_splits(units, passes, d.row_groups == 2 ? kPairCost : kUnitCost, most);
+    d.units = d.row_groups > 1 && un.cost < one.cost;
+    d.items = d.units ? units : d.heads;
+    d.splits = d.units ? un.splits : one.splits;
+    d.tps = num_kv_tokens > 0 ? (num_kv_tokens + d.splits - 1) / d.splits : 0;
+    if (d.tps > 0) d.splits = (num_kv_tokens + d.tps - 1) / d.tps;
+    d.blocks = (size_t)d.splits * d.items;
+    d.ws_bytes = d.splits * per_split;
     return d;
 }
 template <int SCH, int D>
@@ -2902,23 +2953,37 @@ void launch_decode_attention(const uint16_t* query, const uint8_t* pool, const i
     using namespace mfma;
     if (d.combine_blocks > INT32_MAX)
         throw Error(std::string(combine_name) + ": too many query rows");
+    if (scratch.ptr) (void)scratch.get(stream, d.limit_bytes, split_name);  // throws past its limit
     char* ws = static_cast<char*>(scratch.get(stream, d.ws_bytes, split_name));
     float* po = reinterpret_cast<float*>(ws);
-    float2* pml = reinterpret_cast<float2*>(ws + d.blocks * kRows * D * sizeof(float));
+    float2* pml = reinterpret_cast<float2*>(ws + (size_t)d.splits * d.heads * kRows * D * sizeof(float));
+    const int S = num_kv_tokens > 0 ? d.splits : 0;
     if (num_kv_tokens > 0) {
         constexpr int kMaxGridYZ = 65535;
-        const dim3 grid = d.row_groups <= kMaxGridYZ && g.H <= kMaxGridYZ
-                              ? dim3(d.splits, g.H, d.row_groups)
-                              : dim3((unsigned)d.blocks);
-        hipLaunchKernelGGL((dec::attn_decode_split_kernel<SCH, D>), grid, dim3(64 * dec::kWaves),
-                           0, stream, query, pool, slots, po, pml, inv, num_queries,
-                           num_kv_tokens, d.tps, d.splits, g);
+        const int groups = d.items / g.H;  // row groups, or units of them
+        const dim3 grid = groups <= kMaxGridYZ && g.H <= kMaxGridYZ ? dim3(d.splits, g.H, groups)
+                                                                    : dim3((unsigned)d.blocks);
+        if (d.units)
+            hipLaunchKernelGGL((unit::attn_unit_split_kernel<SCH, D, false>), grid,
+                               dim3(64 * unit::kWaves), 0, stream, query, pool, slots, po, pml,
+                               inv, num_queries, num_kv_tokens, d.tps, d.splits, g, PagedRows{});
+        else
+            hipLaunchKernelGGL((dec::attn_decode_split_kernel<SCH, D>), grid,
+                               dim3(64 * dec::kWaves), 0, stream, query, pool, slots, po, pml, inv,
+                               num_queries, num_kv_tokens, d.tps, d.splits, g);
         check_launch(split_name);
     }
     // (no partials for an empty context: the combine writes zeros)
-    hipLaunchKernelGGL(dec::attn_decode_combine_kernel<D>, dim3((unsigned)d.combine_blocks),
-                       dim3(64), 0, stream, po, pml, output, g.H, d.rows,
-                       num_kv_tokens > 0 ? d.splits : 0);
+    const dim3 cgrid((unsigned)d.combine_blocks);
+    if (S <= 16)
+        hipLaunchKernelGGL((dec::attn_decode_combine_kernel<D, 2>), cgrid, dim3(64), 0, stream, po,
+                           pml, output, g.H, d.rows, S);
+    else if (S <= 32)
+        hipLaunchKernelGGL((dec::attn_decode_combine_kernel<D, 4>), cgrid, dim3(64), 0, stream, po,
+                           pml, output, g.H, d.rows, S);
+    else
+        hipLaunchKernelGGL((dec::attn_decode_combine_kernel<D, 16>), cgrid, dim3(64), 0, stream, po,
+                           pml, output, g.H, d.rows, S);
     check_launch(combine_name);
 }
 
@@ -3021,7 +3086,8 @@ void launch_attention(Scheme s, const uint16_t* query, const uint8_t* pool, cons
         prod ? "turbo_prod_fused_attn_combine" : "turbo_mse_fused_attn_combine";
     const bool d64 = mfma_attention64_ok(g, pool);
     if (d64 || mfma_attention_ok(g, pool)) {
-        const DecodeSplit d = decode_split(g, num_queries, num_kv_tokens);
+        const DecodeSplit d =
+            decode_split(g, num_queries, num_kv_tokens, scratch.ptr ? scratch.cap : 0);
         // head_dim 64: where a caller's scratch is too small for the padded
         // row groups' partials, or there are too many rows for the combine's
         // grid, the generic decode below takes the call if it can.
