@@ -1112,6 +1112,68 @@ static_assert(256 * 255 + 128 + 4 * kLoCopies <= kOffKV, "the V lo rows end belo
 static_assert(kRows % kWaves == 0 && kWaves == 8, "eight waves, one row per wave and position");
 constexpr int part_stride(int D) { return D + 4; }  // paged partial row: o[D], m, l, pad
 
+// A query or output row held by 16 lanes, so that a wave works on its row of
+// all four positions at once instead of one after another.  Lane p owns elements 4j .. 4j + 3
+// of the 64-element blocks, j = logical(p): in this order j ^ 1, j ^ 2, j ^ 4 and
+// j ^ 8 are quad permutes, the half-row mirror and a row rotation, one DPP
+// operand each: setup and merge of a unit of four, 2 passes, 16.0 -> 14.4 us;
+// a step of 32 sequences (1.34 pieces per workgroup) 98.5 -> 96.0 us.
+__device__ __forceinline__ int logical(int p) { return (p & 4) ? p ^ 3 : p; }
+template <int M>
+__device__ __forceinline__ float partner(float v) {  // v of logical lane j ^ M
+    constexpr int ctrl = M == 1 ? 0xB1 : M == 2 ? 0x4E : M == 4 ? 0x141 : 0x128;
+    static_assert(M == 1 || M == 2 || M == 4 || M == 8, "16 lanes");
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xF, 0xF, true));
+}
+// y[k] += c * (partner's y[k]) for 4 values (v_fmac_f32_dpp; the s_nop gives the
+// two wait states a DPP read needs after the VALU write of its source).
+#define TQ_FMAC4(CTRL)                                                          \
+    asm("s_nop 1\n\t"                                                           \
+        "v_fmac_f32_dpp %0, %0, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\t"     \
+        "v_fmac_f32_dpp %1, %1, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\t"     \
+        "v_fmac_f32_dpp %2, %2, %4 " CTRL " row_mask:0xf bank_mask:0xf\n\t"     \
+        "v_fmac_f32_dpp %3, %3, %4 " CTRL " row_mask:0xf bank_mask:0xf"         \
+        : "+v"(y[k]), "+v"(y[k + 1]), "+v"(y[k + 2]), "+v"(y[k + 3])            \
+        : "v"(c))
+template <int M, int E>
+__device__ __forceinline__ void wht_across(float (&y)[E], int j) {
+    const float c = (j & M) ? -1.0f : 1.0f;
+#pragma unroll
+    for (int k = 0; k < E; k += 4) {
+        if constexpr (M == 1)
+            TQ_FMAC4("quad_perm:[1,0,3,2]");
+        else if constexpr (M == 2)
+            TQ_FMAC4("quad_perm:[2,3,0,1]");
+        else if constexpr (M == 4)
+            TQ_FMAC4("row_half_mirror");
+        else
+            TQ_FMAC4("row_ror:8");
+    }
+}
+#undef TQ_FMAC4
+// Walsh-Hadamard transform of the row, left with a lane's sign
+// (-1)^popcount(j) (each lane adds +-1 times its partner's value; both lanes of
+// a pair carry the same sign).
+template <int E>
+__device__ __forceinline__ void wht_row16(float (&y)[E], int j) {
+#pragma unroll
+    for (int m = 1; m < E; m <<= 1)  // dims 1, 2 and (E = 8) 64
+#pragma unroll
+        for (int k = 0; k < E; ++k)
+            if (!(k & m)) {
+                const float a = y[k] + y[k + m], b = y[k] - y[k + m];
+                y[k] = a;
+                y[k + m] = b;
+            }
+    wht_across<1>(y, j);
+    wht_across<2>(y, j);
+    wht_across<4>(y, j);
+    wht_across<8>(y, j);
+}
+__device__ __forceinline__ float lane_sign(int j) {
+    return (__builtin_popcount(j & 15) & 1) ? -1.0f : 1.0f;
+}
+
 template <int SCH, int D, bool PAGED>
 __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
     const uint16_t* __restrict__ query, const uint8_t* __restrict__ pool,
@@ -1123,7 +1185,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
     static_assert(D == 128 || D == 64, "head_dim 64 or 128");
     constexpr int kS = D / 32;   // QK k-steps; lane group gq holds dims [D/4 gq, D/4 gq + D/4)
     constexpr int kND = D / 16;  // PV tiles: lane i holds dims kND i .. + kND - 1
-    constexpr int kL = D / 2;    // lanes of a row held two values per lane
+    constexpr int kE = D / 16;   // elements per lane of a row held by 16 lanes
     constexpr bool VLO = D == 64, QSCALE = D == 64, KLO = D == 64 && PROD;
     static_assert(kNT * sizeof(float) * kWaves * kMoRows * D <= 4 * kTabWords, "merge spaces");
     __shared__ __attribute__((aligned(256))) uint32_t lut[kTabWords];
@@ -1147,7 +1209,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         const int lane = tid & 63;
         const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar)
         const int i = lane & 15, gq = lane >> 4;
-        const int jl = lane & (kL - 1);  // this lane's pair of a row (D = 64: lanes l, l + 32 alike)
+        // Setup and merge: lane group gq holds the wave's row of position gq.
+        const int j16 = logical(i);
         // Paged rows: the unit's sequence and per-row kv lengths (causal limit).
         // A piece past every row's length has no partial (the combine does not
         // read it).  Per position: the group's longest row; per tile: this
@@ -1159,14 +1222,13 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         // issue them right after the row lengths and the sequence, so the
         // length processing waits only for those (the vector-memory counter is
         // in order) while the queries are in flight.
-        uint32_t qraw[kNP];
+        uint32_t qraw[kE / 2];
         auto load_queries = [&]() {
+            const int qi = min(rg * kRows + w + gq * kWaves, num_queries - 1);
+            const uint32_t* qp = reinterpret_cast<const uint32_t*>(
+                query + ((size_t)qi * g.H + h) * D + 4 * j16);
 #pragma unroll
-            for (int k = 0; k < kNP; ++k) {
-                const int qi = min(rg * kRows + w + k * kWaves, num_queries - 1);
-                qraw[k] = *reinterpret_cast<const uint32_t*>(query + ((size_t)qi * g.H + h) * D +
-                                                              2 * jl);
-            }
+            for (int k = 0; k < kE / 2; ++k) qraw[k] = qp[(k & 1) + 32 * (k >> 1)];
         };
         if constexpr (!PAGED) load_queries();
         if constexpr (PAGED) {
@@ -1185,14 +1247,18 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
             for (int p = 0; p < kNP; ++p) {
                 const int rr = (rg + p) * kRows + (lane & 7);
                 const int lv = p < npos && rr < num_queries ? lraw[p] : 0;
-                const int lc = __shfl(lv, i & 7);
+                // column i's row of position p is row i % 8 = lane % 8
                 // (one position: both halves of the tile hold its rows, hi and lo)
-                if (npos == 1 ? p == 0 : (i >> 3) == (p & 1)) rl_col[p >> 1] = lc;
-                int m = max(lv, __shfl_xor(lv, 1)), n = min(lv, __shfl_xor(lv, 1));
-                m = max(m, __shfl_xor(m, 2));
-                n = min(n, __shfl_xor(n, 2));
-                m = max(m, __shfl_xor(m, 4));
-                n = min(n, __shfl_xor(n, 4));
+                if (npos == 1 ? p == 0 : (i >> 3) == (p & 1)) rl_col[p >> 1] = lv;
+                // over the 8 rows: lane ^ 1, ^ 2, then 7 - lane of each 8
+                int m = lv, n = lv;
+                const auto over = [&](auto ctrl) {
+                    m = max(m, __builtin_amdgcn_mov_dpp(m, decltype(ctrl)::value, 0xF, 0xF, true));
+                    n = min(n, __builtin_amdgcn_mov_dpp(n, decltype(ctrl)::value, 0xF, 0xF, true));
+                };
+                over(std::integral_constant<int, 0xB1>{});
+                over(std::integral_constant<int, 0x4E>{});
+                over(std::integral_constant<int, 0x141>{});
                 gend[p] = __builtin_amdgcn_readfirstlane(m);
                 const int gmin = __builtin_amdgcn_readfirstlane(n);
                 kv_end = max(kv_end, gend[p]);
@@ -1319,50 +1385,60 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         const int slot0 = load_slot(t0);
         // Query halves to fp32 (times the sign flip) before the code loads are
         // issued, so waiting for them never waits for the codes.
-        float qf[kNP][2];
+        float qf[kE];
         {
             const float sh = (h & 1) ? -1.0f : 1.0f;
 #pragma unroll
-            for (int k = 0; k < kNP; ++k) {
-                qf[k][0] = h2f(qraw[k] & 0xffff) * sh;
-                qf[k][1] = h2f(qraw[k] >> 16) * (-sh);
+            for (int k = 0; k < kE; k += 2) {
+                qf[k] = h2f(qraw[k / 2] & 0xffff) * sh;
+                qf[k + 1] = h2f(qraw[k / 2] >> 16) * (-sh);
             }
         }
         Chunk cur;
         fetch(t0, slot0, cur);  // in flight during the setup below (empty waves: all invalid)
         __builtin_amdgcn_sched_barrier(0);  // the first chunk's loads go out before the setup
-        // The decode tables from registers, and each wave's rotated rows
-        // (position k: row w of group rg + k) as fp16 hi and lo parts straight
-        // into the QK B operand: one barrier for the setup.  Lane l holds d = 2l,
-        // 2l + 1: k-group l / (4 kS), k-step (l / 4) % kS, halves 2(l % 4), + 1 of
-        // the half8.  Two or more positions: tile k / 2, column 8(k % 2) + w, hi
-        // in operand 2(k / 2), lo in 2(k / 2) + 1; one position: tile 0, hi in
-        // column w, lo in column w + 8.
+        // The decode tables from registers, and each wave's rotated rows (lane
+        // group k: row w of group rg + k) as fp16 hi and lo parts straight into
+        // the QK B operand: one barrier for the setup.  A lane's dims 4j .. 4j + 3
+        // (and 64 + 4j ..) lie in k-group d / (8 kS), k-step (j / 2) % kS, halves
+        // 4(j % 2) .. of the half8.  Two or more positions: tile k / 2, column
+        // 8(k % 2) + w, hi in operand 2(k / 2), lo in 2(k / 2) + 1; one position:
+        // tile 0, hi in column w, lo in column w + 8.
         {
             const TableWords<PROD> tw = decode_table_words<PROD, KLO>(w, lane);
-            const int s_l = (jl >> 2) & (kS - 1), g_l = jl / (4 * kS);
+            wht_row16(qf, j16);
+            const bool live = gq < npos && rg * kRows + w + gq * kWaves < num_queries;
+            const float qs = live ? inv * lane_sign(j16) : 0.0f;
 #pragma unroll
-            for (int k = 0; k < kNP; ++k) {
-                if (k >= 2 * ntile || (npos == 1 && k > 0)) continue;  // never read (wave-uniform)
-                float q0 = qf[k][0], q1 = qf[k][1];
-                wht_pair<kL>(q0, q1, lane);
-                const bool live = k < npos && rg * kRows + w + k * kWaves < num_queries;
-                q0 = live ? q0 * inv : 0.0f;
-                q1 = live ? q1 * inv : 0.0f;
-                if constexpr (QSCALE) {
-                    const int ex = scale_exp(max_lanes<kL>(fmaxf(fabsf(q0), fabsf(q1))));
-                    q0 = __builtin_amdgcn_ldexpf(q0, -ex);
-                    q1 = __builtin_amdgcn_ldexpf(q1, -ex);
-                    if (lane == 0) rsc[k * kRows + w] = __builtin_amdgcn_ldexpf(1.0f, ex);
-                }
-                const uint32_t hi = pack_h2(q0, q1);
-                const uint32_t lo = lo_pair(q0, q1, hi);
-                const int col_hi = npos == 1 ? w : 8 * (k & 1) + w;
+            for (int k = 0; k < kE; ++k) qf[k] = live ? qf[k] * qs : 0.0f;
+            if constexpr (QSCALE) {
+                float m = 0.0f;
+#pragma unroll
+                for (int k = 0; k < kE; ++k) m = fmaxf(m, fabsf(qf[k]));
+                m = fmaxf(m, partner<1>(m));
+                m = fmaxf(m, partner<2>(m));
+                m = fmaxf(m, partner<4>(m));
+                m = fmaxf(m, partner<8>(m));
+                const int ex = scale_exp(m);
+#pragma unroll
+                for (int k = 0; k < kE; ++k) qf[k] = __builtin_amdgcn_ldexpf(qf[k], -ex);
+                if (i == 0) rsc[gq * kRows + w] = __builtin_amdgcn_ldexpf(1.0f, ex);
+            }
+            if (npos == 1 ? gq == 0 : gq < 2 * ntile) {  // (the other rows are never read)
+                const int col_hi = npos == 1 ? w : 8 * (gq & 1) + w;
                 const int col_lo = npos == 1 ? w + 8 : col_hi;
-                const int op_hi = npos == 1 ? 0 : 2 * (k >> 1);
+                const int op_hi = npos == 1 ? 0 : 2 * (gq >> 1);
                 const int op_lo = npos == 1 ? 0 : op_hi + 1;
-                reinterpret_cast<uint32_t*>(&bqs[op_hi][s_l][16 * g_l + col_hi])[jl & 3] = hi;
-                reinterpret_cast<uint32_t*>(&bqs[op_lo][s_l][16 * g_l + col_lo])[jl & 3] = lo;
+                const int s_l = (j16 >> 1) & (kS - 1), g_l = j16 / (2 * kS);
+#pragma unroll
+                for (int k = 0; k < kE; k += 4) {
+                    const uint32_t h0 = pack_h2(qf[k], qf[k + 1]), h1 = pack_h2(qf[k + 2], qf[k + 3]);
+                    const int at = 16 * (g_l + k / 2);  // (second block: two k-groups on)
+                    reinterpret_cast<uint2*>(&bqs[op_hi][s_l][at + col_hi])[j16 & 1] =
+                        make_uint2(h0, h1);
+                    reinterpret_cast<uint2*>(&bqs[op_lo][s_l][at + col_lo])[j16 & 1] =
+                        make_uint2(lo_pair(qf[k], qf[k + 1], h0), lo_pair(qf[k + 2], qf[k + 3], h1));
+                }
             }
             store_decode_tables<PROD>(lut, kOffKV / 4, w, lane, tw);
             if constexpr (VLO && PROD) {
@@ -1709,59 +1785,11 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
             }
         }
         const float iav = 1.0f / kAlphaV;
-        const float s0 = (h & 1) ? -inv : inv;
-        // Row rr of tile t from the merge space mt (the 8 waves' o rows): the
-        // waves' (m, l, o) merged, the inverse WHT and sign flip, the partial.
-        auto merge_row = [&](int t, int rr, float(*mt)[kMoRows][D]) {
-            const int r = kMoRows * t + rr;  // row of the workgroup
-            const int p = r / kRows;
-            bool keep = p < npos;
-            if constexpr (PAGED)
-                keep = keep && t_begin < gend[p];
-            else
-                keep = keep && rg * kRows + r < num_queries;
-            if (!keep) return;  // wave-uniform
-            float M = mm[0][r];
-#pragma unroll
-            for (int u = 1; u < kWaves; ++u) M = fmaxf(M, mm[u][r]);
-            float L = 0.f, o0 = 0.f, o1 = 0.f;
-#pragma unroll
-            for (int u = 0; u < kWaves; ++u) {
-                const float wt = __builtin_amdgcn_exp2f(mm[u][r] - M);  // (argument <= 0)
-                L += ml[u][r] * wt;
-                o0 += mt[u][rr][2 * jl] * wt;
-                o1 += mt[u][rr][2 * jl + 1] * wt;
-            }
-            if (npos == 1) {  // one position: + its lo columns 8-15
-#pragma unroll
-                for (int u = 0; u < kWaves; ++u) {
-                    const float wt = __builtin_amdgcn_exp2f(mm[u][r] - M);  // (argument <= 0)
-                    o0 += mt[u][rr + kRows][2 * jl] * wt;
-                    o1 += mt[u][rr + kRows][2 * jl + 1] * wt;
-                }
-            }
-            wht_pair<kL>(o0, o1, lane);
-            if constexpr (PAGED) {
-                float* part = ws + ((pid * kNP + p) * kRows + r % kRows) * part_stride(D);
-                if (D == 128 || lane < kL) {
-                    part[2 * jl] = o0 * s0;
-                    part[2 * jl + 1] = o1 * -s0;
-                }
-                if (lane == 0) {
-                    part[D] = M;
-                    part[D + 1] = L;
-                }
-            } else {  // the layout of dec's partials (attn_decode_combine_kernel)
-                const size_t it = (size_t)(rg + p) * g.H + h;
-                const size_t row = (it * num_splits + pid) * kRows + r % kRows;
-                if (D == 128 || lane < kL)
-                    *reinterpret_cast<float2*>(ws + row * D + 2 * jl) = make_float2(o0 * s0, o1 * -s0);
-                if (lane == 0) pml[(it * kRows + r % kRows) * num_splits + pid] = make_float2(M, L);
-            }
-        };
-        // Both tiles at once: tile t's merge space at table word 16384 t (the
-        // tables are no longer read), three barriers per piece instead of four,
-        // and each wave's four rows merged without a barrier between them.
+        // Both tiles at once, tile t's merge space at table word 16384 t (the
+        // tables are no longer read).  Then wave w merges row w of every
+        // position: lane group gq the waves' (m, l, o) of position gq, elements
+        // 4j .. 4j + 3 (and 64 + 4j ..) per lane, then the inverse WHT and sign
+        // flip, and the partial.
         auto mot = [&](int t) { return reinterpret_cast<float(*)[kMoRows][D]>(&lut[16384 * t]); };
         __syncthreads();  // every wave is done with the tables
 #pragma unroll
@@ -1777,10 +1805,60 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 }
         }
         __syncthreads();
+        {
+            const int rr = 8 * (gq & 1) + w;  // this lane group's row of its tile
+            const int r = kMoRows * (gq >> 1) + rr;
+            // (a unit of one position: group 1 holds the same rows' lo columns;
+            // with one tile, groups 2 and 3 merge tile 0's rows and drop them)
+            const float(*mt)[kMoRows][D] = mot(ntile == 2 ? gq >> 1 : 0);
+            float pm[kWaves], pl[kWaves];
 #pragma unroll
-        for (int t = 0; t < kNT; ++t)
+            for (int u = 0; u < kWaves; ++u) pm[u] = mm[u][r], pl[u] = ml[u][r];
+            float M = pm[0];
 #pragma unroll
-            for (int k = 0; k < kMoRows / kWaves; ++k) merge_row(t, w + k * kWaves, mot(t));
+            for (int u = 1; u < kWaves; ++u) M = fmaxf(M, pm[u]);
+            float L = 0.f, o[kE];
+#pragma unroll
+            for (int k = 0; k < kE; ++k) o[k] = 0.f;
+#pragma unroll
+            for (int u = 0; u < kWaves; ++u) {
+                const float wt = __builtin_amdgcn_exp2f(pm[u] - M);  // (argument <= 0)
+                L += pl[u] * wt;
+#pragma unroll
+                for (int k = 0; k < kE; k += 4) {
+                    const float4 x = *reinterpret_cast<const float4*>(&mt[u][rr][4 * j16 + 16 * k]);
+                    o[k] += x.x * wt;
+                    o[k + 1] += x.y * wt;
+                    o[k + 2] += x.z * wt;
+                    o[k + 3] += x.w * wt;
+                }
+            }
+            if (npos == 1) {  // + the lo columns (wave-uniform)
+#pragma unroll
+                for (int k = 0; k < kE; ++k) o[k] += lane_xor<16>(o[k]);
+            }
+            wht_row16(o, j16);
+            const float s0 = ((h & 1) ? -inv : inv) * lane_sign(j16);
+            bool keep = gq < npos;
+            if constexpr (PAGED)
+                keep = keep && t_begin < (gq == 0 ? gend[0] : gq == 1 ? gend[1] : gq == 2 ? gend[2] : gend[3]);
+            else
+                keep = keep && rg * kRows + r < num_queries;
+            // paged: rows of part_stride with (m, l) behind them; slot-mapped:
+            // the layout of dec's partials (attn_decode_combine_kernel)
+            const size_t it = (size_t)(rg + gq) * g.H + h;
+            float* po = PAGED ? ws + ((pid * kNP + gq) * kRows + w) * part_stride(D)
+                              : ws + ((it * num_splits + pid) * kRows + w) * D;
+            float2* pm2 = PAGED ? reinterpret_cast<float2*>(po + D)
+                                : pml + (it * kRows + w) * num_splits + pid;
+            if (keep) {
+#pragma unroll
+                for (int k = 0; k < kE; k += 4)
+                    *reinterpret_cast<float4*>(po + 4 * j16 + 16 * k) =
+                        make_float4(o[k] * s0, o[k + 1] * -s0, o[k + 2] * s0, o[k + 3] * -s0);
+                if (i == 0) *pm2 = make_float2(M, L);
+            }
+        }
         // the next piece's setup writes its decode tables over the merge spaces
         if constexpr (PAGED) __syncthreads();
     };  // item
@@ -2880,13 +2958,13 @@ struct DecodeSplit {
 };
 // Cost of a split kernel's workgroup: a setup and merge, and a pass of 256
 // tokens, in 0.1 us (measured at D = 128, turbo_prod, 2 heads, 250 to 32,768
-// tokens, kernel trace: one group 5.9 us at one pass, 10.4 at two, 14.8 at
-// four, 22.5 at eight; a unit of two groups 8.3 at one, of four 12.0 at one,
-// 16.0 at two, 32.5 at seven).
+// tokens, kernel trace: one group 5.9-7.1 us at one pass, 9.8 at two, 14.8 at
+// four, 22.5 at eight; a unit of two groups 8.2-9.2 at one, of four 11.6 at
+// one, 14.4-15.3 at two, 30.7 at seven).
 struct SplitCost {
     int setup, pass;
 };
-constexpr SplitCost kGroupCost{51, 20}, kPairCost{70, 20}, kUnitCost{90, 33};
+constexpr SplitCost kGroupCost{51, 20}, kPairCost{60, 22}, kUnitCost{78, 33};
 // The split count and its cost: one workgroup runs on a CU at a time, so of
 // the counts that fill one to four rounds of the CUs the cheapest is taken
 // (the fewest splits among equals: the merge reads every split's partials).
