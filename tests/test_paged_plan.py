@@ -44,6 +44,19 @@ def _passes(S, n, w, b0, b1):
     return x0, x1
 
 
+def test_pass_per_segment():
+    """A step with no more passes than segments: weight 1, no lead, as many
+    segments as passes, so each holds exactly the pass of its own number."""
+    for total in (1, 2, 7, 64, 127, 256):
+        for s in range(total):
+            assert (_bound(s, total, total), _bound(s + 1, total, total)) == (s, s + 1)
+            assert _segment_of(s, total, total) == s
+        for S, n in ((0, total), (total // 3, total - total // 3)):
+            for s in range(total):
+                x0, x1 = _passes(S, n, 1, s, s + 1)
+                assert (x0, x1) == ((s - S, s - S + 1) if s >= S else (0, 0))
+
+
 def test_paged_plan_pieces_partition_every_item():
     rng = np.random.default_rng(77)
     for _ in range(400):

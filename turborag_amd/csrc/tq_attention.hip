@@ -308,18 +308,23 @@ __device__ __forceinline__ half8 as_h8(uint32_t a, uint32_t b, uint32_t c, uint3
 // at work positions [start, start + w*n) of its head's work (every head has
 // the same work, split into segments per head).
 struct PagedUnit {
-    int32_t first, npos, kv_end, start, n, w, index, pad;  // index: the unit's number
+    // index: the unit's number; group_kv: in a row group's copy, the group's
+    // own longest row
+    int32_t first, npos, kv_end, start, n, w, index, group_kv;
 };
 struct PagedRows {
     const int32_t* block_tables;
     const int32_t* row_seq;
     const int32_t* row_kv_len;
     int max_blocks;
-    // The step's plan (paged_plan_kernel): plan[0] units, then a sentinel
-    // whose start is the total work plan[1]; a copy of each row group's unit.
+    // The step's plan: plan[0] units, then a sentinel whose start is the total
+    // work plan[1], in plan[2] segments per head; a copy of each row group's
+    // unit.  From paged_plan_kernel, or (units null: up to unit::kPlanGroups
+    // row groups) computed by every split workgroup for itself, the first one
+    // leaving group_unit and plan for the merge.
     const PagedUnit* units;
-    const PagedUnit* group_unit;
-    const int32_t* plan;
+    PagedUnit* group_unit;
+    int32_t* plan;
     // A page-sized region of the workspace that masked tokens' loads address
     // (always valid memory; what they read is not used)
     const uint8_t* spare_page;
@@ -1111,6 +1116,125 @@ static_assert(kOffKV + 256 * 256 <= 4 * kTabWords, "K|V rows");
 static_assert(256 * 255 + 128 + 4 * kLoCopies <= kOffKV, "the V lo rows end below the K table");
 static_assert(kRows % kWaves == 0 && kWaves == 8, "eight waves, one row per wave and position");
 constexpr int part_stride(int D) { return D + 4; }  // paged partial row: o[D], m, l, pad
+// A pass's weight in work positions: 4 for a unit of more than two positions
+// (the two-tile loop), 3 otherwise, about their measured cost ratio.
+__device__ __forceinline__ int pass_weight(int npos) { return npos > 2 ? 4 : 3; }
+// Paged steps: the work positions a unit's setup counts for (a two-tile pass
+// weighs 4), before its first pass (32 sequences of 1K-32K tokens: 139 us per
+// step with 0, 135 with 4, 131-133 with 8, 12 or 16).
+#ifndef TQ_PAGED_PIECE_COST
+#define TQ_PAGED_PIECE_COST 8
+#endif
+constexpr int kPieceCost = TQ_PAGED_PIECE_COST;
+// Row groups a split workgroup plans by itself (one wave, four groups per
+// lane; the unit records take 12 bytes of LDS each).
+constexpr int kPlanGroups = 256;
+struct UnitRec {
+    int32_t start, kv_end;
+    int16_t first, npos;
+};
+
+// The step's plan as paged_plan_kernel makes it, by one workgroup for itself:
+// units in rec, then a sentinel; plan[0..2] = units, total work, segments per
+// head.  Where the step has no more passes than Gh, every pass is a segment
+// of its own (weight 1, no lead): no workgroup takes two while another has
+// none, and the merge of a unit looks at its n passes instead of the segments
+// they are scattered over.  `scratch`: LDS of 2 (kPlanGroups + 8) words.
+// leave: write group_unit and plan for the merge.
+__device__ __forceinline__ void plan_step(const PagedRows& pr, int num_rows, int max_kv_len, int Gh,
+                                          bool leave, int* scratch, UnitRec* rec, int* plan) {
+    const int groups = (num_rows + kRows - 1) / kRows;
+    int* s_sq = scratch + 4;  // sequence of group g at [g], with room before and after
+    int* s_gk = s_sq + kPlanGroups + 8;
+    if (threadIdx.x < kPlanGroups) {
+        // (unconditional loads: a group or row past the end re-reads the last)
+        const int g = threadIdx.x, gc = min(g, groups - 1);
+        int v[kRows];
+        const int sq = pr.row_seq[(size_t)gc * kRows];
+#pragma unroll
+        for (int k = 0; k < kRows; ++k) v[k] = pr.row_kv_len[min(gc * kRows + k, num_rows - 1)];
+        int m = 0;
+#pragma unroll
+        for (int k = 0; k < kRows; ++k)
+            if (gc * kRows + k < num_rows) m = max(m, v[k]);
+        s_sq[g] = sq;
+        s_gk[g] = g < groups ? min(m, max_kv_len) : 0;
+    }
+    __syncthreads();
+    if (threadIdx.x < 64) {
+        const int lane = threadIdx.x, g0 = 4 * lane;
+        int sq[8], gk[7];  // sequences of groups g0 - 1 .. g0 + 6, lengths from g0
+#pragma unroll
+        for (int k = 0; k < 8; ++k) sq[k] = s_sq[min(max(g0 + k - 1, 0), kPlanGroups - 1)];
+#pragma unroll
+        for (int k = 0; k < 7; ++k) gk[k] = g0 + k < kPlanGroups ? s_gk[g0 + k] : 0;
+        // The run each group is in: the last group at or before it that starts one.
+        int last = -1;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (g0 + k < groups && (g0 + k == 0 || sq[k + 1] != sq[k])) last = g0 + k;
+        const uint64_t below = __ballot(last >= 0) & ((1ull << lane) - 1ull);
+        int cur = __shfl(last, below ? 63 - __clzll(below) : 0);
+        int cnt[4], kv[4], n[4], lane_u = 0, lane_n = 0, lane_w = 0;
+        bool start[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const int g = g0 + k;
+            if (g < groups && (g == 0 || sq[k + 1] != sq[k])) cur = g;
+            start[k] = g < groups && ((g - cur) & (kNP - 1)) == 0;
+            cnt[k] = 1;
+            kv[k] = gk[k];
+#pragma unroll
+            for (int m = 1; m < kNP; ++m)
+                if (cnt[k] == m && g + m < groups && sq[k + 1 + m] == sq[k + 1]) {
+                    ++cnt[k];
+                    kv[k] = max(kv[k], gk[k + m]);
+                }
+            n[k] = start[k] ? (kv[k] + kPass - 1) / kPass : 0;
+            lane_u += start[k] ? 1 : 0;
+            lane_n += n[k];
+            lane_w += n[k] > 0 ? kPieceCost + pass_weight(cnt[k]) * n[k] : 0;
+        }
+        int su = lane_u, sn = lane_n, sw = lane_w;  // inclusive scans over the lanes
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const int a = __shfl_up(su, d), b = __shfl_up(sn, d), c = __shfl_up(sw, d);
+            if (lane >= d) su += a, sn += b, sw += c;
+        }
+        const int units = __shfl(su, 63), tn = __shfl(sn, 63), tw = __shfl(sw, 63);
+        const bool single = tn <= Gh;
+        const int total = single ? tn : tw, segs = single ? max(tn, 1) : Gh;
+        int u = su - lane_u, x = single ? sn - lane_n : sw - lane_w;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            if (!start[k]) continue;
+            const int w = single ? 1 : pass_weight(cnt[k]);
+            x += !single && n[k] > 0 ? kPieceCost : 0;
+            rec[u] = UnitRec{x, kv[k], (int16_t)(g0 + k), (int16_t)cnt[k]};
+            if (leave) {
+#pragma unroll
+                for (int m = 0; m < kNP; ++m)
+                    if (m < cnt[k])
+                        pr.group_unit[g0 + k + m] =
+                            PagedUnit{g0 + k, cnt[k], kv[k], x, n[k], w, u, gk[k + m]};
+            }
+            x += w * n[k];
+            ++u;
+        }
+        if (lane == 0) {
+            rec[units] = UnitRec{total, 0, 0, 0};
+            plan[0] = units;
+            plan[1] = total;
+            plan[2] = segs;
+            if (leave) {
+                pr.plan[0] = units;
+                pr.plan[1] = total;
+                pr.plan[2] = segs;
+            }
+        }
+    }
+    __syncthreads();
+}
 
 // A query or output row held by 16 lanes, so that a wave works on its row of
 // all four positions at once instead of one after another.  Lane p owns elements 4j .. 4j + 3
@@ -1872,20 +1996,37 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         // of a token share its cache lines (cell tib * H + h), and the second
         // reader finds them in that XCD's L2.  The segments of one XCD are
         // consecutive, so the units of a sequence mostly share it too.
+        // (A step planned here with one pass per segment spreads its segments
+        // over the XCDs instead; the heads of one still share an XCD.)
         const int Gh = (int)gridDim.x / g.H;
         const int hh = (int)blockIdx.x / Gh;
         const int bl = (int)blockIdx.x - hh * Gh;
-        const int seg = (bl & 7) * (Gh >> 3) + (bl >> 3);
-        const int nu = __builtin_amdgcn_readfirstlane(pr.plan[0]);
-        const int total = __builtin_amdgcn_readfirstlane(pr.plan[1]);
-        const Segments sg(total, Gh);
+        __shared__ UnitRec s_units[kPlanGroups + 1];
+        __shared__ int s_plan[3];
+        const bool planned = pr.units != nullptr;  // by paged_plan_kernel
+        if (planned) {
+            if (threadIdx.x < 3) s_plan[threadIdx.x] = pr.plan[threadIdx.x];
+            __syncthreads();
+        } else {
+            plan_step(pr, num_queries, num_kv_tokens, Gh, blockIdx.x == 0,
+                      reinterpret_cast<int*>(lut), s_units, s_plan);
+        }
+        const int nu = __builtin_amdgcn_readfirstlane(s_plan[0]);
+        const int total = __builtin_amdgcn_readfirstlane(s_plan[1]);
+        const int segs = __builtin_amdgcn_readfirstlane(s_plan[2]);
+        const bool single = segs != Gh;  // (segs == Gh == total: either numbering)
+        const int seg = single ? bl : (bl & 7) * (Gh >> 3) + (bl >> 3);
+        if (seg >= segs || total == 0) return;
+        const Segments sg(total, segs);
         const int b0 = sg.bound(seg), b1 = sg.bound(seg + 1);
         if (b0 >= b1) return;  // an empty segment (less work than workgroups)
+        const bool ones = !planned && segs == total;  // weight 1 per pass
+        auto start_of = [&](int u) { return planned ? pr.units[u].start : s_units[u].start; };
         // The unit holding work position b0: exactly one u has start(u) <= b0 <
         // start(u + 1), or b0 lies before the first unit's first pass (unit 0).
         __shared__ int s_unit;
         for (int u = threadIdx.x; u < nu; u += 64 * kWaves)
-            if ((u == 0 || pr.units[u].start <= b0) && b0 < pr.units[u + 1].start) s_unit = u;
+            if ((u == 0 || start_of(u) <= b0) && b0 < start_of(u + 1)) s_unit = u;
         __syncthreads();
         // The walk over the units overlapping the segment, in work order.  Its
         // position lives in LDS (one copy per wave, volatile accesses), so no
@@ -1900,17 +2041,28 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         for (;;) {
             const int u = __builtin_amdgcn_readfirstlane(walk[0]);
             if (u >= nu) break;
-            const PagedUnit un = pr.units[u];
-            if (un.start >= b1) break;
+            int first, npos, kv_end, start;
+            if (planned) {
+                const PagedUnit un = pr.units[u];
+                first = un.first, npos = un.npos, kv_end = un.kv_end, start = un.start;
+            } else {
+                const UnitRec un = s_units[u];
+                first = __builtin_amdgcn_readfirstlane((int)un.first);
+                npos = __builtin_amdgcn_readfirstlane((int)un.npos);
+                kv_end = __builtin_amdgcn_readfirstlane(un.kv_end);
+                start = __builtin_amdgcn_readfirstlane(un.start);
+            }
+            if (start >= b1) break;
             if ((threadIdx.x & 63) == 0) walk[0] = u + 1;
             int x0, x1;
-            item_passes(un.start, un.n, un.w, b0, b1, x0, x1);
+            item_passes(start, (kv_end + kPass - 1) / kPass, ones ? 1 : pass_weight(npos), b0, b1,
+                        x0, x1);
             if (x0 < x1) {
                 int tid = threadIdx.x;
                 asm volatile("" : "+v"(tid));  // opaque per item (see item)
                 // partial slot: (unit + segment) * H + head, unique (the
                 // pieces of one head form a staircase in (unit, segment))
-                item(tid, hh, un.first, un.npos, x0 * kPass, min(x1 * kPass, un.kv_end),
+                item(tid, hh, first, npos, x0 * kPass, min(x1 * kPass, kv_end),
                      (size_t)(u + seg) * g.H + hh);
             }
         }
@@ -2071,69 +2223,70 @@ __global__ __launch_bounds__(256) void attn_mfma_combine_items_kernel(
         make_uint2(fin(acc.x) | (fin(acc.y) << 16), fin(acc.z) | (fin(acc.w) << 16));
 }
 
-// Merge of a paged step's partials: one block per (row group, kv head), laid
-// out as in attn_mfma_combine_items_kernel.  The row group is position p of
-// unit u; its item's passes were cut at segment bounds into pieces, one
-// partial per segment they start in (slot item + segment, position p), and
-// a piece starting at or past the group's longest row wrote none.
-template <int D>
-__global__ __launch_bounds__(2 * D) void attn_paged_combine_kernel(
+// Merge of a paged step's partials.  A row group is position p of unit u; its
+// item's passes were cut at segment bounds into pieces, one partial per
+// segment they start in (slot unit + segment, position p), and a piece
+// starting at or past the group's longest row wrote none.  One wave per (row,
+// slice of 4 LS elements): 64 / LS lane groups take the segments in turn, kB
+// at a time (every load of a batch in flight together), merge them with a
+// running maximum, then the groups are merged across lanes.  LS = 8 (one
+// 128-byte line, 8 groups) for few rows, whose unit may lie in a hundred
+// segments; LS = D / 4 (a whole row) for many, which have a few each.  Bound by
+// its chain of dependent loads: 3 row groups x 4 heads 8.4 -> 4.2 us, 160 x 2
+// 6.5 -> 5.3 us, against a block of 256 threads per item that read eight
+// segments at a time.
+template <int D, int LS>
+__global__ __launch_bounds__(64) void attn_paged_combine_kernel(
     const float* __restrict__ ws, uint16_t* __restrict__ output, int H, int num_queries,
-    int num_segments, mfma::PagedRows pr) {
+    mfma::PagedRows pr) {
     using namespace mfma;
-    constexpr int positions = unit::kNP, pass = unit::kPass;
-    constexpr int kT = D / 4;     // threads per row
-    const int item = blockIdx.x;  // h + H * rg
-    const int h = item % H, rg = item / H;
-    const int t = threadIdx.x, r = t / kT, d0 = 4 * (t % kT);
+    constexpr int kG = 64 / LS, kSlices = D / (4 * LS), kB = 4;
+    const int t = threadIdx.x, grp = t / LS;
+    const int d0 = 4 * LS * (blockIdx.x % kSlices) + 4 * (t % LS);
+    const int row = blockIdx.x / kSlices;  // ((row group) * H + head) * 8 + row
+    const int r = row % kRows, item = row / kRows, h = item % H, rg = item / H;
+    const int q = rg * kRows + r;
+    if (q >= num_queries) return;
     const PagedUnit un = pr.group_unit[rg];
-    const int u = un.index;
-    const int total = pr.plan[1], G = num_segments;
-    const int p = rg - un.first;
-    // The group's longest row: the row lengths are loaded unconditionally (a
-    // row past the end re-reads the last row), so the loads go out together
-    // with the unit's record instead of one after another in branches.
-    int kvr[kRows];
-#pragma unroll
-    for (int k = 0; k < kRows; ++k) kvr[k] = pr.row_kv_len[min(rg * kRows + k, num_queries - 1)];
-    int kv = 0;
-#pragma unroll
-    for (int k = 0; k < kRows; ++k)
-        if (rg * kRows + k < num_queries) kv = max(kv, kvr[k]);
-    const int S = un.start;  // every head has the unit's work range, in its own segments
-    // segments holding the item's first and last pass starts
+    const int total = pr.plan[1], G = pr.plan[2];
+    const int p = rg - un.first, kv = un.group_kv, S = un.start;
+    // Segment gs holds the item's passes [first(bound(gs)), first(bound(gs + 1))).
+    const auto first = [&](int b) {
+        const int v = max(b - S, 0);
+        return min(un.n, un.w == 4 ? (v + 3) >> 2 : un.w == 3 ? (v + 2) / 3 : v);
+    };
     int g_lo = 0, g_hi = -1;
     const Segments sg(max(total, 1), G);
     if (un.n > 0 && kv > 0) {
         g_lo = sg.of(S, total);
         g_hi = sg.of(S + un.w * (un.n - 1), total);
     }
-    const size_t unit0 = (size_t)u;
+    const float* base = ws + ((((size_t)un.index * H + h) * unit::kNP + p) * kRows + r) *
+                                 unit::part_stride(D);
+    const size_t seg_stride = (size_t)H * unit::kNP * kRows * unit::part_stride(D);
     float M = kInitMax, L = 0.f;
     float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-    for (int b = g_lo; b <= g_hi; b += 8) {
-        float pm[8], pl[8];
-        float4 po[8];
-        float2 mlr[8];
-        int okv[8];
+    for (int b = g_lo + grp; b <= g_hi; b += kG * kB) {
+        float4 po[kB];
+        float2 mlr[kB];
+        int okv[kB];
         // (slot gs <= g_hi is one of the item's pieces: the loads are
         // unconditional and all in flight together; the pieces that wrote
         // nothing are dropped after, by a per-lane select rather than a branch
         // whose join would wait for each load in turn)
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            const int gs = min(b + k, g_hi);
-            int x0, x1;
-            item_passes(S, un.n, un.w, sg.bound(gs), sg.bound(gs + 1), x0, x1);
-            okv[k] = b + k <= g_hi && x0 < x1 && x0 * pass < kv;
-            const float* pp =
-                ws + ((((unit0 + gs) * H + h) * positions + p) * kRows + r) * unit::part_stride(D);
+        for (int k = 0; k < kB; ++k) {
+            const int gs = min(b + kG * k, g_hi);
+            const float* pp = base + seg_stride * gs;
             mlr[k] = *reinterpret_cast<const float2*>(pp + D);
             po[k] = *reinterpret_cast<const float4*>(pp + d0);
+            const int x0 = first(sg.bound(gs));
+            okv[k] = b + kG * k <= g_hi && x0 < first(sg.bound(gs + 1)) && x0 * unit::kPass < kv;
         }
         __builtin_amdgcn_sched_barrier(0);
+        float pm[kB], pl[kB];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
+        for (int k = 0; k < kB; ++k) {
             int ok = okv[k];
             asm volatile("" : "+v"(ok));
             pm[k] = ok ? mlr[k].x : kInitMax;
@@ -2142,7 +2295,7 @@ __global__ __launch_bounds__(2 * D) void attn_paged_combine_kernel(
         }
         float mb = M;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) mb = fmaxf(mb, pm[k]);
+        for (int k = 0; k < kB; ++k) mb = fmaxf(mb, pm[k]);
         const float sc = __builtin_amdgcn_exp2f(M - mb);  // (argument <= 0)
         L *= sc;
         acc.x *= sc;
@@ -2150,7 +2303,7 @@ __global__ __launch_bounds__(2 * D) void attn_paged_combine_kernel(
         acc.z *= sc;
         acc.w *= sc;
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
+        for (int k = 0; k < kB; ++k) {
             const float wt = __builtin_amdgcn_exp2f(pm[k] - mb);
             L += pl[k] * wt;
             acc.x += po[k].x * wt;
@@ -2160,8 +2313,24 @@ __global__ __launch_bounds__(2 * D) void attn_paged_combine_kernel(
         }
         M = mb;
     }
-    const int q = rg * kRows + r;
-    if (q >= num_queries) return;
+    // The lane groups (lanes LS apart), pairwise.
+    const auto merge = [&](auto lanes) {
+        constexpr int X = decltype(lanes)::value;
+        if constexpr (X >= LS) {
+            const float Mp = lane_xor<X>(M), mn = fmaxf(M, Mp);
+            const float a = __builtin_amdgcn_exp2f(M - mn), c = __builtin_amdgcn_exp2f(Mp - mn);
+            L = L * a + lane_xor<X>(L) * c;
+            acc.x = acc.x * a + lane_xor<X>(acc.x) * c;
+            acc.y = acc.y * a + lane_xor<X>(acc.y) * c;
+            acc.z = acc.z * a + lane_xor<X>(acc.z) * c;
+            acc.w = acc.w * a + lane_xor<X>(acc.w) * c;
+            M = mn;
+        }
+    };
+    merge(std::integral_constant<int, 8>{});
+    merge(std::integral_constant<int, 16>{});
+    merge(std::integral_constant<int, 32>{});
+    if (t >= LS) return;
     const auto fin = [&](float o) { return (uint32_t)f2h(L > 0.f ? o / L : o); };
     *reinterpret_cast<uint2*>(output + ((size_t)q * H + h) * D + d0) =
         make_uint2(fin(acc.x) | (fin(acc.y) << 16), fin(acc.z) | (fin(acc.w) << 16));
@@ -2192,15 +2361,8 @@ __device__ int block_scan_1024(int v, int ident, int* s_tot, Op op) {
     return op(pre, v);
 }
 
-// Paged steps: the work positions a unit's setup counts for (a two-tile pass
-// weighs 4), before its first pass (32 sequences of 1K-32K tokens: 139 us per step
-// with 0, 135 with 4, 131-133 with 8, 12 or 16).
-#ifndef TQ_PAGED_PIECE_COST
-#define TQ_PAGED_PIECE_COST 8
-#endif
-constexpr int kPieceCost = TQ_PAGED_PIECE_COST;
-
-// The plan of a paged step, one block of 1024 threads.  Row groups (8 rows
+// The plan of a paged step of more than unit::kPlanGroups row groups, one
+// block of 1024 threads.  Row groups (8 rows
 // of one sequence) form units: each run of consecutive groups of one
 // sequence is cut into units of U groups from its start, the last one
 // shorter.  A unit's items (one per kv head) are n = ceil(kv_end / pass)
@@ -2216,7 +2378,7 @@ constexpr int kPieceCost = TQ_PAGED_PIECE_COST;
 template <int U>
 __global__ __launch_bounds__(1024) void paged_plan_kernel(
     const int32_t* __restrict__ row_seq, const int32_t* __restrict__ row_kv_len, int num_rows,
-    int groups, int pass, int max_kv_len, mfma::PagedUnit* __restrict__ units,
+    int groups, int pass, int max_kv_len, int segments, mfma::PagedUnit* __restrict__ units,
     mfma::PagedUnit* __restrict__ group_unit, int32_t* __restrict__ plan) {
     static_assert(U >= 1 && U <= 4 && (U & (U - 1)) == 0, "1, 2 or 4 groups per unit");
     using mfma::kRows;
@@ -2278,9 +2440,9 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(
                 ++c;
                 kv = max(kv, s_gk[j + k]);
             }
-        const int w = U > 2 ? (c > 2 ? 4 : 3) : 1;
+        const int w = U > 2 ? unit::pass_weight(c) : 1;
         const int n = (kv + pass - 1) / pass;
-        const int lead = n > 0 ? kPieceCost : 0;
+        const int lead = n > 0 ? unit::kPieceCost : 0;
         const int work = start ? lead + w * n : 0;  // per kv head (every head has it)
         const int ui = block_scan_1024(start ? 1 : 0, 0, s_tot, add);
         const int wi = block_scan_1024(work, 0, s_tot, add);
@@ -2288,7 +2450,11 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(
             const int o = c_units + ui - 1;
             const mfma::PagedUnit rec{gi, c, kv, c_work + wi - work + lead, n, w, o, 0};
             units[o] = rec;
-            for (int k = 0; k < c; ++k) group_unit[gi + k] = rec;
+            for (int k = 0; k < c; ++k) {
+                mfma::PagedUnit gu = rec;
+                gu.group_kv = s_gk[j + k];
+                group_unit[gi + k] = gu;
+            }
         }
         if (j == kWin - 1) {  // window totals (inclusive scans at the last thread)
             s_carry[0] = ui;
@@ -2307,6 +2473,7 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(
         units[c_units] = mfma::PagedUnit{0, 0, 0, c_work, 0, 1, c_units, 0};  // sentinel
         plan[0] = c_units;
         plan[1] = c_work;
+        plan[2] = segments;
     }
 }
 
@@ -3134,20 +3301,32 @@ void launch_paged_units(const uint16_t* query, const uint8_t* pool, const int32_
     PagedUnit* units = reinterpret_cast<PagedUnit*>(wsb + part_bytes);
     PagedUnit* group_unit = units + row_groups + 1;
     int32_t* plan = reinterpret_cast<int32_t*>(wsb + part_bytes + unit_bytes);
-    const PagedRows pr{block_tables, row_seq,    row_kv_len, max_blocks, units, group_unit, plan,
-                       reinterpret_cast<const uint8_t*>(wsb + spare_at)};
-    hipLaunchKernelGGL(paged_plan_kernel<unit::kNP>, dim3(1), dim3(1024), 0, stream, row_seq,
-                       row_kv_len, num_rows, row_groups, unit::kPass, max_kv_len, units,
-                       group_unit, plan);
-    check_launch(prod ? "turbo_prod_paged_attn_plan" : "turbo_mse_paged_attn_plan");
-    if (max_kv_len > 0) {
+    // Up to kPlanGroups row groups: each split workgroup makes the plan for
+    // itself, its row lengths read in place of the plan's records, and the
+    // plan launch (5.5 us of a step) is gone.
+    const bool self = row_groups <= unit::kPlanGroups;
+    const PagedRows pr{block_tables, row_seq,    row_kv_len, max_blocks, self ? nullptr : units,
+                       group_unit,   plan,       reinterpret_cast<const uint8_t*>(wsb + spare_at)};
+    if (!self) {
+        hipLaunchKernelGGL(paged_plan_kernel<unit::kNP>, dim3(1), dim3(1024), 0, stream, row_seq,
+                           row_kv_len, num_rows, row_groups, unit::kPass, max_kv_len, Gh, units,
+                           group_unit, plan);
+        check_launch(prod ? "turbo_prod_paged_attn_plan" : "turbo_mse_paged_attn_plan");
+    }
+    if (max_kv_len > 0 || self) {
         hipLaunchKernelGGL((unit::attn_unit_split_kernel<SCH, D, true>), dim3(G),
                            dim3(64 * unit::kWaves), 0, stream, query, pool, nullptr, ws, nullptr,
                            inv_sqrt_d(D), num_rows, max_kv_len, 0, 0, g, pr);
         check_launch(prod ? "turbo_prod_paged_attn_split" : "turbo_mse_paged_attn_split");
     }
-    hipLaunchKernelGGL(attn_paged_combine_kernel<D>, dim3(heads), dim3(2 * D), 0, stream, ws,
-                       output, g.H, num_rows, Gh, pr);
+    // One wave per row, or per 128-byte line of it while that is few waves.
+    const long long lines = (long long)heads * kRows * (D / 32);
+    if (lines <= 4096)
+        hipLaunchKernelGGL((attn_paged_combine_kernel<D, 8>), dim3((unsigned)lines), dim3(64), 0,
+                           stream, ws, output, g.H, num_rows, pr);
+    else
+        hipLaunchKernelGGL((attn_paged_combine_kernel<D, D / 4>), dim3((unsigned)heads * kRows), dim3(64), 0,
+                           stream, ws, output, g.H, num_rows, pr);
     check_launch(prod ? "turbo_prod_paged_attn_combine" : "turbo_mse_paged_attn_combine");
 }
 }  // namespace
@@ -3217,7 +3396,7 @@ void launch_paged_attention(Scheme s, const uint16_t* query, const uint8_t* pool
     const int row_groups = (num_rows + mfma::kRows - 1) / mfma::kRows;
     const bool countable =
         (long long)row_groups *
-            (4LL * ((std::max(max_kv_len, 0) + unit::kPass - 1) / unit::kPass) + kPieceCost) <=
+            (4LL * ((std::max(max_kv_len, 0) + unit::kPass - 1) / unit::kPass) + unit::kPieceCost) <=
         INT32_MAX;
     const bool d64 = mfma_attention64_ok(g, pool) && countable;
     if (!(d64 || mfma_attention_ok(g, pool)) || extent > 0xFFFFFFFFu) {
