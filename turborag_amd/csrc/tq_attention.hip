@@ -3139,8 +3139,7 @@ struct SplitChoice {
     int splits;
     long long cost;
 };
-SplitChoice choose_splits(int items, int passes, SplitCost c, int most) {
-    const int cus = num_cus();
+SplitChoice choose_splits(int items, int passes, SplitCost c, int most, int cus) {
     SplitChoice best{1, -1};
     for (int r = 1; r <= 4; ++r) {
         int s = std::min({std::max(1, (int)((long long)r * cus / items)), passes, most});
@@ -3157,6 +3156,7 @@ SplitChoice choose_splits(int items, int passes, SplitCost c, int most) {
 DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens, size_t cap) {
     using namespace mfma;
     DecodeSplit d{};
+    const int cus = num_cus();
     d.rows = num_queries * g.H;
     d.row_groups = (num_queries + kRows - 1) / kRows;
     d.heads = g.H * d.row_groups;
@@ -3169,7 +3169,7 @@ DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens, 
         // 256-token split per workgroup, or longer splits once there are more
         // than ~2 workgroups per CU and row group.  The launch itself takes no
         // more splits than fit.
-        const int want = std::max(1, (kSplitBlocksPerCU * num_cus() + d.heads - 1) / d.heads);
+        const int want = std::max(1, (kSplitBlocksPerCU * cus + d.heads - 1) / d.heads);
         int splits = std::min(std::min(passes, want), 1024);
         const int tps = num_kv_tokens > 0 ? (num_kv_tokens + splits - 1) / splits : 0;
         if (tps > 0) splits = (num_kv_tokens + tps - 1) / tps;
@@ -3177,9 +3177,9 @@ DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens, 
     }
     const int most = cap ? (int)std::min<size_t>(1024, std::max<size_t>(1, cap / per_split)) : 1024;
     const int units = g.H * ((d.row_groups + unit::kNP - 1) / unit::kNP);
-    const SplitChoice one = choose_splits(d.heads, passes, kGroupCost, most);
+    const SplitChoice one = choose_splits(d.heads, passes, kGroupCost, most, cus);
     const SplitChoice un =
-        choose_splits(units, passes, d.row_groups == 2 ? kPairCost : kUnitCost, most);
+        choose_splits(units, passes, d.row_groups == 2 ? kPairCost : kUnitCost, most, cus);
     d.units = d.row_groups > 1 && un.cost < one.cost;
     d.items = d.units ? units : d.heads;
     d.splits = d.units ? un.splits : one.splits;

@@ -7,6 +7,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdlib>
 #include <cstdio>
@@ -272,17 +273,16 @@ DenseGeom dense_geom(const TQConfig& cfg, const TQDensePageLayout& l) {
 }
 
 int num_cus() {
-    static std::mutex mu;
-    static std::map<int, int> cache;
+    constexpr int kDevices = 64;
+    static std::atomic<int> cache[kDevices] = {};
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) throw Error("hipGetDevice failed");
-    std::lock_guard<std::mutex> lock(mu);
-    auto it = cache.find(dev);
-    if (it != cache.end()) return it->second;
-    int n = 0;
+    const bool known = dev >= 0 && dev < kDevices;
+    int n = known ? cache[dev].load(std::memory_order_relaxed) : 0;
+    if (n > 0) return n;
     if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n <= 0)
         n = 256;
-    cache[dev] = n;
+    if (known) cache[dev].store(n, std::memory_order_relaxed);
     return n;
 }
 

@@ -240,6 +240,27 @@ SIGNATURES: dict[str, tuple[list, object]] = {
 }
 
 
+_DATA_POINTERS = (_P(c_int32), _P(c_uint8), _P(c_float))
+
+
+def _ready(t, dtype: torch.dtype, numel: int) -> bool:
+    """What TurboQuantWrapper._check asks of one tensor (is_cuda: device.type is
+    "cuda", without making a device object and its string on every call)."""
+    return (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype and t.is_contiguous()
+            and t.numel() >= numel)
+
+
+def _ready_pointers(tensors, dtype: torch.dtype, numel: int):
+    """Their device pointers as a C array, or None if one of them is not ready."""
+    out = []
+    for t in tensors:
+        if not (isinstance(t, torch.Tensor) and t.is_cuda and t.dtype is dtype
+                and t.is_contiguous() and t.numel() >= numel):
+            return None
+        out.append(t.data_ptr())
+    return (c_void_p * max(len(out), 1))(*out)
+
+
 class TurboQuantWrapper:
     """Wrapper around libturboquant.so.
 
@@ -257,6 +278,15 @@ class TurboQuantWrapper:
         self.lib_path = path
         self._lib = ctypes.CDLL(str(path))
         self._bind_symbols()
+        # The launches' own bindings: data pointers as plain integers (a
+        # ctypes.cast per pointer cost ~0.6 us of a call), struct pointers
+        # typed as in `lib`.
+        self._fast = ctypes.CDLL(str(path))
+        for name, (argtypes, restype) in SIGNATURES.items():
+            if name.startswith(("tq_launch_", "tq_load_")):
+                fn = getattr(self._fast, name)
+                fn.argtypes = [c_void_p if a in _DATA_POINTERS else a for a in argtypes]
+                fn.restype = restype
 
     def _bind_symbols(self) -> None:
         for name, (argtypes, restype) in SIGNATURES.items():
@@ -302,26 +332,12 @@ class TurboQuantWrapper:
     # ── pointer helpers ─────────────────────────────────────────────── #
 
     @staticmethod
-    def _vp(t: torch.Tensor) -> c_void_p:
-        return c_void_p(t.data_ptr())
-
-    @staticmethod
-    def _i32p(t: torch.Tensor):
-        return ctypes.cast(c_void_p(t.data_ptr()), POINTER(c_int32))
-
-    @staticmethod
-    def _u8p(t: torch.Tensor):
-        return ctypes.cast(c_void_p(t.data_ptr()), POINTER(c_uint8))
-
-    @staticmethod
-    def _f32p(t: torch.Tensor):
-        return ctypes.cast(c_void_p(t.data_ptr()), POINTER(c_float))
-
-    @staticmethod
     def _check(scheme: str, op: str, **tensors: tuple[torch.Tensor, torch.dtype, int]) -> None:
         """Each tensor must live on a GPU, be contiguous, have the dtype and
         hold at least the given number of elements."""
         for name, (t, dtype, numel) in tensors.items():
+            if _ready(t, dtype, numel):
+                continue
             if not isinstance(t, torch.Tensor) or t.device.type != "cuda":
                 raise ValueError(f"{scheme} {op}: {name} must be a GPU tensor")
             if t.dtype != dtype:
@@ -333,8 +349,8 @@ class TurboQuantWrapper:
                                  f"needs {numel}")
 
     @staticmethod
-    def _stream(stream: int) -> c_void_p:
-        return c_void_p(int(stream) if stream else 0)
+    def _stream(stream: int) -> int | None:
+        return int(stream) if stream else None
 
     # ── turbo_prod ──────────────────────────────────────────────────── #
 
@@ -344,8 +360,8 @@ class TurboQuantWrapper:
         self._check("turbo_prod", "pack_kv", key=(key, torch.float16, thd),
                     value=(value, torch.float16, thd), slot_mapping=(slot_mapping, torch.int32, N),
                     page_pool=(page_pool, torch.uint8, 0))
-        rc = self._lib.tq_launch_turbo_prod_pack_kv(
-            self._vp(key), self._vp(value), self._i32p(slot_mapping), self._u8p(page_pool),
+        rc = self._fast.tq_launch_turbo_prod_pack_kv(
+            key.data_ptr(), value.data_ptr(), slot_mapping.data_ptr(), page_pool.data_ptr(),
             ctypes.byref(layout), ctypes.byref(cfg), N, self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, "turbo_prod", "pack_kv")
@@ -367,10 +383,10 @@ class TurboQuantWrapper:
                for n in ("k_rot", "v_rot", "kn", "vn")}
         out.update({n: torch.empty(N, H, D, dtype=torch.int32, device=key.device)
                     for n in ("kidx", "vidx")})
-        rc = self._lib.tq_launch_turbo_prod_pack_kv_debug(
-            self._vp(key), self._vp(value), self._i32p(slot_mapping), self._u8p(page_pool),
+        rc = self._fast.tq_launch_turbo_prod_pack_kv_debug(
+            key.data_ptr(), value.data_ptr(), slot_mapping.data_ptr(), page_pool.data_ptr(),
             ctypes.byref(layout), ctypes.byref(cfg), N, self._stream(stream),
-            *[self._vp(out[n]) for n in ("k_rot", "v_rot", "kn", "vn", "kidx", "vidx")])
+            *[out[n].data_ptr() for n in ("k_rot", "v_rot", "kn", "vn", "kidx", "vidx")])
         if rc != 0:
             self._kernel_raise(rc, "turbo_prod", "pack_kv")
         return out
@@ -382,9 +398,9 @@ class TurboQuantWrapper:
         self._check("turbo_prod", "dequant_kv", page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, N),
                     out_key=(out_key, torch.float16, thd), out_value=(out_value, torch.float16, thd))
-        rc = self._lib.tq_launch_turbo_prod_dequant_kv(
-            self._u8p(page_pool), self._i32p(slot_mapping), self._vp(out_key),
-            self._vp(out_value), ctypes.byref(layout), ctypes.byref(cfg), N,
+        rc = self._fast.tq_launch_turbo_prod_dequant_kv(
+            page_pool.data_ptr(), slot_mapping.data_ptr(), out_key.data_ptr(),
+            out_value.data_ptr(), ctypes.byref(layout), ctypes.byref(cfg), N,
             self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, "turbo_prod", "dequant_kv")
@@ -399,8 +415,8 @@ class TurboQuantWrapper:
                     page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, num_kv_tokens),
                     logits=(logits, torch.float32, num_queries * H * num_kv_tokens))
-        rc = self._lib.tq_launch_turbo_prod_fused_attention_logits(
-            self._vp(query), self._u8p(page_pool), self._i32p(slot_mapping), self._f32p(logits),
+        rc = self._fast.tq_launch_turbo_prod_fused_attention_logits(
+            query.data_ptr(), page_pool.data_ptr(), slot_mapping.data_ptr(), logits.data_ptr(),
             ctypes.byref(layout), ctypes.byref(cfg), num_queries, num_kv_tokens,
             self._stream(stream))
         if rc != 0:
@@ -415,8 +431,8 @@ class TurboQuantWrapper:
                     page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, num_kv_tokens),
                     output=(output, torch.float16, num_queries * H * D))
-        rc = self._lib.tq_launch_turbo_prod_fused_attention_output(
-            self._vp(query), self._u8p(page_pool), self._i32p(slot_mapping), self._vp(output),
+        rc = self._fast.tq_launch_turbo_prod_fused_attention_output(
+            query.data_ptr(), page_pool.data_ptr(), slot_mapping.data_ptr(), output.data_ptr(),
             ctypes.byref(layout), ctypes.byref(cfg), num_queries, num_kv_tokens,
             self._stream(stream))
         if rc != 0:
@@ -433,8 +449,8 @@ class TurboQuantWrapper:
                     page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, num_kv_tokens),
                     output=(output, torch.float16, num_queries * H * D))
-        rc = self._lib.tq_launch_turbo_prod_fused_attention_output_noalloc(
-            self._vp(query), self._u8p(page_pool), self._i32p(slot_mapping), self._vp(output),
+        rc = self._fast.tq_launch_turbo_prod_fused_attention_output_noalloc(
+            query.data_ptr(), page_pool.data_ptr(), slot_mapping.data_ptr(), output.data_ptr(),
             ctypes.byref(layout), ctypes.byref(cfg), num_queries, num_kv_tokens,
             self._stream(stream))
         if rc != 0:
@@ -448,8 +464,8 @@ class TurboQuantWrapper:
         self._check("turbo_mse", "pack_kv", key=(key, torch.float16, thd),
                     value=(value, torch.float16, thd), slot_mapping=(slot_mapping, torch.int32, N),
                     page_pool=(page_pool, torch.uint8, 0))
-        rc = self._lib.tq_launch_turbo_mse_pack_kv(
-            self._vp(key), self._vp(value), self._i32p(slot_mapping), self._u8p(page_pool),
+        rc = self._fast.tq_launch_turbo_mse_pack_kv(
+            key.data_ptr(), value.data_ptr(), slot_mapping.data_ptr(), page_pool.data_ptr(),
             ctypes.byref(layout), ctypes.byref(cfg), N, self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, "turbo_mse", "pack_kv")
@@ -461,9 +477,9 @@ class TurboQuantWrapper:
         self._check("turbo_mse", "dequant_kv", page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, N),
                     out_key=(out_key, torch.float16, thd), out_value=(out_value, torch.float16, thd))
-        rc = self._lib.tq_launch_turbo_mse_dequant_kv(
-            self._u8p(page_pool), self._i32p(slot_mapping), self._vp(out_key),
-            self._vp(out_value), ctypes.byref(layout), ctypes.byref(cfg), N,
+        rc = self._fast.tq_launch_turbo_mse_dequant_kv(
+            page_pool.data_ptr(), slot_mapping.data_ptr(), out_key.data_ptr(),
+            out_value.data_ptr(), ctypes.byref(layout), ctypes.byref(cfg), N,
             self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, "turbo_mse", "dequant_kv")
@@ -476,8 +492,8 @@ class TurboQuantWrapper:
                     page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, num_kv_tokens),
                     output=(output, torch.float16, num_queries * H * D))
-        rc = self._lib.tq_launch_turbo_mse_fused_attention_output(
-            self._vp(query), self._u8p(page_pool), self._i32p(slot_mapping), self._vp(output),
+        rc = self._fast.tq_launch_turbo_mse_fused_attention_output(
+            query.data_ptr(), page_pool.data_ptr(), slot_mapping.data_ptr(), output.data_ptr(),
             ctypes.byref(layout), ctypes.byref(cfg), num_queries, num_kv_tokens,
             self._stream(stream))
         if rc != 0:
@@ -491,10 +507,10 @@ class TurboQuantWrapper:
         self._check(scheme, "dequant_kv_hnd", page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, num_tokens),
                     out_key=(out_key, torch.float16, thd), out_value=(out_value, torch.float16, thd))
-        fn = (self._lib.tq_launch_turbo_prod_dequant_kv_hnd if scheme == "turbo_prod"
-              else self._lib.tq_launch_turbo_mse_dequant_kv_hnd)
-        rc = fn(self._u8p(page_pool), self._i32p(slot_mapping), self._vp(out_key),
-                self._vp(out_value), ctypes.byref(layout), ctypes.byref(cfg), num_tokens,
+        fn = (self._fast.tq_launch_turbo_prod_dequant_kv_hnd if scheme == "turbo_prod"
+              else self._fast.tq_launch_turbo_mse_dequant_kv_hnd)
+        rc = fn(page_pool.data_ptr(), slot_mapping.data_ptr(), out_key.data_ptr(),
+                out_value.data_ptr(), ctypes.byref(layout), ctypes.byref(cfg), num_tokens,
                 self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, scheme, "dequant_kv_hnd")
@@ -519,20 +535,21 @@ class TurboQuantWrapper:
             raise ValueError("pack_layers: one key, value and pool per layer")
         num_tokens = keys[0].shape[0] if n else 0
         thd = num_tokens * cfg.num_kv_heads * cfg.head_dim
+        ks = _ready_pointers(keys, torch.float16, thd)
+        vs = _ready_pointers(values, torch.float16, thd)
+        pools = _ready_pointers(page_pools, torch.uint8, 0)
+        ready = ks and vs and pools and _ready(slot_mapping, torch.int32, num_tokens)
         for l in range(n):
-            self._check(scheme, "pack_kv_layers", key=(keys[l], torch.float16, thd),
-                        value=(values[l], torch.float16, thd),
-                        slot_mapping=(slot_mapping, torch.int32, num_tokens),
-                        page_pool=(page_pools[l], torch.uint8, 0))
+            if not ready:
+                self._check(scheme, "pack_kv_layers", key=(keys[l], torch.float16, thd),
+                            value=(values[l], torch.float16, thd),
+                            slot_mapping=(slot_mapping, torch.int32, num_tokens),
+                            page_pool=(page_pools[l], torch.uint8, 0))
             if keys[l].shape[0] != num_tokens:
                 raise ValueError("pack_layers: every layer has the same number of tokens")
-        arr = c_void_p * max(n, 1)
-        ks = arr(*[t.data_ptr() for t in keys])
-        vs = arr(*[t.data_ptr() for t in values])
-        pools = arr(*[p.data_ptr() for p in page_pools])
-        fn = (self._lib.tq_launch_turbo_prod_pack_kv_layers if scheme == "turbo_prod"
-              else self._lib.tq_launch_turbo_mse_pack_kv_layers)
-        rc = fn(ks, vs, self._i32p(slot_mapping), pools, n, ctypes.byref(layout),
+        fn = (self._fast.tq_launch_turbo_prod_pack_kv_layers if scheme == "turbo_prod"
+              else self._fast.tq_launch_turbo_mse_pack_kv_layers)
+        rc = fn(ks, vs, slot_mapping.data_ptr(), pools, n, ctypes.byref(layout),
                 ctypes.byref(cfg), num_tokens, self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, scheme, "pack_kv_layers")
@@ -547,18 +564,18 @@ class TurboQuantWrapper:
         if not (len(out_keys) == len(out_values) == n):
             raise ValueError("dequant_layers: one pool and two outputs per layer")
         thd = num_tokens * cfg.num_kv_heads * cfg.head_dim
-        for l in range(n):
-            self._check(scheme, "dequant_kv_layers", page_pool=(page_pools[l], torch.uint8, 0),
-                        slot_mapping=(slot_mapping, torch.int32, num_tokens),
-                        out_key=(out_keys[l], torch.float16, thd),
-                        out_value=(out_values[l], torch.float16, thd))
-        arr = c_void_p * max(n, 1)
-        pools = arr(*[p.data_ptr() for p in page_pools])
-        ks = arr(*[t.data_ptr() for t in out_keys])
-        vs = arr(*[t.data_ptr() for t in out_values])
-        fn = (self._lib.tq_launch_turbo_prod_dequant_kv_layers if scheme == "turbo_prod"
-              else self._lib.tq_launch_turbo_mse_dequant_kv_layers)
-        rc = fn(pools, self._i32p(slot_mapping), ks, vs, n, ctypes.byref(layout),
+        pools = _ready_pointers(page_pools, torch.uint8, 0)
+        ks = _ready_pointers(out_keys, torch.float16, thd)
+        vs = _ready_pointers(out_values, torch.float16, thd)
+        if not (ks and vs and pools and _ready(slot_mapping, torch.int32, num_tokens)):
+            for l in range(n):
+                self._check(scheme, "dequant_kv_layers", page_pool=(page_pools[l], torch.uint8, 0),
+                            slot_mapping=(slot_mapping, torch.int32, num_tokens),
+                            out_key=(out_keys[l], torch.float16, thd),
+                            out_value=(out_values[l], torch.float16, thd))
+        fn = (self._fast.tq_launch_turbo_prod_dequant_kv_layers if scheme == "turbo_prod"
+              else self._fast.tq_launch_turbo_mse_dequant_kv_layers)
+        rc = fn(pools, slot_mapping.data_ptr(), ks, vs, n, ctypes.byref(layout),
                 ctypes.byref(cfg), num_tokens, int(head_major), self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, scheme, "dequant_kv_layers")
@@ -576,22 +593,24 @@ class TurboQuantWrapper:
         thd = num_tokens * cfg.num_kv_heads * cfg.head_dim
         for l in range(L):
             hp = host_pools[l]
-            if hp.device.type != "cpu" or hp.dtype != torch.uint8 or not hp.is_contiguous() \
+            if not hp.is_cpu or hp.dtype != torch.uint8 or not hp.is_contiguous() \
                     or hp.numel() != nbytes:
                 raise ValueError(f"{scheme} load_layers: host_pools[{l}] must be a contiguous "
                                  f"CPU uint8 tensor of {nbytes} bytes")
-            self._check(scheme, "load_layers", device_pool=(device_pools[l], torch.uint8, nbytes),
-                        out_key=(out_keys[l], torch.float16, thd),
-                        out_value=(out_values[l], torch.float16, thd))
+        dps = _ready_pointers(device_pools, torch.uint8, nbytes)
+        oks = _ready_pointers(out_keys, torch.float16, thd)
+        ovs = _ready_pointers(out_values, torch.float16, thd)
+        if not (dps and oks and ovs):
+            for l in range(L):
+                self._check(scheme, "load_layers",
+                            device_pool=(device_pools[l], torch.uint8, nbytes),
+                            out_key=(out_keys[l], torch.float16, thd),
+                            out_value=(out_values[l], torch.float16, thd))
         self._check(scheme, "load_layers", slot_mapping=(slot_mapping, torch.int32, num_tokens))
-        arr = c_void_p * max(L, 1)
-        hps = arr(*[t.data_ptr() for t in host_pools])
-        dps = arr(*[t.data_ptr() for t in device_pools])
-        oks = arr(*[t.data_ptr() for t in out_keys])
-        ovs = arr(*[t.data_ptr() for t in out_values])
-        fn = (self._lib.tq_load_turbo_prod_layers if scheme == "turbo_prod"
-              else self._lib.tq_load_turbo_mse_layers)
-        rc = fn(hps, dps, nbytes, L, self._i32p(slot_mapping), num_tokens, oks, ovs,
+        hps = (c_void_p * max(L, 1))(*[t.data_ptr() for t in host_pools])
+        fn = (self._fast.tq_load_turbo_prod_layers if scheme == "turbo_prod"
+              else self._fast.tq_load_turbo_mse_layers)
+        rc = fn(hps, dps, nbytes, L, slot_mapping.data_ptr(), num_tokens, oks, ovs,
                 ctypes.byref(layout), ctypes.byref(cfg), self._stream(copy_stream),
                 self._stream(compute_stream))
         if rc != 0:
@@ -617,11 +636,11 @@ class TurboQuantWrapper:
                     row_seq=(row_seq, torch.int32, num_rows),
                     row_kv_len=(row_kv_len, torch.int32, num_rows),
                     output=(output, torch.float16, num_rows * H * D))
-        fn = (self._lib.tq_launch_turbo_prod_paged_attention if scheme == "turbo_prod"
-              else self._lib.tq_launch_turbo_mse_paged_attention)
-        rc = fn(self._vp(query), self._u8p(page_pool), self._i32p(block_tables),
-                block_tables.shape[1], self._i32p(row_seq), self._i32p(row_kv_len),
-                self._vp(output), ctypes.byref(layout), ctypes.byref(cfg), num_rows, max_kv_len,
+        fn = (self._fast.tq_launch_turbo_prod_paged_attention if scheme == "turbo_prod"
+              else self._fast.tq_launch_turbo_mse_paged_attention)
+        rc = fn(query.data_ptr(), page_pool.data_ptr(), block_tables.data_ptr(),
+                block_tables.shape[1], row_seq.data_ptr(), row_kv_len.data_ptr(),
+                output.data_ptr(), ctypes.byref(layout), ctypes.byref(cfg), num_rows, max_kv_len,
                 self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, scheme, "paged_attn_output")
@@ -652,8 +671,8 @@ class TurboQuantWrapper:
         self._check(scheme, "pack_kv", key=(key, torch.float16, thd),
                     value=(value, torch.float16, thd), slot_mapping=(slot_mapping, torch.int32, N),
                     page_pool=(page_pool, torch.uint8, 0))
-        rc = getattr(self._lib, fn)(self._vp(key), self._vp(value), self._i32p(slot_mapping),
-                                    self._u8p(page_pool), ctypes.byref(layout), ctypes.byref(cfg),
+        rc = getattr(self._fast, fn)(key.data_ptr(), value.data_ptr(), slot_mapping.data_ptr(),
+                                    page_pool.data_ptr(), ctypes.byref(layout), ctypes.byref(cfg),
                                     N, self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, scheme, "pack_kv")
@@ -665,8 +684,8 @@ class TurboQuantWrapper:
         self._check(scheme, "dequant_kv", page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, N),
                     out_key=(out_key, torch.float16, thd), out_value=(out_value, torch.float16, thd))
-        rc = getattr(self._lib, fn)(self._u8p(page_pool), self._i32p(slot_mapping),
-                                    self._vp(out_key), self._vp(out_value), ctypes.byref(layout),
+        rc = getattr(self._fast, fn)(page_pool.data_ptr(), slot_mapping.data_ptr(),
+                                    out_key.data_ptr(), out_value.data_ptr(), ctypes.byref(layout),
                                     ctypes.byref(cfg), N, self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, scheme, "dequant_kv")
@@ -689,8 +708,8 @@ class TurboQuantWrapper:
                     page_pool=(page_pool, torch.uint8, 0),
                     slot_mapping=(slot_mapping, torch.int32, num_kv_tokens),
                     output=(output, torch.float16, num_queries * H * D))
-        rc = self._lib.tq_launch_qjl_fused_attention_output(
-            self._vp(query), self._u8p(page_pool), self._i32p(slot_mapping), self._vp(output),
+        rc = self._fast.tq_launch_qjl_fused_attention_output(
+            query.data_ptr(), page_pool.data_ptr(), slot_mapping.data_ptr(), output.data_ptr(),
             ctypes.byref(layout), ctypes.byref(cfg), num_queries, num_kv_tokens,
             self._stream(stream))
         if rc != 0:
@@ -726,9 +745,9 @@ class TurboQuantWrapper:
                     output=(output, torch.float16, num_queries * H * D),
                     logit_scratch=(logit_scratch, torch.float32,
                                    num_queries * H * num_kv_tokens))
-        rc = self._lib.tq_launch_attention_ref(
-            self._vp(query), self._vp(key), self._vp(value), self._vp(output),
-            self._f32p(logit_scratch), ctypes.byref(cfg), num_queries, num_kv_tokens,
+        rc = self._fast.tq_launch_attention_ref(
+            query.data_ptr(), key.data_ptr(), value.data_ptr(), output.data_ptr(),
+            logit_scratch.data_ptr(), ctypes.byref(cfg), num_queries, num_kv_tokens,
             self._stream(stream))
         if rc != 0:
             self._kernel_raise(rc, "sdpa", "attention_ref")
