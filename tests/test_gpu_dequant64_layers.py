@@ -1,0 +1,60 @@
+"""Multi-layer dequant at head_dim 64 (a row per lane, one launch per 64
+layers): edges of a wave's 64 rows, more layers than a launch takes, unmapped
+tokens, division paths and buffers that fall back to the per-layer kernels,
+bit-exact against the oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from turborag_amd.synthetic import as_u16, kv_tokens_major, permuted_slots
+
+pytestmark = pytest.mark.gpu
+D = 64
+
+
+@pytest.mark.parametrize("scheme,NL,N,H,B,head_major,holes,shift", [
+    ("turbo_prod", 2, 32, 2, 16, False, False, 0),   # one wave's rows exactly
+    ("turbo_mse", 3, 33, 2, 16, True, False, 0),     # and two more
+    ("turbo_prod", 5, 777, 3, 8, True, True, 0),     # 3 heads: division paths
+    ("turbo_mse", 66, 65, 1, 16, False, True, 0),    # two launches
+    ("turbo_mse", 2, 300, 2, 7, False, True, 0),     # 7-token blocks
+    ("turbo_prod", 2, 300, 1, 7, False, False, 0),   # 490-byte pages: the per-layer kernels
+    ("turbo_prod", 2, 300, 2, 16, False, False, 4),  # pools not 16-byte aligned: likewise
+])
+def test_layers(tq, oracle, cuda, scheme, NL, N, H, B, head_major, holes, shift):
+    print(f"[dequant64 layers {scheme}] {NL} x {N} H={H} B={B} head_major={head_major}", flush=True)
+    prod = scheme == "turbo_prod"
+    cfg = tq.default_config()
+    cfg.num_kv_heads, cfg.head_dim, cfg.block_size = H, D, B
+    lay = tq.make_layout_for(cfg) if prod else tq.make_mse_layout_for(cfg)
+    slots = permuted_slots(N, B, seed=660 + N)
+    pages = int(slots.max()) // B + 1
+    pack = oracle.prod_pack if prod else oracle.mse_pack
+    pools_np = []
+    for layer in range(NL):
+        k, v = kv_tokens_major(N, H, D, seed=661 + layer)
+        pools_np.append(pack(as_u16(k), as_u16(v), slots.numpy(), pages, B))
+    if holes:
+        slots[::5] = -1
+    pools = []
+    for p in pools_np:
+        buf = torch.zeros(p.size + shift, dtype=torch.uint8, device=cuda)
+        buf[shift:] = torch.from_numpy(p).to(cuda)
+        pools.append(buf[shift:])
+    shape = (1, H, N, D) if head_major else (N, H, D)
+    oks = [torch.full(shape, 7.0, dtype=torch.float16, device=cuda) for _ in range(NL)]
+    ovs = [torch.full(shape, 7.0, dtype=torch.float16, device=cuda) for _ in range(NL)]
+    tq.dequant_layers(scheme, pools, slots.to(cuda), oks, ovs, lay, cfg, N, head_major=head_major)
+    torch.cuda.synchronize()
+    fn = oracle.prod_dequant if prod else oracle.mse_dequant
+    sl = slots.numpy()
+    live, seven = sl >= 0, np.float16(7.0).view(np.uint16)
+    for layer in range(NL):
+        wk, wv = fn(pools_np[layer], sl, H, D, B)
+        for got, want in ((as_u16(oks[layer]), wk), (as_u16(ovs[layer]), wv)):
+            if head_major:
+                got = got[0].transpose(1, 0, 2)
+            assert np.array_equal(got[live], want[live]), layer
+            assert np.all(got[~live] == seven), layer

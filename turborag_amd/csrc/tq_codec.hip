@@ -818,8 +818,8 @@ __global__ __launch_bounds__(kBlock) void dequant_stream_kernel(
 }
 
 // ---------------------------------------------------------------------------
-// Dequant, one row (E = 128) or half a row (E = 64) per lane (D = 128;
-// turbo_prod and turbo_mse).  With a whole row every WHT stage and both
+// Dequant, E elements of a row of HD = 128 or 64 per lane: a whole row (E = HD)
+// or half a row (E = 64, HD = 128) (turbo_prod and turbo_mse).  With a whole row every WHT stage and both
 // decode tables stay inside the lane: no cross-lane butterfly (a DPP move
 // plus an fmac per value per stage) and one table build per row instead of
 // one per lane of a row: 45 VALU instructions per row against 72 for the
@@ -834,6 +834,11 @@ __global__ __launch_bounds__(kBlock) void dequant_stream_kernel(
 // store r of the wave writes the lines of lanes 8r .. 8r + 7, eight whole
 // lines per buffer store.  Waves walk (layer, row group) pairs grid-stride
 // with the next pair's slot, codes and scales in flight.
+// HD = 64 (one line per row) serves the multi-layer launches only: a single
+// layer has too few row groups to fill the chip at a row per lane, and stays
+// with dequant_stream_kernel's two lanes per row.  8 layers of 32,768 tokens x
+// 2 heads at HD = 64 in one launch: 31.3 us, 5.5 TB/s (68.8 us as launches of
+// the stream kernel); 24 layers of 8,192: 58.3 us host-bound (168.5).
 // ---------------------------------------------------------------------------
 constexpr int kRowStageBytes = 144;  // staged bytes per lane: one output line + 16 of pad
 // The row kernels store through buffer descriptors of a layer's output,
@@ -841,7 +846,7 @@ constexpr int kRowStageBytes = 144;  // staged bytes per lane: one output line +
 // the end of every buffer the launchers allow (rows up to kBufMaxRows), so
 // the hardware's range check drops its stores without a branch.
 constexpr uint32_t kBufSkip = 0x80000000u;
-constexpr int kBufMaxRows = (int)(kBufSkip / 256u) - 1;
+constexpr int kBufMaxRows = (int)(kBufSkip / 256u) - 1;  // (head_dim 64, 128-byte rows: the same limit)
 constexpr uint32_t kBufWord3 = 0x00020000u;  // descriptor word 3 on gfx9: 32-bit data format
 // Row-per-lane dequant: staged output lines (and their row offsets) read
 // from LDS this many stores ahead of the store that writes them, 1..7 (36
@@ -853,7 +858,7 @@ constexpr uint32_t kBufWord3 = 0x00020000u;  // descriptor word 3 on gfx9: 32-bi
 constexpr int kStoreAhead = TQ_DEQ_STORE_AHEAD;
 static_assert(kStoreAhead >= 1 && kStoreAhead <= 7, "1 to 7 stores ahead");
 
-template <int SCH, int ML, int E>
+template <int SCH, int ML, int E, int HD = 128>
 __global__ __launch_bounds__(kBlock, 2) void dequant_rows_kernel(
     const LayerSet<ML> layers, const int32_t* __restrict__ slots, PageGeom g, int num_rows,
     int num_layers, float inv, OutLayout ol) {
@@ -862,8 +867,9 @@ __global__ __launch_bounds__(kBlock, 2) void dequant_rows_kernel(
     // E = 128: lane l owns row l of the group's 64; E = 64: lanes 2r and
     // 2r + 1 own halves 0 and 1 (elements 64j .. 64j + 63) of row r of 32, and
     // the last WHT stage (len = 64) pairs them across the lane pair.
-    static_assert(E == 128 || E == 64, "a whole row or half a row per lane");
-    constexpr int LPR = 128 / E;   // lanes per row
+    static_assert(HD == 128 || HD == 64, "head_dim 128 or 64");
+    static_assert((E == 128 || E == 64) && E <= HD, "a whole row or half a row per lane");
+    constexpr int LPR = HD / E;    // lanes per row
     constexpr int RPG = 64 / LPR;  // rows per wave group
     constexpr int NQ = E / 32;     // 16-byte code loads per tensor and lane
     constexpr int kWaves = kBlock / 64;
@@ -957,7 +963,7 @@ __global__ __launch_bounds__(kBlock, 2) void dequant_rows_kernel(
     // elements 64j + 8(4q + e) .. + 7).
     auto load_codes = [&](const Loc& c, uint64_t off, uint4 (&w)[NQ]) {
         const uint4* p = reinterpret_cast<const uint4*>(
-            c.live ? c.base + off + (size_t)c.cell * 64 + 32 * half_j : c.dummy);
+            c.live ? c.base + off + (size_t)c.cell * (HD / 2) + 32 * half_j : c.dummy);
 #pragma unroll
         for (int q = 0; q < NQ; ++q) w[q] = p[q];
     };
@@ -1090,10 +1096,10 @@ __global__ __launch_bounds__(kBlock, 2) void dequant_rows_kernel(
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
         const float se = (h & 1) ? -inv : inv;  // s(2j, h) * inv; s(2j+1, h) = -s(2j, h)
-        // The layer's K and V outputs as buffers of num_rows * 256 bytes
+        // The layer's K and V outputs as buffers of num_rows * 2 HD bytes
         // (below kBufSkip: the launchers' row limit).
         const int lyr = __builtin_amdgcn_readfirstlane(cur.layer);
-        const uint32_t out_bytes = (uint32_t)num_rows * 256u;
+        const uint32_t out_bytes = (uint32_t)num_rows * (2u * HD);
         transform(kw, 0, se,
                   __builtin_amdgcn_make_buffer_rsrc(layers.out_key[lyr], 0, out_bytes, kBufWord3));
         load_codes(nxt, g.kc_off, kw);
@@ -1109,8 +1115,8 @@ __global__ __launch_bounds__(kBlock, 2) void dequant_rows_kernel(
 // The row-per-lane kernel reads codes as 16-byte pieces.
 bool rows_dequant_ok(const PageGeom& g, const void* pool, const void* ok, const void* ov) {
     const auto al = [](uint64_t v, uint64_t a) { return (v & (a - 1)) == 0; };
-    return g.D == 128 && g.code_stride == 64 && al(g.page_size, 16) && al(g.kc_off, 16) &&
-           al(g.vc_off, 16) && al(g.ks_off, 2) && al(g.vs_off, 2) && al(g.kres_off, 2) &&
+    return (g.D == 128 || g.D == 64) && g.code_stride == g.D / 2 && al(g.page_size, 16) &&
+           al(g.kc_off, 16) && al(g.vc_off, 16) && al(g.ks_off, 2) && al(g.vs_off, 2) && al(g.kres_off, 2) &&
            al(reinterpret_cast<uintptr_t>(pool), 16) &&
            al(reinterpret_cast<uintptr_t>(ok), 16) && al(reinterpret_cast<uintptr_t>(ov), 16);
 }
@@ -1316,7 +1322,7 @@ void launch_dequant(Scheme s, const uint8_t* pool, const int32_t* slots, uint16_
     // D = 128 with 16-byte aligned codes: half a row per lane (2,048 waves
     // for a 32K-token, two-head layer: two per SIMD; 9.8 against 10.05 us for
     // the four-lanes-per-row kernel, 12.8 for a whole row per lane).
-    if (rows <= kBufMaxRows && rows_dequant_ok(g, pool, out_key, out_value)) {
+    if (g.D == 128 && rows <= kBufMaxRows && rows_dequant_ok(g, pool, out_key, out_value)) {
         constexpr int E1 = 64;
         const int rows_per_block = kBlock * E1 / 128;
         const int blocks_needed = (rows + rows_per_block - 1) / rows_per_block;
@@ -1370,10 +1376,16 @@ void launch_dequant_layers(Scheme s, const uint8_t* const* pools, const int32_t*
                            int num_tokens, int num_layers, hipStream_t stream, bool head_major) {
     const int rows = num_tokens * g.H;
     if (rows <= 0 || num_layers <= 0) return;
-    bool wide = g.D == 128;
+    // A whole row per lane when every layer's buffers allow 16-byte code
+    // loads (D = 128, half a row per lane: 9.1 against 8.0 us per 32K-token
+    // layer).
+    bool rows_ok = rows <= kBufMaxRows;
+    for (int l = 0; l < num_layers && rows_ok; ++l)
+        rows_ok = rows_dequant_ok(g, pools[l], out_key[l], out_value[l]);
+    bool wide = g.D == 128 || rows_ok;
     for (int l = 0; l < num_layers && wide; ++l)
         wide = wide_dequant_ok(g, pools[l], out_key[l], out_value[l]);
-    if (!wide) {  // the per-layer kernels (other head dims, unaligned buffers)
+    if (!wide || num_layers == 1) {  // the per-layer kernels (other head dims, unaligned buffers)
         for (int l = 0; l < num_layers; ++l)
             launch_dequant(s, pools[l], slots, out_key[l], out_value[l], g, num_tokens, stream,
                            head_major);
@@ -1384,11 +1396,6 @@ void launch_dequant_layers(Scheme s, const uint8_t* const* pools, const int32_t*
     ol.tok = head_major ? (uint64_t)g.D : (uint64_t)g.H * g.D;
     ol.head = head_major ? (uint64_t)num_tokens * g.D : (uint64_t)g.D;
     const bool prod = s == Scheme::Prod;
-    // A whole row per lane when every layer's buffers allow 16-byte code
-    // loads (half a row per lane: 9.1 against 8.0 us per 32K-token layer).
-    bool rows_ok = rows <= kBufMaxRows;
-    for (int l = 0; l < num_layers && rows_ok; ++l)
-        rows_ok = rows_dequant_ok(g, pools[l], out_key[l], out_value[l]);
     const int rows_per_block = rows_ok ? kBlock : kBlock / (g.D / 32);
     // The kernel counts (layer, row group) pairs in int32: keep them below 2^30.
     const int groups = (rows + 15) / 16;
@@ -1407,19 +1414,17 @@ void launch_dequant_layers(Scheme s, const uint8_t* const* pools, const int32_t*
         const int per_cu = rows_ok ? TQ_DEQ_ROWS_BLOCKS_PER_CU : TQ_DEQ_LAYERS_BLOCKS_PER_CU;
         const dim3 grid((unsigned)std::max(
             1LL, std::min<long long>(blocks_needed, (long long)per_cu * num_cus())));
-        if (rows_ok) {
-            if (prod)
-                hipLaunchKernelGGL((dequant_rows_kernel<1, kMaxLayersPerLaunch, 128>), grid,
-                                   dim3(kBlock), 0, stream, set, slots, g, rows, n, inv, ol);
-            else
-                hipLaunchKernelGGL((dequant_rows_kernel<0, kMaxLayersPerLaunch, 128>), grid,
-                                   dim3(kBlock), 0, stream, set, slots, g, rows, n, inv, ol);
-        } else if (prod)
-            hipLaunchKernelGGL((dequant_stream_kernel<128, 1, kMaxLayersPerLaunch>), grid,
-                               dim3(kBlock), 0, stream, set, slots, g, rows, n, inv, ol);
+        auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, stream, set, slots, g, rows, n, inv,
+                               ol);
+        };
+        constexpr int ML = kMaxLayersPerLaunch;
+        if (rows_ok && g.D == 64)
+            prod ? go(dequant_rows_kernel<1, ML, 64, 64>) : go(dequant_rows_kernel<0, ML, 64, 64>);
+        else if (rows_ok)
+            prod ? go(dequant_rows_kernel<1, ML, 128>) : go(dequant_rows_kernel<0, ML, 128>);
         else
-            hipLaunchKernelGGL((dequant_stream_kernel<128, 0, kMaxLayersPerLaunch>), grid,
-                               dim3(kBlock), 0, stream, set, slots, g, rows, n, inv, ol);
+            prod ? go(dequant_stream_kernel<128, 1, ML>) : go(dequant_stream_kernel<128, 0, ML>);
         check_launch(prod ? "turbo_prod_dequant_kv_layers" : "turbo_mse_dequant_kv_layers");
     }
 }
