@@ -26,6 +26,7 @@ B = 16
     ("turbo_mse", 32, 64, 1025, True),     # four
     ("turbo_prod", 33, 64, 1500, False),   # four and one
     ("turbo_mse", 41, 64, 2000, False),    # four and two
+    ("turbo_prod", 33, 64, 500, True),     # one split: the units write the output
 ])
 def test_units(tq, oracle, cuda, scheme, Q, H, N, holes, D):
     print(f"[decode rows {scheme}] Q={Q} H={H} N={N} D={D}", flush=True)

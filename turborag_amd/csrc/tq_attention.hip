@@ -1301,8 +1301,8 @@ __device__ __forceinline__ float lane_sign(int j) {
 template <int SCH, int D, bool PAGED>
 __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
     const uint16_t* __restrict__ query, const uint8_t* __restrict__ pool,
-    const int32_t* __restrict__ slots, float* __restrict__ ws, float2* __restrict__ pml, float inv,
-    int num_queries, int num_kv_tokens, int tokens_per_split, int num_splits, PageGeom g,
+    const int32_t* __restrict__ slots, float* __restrict__ ws, float2* __restrict__ pml,
+    uint16_t* __restrict__ output, float inv, int num_queries, int num_kv_tokens, int tokens_per_split, int num_splits, PageGeom g,
     PagedRows pr) {
     constexpr bool PROD = SCH == kSchProd;
     static_assert(SCH == kSchProd || SCH == kSchMse, "turbo_prod or turbo_mse pages");
@@ -1975,7 +1975,17 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                               : ws + ((it * num_splits + pid) * kRows + w) * D;
             float2* pm2 = PAGED ? reinterpret_cast<float2*>(po + D)
                                 : pml + (it * kRows + w) * num_splits + pid;
-            if (keep) {
+            if (!PAGED && num_splits == 1) {  // nothing to merge: the output itself
+                uint16_t* out = output + ((size_t)(rg * kRows + r) * g.H + h) * D + 4 * j16;
+                const auto fin = [&](float x) { return (uint32_t)f2h(L > 0.f ? x / L : x); };
+                if (keep) {
+#pragma unroll
+                    for (int k = 0; k < kE; k += 4)
+                        *reinterpret_cast<uint2*>(out + 16 * k) =
+                            make_uint2(fin(o[k] * s0) | (fin(o[k + 1] * -s0) << 16),
+                                       fin(o[k + 2] * s0) | (fin(o[k + 3] * -s0) << 16));
+                }
+            } else if (keep) {
 #pragma unroll
                 for (int k = 0; k < kE; k += 4)
                     *reinterpret_cast<float4*>(po + 4 * j16 + 16 * k) =
@@ -2573,8 +2583,8 @@ template <int SCH, int D>
 __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     const uint16_t* __restrict__ query, const uint8_t* __restrict__ pool,
     const int32_t* __restrict__ slots, float* __restrict__ po, float2* __restrict__ pml,
-    float inv, int num_queries, int num_kv_tokens, int tokens_per_split, int num_splits,
-    PageGeom g) {
+    uint16_t* __restrict__ output, float inv, int num_queries, int num_kv_tokens,
+    int tokens_per_split, int num_splits, PageGeom g) {
     constexpr bool PROD = SCH == kSchProd;
     static_assert(SCH == kSchProd || SCH == kSchMse, "turbo_prod or turbo_mse pages");
     static_assert(D == 128 || D == 64, "head_dim 64 or 128");
@@ -2948,6 +2958,16 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     }
     wht_pair<kL>(o0, o1, lane);
     const float s0 = (h & 1) ? -inv : inv;
+    if (num_splits == 1) {  // nothing to merge: the output itself
+        o0 *= s0;
+        o1 *= -s0;
+        if (D == 128 || lane < kL)
+            *reinterpret_cast<uint32_t*>(
+                output + ((size_t)(rg * kRows + r) * g.H + h) * D + 2 * jl) =
+                (uint32_t)f2h(L > 0.f ? o0 / L : o0) |
+                ((uint32_t)f2h(L > 0.f ? o1 / L : o1) << 16);
+        return;
+    }
     const size_t item = (size_t)rg * g.H + h;
     const size_t pid = item * num_splits + split;
     if (D == 128 || lane < kL)
@@ -3132,23 +3152,28 @@ struct SplitCost {
     int setup, pass;
 };
 constexpr SplitCost kGroupCost{51, 20}, kPairCost{60, 22}, kUnitCost{78, 33};
+// The merge launch, which a single split does without (its kernel writes the
+// output: 64-250 tokens 11.8 -> 6.2 us per call, 500 tokens 11.8 -> 7.2-7.6).
+constexpr int kMergeCost = 30;
 // The split count and its cost: one workgroup runs on a CU at a time, so of
-// the counts that fill one to four rounds of the CUs the cheapest is taken
-// (the fewest splits among equals: the merge reads every split's partials).
+// the counts that fill one to four rounds of the CUs, and one split, the
+// cheapest is taken (the fewest splits among equals: the merge reads every
+// split's partials).
 struct SplitChoice {
     int splits;
     long long cost;
 };
 SplitChoice choose_splits(int items, int passes, SplitCost c, int most, int cus) {
-    SplitChoice best{1, -1};
+    const long long whole = ((long long)items + cus - 1) / cus * (c.setup + (long long)c.pass * passes);
+    SplitChoice best{1, whole};
     for (int r = 1; r <= 4; ++r) {
         int s = std::min({std::max(1, (int)((long long)r * cus / items)), passes, most});
         const int per = (passes + s - 1) / s;
         s = (passes + per - 1) / per;
         const long long rounds = ((long long)items * s + cus - 1) / cus;
-        const long long cost = rounds * (c.setup + (long long)c.pass * per);
-        if (best.cost < 0 || cost < best.cost || (cost == best.cost && s < best.splits))
-            best = {s, cost};
+        const long long cost =
+            rounds * (c.setup + (long long)c.pass * per) + (s > 1 ? kMergeCost : 0);
+        if (cost < best.cost || (cost == best.cost && s < best.splits)) best = {s, cost};
     }
     return best;
 }
@@ -3199,10 +3224,11 @@ void launch_decode_attention(const uint16_t* query, const uint8_t* pool, const i
     if (d.combine_blocks > INT32_MAX)
         throw Error(std::string(combine_name) + ": too many query rows");
     if (scratch.ptr) (void)scratch.get(stream, d.limit_bytes, split_name);  // throws past its limit
-    char* ws = static_cast<char*>(scratch.get(stream, d.ws_bytes, split_name));
-    float* po = reinterpret_cast<float*>(ws);
-    float2* pml = reinterpret_cast<float2*>(ws + (size_t)d.splits * d.heads * kRows * D * sizeof(float));
     const int S = num_kv_tokens > 0 ? d.splits : 0;
+    char* ws = S == 1 ? nullptr : static_cast<char*>(scratch.get(stream, d.ws_bytes, split_name));
+    float* po = reinterpret_cast<float*>(ws);
+    float2* pml = reinterpret_cast<float2*>(
+        reinterpret_cast<uintptr_t>(ws) + (size_t)d.splits * d.heads * kRows * D * sizeof(float));
     if (num_kv_tokens > 0) {
         constexpr int kMaxGridYZ = 65535;
         const int groups = d.items / g.H;  // row groups, or units of them
@@ -3211,13 +3237,14 @@ void launch_decode_attention(const uint16_t* query, const uint8_t* pool, const i
         if (d.units)
             hipLaunchKernelGGL((unit::attn_unit_split_kernel<SCH, D, false>), grid,
                                dim3(64 * unit::kWaves), 0, stream, query, pool, slots, po, pml,
-                               inv, num_queries, num_kv_tokens, d.tps, d.splits, g, PagedRows{});
+                               output, inv, num_queries, num_kv_tokens, d.tps, d.splits, g, PagedRows{});
         else
             hipLaunchKernelGGL((dec::attn_decode_split_kernel<SCH, D>), grid,
-                               dim3(64 * dec::kWaves), 0, stream, query, pool, slots, po, pml, inv,
-                               num_queries, num_kv_tokens, d.tps, d.splits, g);
+                               dim3(64 * dec::kWaves), 0, stream, query, pool, slots, po, pml, output,
+                               inv, num_queries, num_kv_tokens, d.tps, d.splits, g);
         check_launch(split_name);
     }
+    if (S == 1) return;  // (the split kernel wrote the output)
     // (no partials for an empty context: the combine writes zeros)
     const dim3 cgrid((unsigned)d.combine_blocks);
     if (S <= 16)
@@ -3316,7 +3343,7 @@ void launch_paged_units(const uint16_t* query, const uint8_t* pool, const int32_
     if (max_kv_len > 0 || self) {
         hipLaunchKernelGGL((unit::attn_unit_split_kernel<SCH, D, true>), dim3(G),
                            dim3(64 * unit::kWaves), 0, stream, query, pool, nullptr, ws, nullptr,
-                           inv_sqrt_d(D), num_rows, max_kv_len, 0, 0, g, pr);
+                           nullptr, inv_sqrt_d(D), num_rows, max_kv_len, 0, 0, g, pr);
         check_launch(prod ? "turbo_prod_paged_attn_split" : "turbo_mse_paged_attn_split");
     }
     // One wave per row, or per 128-byte line of it while that is few waves.
