@@ -115,3 +115,38 @@ def test_paged(tq, oracle, cuda, scheme, H, lens, widths):
     print(f"    {u:.2f} row-max ulps", flush=True)
     b.close()
     assert u <= 1.0
+
+
+@pytest.mark.parametrize("Q,H,N,scale", [(1, 1, 17, 1.0), (8, 2, 127, 1.0), (9, 3, 128, 1.0),
+                                         (17, 2, 1001, 1.0), (8, 2, 300, 2.0 ** 13),
+                                         (8, 2, 300, 2.0 ** -11)])
+def test_logits(tq, oracle, cuda, Q, H, N, scale):
+    """The turbo_prod logits entry on the matrix cores: wave and workgroup
+    edges, unaligned rows, unmapped tokens, query magnitudes; within 1e-5 of the
+    row's largest logit (fp32 sums of hi/lo parts: ~2^-22 per term)."""
+    print(f"[logits64] Q={Q} H={H} N={N} scale={scale:g}", flush=True)
+    k, v = kv_tokens_major(N, H, D, seed=20 + N)
+    slots = permuted_slots(N, B, seed=21 + N)
+    q = (kv_tokens_major(Q, H, D, seed=22 + N)[0].float().clamp(-7.9, 7.9) * scale)
+    d = torch.arange(D)
+    for h in range(H):  # a row whose rotation is one spike of 8 x its entries
+        q[0, h] = (1 - 2 * ((d + h) % 2)).float() * 7.9 * scale
+    q = q.half()
+    cfg = tq.default_config()
+    cfg.num_kv_heads, cfg.head_dim = H, D
+    lay = tq.make_layout_for(cfg)
+    pool = oracle.prod_pack(as_u16(k), as_u16(v), slots.numpy(), int(slots.max()) // B + 1, B)
+    if N > 100:
+        slots[::9] = -1
+    _, ref = oracle.prod_attention_f64(as_u16(q), pool, slots.numpy(), B, want_logits=True)
+    out = torch.full((Q, H, N), 7.0, device=cuda)
+    tq.fused_attn_logits(q.to(cuda), torch.from_numpy(pool).to(cuda), slots.to(cuda), out, lay, cfg,
+                         Q, N)
+    torch.cuda.synchronize()
+    got, ref = out.cpu().double().numpy().reshape(-1, N), ref.reshape(-1, N)
+    live = slots.numpy() >= 0
+    assert np.all(np.isneginf(got[:, ~live]))
+    got, ref = got[:, live], ref[:, live]
+    err = (np.abs(got - ref).max(axis=1) / np.abs(ref).max(axis=1)).max()
+    print(f"    rel err {err:.2e}", flush=True)
+    assert err < 1e-5

@@ -526,7 +526,7 @@ __device__ __forceinline__ void store_decode_tables(uint32_t* lut, int kv_words,
 }  // namespace mfma
 
 // ---------------------------------------------------------------------------
-// turbo_prod logits on the matrix cores (D = 128; :346-434, 628-648).
+// turbo_prod logits on the matrix cores (D = 64, 128; :346-434, 628-648).
 //
 // Per (token, row): logit = ks (s1 + re s2) / sqrt(D), the reference's
 // s1*ks + s2*ks*re, with s1 = sum_d q_d K3[c_d] and s2 = sum_d q_d u3_d
@@ -547,8 +547,8 @@ __device__ __forceinline__ void store_decode_tables(uint32_t* lut, int kv_words,
 // A workgroup of 8 waves takes 128 tokens of one kv head and one group of up
 // to 8 query rows; wave w takes tokens 16w .. 16w + 15 (one MFMA tile) and
 // rotates query row w.  Lane (i, g) = (lane % 16, lane / 16)
-// holds A rows of token i over dims 32g .. 32g + 31: the contraction runs
-// over the dims in the order (block kk, lane group g, e) -> dim
+// holds A rows of token i over dims 32g .. 32g + 31 (D = 128): the contraction
+// runs over the dims in the order (block kk, lane group g, e) -> dim
 // 32g + 8kk + e, so each lane's codes of a tile are one 16-byte load (code
 // dword kk = block kk).  The MFMA output lane (n, g) holds tokens 4g .. 4g + 3
 // of column n; its token scales come from lanes 16g + m (ks) and
@@ -616,13 +616,20 @@ __device__ __forceinline__ int row_bcast_i(int v) {
 }
 
 // VEC: the logits rows are 16-byte aligned and num_kv_tokens % 4 == 0.
-template <bool VEC>
+// D = 64: two blocks kk instead of four (8 code bytes per lane), and a power of
+// two per query row that holds its fp16 parts in range whatever its magnitude
+// (the fp32 kernel it replaces there took any).  8 rows x 2 heads x 32,768
+// tokens at D = 64: 4.6 us, 16 rows 6.2 us per call, against 10.2 and 18.8 for
+// one thread per (token, row).
+template <bool VEC, int D>
 __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
     const uint16_t* __restrict__ query, const uint8_t* __restrict__ pool,
     const int32_t* __restrict__ slots, float* __restrict__ logits, PageGeom g, int num_queries,
     int num_kv_tokens, float inv) {
-    constexpr int D = 128;
-    __shared__ uint32_t bq[4][64][4];  // B operands: [block kk][lane][dword], fp16 pairs
+    constexpr int kS = D / 32;           // blocks kk
+    constexpr bool QSCALE = D == 64;
+    __shared__ uint32_t bq[kS][64][4];  // B operands: [block kk][lane][dword], fp16 pairs
+    __shared__ float rsc[kRows];         // QSCALE: the rows' power of two
     // Every kernel argument the loads need, fetched in the first batch of
     // scalar loads (one wait) rather than each before its first use.
     asm volatile("" ::"s"(pool), "s"(slots), "s"(logits), "s"(g.page_size), "s"(g.kc_off),
@@ -631,6 +638,7 @@ __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
     const int nrows = min(kRows, num_queries - rg * kRows);
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const int i = lane & 15, gq = lane >> 4;
+    const int jl = lane & (D / 2 - 1);  // this lane's pair of a row
     const int t0 = blockIdx.x * kTokens + w * (kTilesW * kTile);
     // Loads first, in dependency order: the wave's two query rows (raw), the
     // slots of the lane's code token (i) and scale token (4 gq + lane % 4) of
@@ -644,7 +652,7 @@ __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
     for (int e = 0; e < kRowsW; ++e) {
         const int r = w + kWaves * e;
         qq[e] = r < nrows ? *reinterpret_cast<const uint32_t*>(
-                                query + ((size_t)(rg * kRows + r) * g.H + h) * D + 2 * lane)
+                                query + ((size_t)(rg * kRows + r) * g.H + h) * D + 2 * jl)
                           : 0u;
     }
     int slot_c[kTilesW], slot_s[kTilesW];
@@ -656,8 +664,9 @@ __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
     }
     const uint64_t dummy = reinterpret_cast<uint64_t>(query);
     const uint64_t soff = (lane & 4) ? g.kres_off : g.ks_off;
-    typedef uint32_t u32x4a4 __attribute__((ext_vector_type(4), aligned(4)));
-    u32x4 code[kTilesW];
+    typedef uint32_t codes __attribute__((ext_vector_type(kS)));
+    typedef uint32_t codes_a4 __attribute__((ext_vector_type(kS), aligned(4)));
+    codes code[kTilesW];
     uint16_t sraw[kTilesW];
 #pragma unroll
     for (int tt = 0; tt < kTilesW; ++tt) {
@@ -667,7 +676,7 @@ __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
         uint64_t ac = slot_c[tt] >= 0
                           ? reinterpret_cast<uint64_t>(pool) +
                                 (uint64_t)(uint32_t)page * (uint32_t)g.page_size + g.kc_off +
-                                (uint32_t)((tib * g.H + h) * g.code_stride + 16 * gq)
+                                (uint32_t)((tib * g.H + h) * g.code_stride + 4 * kS * gq)
                           : dummy;
         split_slot(slot_s[tt] >= 0 ? slot_s[tt] : 0, g, page, tib);
         uint64_t as = slot_s[tt] >= 0
@@ -676,28 +685,34 @@ __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
                                 (uint32_t)((tib * g.H + h) * g.scale_stride)
                           : dummy;
         asm volatile("" : "+v"(ac), "+v"(as));
-        // 16 code bytes at a 4-byte aligned address (one multi-dword load;
+        // 4 kS code bytes at a 4-byte aligned address (one multi-dword load;
         // global loads need dword alignment only).
-        code[tt] = *reinterpret_cast<const __attribute__((address_space(1))) u32x4a4*>(ac);
+        code[tt] = *reinterpret_cast<const __attribute__((address_space(1))) codes_a4*>(ac);
         sraw[tt] = *reinterpret_cast<const __attribute__((address_space(1))) uint16_t*>(as);
     }
 
     // Rotate the wave's query rows w + 8e / kWaves (sign flip, orthonormal
-    // WHT) while the codes load; lane j holds dims 2j, 2j + 1: block kk = (j % 16) / 4, lane group
-    // g = j / 16, dword j % 4 of columns 2r (hi) and 2r + 1 (lo).
+    // WHT) while the codes load; lane j holds dims 2j, 2j + 1: block kk = (j / 4) % kS, lane group
+    // g = j / (4 kS), dword j % 4 of columns 2r (hi) and 2r + 1 (lo).
     {
         const float sh = (h & 1) ? -1.0f : 1.0f;
-        const int kk = (lane & 15) >> 2, cg = 16 * (lane >> 4);
+        const int kk = (jl >> 2) & (kS - 1), cg = 16 * (jl / (4 * kS));
 #pragma unroll
         for (int e = 0; e < kRowsW; ++e) {
             float q0 = h2f(qq[e] & 0xffff) * sh, q1 = h2f(qq[e] >> 16) * (-sh);
             wht_pair<D / 2>(q0, q1, lane);
             q0 *= inv;
             q1 *= inv;
+            if constexpr (QSCALE) {
+                const int ex = scale_exp(max_lanes<D / 2>(fmaxf(fabsf(q0), fabsf(q1))));
+                q0 = __builtin_amdgcn_ldexpf(q0, -ex);
+                q1 = __builtin_amdgcn_ldexpf(q1, -ex);
+                if (lane == 0) rsc[w + kWaves * e] = __builtin_amdgcn_ldexpf(1.0f, ex);
+            }
             const uint32_t hi = pack_h2(q0, q1);
             const int col = 2 * (w + kWaves * e) + cg;
-            bq[kk][col][lane & 3] = hi;
-            bq[kk][col + 1][lane & 3] = lo_pair(q0, q1, hi);
+            bq[kk][col][jl & 3] = hi;
+            bq[kk][col + 1][jl & 3] = lo_pair(q0, q1, hi);
         }
     }
     // Register tables for the K operands (values in VGPRs: v_perm reads at
@@ -707,19 +722,20 @@ __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
     __builtin_amdgcn_sched_barrier(0);
     lds_barrier();
     __builtin_amdgcn_sched_barrier(0);
-    half8 b[4];
+    half8 b[kS];
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk)
+    for (int kk = 0; kk < kS; ++kk)
         b[kk] = __builtin_bit_cast(half8, *reinterpret_cast<const u32x4*>(bq[kk][lane]));
 
     const int r = i >> 1;
+    const float qinv = QSCALE ? inv * rsc[r] : inv;
     const bool writer = (i & 1) == 0 && r < nrows;
     float* const row_out = logits + ((size_t)(rg * kRows + r) * g.H + h) * num_kv_tokens;
 #pragma unroll
     for (int tt = 0; tt < kTilesW; ++tt) {
         f32x4 s1 = {0.f, 0.f, 0.f, 0.f}, s2 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int kk = 0; kk < 4; ++kk) {
+        for (int kk = 0; kk < kS; ++kk) {
             const AOps a = a_ops(code[tt][kk], hil, hih, lol, loh);
             s1 = mma(a.hi, b[kk], s1);
             s2 = mma(a.u3, b[kk], s2);
@@ -739,7 +755,7 @@ __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
         for (int m = 0; m < 4; ++m) {
             float x = s1[m] + rem[m] * s2[m];
             x += lane_xor<1>(x);
-            out[m] = okm[m] < 0 ? -INFINITY : x * ksm[m] * inv;
+            out[m] = okm[m] < 0 ? -INFINITY : x * ksm[m] * qinv;
         }
         const int tf = t0 + kTile * tt + 4 * gq;
         if (writer) {
@@ -3492,19 +3508,21 @@ void launch_logits(const uint16_t* query, const uint8_t* pool, const int32_t* sl
     const int tiles = (num_kv_tokens + 255) / 256;
     const float inv = inv_sqrt_d(g.D);
     const int row_groups = (num_queries + 7) / 8;
-    if (g.D == 128 && g.code_stride == 64 && (g.kc_off & 3) == 0 && (g.page_size & 3) == 0 &&
+    if ((g.D == 128 || g.D == 64) && g.code_stride == g.D / 2 && (g.kc_off & 3) == 0 && (g.page_size & 3) == 0 &&
         (g.ks_off & 1) == 0 && (g.kres_off & 1) == 0 &&
         (reinterpret_cast<uintptr_t>(pool) & 3) == 0 && g.H <= 65535 && row_groups <= 65535 &&
         g.page_size <= 0xFFFFFFFFull) {
         const bool vec = (num_kv_tokens & 3) == 0 && (reinterpret_cast<uintptr_t>(logits) & 15) == 0;
         const dim3 grid((num_kv_tokens + lgt::kTokens - 1) / lgt::kTokens, g.H, row_groups);
         const dim3 block(64 * lgt::kWaves);
-        if (vec)
-            hipLaunchKernelGGL((lgt::prod_logits_mfma_kernel<true>), grid, block, 0, stream, query,
-                               pool, slots, logits, g, num_queries, num_kv_tokens, inv);
+        const auto go = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, grid, block, 0, stream, query, pool, slots, logits, g,
+                               num_queries, num_kv_tokens, inv);
+        };
+        if (g.D == 128)
+            vec ? go(lgt::prod_logits_mfma_kernel<true, 128>) : go(lgt::prod_logits_mfma_kernel<false, 128>);
         else
-            hipLaunchKernelGGL((lgt::prod_logits_mfma_kernel<false>), grid, block, 0, stream, query,
-                               pool, slots, logits, g, num_queries, num_kv_tokens, inv);
+            vec ? go(lgt::prod_logits_mfma_kernel<true, 64>) : go(lgt::prod_logits_mfma_kernel<false, 64>);
         check_launch("turbo_prod_fused_attention_logits_kernel");
         return;
     }
