@@ -58,3 +58,35 @@ def test_layers(tq, oracle, cuda, scheme, NL, N, H, B, head_major, holes, shift)
                 got = got[0].transpose(1, 0, 2)
             assert np.array_equal(got[live], want[live]), layer
             assert np.all(got[~live] == seven), layer
+
+
+@pytest.mark.parametrize("scheme,head_major", [("turbo_prod", False), ("turbo_mse", True)])
+@pytest.mark.parametrize("N", [24575, 24576])
+def test_one_large_layer(tq, oracle, cuda, scheme, head_major, N):
+    """Both sides of the row count (49,152) from which one layer takes a row per
+    lane, with unmapped tokens."""
+    H, B = 2, 16
+    print(f"[dequant64 one layer {scheme}] N={N} head_major={head_major}", flush=True)
+    oracle.nthreads = 16
+    prod = scheme == "turbo_prod"
+    cfg = tq.default_config()
+    cfg.num_kv_heads, cfg.head_dim = H, D
+    lay = tq.make_layout_for(cfg) if prod else tq.make_mse_layout_for(cfg)
+    slots = permuted_slots(N, B, seed=680)
+    k, v = kv_tokens_major(N, H, D, seed=681)
+    pool = (oracle.prod_pack if prod else oracle.mse_pack)(as_u16(k), as_u16(v), slots.numpy(),
+                                                           int(slots.max()) // B + 1, B)
+    slots[::11] = -1
+    shape = (1, H, N, D) if head_major else (N, H, D)
+    ok = torch.full(shape, 7.0, dtype=torch.float16, device=cuda)
+    ov = torch.full_like(ok, 7.0)
+    fn = {(True, False): tq.dequant, (False, True): tq.mse_dequant_hnd}[(prod, head_major)]
+    fn(torch.from_numpy(pool).to(cuda), slots.to(cuda), ok, ov, lay, cfg,
+       *((N,) if head_major else ()))
+    torch.cuda.synchronize()
+    wk, wv = (oracle.prod_dequant if prod else oracle.mse_dequant)(pool, slots.numpy(), H, D, B)
+    live, seven = slots.numpy() >= 0, np.float16(7.0).view(np.uint16)
+    for got, want in ((as_u16(ok), wk), (as_u16(ov), wv)):
+        if head_major:
+            got = got[0].transpose(1, 0, 2)
+        assert np.array_equal(got[live], want[live]) and np.all(got[~live] == seven)

@@ -834,9 +834,9 @@ __global__ __launch_bounds__(kBlock) void dequant_stream_kernel(
 // store r of the wave writes the lines of lanes 8r .. 8r + 7, eight whole
 // lines per buffer store.  Waves walk (layer, row group) pairs grid-stride
 // with the next pair's slot, codes and scales in flight.
-// HD = 64 (one line per row) serves the multi-layer launches only: a single
-// layer has too few row groups to fill the chip at a row per lane, and stays
-// with dequant_stream_kernel's two lanes per row.  8 layers of 32,768 tokens x
+// HD = 64 (one line per row) serves the multi-layer launches and large single
+// layers; a smaller one has too few row groups to fill the chip at a row per
+// lane, and stays with dequant_stream_kernel's two lanes per row.  8 layers of 32,768 tokens x
 // 2 heads at HD = 64 in one launch: 31.3 us, 5.5 TB/s (68.8 us as launches of
 // the stream kernel); 24 layers of 8,192: 58.3 us host-bound (168.5).
 // ---------------------------------------------------------------------------
@@ -1112,6 +1112,11 @@ __global__ __launch_bounds__(kBlock, 2) void dequant_rows_kernel(
     }
 }
 
+// head_dim 64, one layer: from this many rows on a row per lane (768 waves)
+// beats the stream kernel's two lanes per row (32,768 rows: 7.0 against 6.2 us;
+// 65,536: 7.8 against 8.8; 131,072: 9.6 against 12.4).
+constexpr int kOneLayerRows64 = 3 << 14;
+
 // The row-per-lane kernel reads codes as 16-byte pieces.
 bool rows_dequant_ok(const PageGeom& g, const void* pool, const void* ok, const void* ov) {
     const auto al = [](uint64_t v, uint64_t a) { return (v & (a - 1)) == 0; };
@@ -1334,6 +1339,20 @@ void launch_dequant(Scheme s, const uint8_t* pool, const int32_t* slots, uint16_
         else
             hipLaunchKernelGGL((dequant_rows_kernel<0, 1, E1>), grid, dim3(kBlock), 0, stream, one,
                                slots, g, rows, 1, inv, ol);
+        check_launch(s == Scheme::Prod ? "turbo_prod_dequant_kv_kernel" : "turbo_mse_dequant_kv_kernel");
+        return;
+    }
+    if (g.D == 64 && rows >= kOneLayerRows64 && rows <= kBufMaxRows &&
+        rows_dequant_ok(g, pool, out_key, out_value)) {
+        const int blocks_needed = (rows + kBlock - 1) / kBlock;
+        const dim3 grid(std::min(blocks_needed, TQ_DEQ_ONE_BLOCKS_PER_CU * num_cus()));
+        const LayerSet<1> one{{pool}, {out_key}, {out_value}};
+        if (s == Scheme::Prod)
+            hipLaunchKernelGGL((dequant_rows_kernel<1, 1, 64, 64>), grid, dim3(kBlock), 0, stream,
+                               one, slots, g, rows, 1, inv, ol);
+        else
+            hipLaunchKernelGGL((dequant_rows_kernel<0, 1, 64, 64>), grid, dim3(kBlock), 0, stream,
+                               one, slots, g, rows, 1, inv, ol);
         check_launch(s == Scheme::Prod ? "turbo_prod_dequant_kv_kernel" : "turbo_mse_dequant_kv_kernel");
         return;
     }
