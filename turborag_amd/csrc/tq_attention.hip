@@ -308,9 +308,9 @@ __device__ __forceinline__ half8 as_h8(uint32_t a, uint32_t b, uint32_t c, uint3
 // at work positions [start, start + w*n) of its head's work (every head has
 // the same work, split into segments per head).
 struct PagedUnit {
-    // index: the unit's number; group_kv: in a row group's copy, the group's
-    // own longest row
-    int32_t first, npos, kv_end, start, n, w, index, group_kv;
+    // index: the unit's number; seq_kv: the unit's sequence, or in a row
+    // group's copy the group's own longest row
+    int32_t first, npos, kv_end, start, n, w, index, seq_kv;
 };
 struct PagedRows {
     const int32_t* block_tables;
@@ -1143,10 +1143,10 @@ __device__ __forceinline__ int pass_weight(int npos) { return npos > 2 ? 4 : 3; 
 #endif
 constexpr int kPieceCost = TQ_PAGED_PIECE_COST;
 // Row groups a split workgroup plans by itself (one wave, four groups per
-// lane; the unit records take 12 bytes of LDS each).
+// lane; the unit records take 16 bytes of LDS each).
 constexpr int kPlanGroups = 256;
 struct UnitRec {
-    int32_t start, kv_end;
+    int32_t start, kv_end, seq;
     int16_t first, npos;
 };
 
@@ -1226,7 +1226,7 @@ __device__ __forceinline__ void plan_step(const PagedRows& pr, int num_rows, int
             if (!start[k]) continue;
             const int w = single ? 1 : pass_weight(cnt[k]);
             x += !single && n[k] > 0 ? kPieceCost : 0;
-            rec[u] = UnitRec{x, kv[k], (int16_t)(g0 + k), (int16_t)cnt[k]};
+            rec[u] = UnitRec{x, kv[k], sq[k + 1], (int16_t)(g0 + k), (int16_t)cnt[k]};
             if (leave) {
 #pragma unroll
                 for (int m = 0; m < kNP; ++m)
@@ -1238,7 +1238,7 @@ __device__ __forceinline__ void plan_step(const PagedRows& pr, int num_rows, int
             ++u;
         }
         if (lane == 0) {
-            rec[units] = UnitRec{total, 0, 0, 0};
+            rec[units] = UnitRec{total, 0, 0, 0, 0};
             plan[0] = units;
             plan[1] = total;
             plan[2] = segs;
@@ -1338,78 +1338,25 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
     // logit scale per unit ks (log2(e) / alpha folded at compile time: no run-time division)
     const float ck = inv * (PROD ? kLog2e / kAlphaK : kLog2e / kAlphaV);
     const float cr = inv * kLog2e;                                 // residual: ks * re
-    // One work item: kv head h, row groups rg .. rg + npos - 1, tokens
-    // [t_begin, t_cap) (paged: and below each row's length), partial slot pid
+    // One work item: kv head h, row groups rg .. rg + npos - 1 (paged: of
+    // sequence seq), tokens [t_begin, t_end) (paged: t_end is at most the unit's
+    // longest row, and each row stops at its own length), partial slot pid
     // (slot-mapped: split pid).
     // (tid is a parameter so that a caller looping over items can keep the
     // per-thread values derived from it from being hoisted out of the loop
     // and held across the token loop.)
-    auto item = [&](const int tid, const int h, const int rg, const int npos, const int t_begin,
-                    const int t_cap, const size_t pid) {
+    auto item = [&](const int tid, const int h, const int rg, const int npos, const int seq,
+                    const int t_begin, const int t_end, const size_t pid) {
         const int lane = tid & 63;
         const int w = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (scalar)
         const int i = lane & 15, gq = lane >> 4;
         // Setup and merge: lane group gq holds the wave's row of position gq.
         const int j16 = logical(i);
-        // Paged rows: the unit's sequence and per-row kv lengths (causal limit).
-        // A piece past every row's length has no partial (the combine does not
-        // read it).  Per position: the group's longest row; per tile: this
-        // lane's column row length; the shortest live row.
-        int kv_end = num_kv_tokens, seq = 0;
+        // Paged rows: per-row kv lengths (causal limit).  A piece past every
+        // row's length has no partial (the combine does not read it).  Per
+        // position: the group's longest row; per tile: this lane's column row
+        // length; the shortest live row.
         int gend[kNP] = {}, rl_col[kNT] = {}, gmin_live = 0x7fffffff;
-        // This wave's query rows (row r of the workgroup is row r % 8 of group
-        // rg + r / 8: rows rg * 8 + r), loaded before anything waits: paged rows
-        // issue them right after the row lengths and the sequence, so the
-        // length processing waits only for those (the vector-memory counter is
-        // in order) while the queries are in flight.
-        uint32_t qraw[kE / 2];
-        auto load_queries = [&]() {
-            const int qi = min(rg * kRows + w + gq * kWaves, num_queries - 1);
-            const uint32_t* qp = reinterpret_cast<const uint32_t*>(
-                query + ((size_t)qi * g.H + h) * D + 4 * j16);
-#pragma unroll
-            for (int k = 0; k < kE / 2; ++k) qraw[k] = qp[(k & 1) + 32 * (k >> 1)];
-        };
-        if constexpr (!PAGED) load_queries();
-        if constexpr (PAGED) {
-            kv_end = 0;
-            // Every row length and the sequence are loaded unconditionally (rows
-            // past the end re-read the last row), so the loads go out together:
-            // a load under a condition sits in a branch whose join waits for it.
-            int lraw[kNP];
-#pragma unroll
-            for (int p = 0; p < kNP; ++p)
-                lraw[p] = pr.row_kv_len[min((rg + p) * kRows + (lane & 7), num_queries - 1)];
-            const int seq_raw = pr.row_seq[rg * kRows];
-            load_queries();
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int p = 0; p < kNP; ++p) {
-                const int rr = (rg + p) * kRows + (lane & 7);
-                const int lv = p < npos && rr < num_queries ? lraw[p] : 0;
-                // column i's row of position p is row i % 8 = lane % 8
-                // (one position: both halves of the tile hold its rows, hi and lo)
-                if (npos == 1 ? p == 0 : (i >> 3) == (p & 1)) rl_col[p >> 1] = lv;
-                // over the 8 rows: lane ^ 1, ^ 2, then 7 - lane of each 8
-                int m = lv, n = lv;
-                const auto over = [&](auto ctrl) {
-                    m = max(m, __builtin_amdgcn_mov_dpp(m, decltype(ctrl)::value, 0xF, 0xF, true));
-                    n = min(n, __builtin_amdgcn_mov_dpp(n, decltype(ctrl)::value, 0xF, 0xF, true));
-                };
-                over(std::integral_constant<int, 0xB1>{});
-                over(std::integral_constant<int, 0x4E>{});
-                over(std::integral_constant<int, 0x141>{});
-                gend[p] = __builtin_amdgcn_readfirstlane(m);
-                const int gmin = __builtin_amdgcn_readfirstlane(n);
-                kv_end = max(kv_end, gend[p]);
-                if (p < npos) gmin_live = min(gmin_live, gmin);
-            }
-            seq = __builtin_amdgcn_readfirstlane(seq_raw);
-            // (a piece always starts below its unit's kv end: the walk calls
-            // this only for work positions below ceil(kv_end / pass); a piece
-            // past every row would run no chunk and write no partial)
-        }
-        const int t_end = min(kv_end, t_cap);
         const int ntile = (npos + 1) >> 1;  // tiles of 16 columns in use
 
         // A chunk's codes and per-token scales, loaded ahead of its compute.
@@ -1518,11 +1465,31 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
             }
         };
 
-        // Issue order matters (the vector-memory counter is in order): the
-        // query rows (above), then the first chunk's slots; the decode tables
-        // are built while they are in flight.
+        // Issue order matters (the vector-memory counter is in order): the first
+        // chunk's slots, which the code loads wait for; this wave's query rows
+        // (row r of the workgroup is row r % 8 of group rg + r / 8: rows rg * 8 +
+        // r); paged rows' lengths, which nothing needs before the codes are out.
+        // (The unit's sequence and end come with the plan: read here before the
+        // slots, they were one more memory latency ahead of every piece.)
         int t0 = t_begin + w * kChunk;
         const int slot0 = load_slot(t0);
+        uint32_t qraw[kE / 2];
+        {
+            const int qi = min(rg * kRows + w + gq * kWaves, num_queries - 1);
+            const uint32_t* qp = reinterpret_cast<const uint32_t*>(
+                query + ((size_t)qi * g.H + h) * D + 4 * j16);
+#pragma unroll
+            for (int k = 0; k < kE / 2; ++k) qraw[k] = qp[(k & 1) + 32 * (k >> 1)];
+        }
+        // (every length unconditionally, rows past the end re-read the last
+        // row: a load under a condition sits in a branch whose join waits for it)
+        int lraw[kNP];
+        if constexpr (PAGED) {
+#pragma unroll
+            for (int p = 0; p < kNP; ++p)
+                lraw[p] = pr.row_kv_len[min((rg + p) * kRows + (lane & 7), num_queries - 1)];
+        }
+        __builtin_amdgcn_sched_barrier(0);
         // Query halves to fp32 (times the sign flip) before the code loads are
         // issued, so waiting for them never waits for the codes.
         float qf[kE];
@@ -1537,6 +1504,28 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         Chunk cur;
         fetch(t0, slot0, cur);  // in flight during the setup below (empty waves: all invalid)
         __builtin_amdgcn_sched_barrier(0);  // the first chunk's loads go out before the setup
+        if constexpr (PAGED) {
+#pragma unroll
+            for (int p = 0; p < kNP; ++p) {
+                const int rr = (rg + p) * kRows + (lane & 7);
+                const int lv = p < npos && rr < num_queries ? lraw[p] : 0;
+                // column i's row of position p is row i % 8 = lane % 8
+                // (one position: both halves of the tile hold its rows, hi and lo)
+                if (npos == 1 ? p == 0 : (i >> 3) == (p & 1)) rl_col[p >> 1] = lv;
+                // over the 8 rows: lane ^ 1, ^ 2, then 7 - lane of each 8
+                int m = lv, n = lv;
+                const auto over = [&](auto ctrl) {
+                    m = max(m, __builtin_amdgcn_mov_dpp(m, decltype(ctrl)::value, 0xF, 0xF, true));
+                    n = min(n, __builtin_amdgcn_mov_dpp(n, decltype(ctrl)::value, 0xF, 0xF, true));
+                };
+                over(std::integral_constant<int, 0xB1>{});
+                over(std::integral_constant<int, 0x4E>{});
+                over(std::integral_constant<int, 0x141>{});
+                gend[p] = __builtin_amdgcn_readfirstlane(m);
+                const int gmin = __builtin_amdgcn_readfirstlane(n);
+                if (p < npos) gmin_live = min(gmin_live, gmin);
+            }
+        }
         // The decode tables from registers, and each wave's rotated rows (lane
         // group k: row w of group rg + k) as fp16 hi and lo parts straight into
         // the QK B operand: one barrier for the setup.  A lane's dims 4j .. 4j + 3
@@ -2067,16 +2056,17 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         for (;;) {
             const int u = __builtin_amdgcn_readfirstlane(walk[0]);
             if (u >= nu) break;
-            int first, npos, kv_end, start;
+            int first, npos, kv_end, start, useq;
             if (planned) {
                 const PagedUnit un = pr.units[u];
-                first = un.first, npos = un.npos, kv_end = un.kv_end, start = un.start;
+                first = un.first, npos = un.npos, kv_end = un.kv_end, start = un.start, useq = un.seq_kv;
             } else {
                 const UnitRec un = s_units[u];
                 first = __builtin_amdgcn_readfirstlane((int)un.first);
                 npos = __builtin_amdgcn_readfirstlane((int)un.npos);
                 kv_end = __builtin_amdgcn_readfirstlane(un.kv_end);
                 start = __builtin_amdgcn_readfirstlane(un.start);
+                useq = __builtin_amdgcn_readfirstlane(un.seq);
             }
             if (start >= b1) break;
             if ((threadIdx.x & 63) == 0) walk[0] = u + 1;
@@ -2088,7 +2078,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 asm volatile("" : "+v"(tid));  // opaque per item (see item)
                 // partial slot: (unit + segment) * H + head, unique (the
                 // pieces of one head form a staircase in (unit, segment))
-                item(tid, hh, first, npos, x0 * kPass, min(x1 * kPass, kv_end),
+                item(tid, hh, first, npos, useq, x0 * kPass, min(x1 * kPass, kv_end),
                      (size_t)(u + seg) * g.H + hh);
             }
         }
@@ -2108,8 +2098,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
             un = hr / g.H;
         }
         const int t_begin = split * tokens_per_split;
-        item(threadIdx.x, h, un * kNP, min(kNP, groups - un * kNP), t_begin,
-             t_begin + tokens_per_split, (size_t)split);
+        item(threadIdx.x, h, un * kNP, min(kNP, groups - un * kNP), 0, t_begin,
+             min(t_begin + tokens_per_split, num_kv_tokens), (size_t)split);
     }
 }
 }  // namespace unit
@@ -2275,7 +2265,7 @@ __global__ __launch_bounds__(64) void attn_paged_combine_kernel(
     if (q >= num_queries) return;
     const PagedUnit un = pr.group_unit[rg];
     const int total = pr.plan[1], G = pr.plan[2];
-    const int p = rg - un.first, kv = un.group_kv, S = un.start;
+    const int p = rg - un.first, kv = un.seq_kv, S = un.start;
     // Segment gs holds the item's passes [first(bound(gs)), first(bound(gs + 1))).
     const auto first = [&](int b) {
         const int v = max(b - S, 0);
@@ -2474,11 +2464,11 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(
         const int wi = block_scan_1024(work, 0, s_tot, add);
         if (start) {
             const int o = c_units + ui - 1;
-            const mfma::PagedUnit rec{gi, c, kv, c_work + wi - work + lead, n, w, o, 0};
+            const mfma::PagedUnit rec{gi, c, kv, c_work + wi - work + lead, n, w, o, sq};
             units[o] = rec;
             for (int k = 0; k < c; ++k) {
                 mfma::PagedUnit gu = rec;
-                gu.group_kv = s_gk[j + k];
+                gu.seq_kv = s_gk[j + k];
                 group_unit[gi + k] = gu;
             }
         }
