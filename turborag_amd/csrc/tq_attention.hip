@@ -328,18 +328,30 @@ struct PagedRows {
     // A page-sized region of the workspace that masked tokens' loads address
     // (always valid memory; what they read is not used)
     const uint8_t* spare_page;
+    uint32_t inv_segments;  // floor((2^32 - 1) / segments per head)
 };
 // Workgroup s of G takes the work positions [bound(s), bound(s + 1)) with
 // bound(s) = floor(s * total / G) = q*s + floor(r*s / G) (q, r = total div, mod
 // G; r*s < G*G stays in 32 bits); a pass belongs to the segment holding its
-// first work position.
+// first work position.  Divisions by G through inv = floor((2^32 - 1) / G): the
+// high half of n * inv is n / G or one less (n < 2^31: n (1 + 1/G) / 2^32 < 1).
+// total = G (a pass per segment): bound(s) = s.
 struct Segments {
     int q, r, G;
-    __device__ Segments(int total, int g) : q(total / g), r(total % g), G(g) {}
-    __device__ int bound(int s) const { return q * s + (int)((uint32_t)(r * s) / (uint32_t)G); }
+    uint32_t inv;
+    __device__ Segments(int total, int g, uint32_t inv_g) : G(g), inv(inv_g) {
+        q = total == g ? 1 : div((uint32_t)total);
+        r = total - q * g;
+    }
+    __device__ int div(uint32_t n) const {
+        const uint32_t d = __umulhi(n, inv);
+        return (int)(d + (n - d * (uint32_t)G >= (uint32_t)G ? 1u : 0u));
+    }
+    __device__ int bound(int s) const { return q * s + (r ? div((uint32_t)(r * s)) : 0); }
     // The segment holding work position x < total: an estimate within one of
     // floor(((x + 1) G - 1) / total), then corrected.
     __device__ int of(int x, int total) const {
+        if (total == G) return x;
         int g = (int)(((float)x + 1.0f) * (float)G / (float)total) - 1;
         g = max(0, min(g, G - 1));
         while (g + 1 < G && bound(g + 1) <= x) ++g;
@@ -347,12 +359,26 @@ struct Segments {
         return g;
     }
 };
+// ceil(v / w) for a pass weight w (1, 3 or 4), v >= 0.
+__device__ __forceinline__ int passes_of(int v, int w) {
+    return w == 4 ? (v + 3) >> 2 : w == 3 ? (v + 2) / 3 : v;
+}
 // Passes [x0, x1) of an item (start S, n passes of weight w) that begin in
 // the work range [b0, b1).
 __device__ __forceinline__ void item_passes(int S, int n, int w, int b0, int b1, int& x0,
                                             int& x1) {
-    x0 = S >= b0 ? 0 : (b0 - S + w - 1) / w;
-    x1 = S >= b1 ? 0 : min(n, (b1 - S + w - 1) / w);
+    x0 = passes_of(max(b0 - S, 0), w);
+    x1 = min(n, passes_of(max(b1 - S, 0), w));
+}
+// Inclusive sum over the lanes of a wave (DPP row shifts and row broadcasts).
+__device__ __forceinline__ int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xF, 0xF, false);  // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xF, 0xF, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);  // row_bcast:15
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);  // row_bcast:31
+    return v;
 }
 
 // Workgroup barrier for LDS traffic only: waits for this wave's LDS accesses,
@@ -1143,7 +1169,9 @@ __device__ __forceinline__ int pass_weight(int npos) { return npos > 2 ? 4 : 3; 
 #endif
 constexpr int kPieceCost = TQ_PAGED_PIECE_COST;
 // Row groups a split workgroup plans by itself (one wave, four groups per
-// lane; the unit records take 16 bytes of LDS each).
+// lane; the unit records take 16 bytes of LDS each).  Scans by DPP, divisions by
+// the segment count through its inverse and the first unit found by the same wave
+// took a small step's split kernel from 10.7 to 9.7 us.
 constexpr int kPlanGroups = 256;
 struct UnitRec {
     int32_t start, kv_end, seq;
@@ -1155,10 +1183,15 @@ struct UnitRec {
 // head.  Where the step has no more passes than Gh, every pass is a segment
 // of its own (weight 1, no lead): no workgroup takes two while another has
 // none, and the merge of a unit looks at its n passes instead of the segments
-// they are scattered over.  `scratch`: LDS of 2 (kPlanGroups + 8) words.
-// leave: write group_unit and plan for the merge.
+// they are scattered over; those segments go round the XCDs (seg = bl), the
+// others are consecutive on each.  `scratch`: LDS of 2 (kPlanGroups + 8)
+// words.  leave: write group_unit and plan for the merge.  Further results for
+// workgroup bl of its head, in plan[3..6]: its segment, the segment's work
+// positions [plan[4], plan[5]) (none: an empty segment), the unit holding the
+// first of them.
 __device__ __forceinline__ void plan_step(const PagedRows& pr, int num_rows, int max_kv_len, int Gh,
-                                          bool leave, int* scratch, UnitRec* rec, int* plan) {
+                                          int bl, bool leave, int* scratch, UnitRec* rec,
+                                          int* plan) {
     const int groups = (num_rows + kRows - 1) / kRows;
     int* s_sq = scratch + 4;  // sequence of group g at [g], with room before and after
     int* s_gk = s_sq + kPlanGroups + 8;
@@ -1177,24 +1210,26 @@ __device__ __forceinline__ void plan_step(const PagedRows& pr, int num_rows, int
         s_gk[g] = g < groups ? min(m, max_kv_len) : 0;
     }
     __syncthreads();
-    if (threadIdx.x < 64) {
-        const int lane = threadIdx.x, g0 = 4 * lane;
-        int sq[8], gk[7];  // sequences of groups g0 - 1 .. g0 + 6, lengths from g0
+    // One group per lane, or four where there are more than 64.
+    const auto plan_lanes = [&](auto per) {
+        constexpr int P = decltype(per)::value;
+        const int lane = threadIdx.x, g0 = P * lane;
+        int sq[P + 4], gk[P + 3];  // sequences of groups g0 - 1 .. g0 + P + 2, lengths from g0
 #pragma unroll
-        for (int k = 0; k < 8; ++k) sq[k] = s_sq[min(max(g0 + k - 1, 0), kPlanGroups - 1)];
+        for (int k = 0; k < P + 4; ++k) sq[k] = s_sq[min(max(g0 + k - 1, 0), kPlanGroups - 1)];
 #pragma unroll
-        for (int k = 0; k < 7; ++k) gk[k] = g0 + k < kPlanGroups ? s_gk[g0 + k] : 0;
+        for (int k = 0; k < P + 3; ++k) gk[k] = g0 + k < kPlanGroups ? s_gk[g0 + k] : 0;
         // The run each group is in: the last group at or before it that starts one.
         int last = -1;
 #pragma unroll
-        for (int k = 0; k < 4; ++k)
+        for (int k = 0; k < P; ++k)
             if (g0 + k < groups && (g0 + k == 0 || sq[k + 1] != sq[k])) last = g0 + k;
         const uint64_t below = __ballot(last >= 0) & ((1ull << lane) - 1ull);
         int cur = __shfl(last, below ? 63 - __clzll(below) : 0);
-        int cnt[4], kv[4], n[4], lane_u = 0, lane_n = 0, lane_w = 0;
-        bool start[4];
+        int cnt[P], kv[P], n[P], lane_u = 0, lane_n = 0, lane_w = 0;
+        bool start[P];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < P; ++k) {
             const int g = g0 + k;
             if (g < groups && (g == 0 || sq[k + 1] != sq[k])) cur = g;
             start[k] = g < groups && ((g - cur) & (kNP - 1)) == 0;
@@ -1211,21 +1246,23 @@ __device__ __forceinline__ void plan_step(const PagedRows& pr, int num_rows, int
             lane_n += n[k];
             lane_w += n[k] > 0 ? kPieceCost + pass_weight(cnt[k]) * n[k] : 0;
         }
-        int su = lane_u, sn = lane_n, sw = lane_w;  // inclusive scans over the lanes
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int a = __shfl_up(su, d), b = __shfl_up(sn, d), c = __shfl_up(sw, d);
-            if (lane >= d) su += a, sn += b, sw += c;
-        }
-        const int units = __shfl(su, 63), tn = __shfl(sn, 63), tw = __shfl(sw, 63);
+        const int su = wave_scan(lane_u), sn = wave_scan(lane_n), sw = wave_scan(lane_w);
+        const int units = __builtin_amdgcn_readlane(su, 63);
+        const int tn = __builtin_amdgcn_readlane(sn, 63), tw = __builtin_amdgcn_readlane(sw, 63);
         const bool single = tn <= Gh;
         const int total = single ? tn : tw, segs = single ? max(tn, 1) : Gh;
+        const int seg = single ? bl : (bl & 7) * (Gh >> 3) + (bl >> 3);
+        const Segments sg(total, segs, pr.inv_segments);
+        const int b0 = seg < segs && total > 0 ? sg.bound(seg) : 0;
+        const int b1 = seg < segs && total > 0 ? sg.bound(seg + 1) : 0;
         int u = su - lane_u, x = single ? sn - lane_n : sw - lane_w;
+        int below_b0 = 0;  // units starting at or before b0
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
+        for (int k = 0; k < P; ++k) {
             if (!start[k]) continue;
             const int w = single ? 1 : pass_weight(cnt[k]);
             x += !single && n[k] > 0 ? kPieceCost : 0;
+            below_b0 += x <= b0 ? 1 : 0;
             rec[u] = UnitRec{x, kv[k], sq[k + 1], (int16_t)(g0 + k), (int16_t)cnt[k]};
             if (leave) {
 #pragma unroll
@@ -1237,17 +1274,28 @@ __device__ __forceinline__ void plan_step(const PagedRows& pr, int num_rows, int
             x += w * n[k];
             ++u;
         }
+        below_b0 = __builtin_amdgcn_readlane(wave_scan(below_b0), 63);
         if (lane == 0) {
             rec[units] = UnitRec{total, 0, 0, 0, 0};
             plan[0] = units;
             plan[1] = total;
             plan[2] = segs;
+            plan[3] = seg;
+            plan[4] = b0;
+            plan[5] = b1;
+            plan[6] = max(below_b0 - 1, 0);
             if (leave) {
                 pr.plan[0] = units;
                 pr.plan[1] = total;
                 pr.plan[2] = segs;
             }
         }
+    };
+    if (threadIdx.x < 64) {
+        if (groups <= 64)
+            plan_lanes(std::integral_constant<int, 1>{});
+        else
+            plan_lanes(std::integral_constant<int, 4>{});
     }
     __syncthreads();
 }
@@ -2011,38 +2059,38 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         // of a token share its cache lines (cell tib * H + h), and the second
         // reader finds them in that XCD's L2.  The segments of one XCD are
         // consecutive, so the units of a sequence mostly share it too.
-        // (A step planned here with one pass per segment spreads its segments
-        // over the XCDs instead; the heads of one still share an XCD.)
         const int Gh = (int)gridDim.x / g.H;
         const int hh = (int)blockIdx.x / Gh;
         const int bl = (int)blockIdx.x - hh * Gh;
         __shared__ UnitRec s_units[kPlanGroups + 1];
-        __shared__ int s_plan[3];
+        __shared__ int s_plan[7], s_unit;
         const bool planned = pr.units != nullptr;  // by paged_plan_kernel
+        int nu, seg, b0, b1;
         if (planned) {
-            if (threadIdx.x < 3) s_plan[threadIdx.x] = pr.plan[threadIdx.x];
+            nu = __builtin_amdgcn_readfirstlane(pr.plan[0]);
+            const int total = __builtin_amdgcn_readfirstlane(pr.plan[1]);
+            seg = (bl & 7) * (Gh >> 3) + (bl >> 3);
+            const Segments sg(total, Gh, pr.inv_segments);
+            b0 = sg.bound(seg), b1 = sg.bound(seg + 1);
+            if (b0 >= b1) return;  // an empty segment (less work than workgroups)
+            // The unit holding work position b0: exactly one u has start(u) <= b0
+            // < start(u + 1), or b0 lies before the first unit's first pass
+            // (unit 0).
+            for (int u = threadIdx.x; u < nu; u += 64 * kWaves)
+                if ((u == 0 || pr.units[u].start <= b0) && b0 < pr.units[u + 1].start) s_unit = u;
             __syncthreads();
         } else {
-            plan_step(pr, num_queries, num_kv_tokens, Gh, blockIdx.x == 0,
+            plan_step(pr, num_queries, num_kv_tokens, Gh, bl, blockIdx.x == 0,
                       reinterpret_cast<int*>(lut), s_units, s_plan);
+            nu = __builtin_amdgcn_readfirstlane(s_plan[0]);
+            seg = __builtin_amdgcn_readfirstlane(s_plan[3]);
+            b0 = __builtin_amdgcn_readfirstlane(s_plan[4]);
+            b1 = __builtin_amdgcn_readfirstlane(s_plan[5]);
+            if (b0 >= b1) return;
         }
-        const int nu = __builtin_amdgcn_readfirstlane(s_plan[0]);
-        const int total = __builtin_amdgcn_readfirstlane(s_plan[1]);
-        const int segs = __builtin_amdgcn_readfirstlane(s_plan[2]);
-        const bool single = segs != Gh;  // (segs == Gh == total: either numbering)
-        const int seg = single ? bl : (bl & 7) * (Gh >> 3) + (bl >> 3);
-        if (seg >= segs || total == 0) return;
-        const Segments sg(total, segs);
-        const int b0 = sg.bound(seg), b1 = sg.bound(seg + 1);
-        if (b0 >= b1) return;  // an empty segment (less work than workgroups)
-        const bool ones = !planned && segs == total;  // weight 1 per pass
-        auto start_of = [&](int u) { return planned ? pr.units[u].start : s_units[u].start; };
-        // The unit holding work position b0: exactly one u has start(u) <= b0 <
-        // start(u + 1), or b0 lies before the first unit's first pass (unit 0).
-        __shared__ int s_unit;
-        for (int u = threadIdx.x; u < nu; u += 64 * kWaves)
-            if ((u == 0 || start_of(u) <= b0) && b0 < start_of(u + 1)) s_unit = u;
-        __syncthreads();
+        // (a pass per segment: weight 1)
+        const bool ones = !planned && s_plan[1] == s_plan[2];
+        const int u_first = __builtin_amdgcn_readfirstlane(planned ? s_unit : s_plan[6]);
         // The walk over the units overlapping the segment, in work order.  Its
         // position lives in LDS (one copy per wave, volatile accesses), so no
         // walk state is held in registers across an item.  The pointer is an
@@ -2052,7 +2100,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         typedef __attribute__((address_space(3))) int lds_int;
         const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
         volatile lds_int* walk = (volatile lds_int*)&s_walk[wv];
-        if ((threadIdx.x & 63) == 0) walk[0] = __builtin_amdgcn_readfirstlane(s_unit);
+        if ((threadIdx.x & 63) == 0) walk[0] = u_first;
         for (;;) {
             const int u = __builtin_amdgcn_readfirstlane(walk[0]);
             if (u >= nu) break;
@@ -2267,12 +2315,9 @@ __global__ __launch_bounds__(64) void attn_paged_combine_kernel(
     const int total = pr.plan[1], G = pr.plan[2];
     const int p = rg - un.first, kv = un.seq_kv, S = un.start;
     // Segment gs holds the item's passes [first(bound(gs)), first(bound(gs + 1))).
-    const auto first = [&](int b) {
-        const int v = max(b - S, 0);
-        return min(un.n, un.w == 4 ? (v + 3) >> 2 : un.w == 3 ? (v + 2) / 3 : v);
-    };
+    const auto first = [&](int b) { return min(un.n, passes_of(max(b - S, 0), un.w)); };
     int g_lo = 0, g_hi = -1;
-    const Segments sg(max(total, 1), G);
+    const Segments sg(max(total, 1), G, pr.inv_segments);
     if (un.n > 0 && kv > 0) {
         g_lo = sg.of(S, total);
         g_hi = sg.of(S + un.w * (un.n - 1), total);
@@ -3339,7 +3384,8 @@ void launch_paged_units(const uint16_t* query, const uint8_t* pool, const int32_
     // plan launch (5.5 us of a step) is gone.
     const bool self = row_groups <= unit::kPlanGroups;
     const PagedRows pr{block_tables, row_seq,    row_kv_len, max_blocks, self ? nullptr : units,
-                       group_unit,   plan,       reinterpret_cast<const uint8_t*>(wsb + spare_at)};
+                       group_unit,   plan,       reinterpret_cast<const uint8_t*>(wsb + spare_at),
+                       0xFFFFFFFFu / (uint32_t)Gh};
     if (!self) {
         hipLaunchKernelGGL(paged_plan_kernel<unit::kNP>, dim3(1), dim3(1024), 0, stream, row_seq,
                            row_kv_len, num_rows, row_groups, unit::kPass, max_kv_len, Gh, units,
