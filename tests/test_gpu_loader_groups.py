@@ -76,3 +76,38 @@ def test_placements(tq, cuda, scheme, D, L, N, host, dev, pin):
     for layer in range(L):
         assert torch.equal(devs[layer], pools[layer]), layer
         assert torch.equal(oks[layer], wks[layer]) and torch.equal(ovs[layer], wvs[layer]), layer
+
+
+@pytest.mark.parametrize("shared", ["all", "pairs", "half"])
+def test_shared_outputs(tq, cuda, shared):
+    """Layers that write one output buffer, or overlapping ones, go in order
+    whatever the placement of their pages: the last one's values stay."""
+    print(f"[loader groups] outputs shared: {shared}", flush=True)
+    H, B, D, L, N = 2, 16, 64, 6, 900
+    cfg = tq.default_config()
+    cfg.num_kv_heads, cfg.head_dim = H, D
+    lay = tq.make_mse_layout_for(cfg)
+    slots = permuted_slots(N, B, seed=672).to(cuda)
+    pages = int(slots.max()) // B + 1
+    k, v = (x.to(cuda) for x in kv_tokens_major(N, H, D, seed=673))
+    pools = torch.zeros(L, pages * lay.page_size_bytes, dtype=torch.uint8, device=cuda)
+    for layer in range(L):
+        tq.mse_pack(k.roll(layer, 0).contiguous(), v.roll(layer, 0).contiguous(), slots,
+                    pools[layer], lay, cfg)
+    host = torch.empty(pools.shape, dtype=torch.uint8, pin_memory=True)
+    host.copy_(pools)
+    n = N * H * D
+    flat = torch.full((2 * L * n,), 7.0, dtype=torch.float16, device=cuda)
+    want = flat.clone()
+    at = [{"all": 0, "pairs": l // 2 * n, "half": l * n // 2}[shared] for l in range(L)]
+    out = lambda buf, l, side: buf[side * L * n + at[l]:][:n].view(1, H, N, D)  # noqa: E731
+    for layer in range(L):
+        tq.mse_dequant_hnd(pools[layer], slots, out(want, layer, 0), out(want, layer, 1), lay, cfg, N)
+    copy = torch.cuda.Stream()
+    devs = torch.zeros_like(pools)
+    torch.cuda.synchronize()
+    tq.load_layers("turbo_mse", list(host), list(devs), slots, [out(flat, l, 0) for l in range(L)],
+                   [out(flat, l, 1) for l in range(L)], lay, cfg, N, copy_stream=copy.cuda_stream,
+                   compute_stream=torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    assert torch.equal(flat, want)

@@ -18,9 +18,11 @@
 // hides, so a group is not the whole document.  24 layers of 1.3 MB: 1,070 ->
 // 724 us (0.55 ms of link time); 36 of 0.3 MB: 942 -> 278; 36 of 2.2 MB: 2,413
 // -> 1,610.
+#include <algorithm>
 #include <map>
 #include <memory>
 #include <mutex>
+#include <utility>
 #include <vector>
 
 #include "tq_internal.h"
@@ -107,14 +109,36 @@ void load_layers(Scheme s, const uint8_t* const* host_pools, uint8_t* const* dev
         check(hipStreamWaitEvent(copy_stream, ev[num_layers], 0), "hipStreamWaitEvent");
     }
     // Layers [l, l + n): pages one after another on both sides, inside one
-    // allocation each (so that one copy is the n copies).
+    // allocation each (so that one copy is the n copies), and outputs that meet
+    // neither each other nor the pages (a group's layers are dequantized in
+    // any order; layers that share a buffer are taken one by one).
+    const size_t out_bytes = (size_t)std::max(num_tokens, 0) * g.H * g.D * sizeof(uint16_t);
+    const auto meet = [](const void* a, size_t an, const void* b, size_t bn) {
+        const uintptr_t x = reinterpret_cast<uintptr_t>(a), y = reinterpret_cast<uintptr_t>(b);
+        return x < y + bn && y < x + an;
+    };
+    std::vector<std::pair<uintptr_t, uintptr_t>> taken;  // the group's outputs, sorted
+    const auto take = [&](const void* p) {
+        const uintptr_t x = reinterpret_cast<uintptr_t>(p);
+        const std::pair<uintptr_t, uintptr_t> r{x, x + out_bytes};
+        const auto at = std::lower_bound(taken.begin(), taken.end(), r);
+        if (at != taken.end() && at->first < r.second) return false;
+        if (at != taken.begin() && (at - 1)->second > x) return false;
+        taken.insert(at, r);
+        return true;
+    };
     const auto group_at = [&](int l) {
-        int n = 1;
-        while (l + n < num_layers && n * pool_bytes < kGroupBytes &&
+        taken.clear();
+        int n = 0;
+        while (l + n < num_layers && (n == 0 || n * pool_bytes < kGroupBytes) &&
                host_pools[l + n] == host_pools[l] + n * pool_bytes &&
-               device_pools[l + n] == device_pools[l] + n * pool_bytes)
+               device_pools[l + n] == device_pools[l] + n * pool_bytes && take(out_key[l + n]) &&
+               take(out_value[l + n]))
             ++n;
-        return n;
+        for (const auto& r : taken)
+            if (meet(device_pools[l], n * pool_bytes, reinterpret_cast<void*>(r.first), out_bytes))
+                return 1;
+        return std::max(n, 1);
     };
     size_t host_left = 0, dev_left = 0;  // of the allocations from layer `known` on
     int known = -1;
