@@ -205,8 +205,8 @@ int tq_launch_turbo_mse_pack_kv_layers(const uint16_t* const* keys, const uint16
  * as a document's layers do, cag_store.py:129).  page_pools, out_keys and
  * out_values are HOST arrays of num_layers device pointers, read during the
  * call.  Outputs are [num_tokens, H, D] fp16, or [1, H, num_tokens, D] when
- * head_major != 0.  For D = 128 one launch covers up to 64 layers; the layers
- * run concurrently, so the outputs must not overlap each other. */
+ * head_major != 0.  For D = 64 and 128 one launch covers up to 64 layers; the
+ * layers run concurrently, so the outputs must not overlap each other. */
 int tq_launch_turbo_prod_dequant_kv_layers(const uint8_t* const* page_pools,
                                            const int32_t* slot_mapping,
                                            uint16_t* const* out_keys, uint16_t* const* out_values,
@@ -222,8 +222,11 @@ int tq_launch_turbo_mse_dequant_kv_layers(const uint8_t* const* page_pools,
 /* For each layer l < num_layers: copies pool_bytes bytes from host_pools[l]
  * to device_pools[l] on copy_stream and dequantizes device_pools[l] into
  * out_key[l] / out_value[l] ([1, H, num_tokens, D] fp16) on compute_stream,
- * which waits for layer l's copy only; layer l's dequant overlaps layer
- * l+1's copy.  Copies start after the work already on compute_stream.
+ * which waits for that layer's copy, not the later ones': the dequant overlaps
+ * the copies that follow.  Layers whose pages lie one after another in one
+ * pinned host buffer and one device buffer go in groups of at least 24 MB, one
+ * copy and one dequant launch per group (the results do not change: layers
+ * whose outputs overlap are taken one by one).  Copies start after the work already on compute_stream.
  * slot_mapping is device int32[num_tokens].  Asynchronous: completion is
  * ordered on compute_stream.  Host pages in pinned memory overlap fully;
  * pageable pages are correct but copied at the runtime's staging rate.

@@ -2545,17 +2545,15 @@ __global__ __launch_bounds__(1024) void paged_plan_kernel(
 // turbo_prod / turbo_mse pages.
 //
 // Flash-decoding split-K on a (split, kv head, row group) grid, 8 waves of
-// 32-token chunks per workgroup, the same MFMA formulation as
-// attn_mfma_split_kernel (QK: A = decoded K, B = the rotated query as fp16
-// hi/lo columns; PV: A = P', B = decoded V), with a setup and a chunk loop
-// cut to what the decode needs:
+// 32-token chunks per workgroup (QK: A = decoded K, B = the rotated query as
+// fp16 hi/lo columns; PV: A = P', B = decoded V), with a setup and a chunk
+// loop cut to what the decode needs:
 //  - one LDS lookup per K code byte returns two fp16 pairs: turbo_prod's
 //    aK*K3 pair and its pair of residual signs (+-1; no VALU builds the sign
 //    matrix), turbo_mse's hi and lo parts of aV*V4 (its V lookups read the
 //    hi pair of the same entry);
-//  - the tables are copied into LDS from compile-time constants while the
-//    slots and codes are in flight (no per-entry arithmetic, no staging
-//    pass);
+//  - the tables are built in registers from compile-time constants while the
+//    slots and codes are in flight (no staging pass);
 //  - each wave rotates one query row and stores its fp16 hi and lo parts
 //    straight into the B-operand layout: one barrier for the whole setup;
 //  - P' = p * vs / aV enters the PV product as its fp16 hi part, or on the

@@ -559,7 +559,7 @@ class TurboQuantWrapper:
                        stream: int = 0) -> None:
         """Dequant every layer's pool (one shared slot mapping) into
         out_keys[l] / out_values[l]: [N, H, D] fp16, or [1, H, N, D] with
-        head_major; one launch per 64 layers at head_dim 128."""
+        head_major; one launch per 64 layers at head_dim 64 and 128."""
         n = len(page_pools)
         if not (len(out_keys) == len(out_values) == n):
             raise ValueError("dequant_layers: one pool and two outputs per layer")
@@ -624,7 +624,7 @@ class TurboQuantWrapper:
         query / output [num_rows, H, D] fp16; row r belongs to sequence
         row_seq[r] (aligned groups of 8 rows share one) and attends its first
         row_kv_len[r] tokens; block_tables [num_seqs, max_blocks] int32 page
-        ids.  head_dim 128."""
+        ids."""
         H, D = cfg.num_kv_heads, cfg.head_dim
         num_rows = query.shape[0]
         if block_tables.dim() != 2:
