@@ -1133,7 +1133,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_qjl_split_kernel(
 // Issue-bound at many passes per workgroup (D = 128, 32 sequences of 1K-32K
 // tokens: 94 us), bound by the setup and the merge at few.  A D = 64 step of
 // 8 sequences (500-4,000 tokens, 2 new tokens, 2 heads) with its append takes
-// 26.8 us, against 212.6 on the generic kernels it ran on before.
+// 22.1 us, against 212.6 on the generic kernels it ran on before.
 // ---------------------------------------------------------------------------
 namespace unit {
 using namespace mfma;
