@@ -1829,7 +1829,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                     fetch(t1, slot_nx, cur);
                     slot_nx = load_slot(t1 + kPass);
                 }
-                if (PAGED && t0 + kChunk > gmin_live) {  // a row of the unit ends in this chunk
+                const bool row_ends = PAGED && t0 + kChunk > gmin_live;
+                if (row_ends) {  // a row of the unit ends in this chunk
                     // (wave-uniform; a branch: no selects on every chunk)
                     asm volatile("" ::: "memory");
 #pragma unroll
@@ -1899,13 +1900,29 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 // PV: every tile's hi and lo P against each decoded B operand
                 half8 ah[NTA], al[NTA];
 #pragma unroll
+                for (int t = 0; t < NTA; ++t)
+#pragma unroll
+                    for (int tau = 0; tau < kTiles; ++tau)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) lg[t][tau][e] *= tsc[w][16 * tau + 4 * gq + e].z;
+                if (row_ends) {
+                    // a token past the column's row: 0 also where its V scale is
+                    // infinite or NaN (0 times it is NaN)
+                    asm volatile("" ::: "memory");
+#pragma unroll
+                    for (int t = 0; t < NTA; ++t)
+#pragma unroll
+                        for (int tau = 0; tau < kTiles; ++tau)
+#pragma unroll
+                            for (int e = 0; e < 4; ++e)
+                                if (t0 + 16 * tau + 4 * gq + e >= rl_col[t]) lg[t][tau][e] = 0.0f;
+                }
+#pragma unroll
                 for (int t = 0; t < NTA; ++t) {
                     uint32_t hw[4], lw[4];
 #pragma unroll
                     for (int e = 0; e < 8; e += 2) {
-                        const int tau = e >> 2, ee = e & 3;
-                        const float x0 = lg[t][tau][ee] * tsc[w][16 * tau + 4 * gq + ee].z;
-                        const float x1 = lg[t][tau][ee + 1] * tsc[w][16 * tau + 4 * gq + ee + 1].z;
+                        const float x0 = lg[t][e >> 2][e & 3], x1 = lg[t][e >> 2][(e & 3) + 1];
                         hw[e >> 1] = pack_h2(x0, x1);
                         lw[e >> 1] = lo_pair(x0, x1, hw[e >> 1]);
                     }
