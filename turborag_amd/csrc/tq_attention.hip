@@ -534,6 +534,40 @@ __device__ __forceinline__ half8 sign_octet(uint32_t wd) {
 __device__ __forceinline__ int scale_exp(float x) {
     return __builtin_isfinite(x) ? __builtin_amdgcn_frexp_expf(x) : 0;
 }
+// V's power of two.  P * vs enters PV as an fp16 hi and lo part; with vs as it
+// is, products below 2^-14 fell among fp16's subnormals (step 6e-8, hi and lo
+// alike: V rows of rms 1e-5 were off by 3 ulps of the output).  So a wave's vs
+// are multiplied by the power of two that puts the largest into [2^13, 2^14):
+// products keep ~22 bits down to 2^-28 of it.  `top` is the largest fp16 with
+// the exponent of the largest finite vs so far; a chunk that passes it moves it
+// and rescales the wave's accumulators.  Head_dim 64, and the units over a slot
+// map, carry it; the first chunk's maximum costs 0.05-0.2 us of a call (8 rows x
+// 2 heads x 250 tokens at head_dim 64: 5.7 -> 5.9).  The one-group and paged
+// kernels at head_dim 128 take vs as it is.
+__device__ __forceinline__ float v_scale(uint32_t top) {  // 2^(28 - exponent field)
+    return __uint_as_float((155u - (top >> 10)) << 23);
+}
+__device__ __forceinline__ float v_unscale(uint32_t top) {
+    return __uint_as_float((99u + (top >> 10)) << 23);
+}
+// The bits of a finite vs (0: no token), else 0.
+__device__ __forceinline__ uint32_t v_bits(uint32_t vb) {
+    vb &= 0x7FFFu;
+    return vb < 0x7C00u ? vb : 0u;
+}
+// top for a chunk of v_bits vb, one token in lanes l and l + 32.
+__device__ __forceinline__ uint32_t v_top(uint32_t vb) {
+    const uint32_t m = (uint32_t)max_lanes<32>((float)vb);
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)m) | 0x3FFu;
+}
+// Moves top for a further chunk; rescale(f): the accumulators times f.
+template <class F>
+__device__ __forceinline__ void v_raise(uint32_t vb, uint32_t& top, F rescale) {
+    if (!__any(vb > top)) return;
+    const uint32_t t = v_top(vb);
+    rescale(__uint_as_float((127u + (top >> 10) - (t >> 10)) << 23));
+    top = t;
+}
 template <bool PROD>
 __device__ __forceinline__ void store_decode_tables(uint32_t* lut, int kv_words, int w, int lane,
                                                     const TableWords<PROD>& tw) {
@@ -1128,7 +1162,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_qjl_split_kernel(
 // decode tables).  PAGED: the grid is one workgroup per work segment of the
 // step's plan (paged_plan_kernel).  Slot-mapped: grid (split, kv head, unit).
 // D = 64: half the k-steps and PV tiles per token, the fp16 lo parts of V and
-// turbo_prod's K and a power of two per query row, as
+// turbo_prod's K and powers of two for the query rows and V, as
 // dec::attn_decode_split_kernel.
 // Issue-bound at many passes per workgroup (D = 128, 32 sequences of 1K-32K
 // tokens: 94 us), bound by the setup and the merge at few.  A D = 64 step of
@@ -1375,6 +1409,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
     constexpr int kND = D / 16;  // PV tiles: lane i holds dims kND i .. + kND - 1
     constexpr int kE = D / 16;   // elements per lane of a row held by 16 lanes
     constexpr bool VLO = D == 64, QSCALE = D == 64, KLO = D == 64 && PROD;
+    constexpr bool VSCALE = D == 64 || !PAGED;
     static_assert(kNT * sizeof(float) * kWaves * kMoRows * D <= 4 * kTabWords, "merge spaces");
     __shared__ __attribute__((aligned(256))) uint32_t lut[kTabWords];
     __shared__ uint4 bqs[kNP][kS][64];  // QK B operand (fp16 hi/lo q) of k-step s for lane l
@@ -1666,6 +1701,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 if constexpr (VLO) acl_col[t][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
             }
         }
+        uint32_t vtop = VSCALE ? v_top(v_bits(cur.valid ? cur.vs : 0u)) : 0u;  // wave-uniform
         float qsc[kNT];
 #pragma unroll
         for (int t = 0; t < kNT; ++t)
@@ -1679,8 +1715,21 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
             constexpr bool COLS = decltype(cols)::value;
             static_assert(!COLS || NTA == 1, "one tile");
             while (t0 < t_end) {  // wave-uniform
+                if constexpr (VSCALE)
+                    v_raise(v_bits(cur.valid ? cur.vs : 0u), vtop, [&](float f) {
+#pragma unroll
+                        for (int t = 0; t < NTA; ++t)
+#pragma unroll
+                            for (int v = 0; v < kND; ++v)
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    acc_col[t][v][e] *= f;
+                                    if constexpr (VLO) acl_col[t][v][e] *= f;
+                                }
+                    });
                 {
-                    const float ks = h2f(cur.ks), vs = h2f(cur.vs), re = PROD ? h2f(cur.re) : 0.0f;
+                    const float ks = h2f(cur.ks), re = PROD ? h2f(cur.re) : 0.0f;
+                    const float vs = VSCALE ? h2f(cur.vs) * v_scale(vtop) : h2f(cur.vs);
                     tsc[w][lane & (kChunk - 1)] =
                         cur.valid ? make_float4(ks * ck, PROD ? ks * re * cr : ks * ck * kLoScale,
                                                 0.5f * vs, 0.0f)
@@ -1984,6 +2033,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         // position: lane group gq the waves' (m, l, o) of position gq, elements
         // 4j .. 4j + 3 (and 64 + 4j ..) per lane, then the inverse WHT and sign
         // flip, and the partial.
+        const float vun = 2.0f * iav * (VSCALE ? v_unscale(vtop) : 1.0f);
         auto mot = [&](int t) { return reinterpret_cast<float(*)[kMoRows][D]>(&lut[16384 * t]); };
         __syncthreads();  // every wave is done with the tables
 #pragma unroll
@@ -1995,7 +2045,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 for (int e = 0; e < 4; ++e) {  // (x2: the PV operand was P * vs / 2)
                     float x = acc_col[t][v][e];
                     if constexpr (VLO) x = fmaf(acl_col[t][v][e], kLoScale, x);
-                    mot(t)[w][4 * gq + e][kND * i + v] = x * (2.0f * iav);
+                    mot(t)[w][4 * gq + e][kND * i + v] = x * vun;
                 }
         }
         __syncthreads();
@@ -2638,9 +2688,9 @@ constexpr size_t part_bytes(int D) { return kRows * (D + 2) * sizeof(float); }
 // table's hi parts alone are 5e-5 off in the mean, a quarter of the output's
 // own fp16 rounding) and of turbo_prod's K (in the S table, a third QK
 // product; the signs are built in registers: logits of magnitude 60, outlier
-// channels shared by q and k, are 6e-4 off without it), and a power of two
-// per query row that holds the row's fp16 parts in range whatever its
-// magnitude.  Bound by its dependent loads and
+// channels shared by q and k, are 6e-4 off without it), and powers of two, one
+// per query row and one per wave for V, that hold their fp16 parts in range
+// whatever their magnitudes.  Bound by its dependent loads and
 // the setup, as D = 128: 7 rows x 2 heads x 6,001 tokens (turbo_mse) take 6.0
 // (split) + 2.9 us (combine); the generic one-wave-per-row kernels, whose
 // cross-lane sum per token and serial merge over 147 splits this replaces,
@@ -2657,7 +2707,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
     constexpr int kS = D / 32;       // QK k-steps; lane group gq holds dims [D/4 gq, D/4 gq + D/4)
     constexpr int kNT = D / 16;      // PV tiles: lane i holds dims kNT i .. + kNT - 1
     constexpr int kL = D / 2;        // lanes of a row held two values per lane
-    constexpr bool VLO = D == 64, QSCALE = D == 64, KLO = D == 64 && PROD;
+    constexpr bool VLO = D == 64, QSCALE = D == 64, KLO = D == 64 && PROD, VSCALE = D == 64;
     // The decode tables (layout above); after the chunk loop the space holds
     // the waves' results for the merge.
     __shared__ __attribute__((aligned(256))) uint32_t lut[kLutWords];
@@ -2825,12 +2875,22 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         for (int v = 0; v < kNT; ++v) acl[v] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     bool first = true;
+    uint32_t vtop = VSCALE ? v_top(v_bits(cur.valid ? cur.vs : 0u)) : 0u;  // wave-uniform
 
     while (t0 < t_end) {  // wave-uniform
+        if constexpr (VSCALE)
+            v_raise(v_bits(cur.valid ? cur.vs : 0u), vtop, [&](float f) {
+#pragma unroll
+                for (int v = 0; v < kNT; ++v) {
+                    acc[v] *= f;
+                    if constexpr (VLO) acl[v] *= f;
+                }
+            });
         {
-            const float ks = h2f(cur.ks), vs = h2f(cur.vs), re = PROD ? h2f(cur.re) : 0.0f;
-            const float4 sc = PROD ? make_float4(ks * ck, ks * re * cr, vs * iav, 0.0f)
-                                   : make_float4(ks * ck, ks * ck * kLoScale, vs * iav, 0.0f);
+            const float ks = h2f(cur.ks), re = PROD ? h2f(cur.re) : 0.0f;
+            const float vz = h2f(cur.vs) * (VSCALE ? iav * v_scale(vtop) : iav);
+            const float4 sc = PROD ? make_float4(ks * ck, ks * re * cr, vz, 0.0f)
+                                   : make_float4(ks * ck, ks * ck * kLoScale, vz, 0.0f);
             tsc[w][lane & (kChunk - 1)] = cur.valid ? sc : make_float4(0.f, 0.f, 0.f, -INFINITY);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -3004,6 +3064,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
             x0 = fmaf(acl[v][0] + acl[v][1], kLoScale, x0);
             x1 = fmaf(acl[v][2] + acl[v][3], kLoScale, x1);
         }
+        if constexpr (VSCALE) x0 *= v_unscale(vtop), x1 *= v_unscale(vtop);
         mo[w][2 * gq][kNT * i + v] = x0;
         mo[w][2 * gq + 1][kNT * i + v] = x1;
     }
