@@ -530,43 +530,44 @@ __device__ __forceinline__ half8 sign_octet(uint32_t wd) {
     return as_h8(__builtin_amdgcn_perm(ho, he, 0x040C000Cu), __builtin_amdgcn_perm(ho, he, 0x050C010Cu),
                  __builtin_amdgcn_perm(ho, he, 0x060C020Cu), __builtin_amdgcn_perm(ho, he, 0x070C030Cu));
 }
+// The factor of a logit's low products (K's and q's lo parts, x 2^kLoShift) for
+// a K scale x: 0 beside an infinite one, whose logit takes its sign from the hi
+// products (inf - inf otherwise).
+__device__ __forceinline__ float low_factor(float x) {
+    return __builtin_isinf(x) ? 0.0f : x * kLoScale;
+}
+// v of the even (odd) lane of this lane's pair.
+__device__ __forceinline__ float pair_even(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xA0, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float pair_odd(float v) {
+    return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0xF5, 0xF, 0xF, true));
+}
 // Exponent e with x * 2^-e in [0.5, 1); 0 for a zero or non-finite x.
 __device__ __forceinline__ int scale_exp(float x) {
     return __builtin_isfinite(x) ? __builtin_amdgcn_frexp_expf(x) : 0;
 }
-// V's power of two.  P * vs enters PV as an fp16 hi and lo part; with vs as it
-// is, products below 2^-14 fell among fp16's subnormals (step 6e-8, hi and lo
-// alike: V rows of rms 1e-5 were off by 3 ulps of the output).  So a wave's vs
-// are multiplied by the power of two that puts the largest into [2^13, 2^14):
-// products keep ~22 bits down to 2^-28 of it.  `top` is the largest fp16 with
-// the exponent of the largest finite vs so far; a chunk that passes it moves it
-// and rescales the wave's accumulators.  Head_dim 64, and the units over a slot
-// map, carry it; the first chunk's maximum costs 0.05-0.2 us of a call (8 rows x
-// 2 heads x 250 tokens at head_dim 64: 5.7 -> 5.9).  The one-group and paged
-// kernels at head_dim 128 take vs as it is.
-__device__ __forceinline__ float v_scale(uint32_t top) {  // 2^(28 - exponent field)
-    return __uint_as_float((155u - (top >> 10)) << 23);
+// V's power of two.  P * vs enters PV as an fp16 hi and lo part; with weights
+// of at most 1, products below 2^-14 fell among fp16's subnormals (step 6e-8, hi
+// and lo alike: V rows of rms 1e-5 were off by 3 ulps of the output).  So a
+// wave's softmax reference lies k below its maximum: weights and their sum are
+// 2^k times as large, with k such that the largest vs of the wave's tokens times
+// 2^k is in [2^13, 2^14), and products keep ~22 bits down to 2^-28 of it.  `top` is the largest fp16 with the exponent of the largest
+// finite vs so far; a chunk that passes it lowers k, and the accumulators are
+// rescaled as for a new maximum.  Head_dim 64, and the units over a slot map,
+// carry it.  The one-group and paged kernels at head_dim 128 have k = 0.
+constexpr uint32_t kVTop0 = 0x3FFu;  // (exponent field 0: subnormals and zeros)
+__device__ __forceinline__ float v_power(uint32_t top) {  // k
+    return 28.0f - (float)(int)(top >> 10);
 }
-__device__ __forceinline__ float v_unscale(uint32_t top) {
-    return __uint_as_float((99u + (top >> 10)) << 23);
-}
-// The bits of a finite vs (0: no token), else 0.
-__device__ __forceinline__ uint32_t v_bits(uint32_t vb) {
+// Moves top for a chunk whose vs (fp16 bits; 0: no token) are vb, one token in
+// lanes l and l + 32.
+__device__ __forceinline__ void v_raise(uint32_t vb, uint32_t& top) {
     vb &= 0x7FFFu;
-    return vb < 0x7C00u ? vb : 0u;
-}
-// top for a chunk of v_bits vb, one token in lanes l and l + 32.
-__device__ __forceinline__ uint32_t v_top(uint32_t vb) {
-    const uint32_t m = (uint32_t)max_lanes<32>((float)vb);
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)m) | 0x3FFu;
-}
-// Moves top for a further chunk; rescale(f): the accumulators times f.
-template <class F>
-__device__ __forceinline__ void v_raise(uint32_t vb, uint32_t& top, F rescale) {
+    if (vb >= 0x7C00u) vb = 0u;  // infinite or NaN
     if (!__any(vb > top)) return;
-    const uint32_t t = v_top(vb);
-    rescale(__uint_as_float((127u + (top >> 10) - (t >> 10)) << 23));
-    top = t;
+    const uint32_t m = (uint32_t)max_lanes<32>((float)vb);
+    top = (uint32_t)__builtin_amdgcn_readfirstlane((int)m) | 0x3FFu;
 }
 template <bool PROD>
 __device__ __forceinline__ void store_decode_tables(uint32_t* lut, int kv_words, int w, int lane,
@@ -1410,6 +1411,14 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
     constexpr int kE = D / 16;   // elements per lane of a row held by 16 lanes
     constexpr bool VLO = D == 64, QSCALE = D == 64, KLO = D == 64 && PROD;
     constexpr bool VSCALE = D == 64 || !PAGED;
+    // MLO (turbo_mse): q's lo parts are stored x 2^kLoShift, so that their
+    // product with K's hi parts and that of K's lo parts with q's hi parts share
+    // an accumulator (cs).  KLO: the products with a lo part come first, while
+    // the accumulator (cb) is small.  Added to a sum near the logit each costs a
+    // rounding of it: logits of 20-85 were off by 7-8e-6 instead of 4.2-4.6e-6
+    // (fp32 arithmetic: 3.9-4.8e-6).  With QSCALE log2(e) / sqrt(D) and the row's
+    // power of two enter in the exponent's FMA, for the same reason.
+    constexpr bool MLO = !PROD && (D == 64 || !PAGED);
     static_assert(kNT * sizeof(float) * kWaves * kMoRows * D <= 4 * kTabWords, "merge spaces");
     __shared__ __attribute__((aligned(256))) uint32_t lut[kTabWords];
     __shared__ uint4 bqs[kNP][kS][64];  // QK B operand (fp16 hi/lo q) of k-step s for lane l
@@ -1648,8 +1657,11 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                     const int at = 16 * (g_l + k / 2);  // (second block: two k-groups on)
                     reinterpret_cast<uint2*>(&bqs[op_hi][s_l][at + col_hi])[j16 & 1] =
                         make_uint2(h0, h1);
-                    reinterpret_cast<uint2*>(&bqs[op_lo][s_l][at + col_lo])[j16 & 1] =
-                        make_uint2(lo_pair(qf[k], qf[k + 1], h0), lo_pair(qf[k + 2], qf[k + 3], h1));
+                    uint2 lo = make_uint2(lo_pair(qf[k], qf[k + 1], h0), lo_pair(qf[k + 2], qf[k + 3], h1));
+                    if (MLO && npos > 1)
+                        lo = make_uint2(pack_h2(lo_part(qf[k]), lo_part(qf[k + 1])),
+                                        pack_h2(lo_part(qf[k + 2]), lo_part(qf[k + 3])));
+                    reinterpret_cast<uint2*>(&bqs[op_lo][s_l][at + col_lo])[j16 & 1] = lo;
                 }
             }
             store_decode_tables<PROD>(lut, kOffKV / 4, w, lane, tw);
@@ -1685,7 +1697,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                                                                 : 128u;
 
         int slot_nx = load_slot(t0 + kPass);
-        // One softmax state per lane and tile (its column's row), hi and lo
+        // One softmax state per lane and tile (its column's row; m_col: the
+        // reference, k below the maximum), hi and lo
         // stacked along the reductions.  A unit with fewer positions runs the
         // loop over the tiles it needs; a tile's unused columns compute on zero
         // queries and are dropped.
@@ -1701,11 +1714,11 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 if constexpr (VLO) acl_col[t][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
             }
         }
-        uint32_t vtop = VSCALE ? v_top(v_bits(cur.valid ? cur.vs : 0u)) : 0u;  // wave-uniform
+        uint32_t vtop = kVTop0;  // VSCALE: wave-uniform
         float qsc[kNT];
 #pragma unroll
         for (int t = 0; t < kNT; ++t)
-            qsc[t] = QSCALE && t < ntile ? rsc[npos == 1 ? i & 7 : 16 * t + i] : 1.0f;
+            qsc[t] = QSCALE && t < ntile ? ck * rsc[npos == 1 ? i & 7 : 16 * t + i] : 1.0f;
         // COLS (a unit of one position): one tile whose columns are the
         // position's rows as hi (columns 0-7) and lo (8-15) parts: one MFMA per
         // product instead of two, and the two halves of a column pair summed
@@ -1715,23 +1728,17 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
             constexpr bool COLS = decltype(cols)::value;
             static_assert(!COLS || NTA == 1, "one tile");
             while (t0 < t_end) {  // wave-uniform
-                if constexpr (VSCALE)
-                    v_raise(v_bits(cur.valid ? cur.vs : 0u), vtop, [&](float f) {
-#pragma unroll
-                        for (int t = 0; t < NTA; ++t)
-#pragma unroll
-                            for (int v = 0; v < kND; ++v)
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) {
-                                    acc_col[t][v][e] *= f;
-                                    if constexpr (VLO) acl_col[t][v][e] *= f;
-                                }
-                    });
+                // (before the next chunk is fetched into cur)
+                const uint32_t vtop_old = vtop;
+                if constexpr (VSCALE) v_raise(cur.valid ? cur.vs : 0u, vtop);
                 {
-                    const float ks = h2f(cur.ks), re = PROD ? h2f(cur.re) : 0.0f;
-                    const float vs = VSCALE ? h2f(cur.vs) * v_scale(vtop) : h2f(cur.vs);
+                    const float ks = h2f(cur.ks), vs = h2f(cur.vs), re = PROD ? h2f(cur.re) : 0.0f;
+                    const float kx = QSCALE ? 1.0f : ck, kr = QSCALE ? kAlphaK : cr;
                     tsc[w][lane & (kChunk - 1)] =
-                        cur.valid ? make_float4(ks * ck, PROD ? ks * re * cr : ks * ck * kLoScale,
+                        cur.valid ? make_float4(ks * kx,
+                                                PROD  ? ks * re * kr
+                                                : MLO ? low_factor(ks * kx)
+                                                      : ks * kx * kLoScale,
                                                 0.5f * vs, 0.0f)
                                   : make_float4(0.f, 0.f, 0.f, -INFINITY);
                 }
@@ -1790,14 +1797,17 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                     for (int tau = 0; tau < kTiles; ++tau) {
 #pragma unroll
                         for (int t = 0; t < NTA; ++t) {
-                            cb[t][tau] = mma(o.a[tau], o.bk[2 * t], cb[t][tau]);
-                            if (!COLS) cb[t][tau] = mma(o.a[tau], o.bk[2 * t + 1], cb[t][tau]);
+                            if constexpr (!KLO) cb[t][tau] = mma(o.a[tau], o.bk[2 * t], cb[t][tau]);
+                            if constexpr (!COLS) {
+                                f32x4& c = MLO ? cs[t][tau] : cb[t][tau];
+                                c = mma(o.a[tau], o.bk[2 * t + 1], c);
+                            }
                         }
                         // prod: the +-1 residual signs against the hi and lo query;
                         // mse: the codebook's lo parts (into cs) against the hi query
                         // only: the product of the two lo parts, each below 2^-11
-                        // of its value, is ~2^-22 of the logit (KLO: so K's lo parts,
-                        // into cb)
+                        // of its value, is at most 2^-22 of the logit's terms (KLO: so
+                        // K's lo parts, into cb)
                         half8 sg = o.al[tau];
                         if constexpr (KLO) {
 #pragma unroll
@@ -1811,9 +1821,21 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                             if (!COLS && PROD) cs[t][tau] = mma(sg, o.bk[2 * t + 1], cs[t][tau]);
                         }
                     }
+                    if constexpr (KLO) {
+                        static_assert(kS == 2, "both k-steps' operands in ops");
+                        if (s == kS - 1)
+#pragma unroll
+                            for (int k = 0; k < kS; ++k)
+#pragma unroll
+                                for (int tau = 0; tau < kTiles; ++tau)
+#pragma unroll
+                                    for (int t = 0; t < NTA; ++t)
+                                        cb[t][tau] = mma(ops[k].a[tau], ops[k].bk[2 * t], cb[t][tau]);
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 }
-                // Logits (base 2) of tokens 16*tau + 4*gq + e for this lane's column.
+                // Logits (base 2; QSCALE: before their row's factor qsc) of tokens
+                // 16*tau + 4*gq + e for this lane's column.
                 float lg[NTA][kTiles][4];
 #pragma unroll
                 for (int t = 0; t < NTA; ++t)
@@ -1823,12 +1845,19 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                         for (int e = 0; e < 4; ++e) {
                             const float4 sc = scq[tau][e];
                             float b = cb[t][tau][e], r = cs[t][tau][e];
+                            float low = 0.0f;
                             if constexpr (COLS) {  // + the partner column (lane ^ 8)
-                                b += lane_xor<8>(b);
+                                const float p = lane_xor<8>(b);
+                                const float lo = i & 8 ? b : p;
                                 r += lane_xor<8>(r);
+                                if constexpr (QSCALE && !PROD) r = fmaf(lo, (float)(1 << kLoShift), r);
+                                low = fmaf(r, sc.y, sc.w);
+                                if constexpr (QSCALE && PROD) low = fmaf(lo, sc.x, low);
+                                b = !QSCALE ? b + p : i & 8 ? p : b;
+                            } else {
+                                low = fmaf(r, sc.y, sc.w);
                             }
-                            lg[t][tau][e] = QSCALE ? fmaf(fmaf(b, sc.x, r * sc.y), qsc[t], sc.w)
-                                                   : fmaf(b, sc.x, fmaf(r, sc.y, sc.w));
+                            lg[t][tau][e] = fmaf(b, sc.x, low);
                         }
                 // The V lookups (B operands of PV) go out before the softmax,
                 // whose VALU work hides their LDS latency.
@@ -1895,7 +1924,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 // accumulators are rescaled) only when a logit passes it by more
                 // than 1, so the weights stay <= 2 (the PV operand is P * vs / 2).
                 float mloc[NTA];
-                bool grow = false;
+                bool grow = VSCALE && vtop != vtop_old;
+                const float k_new = VSCALE ? v_power(vtop) : 0.0f;
 #pragma unroll
                 for (int t = 0; t < NTA; ++t) {
                     // (IEEE maximum: no canonicalising of the lane-exchanged
@@ -1906,13 +1936,13 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                         m = __builtin_elementwise_maximum(m, lg[t][k >> 2][k & 3]);
                     const auto mx = [](float x, float y) { return __builtin_elementwise_maximum(x, y); };
                     m = lane_xor_reduce<16>(m, mx);
-                    mloc[t] = lane_xor_reduce<32>(m, mx);
-                    grow = grow || mloc[t] > m_col[t] + 1.0f;
+                    mloc[t] = lane_xor_reduce<32>(m, mx) * (QSCALE ? qsc[t] : 1.0f);
+                    grow = grow || mloc[t] - k_new > m_col[t] + 1.0f;
                 }
                 if (__any(grow)) {  // wave-uniform
 #pragma unroll
                     for (int t = 0; t < NTA; ++t) {
-                        const float m_new = fmaxf(m_col[t], mloc[t]);
+                        const float m_new = fmaxf(m_col[t] + (VSCALE ? v_power(vtop_old) : 0.0f), mloc[t]) - k_new;
                         const float alpha = __builtin_amdgcn_exp2f(m_col[t] - m_new);
                         m_col[t] = m_new;
                         l_col[t] *= alpha;
@@ -1935,7 +1965,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                     for (int tau = 0; tau < kTiles; ++tau)
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            lg[t][tau][e] = __builtin_amdgcn_exp2f(lg[t][tau][e] - m_col[t]);
+                            lg[t][tau][e] = __builtin_amdgcn_exp2f(
+                                QSCALE ? fmaf(lg[t][tau][e], qsc[t], -m_col[t]) : lg[t][tau][e] - m_col[t]);
                     // pairwise: no zero start, and the adds do not wait on one another
                     float part[kTiles];
 #pragma unroll
@@ -2033,7 +2064,6 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
         // position: lane group gq the waves' (m, l, o) of position gq, elements
         // 4j .. 4j + 3 (and 64 + 4j ..) per lane, then the inverse WHT and sign
         // flip, and the partial.
-        const float vun = 2.0f * iav * (VSCALE ? v_unscale(vtop) : 1.0f);
         auto mot = [&](int t) { return reinterpret_cast<float(*)[kMoRows][D]>(&lut[16384 * t]); };
         __syncthreads();  // every wave is done with the tables
 #pragma unroll
@@ -2045,7 +2075,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 for (int e = 0; e < 4; ++e) {  // (x2: the PV operand was P * vs / 2)
                     float x = acc_col[t][v][e];
                     if constexpr (VLO) x = fmaf(acl_col[t][v][e], kLoScale, x);
-                    mot(t)[w][4 * gq + e][kND * i + v] = x * vun;
+                    mot(t)[w][4 * gq + e][kND * i + v] = x * (2.0f * iav);
                 }
         }
         __syncthreads();
@@ -2862,11 +2892,11 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         PROD ? (uint32_t)reinterpret_cast<uintptr_t>(
                    (lds_u32*)&lut[32 + ((lane & 31) < kLoCopies ? lane & 31 : (lane & 31) - kLoCopies)])
              : basek;
-    const float qsc = QSCALE ? rsc[i >> 1] : 1.0f;
+    const float qsc = QSCALE ? ck * rsc[i >> 1] : 1.0f;
     const bool lo_col = (i & 1) != 0;
     const uint32_t lomask = lo_col ? 0xFFFFFFFFu : 0u;
 
-    float m_run = kInitMax, l_run = 0.0f;
+    float m_run = kInitMax, r_run = kInitMax, l_run = 0.0f;  // maximum, reference, sum
     f32x4 acc[kNT], acl[VLO ? kNT : 1];  // PV sums; VLO: of V's lo parts (x 2^kLoShift)
 #pragma unroll
     for (int v = 0; v < kNT; ++v) acc[v] = (f32x4){0.f, 0.f, 0.f, 0.f};
@@ -2875,26 +2905,20 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         for (int v = 0; v < kNT; ++v) acl[v] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     bool first = true;
-    uint32_t vtop = VSCALE ? v_top(v_bits(cur.valid ? cur.vs : 0u)) : 0u;  // wave-uniform
+    uint32_t vtop = kVTop0;  // VSCALE: wave-uniform
 
     while (t0 < t_end) {  // wave-uniform
-        if constexpr (VSCALE)
-            v_raise(v_bits(cur.valid ? cur.vs : 0u), vtop, [&](float f) {
-#pragma unroll
-                for (int v = 0; v < kNT; ++v) {
-                    acc[v] *= f;
-                    if constexpr (VLO) acl[v] *= f;
-                }
-            });
         {
-            const float ks = h2f(cur.ks), re = PROD ? h2f(cur.re) : 0.0f;
-            const float vz = h2f(cur.vs) * (VSCALE ? iav * v_scale(vtop) : iav);
-            const float4 sc = PROD ? make_float4(ks * ck, ks * re * cr, vz, 0.0f)
-                                   : make_float4(ks * ck, ks * ck * kLoScale, vz, 0.0f);
+            const float ks = h2f(cur.ks), vs = h2f(cur.vs), re = PROD ? h2f(cur.re) : 0.0f;
+            const float kx = QSCALE ? 1.0f : ck, kr = QSCALE ? kAlphaK : cr;
+            const float4 sc = PROD ? make_float4(ks * kx, ks * re * kr, vs * iav, 0.0f)
+                                   : make_float4(ks * kx, QSCALE ? low_factor(ks) : ks * kx * kLoScale,
+                                                 vs * iav, 0.0f);
             tsc[w][lane & (kChunk - 1)] = cur.valid ? sc : make_float4(0.f, 0.f, 0.f, -INFINITY);
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if constexpr (VSCALE) v_raise(cur.valid ? cur.vs : 0u, vtop);
         Chunk nxt;
         const int t1 = t0 + kPass;
         if (t1 < t_end) {  // codes of the next chunk, slots of the one after
@@ -2933,14 +2957,17 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
             cs[tau] = cb[tau];
 #pragma unroll
             for (int s = 0; s < kS; ++s) {
-                cb[tau] = mma(ka[tau][s], bq[s], cb[tau]);
-                if constexpr (KLO) {
+                if constexpr (KLO) {  // (K's lo parts first, see unit::)
                     cb[tau] = mma(kb[tau][s], bq[s], cb[tau]);
                     cs[tau] = mma(sign_octet(cur.kw[tau][s]), bq[s], cs[tau]);
                 } else {
+                    cb[tau] = mma(ka[tau][s], bq[s], cb[tau]);
                     cs[tau] = mma(kb[tau][s], bq[s], cs[tau]);  // prod: residual signs; mse: lo parts
                 }
             }
+            if constexpr (KLO)
+#pragma unroll
+                for (int s = 0; s < kS; ++s) cb[tau] = mma(ka[tau][s], bq[s], cb[tau]);
         }
         // V lookups (B operands of PV), in flight during the softmax.
         uint32_t bv[kNT][4];  // [N-tile v = d - kNT i][token pair]
@@ -2977,7 +3004,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
             }
         }
         __builtin_amdgcn_sched_barrier(0);
-        // Logits (base 2) of tokens 16 tau + 4 gq + e; hi + lo columns summed.
+        // Logits (base 2; QSCALE: before their row's factor qsc) of tokens
+        // 16 tau + 4 gq + e; hi + lo columns summed.
         float lg[2][4];
         float mloc = -INFINITY;
 #pragma unroll
@@ -2985,25 +3013,30 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
                 const float4 sc = scv[tau][e];
-                const float sb = cb[tau][e] + quad_xor<1>(cb[tau][e]);
-                const float sr = cs[tau][e] + quad_xor<1>(cs[tau][e]);
-                lg[tau][e] = QSCALE ? fmaf(fmaf(sb, sc.x, sr * sc.y), qsc, sc.w)
-                                    : fmaf(sb, sc.x, fmaf(sr, sc.y, sc.w));
+                const float sb = QSCALE ? pair_even(cb[tau][e]) : cb[tau][e] + quad_xor<1>(cb[tau][e]);
+                float sr = cs[tau][e] + quad_xor<1>(cs[tau][e]);
+                if constexpr (QSCALE && !PROD)
+                    sr = fmaf(pair_odd(cb[tau][e]), (float)(1 << kLoShift), sr);
+                float low = fmaf(sr, sc.y, sc.w);
+                if constexpr (QSCALE && PROD) low = fmaf(pair_odd(cb[tau][e]), sc.x, low);
+                lg[tau][e] = fmaf(sb, sc.x, low);
                 mloc = fmaxf(mloc, lg[tau][e]);
             }
         mloc = lane_xor_reduce<16>(mloc, [](float x, float y) { return fmaxf(x, y); });
         mloc = lane_xor_reduce<32>(mloc, [](float x, float y) { return fmaxf(x, y); });
         // v_exp_f32 without denormal handling: arguments are <= 0 and a weight
         // below 2^-126 of the running maximum is negligible.
-        const float m_new = fmaxf(m_run, mloc);
-        const float alpha = first ? 0.0f : __builtin_amdgcn_exp2f(m_run - m_new);
-        m_run = m_new;
+        m_run = fmaxf(m_run, QSCALE ? mloc * qsc : mloc);
+        const float ref = VSCALE ? m_run - v_power(vtop) : m_run;
+        const float alpha = first ? 0.0f : __builtin_amdgcn_exp2f(r_run - ref);
+        r_run = ref;
         float lsum = 0.0f;
 #pragma unroll
         for (int tau = 0; tau < 2; ++tau)
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                lg[tau][e] = __builtin_amdgcn_exp2f(lg[tau][e] - m_new);
+                lg[tau][e] = __builtin_amdgcn_exp2f(QSCALE ? fmaf(lg[tau][e], qsc, -ref)
+                                                           : lg[tau][e] - ref);
                 lsum += lg[tau][e];
             }
         l_run = l_run * alpha + lsum;
@@ -3052,7 +3085,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         float l_tot = lane_xor_reduce<16>(l_run, [](float x, float y) { return x + y; });
         l_tot = lane_xor_reduce<32>(l_tot, [](float x, float y) { return x + y; });
         if (gq == 0 && !lo_col) {
-            mm[w][i >> 1] = m_run;
+            mm[w][i >> 1] = r_run;
             ml[w][i >> 1] = l_tot;
         }
     }
@@ -3064,7 +3097,6 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
             x0 = fmaf(acl[v][0] + acl[v][1], kLoScale, x0);
             x1 = fmaf(acl[v][2] + acl[v][3], kLoScale, x1);
         }
-        if constexpr (VSCALE) x0 *= v_unscale(vtop), x1 *= v_unscale(vtop);
         mo[w][2 * gq][kNT * i + v] = x0;
         mo[w][2 * gq + 1][kNT * i + v] = x1;
     }
