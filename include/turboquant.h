@@ -290,11 +290,12 @@ int tq_workspace_release(void);
 /* No reference counterpart.  For callers that cannot allocate device memory
  * (code under graph capture, tight serving loops, harnesses that forbid
  * hipMalloc): tq_launch_turbo_prod_fused_attention_output (src/tq_capi.cpp:99
- * semantics, same arguments and result) with its split-K partials in a
- * static 4 MiB device array instead of an allocated workspace; it calls no
- * hipMalloc, hipFree or allocating library routine.  A launch whose
- * partials exceed 4 MiB (more than 1,008 split workgroups of 8 query rows,
- * 4,160 bytes each) returns -2.  Every call on one GPU shares that GPU's array: calls that
+ * semantics, same arguments and, bit for bit, result) with its split-K
+ * partials in a static 16.25 MiB device array instead of an allocated workspace;
+ * it calls no hipMalloc, hipFree or allocating library routine.  A call whose
+ * partials at one 256-token split per workgroup (or two workgroups per CU,
+ * whichever is fewer) exceed 4 MiB (more than 1,008 split workgroups of 8 query
+ * rows, 4,160 bytes each) returns -2.  Every call on one GPU shares that GPU's array: calls that
  * overlap on one GPU (other streams, threads or graph replays) race. */
 int tq_launch_turbo_prod_fused_attention_output_noalloc(
     const uint16_t* query, const uint8_t* page_pool, const int32_t* slot_mapping,

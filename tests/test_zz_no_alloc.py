@@ -132,3 +132,55 @@ def test_noalloc_rejects_launch_beyond_scratch(tq, cuda):
         tq.fused_attn_output_noalloc(q, pool, slots, out, lp, cfg, Q, N)
     torch.cuda.synchronize()
     assert torch.all(out == 3.0)  # nothing ran
+
+
+@pytest.mark.parametrize("D,Q,H,N", [
+    (128, 32, 2, 32768),  # a unit of four row groups over 128 splits: 4.3 MB of partials
+    (128, 192, 2, 8192),
+    (128, 40, 3, 20000),
+    (128, 16, 1, 100),    # one split
+    (64, 8, 2, 3000),
+    (64, 192, 2, 8192),
+    (64, 1, 2048, 300),   # padded row groups of one row: 4.3 MB each split
+])
+def test_noalloc_same_choice_as_allocating_entry(tq, cuda, D, Q, H, N):
+    """Kernel and split count are the allocating entry's, also where its
+    partials are larger than the 4 MiB that a call is held to: the same bits."""
+    print(f"[noalloc choice] D={D} Q={Q} H={H} N={N}", flush=True)
+    cfg, lp = _cfg(tq, H, D)
+    g = torch.Generator(device=cuda).manual_seed(97)
+    k, v = (torch.randn(N, H, D, generator=g, device=cuda).half() for _ in range(2))
+    q = torch.randn(Q, H, D, generator=g, device=cuda).half()
+    slots = permuted_slots(N, 16, seed=98).to(cuda)
+    pool = torch.zeros((N + 15) // 16 * lp.page_size_bytes, dtype=torch.uint8, device=cuda)
+    tq.pack(k, v, slots, pool, lp, cfg)
+    got, want = torch.full_like(q, 3.0), torch.full_like(q, 5.0)
+    tq.fused_attn_output(q, pool, slots, want, lp, cfg, Q, N)
+    tq.fused_attn_output_noalloc(q, pool, slots, got, lp, cfg, Q, N)
+    torch.cuda.synchronize()
+    assert np.array_equal(as_u16(got), as_u16(want))
+
+
+def test_noalloc_limit_at_head_dim_64(tq, cuda):
+    """264 bytes per row and split (the generic decode's partials) within 4 MiB:
+    15,887 rows of one split are accepted, 15,888 refused."""
+    cfg, lp = _cfg(tq, H=1, D=64)
+    N = 16
+    g = torch.Generator(device=cuda).manual_seed(99)
+    k, v = (torch.randn(N, 1, 64, generator=g, device=cuda).half() for _ in range(2))
+    slots = torch.arange(N, dtype=torch.int32, device=cuda)
+    pool = torch.zeros(lp.page_size_bytes, dtype=torch.uint8, device=cuda)
+    tq.pack(k, v, slots, pool, lp, cfg)
+    for Q, ok in ((15887, True), (15888, False)):
+        q = torch.randn(Q, 1, 64, generator=g, device=cuda).half()
+        out, want = torch.full_like(q, 3.0), torch.full_like(q, 5.0)
+        if not ok:
+            with pytest.raises(RuntimeError, match="split-K scratch"):
+                tq.fused_attn_output_noalloc(q, pool, slots, out, lp, cfg, Q, N)
+            torch.cuda.synchronize()
+            assert torch.all(out == 3.0)  # nothing ran
+            continue
+        tq.fused_attn_output_noalloc(q, pool, slots, out, lp, cfg, Q, N)
+        tq.fused_attn_output(q, pool, slots, want, lp, cfg, Q, N)
+        torch.cuda.synchronize()
+        assert np.array_equal(as_u16(out), as_u16(want))

@@ -3293,6 +3293,21 @@ void launch_qjl_mfma(const uint16_t* query, const uint8_t* pool, const int32_t* 
     check_launch(combine_name);
 }
 
+// The generic split-K decode (attn_partial_kernel + attn_combine_kernel, any
+// head_dim and page geometry): one wave per (split, row), enough waves to
+// cover the chip several times, at least 32 tokens per split.
+struct GenericSplit {
+    int splits, tps;
+    size_t ws_bytes;
+};
+GenericSplit generic_split(int rows, int max_tokens, int D) {
+    int splits = (2048 + rows - 1) / rows;
+    splits = std::min(splits, std::max(1, (max_tokens + 31) / 32));
+    splits = std::max(splits, 1);
+    const int tps = max_tokens > 0 ? (max_tokens + splits - 1) / splits : 0;
+    if (tps > 0) splits = (max_tokens + tps - 1) / tps;
+    return {splits, tps, (size_t)splits * rows * (D + 2) * sizeof(float)};
+}
 // The slot-mapped decode (turbo_prod, turbo_mse; D = 64, 128): split + combine,
 // with one row group per workgroup (dec::) or units of up to four that share
 // the decoded chunks (unit::).
@@ -3300,7 +3315,7 @@ struct DecodeSplit {
     int rows, row_groups, heads, items, splits, tps;
     bool units;
     long long combine_blocks;
-    size_t blocks, ws_bytes, limit_bytes;  // limit_bytes: what a fixed scratch is held to
+    size_t blocks, ws_bytes;
 };
 // Cost of a split kernel's workgroup: a setup and merge, and a pass of 256
 // tokens, in 0.1 us (measured at D = 128, turbo_prod, 2 heads, 250 to 32,768
@@ -3322,11 +3337,11 @@ struct SplitChoice {
     int splits;
     long long cost;
 };
-SplitChoice choose_splits(int items, int passes, SplitCost c, int most, int cus) {
+SplitChoice choose_splits(int items, int passes, SplitCost c, int cus) {
     const long long whole = ((long long)items + cus - 1) / cus * (c.setup + (long long)c.pass * passes);
     SplitChoice best{1, whole};
     for (int r = 1; r <= 4; ++r) {
-        int s = std::min({std::max(1, (int)((long long)r * cus / items)), passes, most});
+        int s = std::min({std::max(1, (int)((long long)r * cus / items)), passes, 1024});
         const int per = (passes + s - 1) / s;
         s = (passes + per - 1) / per;
         const long long rounds = ((long long)items * s + cus - 1) / cus;
@@ -3336,8 +3351,21 @@ SplitChoice choose_splits(int items, int passes, SplitCost c, int most, int cus)
     }
     return best;
 }
-// cap: a fixed scratch's bytes, or 0.
-DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens, size_t cap) {
+// What a caller's fixed scratch is held to, whatever the launch takes: at D = 128
+// the partials of one 256-token split per workgroup, or of longer splits once
+// there are more than ~2 workgroups per CU and row group; at D = 64 the generic
+// decode's.
+size_t fixed_scratch_bytes(const PageGeom& g, int num_queries, int num_kv_tokens) {
+    if (g.D == 64) return generic_split(num_queries * g.H, num_kv_tokens, g.D).ws_bytes;
+    const int heads = g.H * ((num_queries + mfma::kRows - 1) / mfma::kRows);
+    const int passes = std::max(1, (num_kv_tokens + kSplitMinTokens - 1) / kSplitMinTokens);
+    const int want = std::max(1, (kSplitBlocksPerCU * num_cus() + heads - 1) / heads);
+    int splits = std::min(std::min(passes, want), 1024);
+    const int tps = num_kv_tokens > 0 ? (num_kv_tokens + splits - 1) / splits : 0;
+    if (tps > 0) splits = (num_kv_tokens + tps - 1) / tps;
+    return (size_t)splits * heads * dec::part_bytes(g.D);
+}
+DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens) {
     using namespace mfma;
     DecodeSplit d{};
     const int cus = num_cus();
@@ -3348,22 +3376,9 @@ DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens, 
     d.combine_blocks = ((long long)d.rows * (g.D / 32) + 7) / 8 * 32;
     const size_t per_split = (size_t)d.heads * dec::part_bytes(g.D);
     const int passes = std::max(1, (num_kv_tokens + kSplitMinTokens - 1) / kSplitMinTokens);
-    if (cap) {
-        // The partials a fixed scratch has to hold for a call to be taken: one
-        // 256-token split per workgroup, or longer splits once there are more
-        // than ~2 workgroups per CU and row group.  The launch itself takes no
-        // more splits than fit.
-        const int want = std::max(1, (kSplitBlocksPerCU * cus + d.heads - 1) / d.heads);
-        int splits = std::min(std::min(passes, want), 1024);
-        const int tps = num_kv_tokens > 0 ? (num_kv_tokens + splits - 1) / splits : 0;
-        if (tps > 0) splits = (num_kv_tokens + tps - 1) / tps;
-        d.limit_bytes = splits * per_split;
-    }
-    const int most = cap ? (int)std::min<size_t>(1024, std::max<size_t>(1, cap / per_split)) : 1024;
     const int units = g.H * ((d.row_groups + unit::kNP - 1) / unit::kNP);
-    const SplitChoice one = choose_splits(d.heads, passes, kGroupCost, most, cus);
-    const SplitChoice un =
-        choose_splits(units, passes, d.row_groups == 2 ? kPairCost : kUnitCost, most, cus);
+    const SplitChoice one = choose_splits(d.heads, passes, kGroupCost, cus);
+    const SplitChoice un = choose_splits(units, passes, d.row_groups == 2 ? kPairCost : kUnitCost, cus);
     d.units = d.row_groups > 1 && un.cost < one.cost;
     d.items = d.units ? units : d.heads;
     d.splits = d.units ? un.splits : one.splits;
@@ -3382,7 +3397,6 @@ void launch_decode_attention(const uint16_t* query, const uint8_t* pool, const i
     using namespace mfma;
     if (d.combine_blocks > INT32_MAX)
         throw Error(std::string(combine_name) + ": too many query rows");
-    if (scratch.ptr) (void)scratch.get(stream, d.limit_bytes, split_name);  // throws past its limit
     const int S = num_kv_tokens > 0 ? d.splits : 0;
     char* ws = S == 1 ? nullptr : static_cast<char*>(scratch.get(stream, d.ws_bytes, split_name));
     float* po = reinterpret_cast<float*>(ws);
@@ -3418,21 +3432,7 @@ void launch_decode_attention(const uint16_t* query, const uint8_t* pool, const i
     check_launch(combine_name);
 }
 
-// The generic split-K decode (attn_partial_kernel + attn_combine_kernel, any
-// head_dim and page geometry): one wave per (split, row), enough waves to
-// cover the chip several times, at least 32 tokens per split.
-struct GenericSplit {
-    int splits, tps;
-    size_t ws_bytes;
-};
-GenericSplit generic_split(int rows, int max_tokens, int D) {
-    int splits = (2048 + rows - 1) / rows;
-    splits = std::min(splits, std::max(1, (max_tokens + 31) / 32));
-    splits = std::max(splits, 1);
-    const int tps = max_tokens > 0 ? (max_tokens + splits - 1) / splits : 0;
-    if (tps > 0) splits = (max_tokens + tps - 1) / tps;
-    return {splits, tps, (size_t)splits * rows * (D + 2) * sizeof(float)};
-}
+// (generic_split)
 template <class Tok>
 void launch_generic_attention(Scheme s, const uint16_t* query, const uint8_t* pool, Tok tok,
                               uint16_t* output, const PageGeom& g, int rows,
@@ -3530,13 +3530,12 @@ void launch_attention(Scheme s, const uint16_t* query, const uint8_t* pool, cons
         prod ? "turbo_prod_fused_attn_combine" : "turbo_mse_fused_attn_combine";
     const bool d64 = mfma_attention64_ok(g, pool);
     if (d64 || mfma_attention_ok(g, pool)) {
-        const DecodeSplit d =
-            decode_split(g, num_queries, num_kv_tokens, scratch.ptr ? scratch.cap : 0);
-        // head_dim 64: where a caller's scratch is too small for the padded
-        // row groups' partials, or there are too many rows for the combine's
-        // grid, the generic decode below takes the call if it can.
-        const bool fits = !d64 || ((!scratch.ptr || d.ws_bytes <= scratch.cap) &&
-                                   d.combine_blocks <= INT32_MAX && d.blocks <= INT32_MAX);
+        const DecodeSplit d = decode_split(g, num_queries, num_kv_tokens);
+        // head_dim 64: where there are too many rows for the combine's grid, the
+        // generic decode below takes the call if it can.
+        const bool fits = !d64 || (d.combine_blocks <= INT32_MAX && d.blocks <= INT32_MAX);
+        if (scratch.ptr)
+            scratch.hold(fixed_scratch_bytes(g, num_queries, num_kv_tokens), split_name);
         const auto go = [&](auto sch) {
             constexpr int kSch = decltype(sch)::value;
             if (d64)
@@ -3557,8 +3556,9 @@ void launch_attention(Scheme s, const uint16_t* query, const uint8_t* pool, cons
         }
     }
     const GenericSplit sp = generic_split(rows, num_kv_tokens, g.D);
-    float* ws = static_cast<float*>(scratch.get(
-        stream, sp.ws_bytes, prod ? "turbo_prod_fused_attn_partial" : "turbo_mse_fused_attn_partial"));
+    const char* partial_name = prod ? "turbo_prod_fused_attn_partial" : "turbo_mse_fused_attn_partial";
+    scratch.hold(sp.ws_bytes, partial_name);
+    float* ws = static_cast<float*>(scratch.get(stream, sp.ws_bytes, partial_name));
     launch_generic_attention(s, query, pool, SlotTokens{slots, num_kv_tokens}, output, g, rows, sp,
                              ws, stream, prod ? "turbo_prod_fused_attn" : "turbo_mse_fused_attn");
 }

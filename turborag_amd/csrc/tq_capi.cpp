@@ -462,12 +462,21 @@ void* workspace(hipStream_t stream, size_t bytes) {
     return p;
 }
 
+namespace {
+[[noreturn]] void too_large(const char* what, size_t bytes, size_t have) {
+    throw Error(std::string(what) + ": needs " + std::to_string(bytes) +
+                " bytes of split-K scratch, more than the " + std::to_string(have) +
+                " bytes available");
+}
+}  // namespace
+
+void Scratch::hold(size_t bytes, const char* what) const {
+    if (ptr && bytes > limit) too_large(what, bytes, limit);
+}
+
 void* Scratch::get(hipStream_t stream, size_t bytes, const char* what) const {
     if (!ptr) return workspace(stream, bytes);
-    if (bytes > cap)
-        throw Error(std::string(what) + ": needs " + std::to_string(bytes) +
-                    " bytes of split-K scratch, more than the " + std::to_string(cap) +
-                    " bytes available");
+    if (bytes > cap) too_large(what, bytes, cap);
     return ptr;
 }
 

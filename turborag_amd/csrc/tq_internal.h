@@ -74,10 +74,12 @@ void check_launch(const char* what);
 void* workspace(hipStream_t stream, size_t bytes);
 // Where an attention launch takes its split-K partials from: the cached
 // per-stream workspace above (ptr null), or memory the caller provides
-// (ptr, cap bytes), in which case a launch that needs more throws.
+// (ptr, cap bytes), in which case a launch that needs more throws, as does one
+// that hold()s it to more than `limit` bytes.
 struct Scratch {
     void* ptr = nullptr;
-    size_t cap = 0;
+    size_t cap = 0, limit = 0;
+    void hold(size_t bytes, const char* what) const;
     void* get(hipStream_t stream, size_t bytes, const char* what) const;
 };
 // Synchronizes the devices and frees every cached workspace (tq_workspace_release).

@@ -4,8 +4,9 @@
 //
 // tq_launch_turbo_prod_fused_attention_output takes its split-K partials
 // from a per-stream workspace that it allocates on first use.  This variant
-// runs the same kernels with the partials in `scratch`, a file-scope device
-// array of kScratchBytes: no hipMalloc, hipFree or allocating library call.
+// runs the same kernels, with the same splits and so the same results, with the
+// partials in `scratch`, a file-scope device array of kScratchBytes: no
+// hipMalloc, hipFree or allocating library call.
 // Each GPU holds its own copy of the array until the process ends; host code
 // uses the per-device address from hipGetSymbolAddress, taken once per
 // device on the first call with that device current (the array's name in
@@ -21,10 +22,15 @@
 
 namespace {
 
-// 4 MiB: the partials of up to 1,008 split workgroups (8 query rows, 4,160
-// bytes each: 4,194,304 / 4,160 = 1,008.2); the
-// GQA 16/2 decode step at 32K context uses 256 (1.08 MB).
-constexpr size_t kScratchBytes = size_t(4) << 20;
+// The most that a launch's partials take: it fills at most four rounds of the
+// 256 CUs with workgroups of up to four row groups of 4,160 bytes (8 query rows
+// at head_dim 128) each, or has one split and no partials.
+constexpr size_t kScratchBytes = size_t(4 * 256 * 4) * 4160;
+// What a call is held to: one 256-token split per workgroup (or two workgroups
+// per CU, whichever is fewer) within 4 MiB, i.e. up to 1,008 split workgroups of
+// 8 query rows (4,194,304 / 4,160 = 1,008.2); the GQA 16/2 decode step at 32K
+// context uses 256.
+constexpr size_t kScratchLimit = size_t(4) << 20;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
 constexpr int kMaxDevices = 64;
@@ -67,6 +73,7 @@ extern "C" int tq_launch_turbo_prod_fused_attention_output_noalloc(
         tq::Scratch s;
         s.ptr = device_scratch();
         s.cap = kScratchBytes;
+        s.limit = kScratchLimit;
         tq::launch_attention(tq::Scheme::Prod, query, page_pool, slot_mapping, output, g,
                              num_queries, num_kv_tokens, static_cast<hipStream_t>(stream), s);
         tq::debug_sync(stream);
