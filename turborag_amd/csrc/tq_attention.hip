@@ -3315,7 +3315,7 @@ struct DecodeSplit {
     int rows, row_groups, heads, items, splits, tps;
     bool units;
     long long combine_blocks;
-    size_t blocks, ws_bytes;
+    size_t blocks, ws_bytes, want_bytes;  // want_bytes: room for any call of as many rows and no more tokens
 };
 // Cost of a split kernel's workgroup: a setup and merge, and a pass of 256
 // tokens, in 0.1 us (measured at D = 128, turbo_prod, 2 heads, 250 to 32,768
@@ -3351,6 +3351,10 @@ SplitChoice choose_splits(int items, int passes, SplitCost c, int cus) {
     }
     return best;
 }
+// At head_dim 64 every call leaves room for the most that a slot-mapped call
+// takes, 8.7 MB (four rounds of the CUs, up to four row groups each): the kernels
+// these replaced fitted nearly every call into the 1 MB that the first one left.
+size_t workspace64() { return (size_t)16 * num_cus() * dec::part_bytes(64); }
 // What a caller's fixed scratch is held to, whatever the launch takes: at D = 128
 // the partials of one 256-token split per workgroup, or of longer splits once
 // there are more than ~2 workgroups per CU and row group; at D = 64 the generic
@@ -3377,6 +3381,9 @@ DecodeSplit decode_split(const PageGeom& g, int num_queries, int num_kv_tokens) 
     const size_t per_split = (size_t)d.heads * dec::part_bytes(g.D);
     const int passes = std::max(1, (num_kv_tokens + kSplitMinTokens - 1) / kSplitMinTokens);
     const int units = g.H * ((d.row_groups + unit::kNP - 1) / unit::kNP);
+    // (the splits need not grow with the tokens: 76,800 take 100 where 32,768 take 128)
+    d.want_bytes = std::min({passes, 1024, (4 * cus + units - 1) / units}) * per_split;
+    if (g.D == 64) d.want_bytes = std::max(d.want_bytes, workspace64());
     const SplitChoice one = choose_splits(d.heads, passes, kGroupCost, cus);
     const SplitChoice un = choose_splits(units, passes, d.row_groups == 2 ? kPairCost : kUnitCost, cus);
     d.units = d.row_groups > 1 && un.cost < one.cost;
@@ -3398,7 +3405,8 @@ void launch_decode_attention(const uint16_t* query, const uint8_t* pool, const i
     if (d.combine_blocks > INT32_MAX)
         throw Error(std::string(combine_name) + ": too many query rows");
     const int S = num_kv_tokens > 0 ? d.splits : 0;
-    char* ws = S == 1 ? nullptr : static_cast<char*>(scratch.get(stream, d.ws_bytes, split_name));
+    char* ws = static_cast<char*>(
+        scratch.get(stream, S == 1 ? 0 : d.ws_bytes, split_name, d.want_bytes));
     float* po = reinterpret_cast<float*>(ws);
     float2* pml = reinterpret_cast<float2*>(
         reinterpret_cast<uintptr_t>(ws) + (size_t)d.splits * d.heads * kRows * D * sizeof(float));
@@ -3482,7 +3490,12 @@ void launch_paged_units(const uint16_t* query, const uint8_t* pool, const int32_
         ((size_t)heads + G) * unit::kNP * kRows * unit::part_stride(D) * sizeof(float);
     const size_t unit_bytes = (2 * (size_t)row_groups + 1) * sizeof(PagedUnit);
     const size_t spare_at = (part_bytes + unit_bytes + 4 * sizeof(int32_t) + 255) & ~(size_t)255;
-    char* wsb = static_cast<char*>(workspace(stream, spare_at + extent));
+    // head_dim 64: room for the steps of up to 240 (row group, head) pairs, which
+    // the kernels these replaced fitted into the least workspace, 1 MB.
+    const size_t more = (size_t)std::max(0, 240 - heads) *
+                        (unit::kNP * kRows * unit::part_stride(D) * sizeof(float) + 2 * sizeof(PagedUnit));
+    char* wsb = static_cast<char*>(workspace(
+        stream, spare_at + extent, D == 64 ? std::max(spare_at + extent + more, workspace64()) : 0));
     float* ws = reinterpret_cast<float*>(wsb);
     PagedUnit* units = reinterpret_cast<PagedUnit*>(wsb + part_bytes);
     PagedUnit* group_unit = units + row_groups + 1;

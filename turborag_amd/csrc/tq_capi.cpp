@@ -287,8 +287,8 @@ int num_cus() {
 }
 
 // Split-K workspace for attention: one buffer per (device, stream).  Calls
-// on one stream run in order, so they can share it.  A call that needs more
-// replaces the buffer; the old one may still be read by kernels already
+// on one stream run in order, so they can share it.  A call that needs (outside
+// a capture: wants) more replaces the buffer; the old one may still be read by kernels already
 // enqueued on the stream, so it is retired with an event recorded behind them
 // and freed once that event has completed (checked on later calls).  A
 // buffer handed out while its stream was being captured into a graph is
@@ -420,14 +420,16 @@ void release_all(bool keep_captured = false) {
 }
 }  // namespace
 
-void* workspace(hipStream_t stream, size_t bytes) {
+void* workspace(hipStream_t stream, size_t bytes, size_t want) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) throw Error("hipGetDevice failed");
     std::lock_guard<std::mutex> lock(g_ws_mu);
     const bool cap = capturing(stream);
+    const size_t need = cap ? bytes : std::max(bytes, want);
     auto it = g_ws.find({dev, stream});
-    if (it != g_ws.end() && it->second.n >= bytes && it->second.p) {
-        it->second.captured = it->second.captured || cap;
+    if (need == 0 || (it != g_ws.end() && it->second.n >= need && it->second.p)) {
+        if (it == g_ws.end()) return nullptr;
+        it->second.captured = it->second.captured || (cap && bytes > 0);
         it->second.last_use = ++g_ws_tick;
         return it->second.p;
     }
@@ -436,10 +438,15 @@ void* workspace(hipStream_t stream, size_t bytes) {
         if (it == g_ws.end() && g_ws.size() >= kMaxStreams) evict_lru();
     }
     WsBuf& b = g_ws[{dev, stream}];
-    size_t n = std::max<size_t>(bytes, 1 << 20);
-    n = std::max(n, b.n * 2);
+    size_t n = std::max({need, b.n * 2, size_t(1) << 20});
     void* p = nullptr;
-    if (hipMalloc(&p, n) != hipSuccess) {
+    bool ok = hipMalloc(&p, n) == hipSuccess;
+    if (!ok && need > bytes) {  // no room for what it wants: what it needs
+        (void)hipGetLastError();
+        if (b.n >= bytes) return b.p;
+        ok = hipMalloc(&p, n = bytes) == hipSuccess;
+    }
+    if (!ok) {
         (void)hipGetLastError();
         throw Error("workspace hipMalloc failed");
     }
@@ -474,8 +481,8 @@ void Scratch::hold(size_t bytes, const char* what) const {
     if (ptr && bytes > limit) too_large(what, bytes, limit);
 }
 
-void* Scratch::get(hipStream_t stream, size_t bytes, const char* what) const {
-    if (!ptr) return workspace(stream, bytes);
+void* Scratch::get(hipStream_t stream, size_t bytes, const char* what, size_t want) const {
+    if (!ptr) return workspace(stream, bytes, want);
     if (bytes > cap) too_large(what, bytes, cap);
     return ptr;
 }

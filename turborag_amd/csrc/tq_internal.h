@@ -70,8 +70,11 @@ float inv_sqrt_d(int D);
 void check_launch(const char* what);
 
 // Per-(device, stream) scratch for split-K partials.  Grows; an outgrown
-// buffer is freed once the stream's earlier kernels have finished.
-void* workspace(hipStream_t stream, size_t bytes);
+// buffer is freed once the stream's earlier kernels have finished.  Outside a
+// stream capture the buffer is made to hold `want` bytes too (null only for 0
+// bytes): a capture cannot allocate, so a call leaves room for the calls like it
+// that need more than it does itself.
+void* workspace(hipStream_t stream, size_t bytes, size_t want = 0);
 // Where an attention launch takes its split-K partials from: the cached
 // per-stream workspace above (ptr null), or memory the caller provides
 // (ptr, cap bytes), in which case a launch that needs more throws, as does one
@@ -80,7 +83,7 @@ struct Scratch {
     void* ptr = nullptr;
     size_t cap = 0, limit = 0;
     void hold(size_t bytes, const char* what) const;
-    void* get(hipStream_t stream, size_t bytes, const char* what) const;
+    void* get(hipStream_t stream, size_t bytes, const char* what, size_t want = 0) const;
 };
 // Synchronizes the devices and frees every cached workspace (tq_workspace_release).
 void release_workspaces();
