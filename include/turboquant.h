@@ -205,8 +205,9 @@ int tq_launch_turbo_mse_pack_kv_layers(const uint16_t* const* keys, const uint16
  * as a document's layers do, cag_store.py:129).  page_pools, out_keys and
  * out_values are HOST arrays of num_layers device pointers, read during the
  * call.  Outputs are [num_tokens, H, D] fp16, or [1, H, num_tokens, D] when
- * head_major != 0.  For D = 64 and 128 one launch covers up to 64 layers; the
- * layers run concurrently, so the outputs must not overlap each other. */
+ * head_major != 0.  For D = 64 and 128 one launch covers up to 64 layers, which
+ * run concurrently.  D = 128: the outputs must not overlap each other; D = 64:
+ * layers whose outputs overlap are launched one by one, in order. */
 int tq_launch_turbo_prod_dequant_kv_layers(const uint8_t* const* page_pools,
                                            const int32_t* slot_mapping,
                                            uint16_t* const* out_keys, uint16_t* const* out_values,

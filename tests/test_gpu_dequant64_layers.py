@@ -90,3 +90,44 @@ def test_one_large_layer(tq, oracle, cuda, scheme, head_major, N):
         if head_major:
             got = got[0].transpose(1, 0, 2)
         assert np.array_equal(got[live], want[live]) and np.all(got[~live] == seven)
+
+
+@pytest.mark.parametrize("scheme", ["turbo_prod", "turbo_mse"])
+@pytest.mark.parametrize("shared", ["both", "keys", "shifted"])
+def test_overlapping_outputs(tq, oracle, cuda, scheme, shared):
+    """Layers that write one output buffer (or buffers that overlap by some
+    rows) are taken in order: the last layer's values."""
+    NL, N, H, B = 12, 3001, 2, 16
+    print(f"[dequant64 overlap {scheme}] {shared}", flush=True)
+    prod = scheme == "turbo_prod"
+    cfg = tq.default_config()
+    cfg.num_kv_heads, cfg.head_dim, cfg.block_size = H, D, B
+    lay = tq.make_layout_for(cfg) if prod else tq.make_mse_layout_for(cfg)
+    slots = permuted_slots(N, B, seed=690)
+    pages = int(slots.max()) // B + 1
+    pack = oracle.prod_pack if prod else oracle.mse_pack
+    pools_np = []
+    for layer in range(NL):
+        k, v = kv_tokens_major(N, H, D, seed=691 + layer)
+        pools_np.append(pack(as_u16(k), as_u16(v), slots.numpy(), pages, B))
+    pools = [torch.from_numpy(p).to(cuda) for p in pools_np]
+    step = {"both": 0, "keys": 0, "shifted": 100}[shared]  # tokens between two layers' outputs
+    kb = torch.full((N + step * (NL - 1), H, D), 7.0, dtype=torch.float16, device=cuda)
+    vb = torch.full_like(kb, 7.0)
+    oks = [kb[step * layer:step * layer + N] for layer in range(NL)]
+    ovs = [vb[step * layer:step * layer + N] if shared != "keys" else torch.full_like(oks[0], 7.0)
+           for layer in range(NL)]
+    tq.dequant_layers(scheme, pools, slots.to(cuda), oks, ovs, lay, cfg, N)
+    torch.cuda.synchronize()
+    fn = oracle.prod_dequant if prod else oracle.mse_dequant
+    want_k = np.full(kb.shape, np.float16(7.0).view(np.uint16))
+    want_v = want_k.copy()
+    for layer in range(NL):
+        wk, wv = fn(pools_np[layer], slots.numpy(), H, D, B)
+        want_k[step * layer:step * layer + N] = wk
+        want_v[step * layer:step * layer + N] = wv
+        if shared == "keys":
+            assert np.array_equal(as_u16(ovs[layer]), wv)
+    assert np.array_equal(as_u16(kb), want_k)
+    if shared != "keys":
+        assert np.array_equal(as_u16(vb), want_v)

@@ -9,6 +9,7 @@
 // to the reference's CUDA kernels (given correctly rounded / and sqrt, which
 // this library is compiled for).
 #include <algorithm>
+#include <vector>
 
 #include "tq_device.h"
 
@@ -1390,6 +1391,18 @@ void launch_dequant(Scheme s, const uint8_t* pool, const int32_t* slots, uint16_
     }
 }
 
+// Whether any two of the layers' 2n outputs of `bytes` bytes overlap.
+static bool outputs_overlap(uint16_t* const* out_key, uint16_t* const* out_value, int n, size_t bytes) {
+    std::vector<uintptr_t> at;
+    at.reserve(2 * (size_t)n);
+    for (int l = 0; l < n; ++l) at.push_back(reinterpret_cast<uintptr_t>(out_key[l]));
+    for (int l = 0; l < n; ++l) at.push_back(reinterpret_cast<uintptr_t>(out_value[l]));
+    if (!std::is_sorted(at.begin(), at.end())) std::sort(at.begin(), at.end());
+    for (size_t k = 1; k < at.size(); ++k)
+        if (at[k] - at[k - 1] < bytes) return true;
+    return false;
+}
+
 void launch_dequant_layers(Scheme s, const uint8_t* const* pools, const int32_t* slots,
                            uint16_t* const* out_key, uint16_t* const* out_value, const PageGeom& g,
                            int num_tokens, int num_layers, hipStream_t stream, bool head_major) {
@@ -1404,6 +1417,11 @@ void launch_dequant_layers(Scheme s, const uint8_t* const* pools, const int32_t*
     bool wide = g.D == 128 || rows_ok;
     for (int l = 0; l < num_layers && wide; ++l)
         wide = wide_dequant_ok(g, pools[l], out_key[l], out_value[l]);
+    // D = 64: layers whose outputs overlap have the last one's values (callers
+    // that use one pair of outputs for all of them, in order).
+    const size_t out_bytes = (size_t)rows * g.D * sizeof(uint16_t);
+    if (wide && g.D == 64 && num_layers > 1)
+        wide = !outputs_overlap(out_key, out_value, num_layers, out_bytes);
     if (!wide || num_layers == 1) {  // the per-layer kernels (other head dims, unaligned buffers)
         for (int l = 0; l < num_layers; ++l)
             launch_dequant(s, pools[l], slots, out_key[l], out_value[l], g, num_tokens, stream,
