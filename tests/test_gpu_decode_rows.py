@@ -56,3 +56,27 @@ def test_units(tq, oracle, cuda, scheme, Q, H, N, holes, D):
     u = (np.abs(got - ref.astype(np.float16).astype(np.float64)).max(axis=1) / ulp).max()
     print(f"    {u:.2f} row-max ulps", flush=True)
     assert u <= 1.0
+
+
+@pytest.mark.parametrize("D", [128, 64])
+@pytest.mark.parametrize("Q,H,N", [(8, 2, 200), (33, 64, 200), (8, 2, 1500)])
+def test_output_at_any_half(tq, cuda, Q, H, N, D):
+    """An output that starts at an odd half (kernels that write the output
+    themselves store 4 and 8 bytes at a time): the bits of an aligned one."""
+    print(f"[decode rows, output] Q={Q} H={H} N={N} D={D}", flush=True)
+    cfg = tq.default_config()
+    cfg.num_kv_heads, cfg.head_dim = H, D
+    lay = tq.make_layout_for(cfg)
+    g = torch.Generator(device=cuda).manual_seed(720)
+    k, v = (torch.randn(N, H, D, generator=g, device=cuda).half() for _ in range(2))
+    q = torch.randn(Q, H, D, generator=g, device=cuda).half()
+    slots = torch.arange(N, dtype=torch.int32, device=cuda)
+    pool = torch.zeros((N + B - 1) // B * lay.page_size_bytes, dtype=torch.uint8, device=cuda)
+    tq.pack(k, v, slots, pool, lay, cfg)
+    want = torch.zeros_like(q)
+    buf = torch.full((Q * H * D + 2,), 7.0, dtype=torch.float16, device=cuda)
+    tq.fused_attn_output(q, pool, slots, want, lay, cfg, Q, N)
+    tq.fused_attn_output(q, pool, slots, buf[1:-1].view(Q, H, D), lay, cfg, Q, N)
+    torch.cuda.synchronize()
+    assert torch.equal(buf[1:-1].view(Q, H, D).view(torch.int16), want.view(torch.int16))
+    assert buf[0] == 7.0 and buf[-1] == 7.0

@@ -283,6 +283,15 @@ constexpr int kRows = 8;     // query rows per workgroup (16 MFMA columns, hi/lo
 constexpr int kSchMse = 0, kSchProd = 1;
 constexpr int kPartStride = 128 + 4;  // QJL: floats per partial row: o[128], m, l, pad (16-B rows)
 
+// Stores of 2 and 4 output halves (an output row may start at any half).
+__device__ __forceinline__ void store_h2(uint16_t* p, uint32_t v) {
+    typedef uint32_t word __attribute__((aligned(2)));
+    *reinterpret_cast<word*>(p) = v;
+}
+__device__ __forceinline__ void store_h4(uint16_t* p, uint32_t v0, uint32_t v1) {
+    typedef uint32_t pair __attribute__((ext_vector_type(2), aligned(2)));
+    *reinterpret_cast<pair*>(p) = (pair){v0, v1};
+}
 __device__ __forceinline__ uint32_t pack_h2(float a, float b) {
     return __builtin_bit_cast(uint32_t, (half2v){(_Float16)a, (_Float16)b});
 }
@@ -2131,9 +2140,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 if (keep) {
 #pragma unroll
                     for (int k = 0; k < kE; k += 4)
-                        *reinterpret_cast<uint2*>(out + 16 * k) =
-                            make_uint2(fin(o[k] * s0) | (fin(o[k + 1] * -s0) << 16),
-                                       fin(o[k + 2] * s0) | (fin(o[k + 3] * -s0) << 16));
+                        store_h4(out + 16 * k, fin(o[k] * s0) | (fin(o[k + 1] * -s0) << 16),
+                                 fin(o[k + 2] * s0) | (fin(o[k + 3] * -s0) << 16));
                 }
             } else if (keep) {
 #pragma unroll
@@ -2490,8 +2498,8 @@ __global__ __launch_bounds__(64) void attn_paged_combine_kernel(
     merge(std::integral_constant<int, 32>{});
     if (t >= LS) return;
     const auto fin = [&](float o) { return (uint32_t)f2h(L > 0.f ? o / L : o); };
-    *reinterpret_cast<uint2*>(output + ((size_t)q * H + h) * D + d0) =
-        make_uint2(fin(acc.x) | (fin(acc.y) << 16), fin(acc.z) | (fin(acc.w) << 16));
+    store_h4(output + ((size_t)q * H + h) * D + d0, fin(acc.x) | (fin(acc.y) << 16),
+             fin(acc.z) | (fin(acc.w) << 16));
 }
 
 // Inclusive scan over the 1024 threads of a block (16 waves) with an
@@ -3121,10 +3129,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         o0 *= s0;
         o1 *= -s0;
         if (D == 128 || lane < kL)
-            *reinterpret_cast<uint32_t*>(
-                output + ((size_t)(rg * kRows + r) * g.H + h) * D + 2 * jl) =
-                (uint32_t)f2h(L > 0.f ? o0 / L : o0) |
-                ((uint32_t)f2h(L > 0.f ? o1 / L : o1) << 16);
+            store_h2(output + ((size_t)(rg * kRows + r) * g.H + h) * D + 2 * jl,
+                     (uint32_t)f2h(L > 0.f ? o0 / L : o0) | ((uint32_t)f2h(L > 0.f ? o1 / L : o1) << 16));
         return;
     }
     const size_t item = (size_t)rg * g.H + h;
