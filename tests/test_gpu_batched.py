@@ -155,17 +155,18 @@ def test_paged_over_a_thousand_row_groups(tq, cuda):
 @pytest.mark.parametrize("scheme,H,D,B", [
     ("turbo_prod", 2, 128, 7),  # 1,876-byte pages: not 16-byte aligned
     ("turbo_prod", 1, 128, 7),  # 938-byte pages
+    ("turbo_prod", 1, 64, 7),   # 490-byte pages: not 8-byte aligned
+    ("turbo_mse", 4, 32, 5),
+    # aligned pages, D = 64 and 128: the matrix-core kernel
     ("turbo_prod", 2, 64, 16),
     ("turbo_mse", 2, 64, 16),
-    ("turbo_mse", 4, 32, 5),
-    # aligned pages, D = 128: the matrix-core kernel
     ("turbo_prod", 2, 128, 16),
     ("turbo_mse", 2, 128, 16),
     ("turbo_prod", 8, 128, 32),
 ])
 def test_paged_geometries(tq, oracle, cuda, scheme, H, D, B):
     """Geometries the matrix-core kernel does not take (unaligned pages, head
-    dims other than 128) run on the generic split-K decode through the block
+    dims other than 64 and 128) run on the generic split-K decode through the block
     table, the others on the matrix-core kernel: every row against the fp64
     oracle over its sequence's first row_kv_len tokens; a row of kv length 0
     gives 0 and a row whose length passes max_kv_len attends max_kv_len tokens,

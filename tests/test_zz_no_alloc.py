@@ -27,9 +27,9 @@ def _case(oracle, N, seed, Q=8, H=2, D=128, B=16):
     return q, pool, slots, ref
 
 
-def _cfg(tq, H=2, D=128):
+def _cfg(tq, H=2, D=128, B=16):
     cfg = tq.default_config()
-    cfg.num_kv_heads, cfg.head_dim = H, D
+    cfg.num_kv_heads, cfg.head_dim, cfg.block_size = H, D, B
     return cfg, tq.make_layout_for(cfg)
 
 
@@ -134,31 +134,37 @@ def test_noalloc_rejects_launch_beyond_scratch(tq, cuda):
     assert torch.all(out == 3.0)  # nothing ran
 
 
-@pytest.mark.parametrize("D,Q,H,N", [
-    (128, 32, 2, 32768),  # a unit of four row groups over 128 splits: 4.3 MB of partials
-    (128, 192, 2, 8192),
-    (128, 40, 3, 20000),
-    (128, 16, 1, 100),    # one split
-    (64, 8, 2, 3000),
-    (64, 192, 2, 8192),
-    (64, 1, 2048, 300),   # padded row groups of one row: 4.3 MB each split
+@pytest.mark.parametrize("D,Q,H,N,B", [
+    (128, 32, 2, 32768, 16),  # a unit of four row groups over 128 splits: 4.3 MB of partials
+    (128, 192, 2, 8192, 16),
+    (128, 40, 3, 20000, 16),
+    (128, 16, 1, 100, 16),    # one split
+    (64, 8, 2, 3000, 16),
+    (64, 192, 2, 8192, 16),
+    (64, 1, 2048, 300, 16),   # padded row groups of one row: 4.3 MB each split
+    (64, 9, 1, 700, 7),       # 490-byte pages: the generic decode
 ])
-def test_noalloc_same_choice_as_allocating_entry(tq, cuda, D, Q, H, N):
+def test_noalloc_same_choice_as_allocating_entry(tq, oracle, cuda, D, Q, H, N, B):
     """Kernel and split count are the allocating entry's, also where its
-    partials are larger than the 4 MiB that a call is held to: the same bits."""
-    print(f"[noalloc choice] D={D} Q={Q} H={H} N={N}", flush=True)
-    cfg, lp = _cfg(tq, H, D)
+    partials are larger than the 4 MiB that a call is held to: the same bits
+    (small head_dim 64 calls against the oracle too)."""
+    print(f"[noalloc choice] D={D} Q={Q} H={H} N={N} B={B}", flush=True)
+    cfg, lp = _cfg(tq, H, D, B)
     g = torch.Generator(device=cuda).manual_seed(97)
     k, v = (torch.randn(N, H, D, generator=g, device=cuda).half() for _ in range(2))
     q = torch.randn(Q, H, D, generator=g, device=cuda).half()
-    slots = permuted_slots(N, 16, seed=98).to(cuda)
-    pool = torch.zeros((N + 15) // 16 * lp.page_size_bytes, dtype=torch.uint8, device=cuda)
+    slots = permuted_slots(N, B, seed=98).to(cuda)
+    pool = torch.zeros((N + B - 1) // B * lp.page_size_bytes, dtype=torch.uint8, device=cuda)
     tq.pack(k, v, slots, pool, lp, cfg)
     got, want = torch.full_like(q, 3.0), torch.full_like(q, 5.0)
     tq.fused_attn_output(q, pool, slots, want, lp, cfg, Q, N)
     tq.fused_attn_output_noalloc(q, pool, slots, got, lp, cfg, Q, N)
     torch.cuda.synchronize()
     assert np.array_equal(as_u16(got), as_u16(want))
+    if D == 64 and Q < 10:
+        oracle.nthreads = 16
+        ref = oracle.prod_attention_f64(as_u16(q), pool.cpu().numpy(), slots.cpu().numpy(), B)
+        assert _rel(got.cpu().float().numpy(), ref) < 1e-3
 
 
 def test_noalloc_limit_at_head_dim_64(tq, cuda):
