@@ -688,9 +688,9 @@ __device__ __forceinline__ int row_bcast_i(int v) {
 // VEC: the logits rows are 16-byte aligned and num_kv_tokens % 4 == 0.
 // D = 64: two blocks kk instead of four (8 code bytes per lane), and a power of
 // two per query row that holds its fp16 parts in range whatever its magnitude
-// (the fp32 kernel it replaces there took any).  8 rows x 2 heads x 32,768
-// tokens at D = 64: 4.6 us, 16 rows 6.2 us per call, against 10.2 and 18.8 for
-// one thread per (token, row).
+// (the fp32 kernel it replaces there took any).  2 heads x 32,768 tokens at D =
+// 64, calls in a row from a graph: 8 rows 4.8 us, 16 rows 6.7, against 11.6 and
+// 20.9 for one thread per (token, row).
 template <bool VEC, int D>
 __global__ __launch_bounds__(64 * kWaves) void prod_logits_mfma_kernel(
     const uint16_t* __restrict__ query, const uint8_t* __restrict__ pool,
@@ -3327,7 +3327,13 @@ struct DecodeSplit {
 // tokens, in 0.1 us (measured at D = 128, turbo_prod, 2 heads, 250 to 32,768
 // tokens, kernel trace: one group 5.9-7.1 us at one pass, 9.8 at two, 14.8 at
 // four, 22.5 at eight; a unit of two groups 8.2-9.2 at one, of four 11.6 at
-// one, 14.4-15.3 at two, 30.7 at seven).
+// one, 14.4-15.3 at two, 30.7 at seven).  The same constants serve D = 64,
+// turbo_mse and other head counts.  Of 594 shapes of 9 to 256 rows at each D (both
+// schemes, 1-8 heads, 64-32,768 tokens, up to 6.3 M rows x heads x tokens) the
+// kernel they choose is the faster one or within 5% of it but for 8 at D = 128
+// and 7 at D = 64; the worst, 192 rows x 8 heads x 1,143 tokens, takes 18.8 us
+// against 12.4 (D = 64: 13.2 against 11.1), since a merge of 1,536 rows costs
+// more than kMergeCost.
 struct SplitCost {
     int setup, pass;
 };

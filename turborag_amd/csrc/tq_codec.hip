@@ -1114,8 +1114,9 @@ __global__ __launch_bounds__(kBlock, 2) void dequant_rows_kernel(
 }
 
 // head_dim 64, one layer: from this many rows on a row per lane (768 waves)
-// beats the stream kernel's two lanes per row (32,768 rows: 7.0 against 6.2 us;
-// 65,536: 7.8 against 8.8; 131,072: 9.6 against 12.4).
+// beats the stream kernel's two lanes per row (calls in a row from a graph,
+// turbo_prod: 32,768 rows 6.7 against 5.6 us, 40,960 6.7 against 6.7, 49,152 6.8
+// against 7.1, 65,536 6.9 against 7.9, 131,072 8.5 against 11.6).
 constexpr int kOneLayerRows64 = 3 << 14;
 
 // The row-per-lane kernel reads codes as 16-byte pieces.

@@ -15,9 +15,10 @@
 // and one multi-layer dequant per group.  A copy and its event cost 15-20 us
 // beside the bytes, as much as 1 MB of link time (57 GB/s), so small layers
 // were bound by their number; the last group's dequant is the one that no copy
-// hides, so a group is not the whole document.  24 layers of 1.3 MB: 1,070 ->
-// 724 us (0.55 ms of link time); 36 of 0.3 MB: 942 -> 278; 36 of 2.2 MB: 2,413
-// -> 1,610.
+// hides, so a group is not the whole document.  Whole calls from Python: 24
+// layers of 1.3 MB 1,087-1,112 -> 709-718 us (0.55 ms of link time); 36 of 0.3 MB
+// 1,031-1,071 -> 371-380; 36 of 2.2 MB 2,146-2,159 -> 1,605-1,610; 8 of 8.8 MB
+// 1,441-1,453 -> 1,367-1,370.
 #include <algorithm>
 #include <map>
 #include <memory>
