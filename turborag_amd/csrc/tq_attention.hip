@@ -564,20 +564,31 @@ __device__ __forceinline__ int scale_exp(float x) {
 // 2^k is in [2^13, 2^14), and products keep ~22 bits down to 2^-28 of it.  `top` is the largest fp16 with the exponent of the largest
 // finite vs so far; a chunk that passes it lowers k, and the accumulators are
 // rescaled as for a new maximum.  Head_dim 64, and the units over a slot map,
-// carry it.  The one-group and paged kernels at head_dim 128 have k = 0.
-constexpr uint32_t kVTop0 = 0x3FFu;  // (exponent field 0: subnormals and zeros)
-__device__ __forceinline__ float v_power(uint32_t top) {  // k
-    return 28.0f - (float)(int)(top >> 10);
-}
-// Moves top for a chunk whose vs (fp16 bits; 0: no token) are vb, one token in
-// lanes l and l + 32.
-__device__ __forceinline__ void v_raise(uint32_t vb, uint32_t& top) {
-    vb &= 0x7FFFu;
-    if (vb >= 0x7C00u) vb = 0u;  // infinite or NaN
-    if (!__any(vb > top)) return;
-    const uint32_t m = (uint32_t)max_lanes<32>((float)vb);
-    top = (uint32_t)__builtin_amdgcn_readfirstlane((int)m) | 0x3FFu;
-}
+// carry it: 0.1-0.2 us of a call (192 rows x 2 heads x 8,192 tokens, head_dim 128:
+// 16.4 -> 16.6; 8 rows x 200 tokens, head_dim 64: 6.3 -> 6.4).  The one-group and paged kernels at head_dim 128 have k = 0.
+struct VPower {  // wave-uniform
+    uint32_t top = 0x3FFu;  // (exponent field 0: subnormals and zeros)
+    float k = 28.0f;        // 28 - exponent field
+    // For a chunk whose vs (fp16 bits; 0: no token) are vb, one token in lanes l
+    // and l + 32.
+    __device__ __forceinline__ void raise(uint32_t vb) {
+        vb &= 0x7FFFu;
+        // above top and finite
+        if (!__any(vb - (top + 1u) < 0x7C00u - (top + 1u))) return;
+        uint32_t m = vb < 0x7C00u ? vb : 0u;
+        const auto over = [&](auto ctrl) {  // the lane's 16-lane row
+            m = max(m, (uint32_t)__builtin_amdgcn_mov_dpp((int)m, decltype(ctrl)::value, 0xF, 0xF, true));
+        };
+        over(std::integral_constant<int, 0xB1>{});   // quad_perm 1032
+        over(std::integral_constant<int, 0x4E>{});   // quad_perm 2301
+        over(std::integral_constant<int, 0x141>{});  // row_half_mirror
+        over(std::integral_constant<int, 0x140>{});  // row_mirror
+        top = max((uint32_t)__builtin_amdgcn_readlane((int)m, 0),
+                  (uint32_t)__builtin_amdgcn_readlane((int)m, 16)) | 0x3FFu;
+        k = __int_as_float(
+            __builtin_amdgcn_readfirstlane(__float_as_int(28.0f - (float)(int)(top >> 10))));
+    }
+};
 template <bool PROD>
 __device__ __forceinline__ void store_decode_tables(uint32_t* lut, int kv_words, int w, int lane,
                                                     const TableWords<PROD>& tw) {
@@ -1723,7 +1734,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 if constexpr (VLO) acl_col[t][v] = (f32x4){0.f, 0.f, 0.f, 0.f};
             }
         }
-        uint32_t vtop = kVTop0;  // VSCALE: wave-uniform
+        VPower vp;  // VSCALE
         float qsc[kNT];
 #pragma unroll
         for (int t = 0; t < kNT; ++t)
@@ -1737,9 +1748,8 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
             constexpr bool COLS = decltype(cols)::value;
             static_assert(!COLS || NTA == 1, "one tile");
             while (t0 < t_end) {  // wave-uniform
-                // (before the next chunk is fetched into cur)
-                const uint32_t vtop_old = vtop;
-                if constexpr (VSCALE) v_raise(cur.valid ? cur.vs : 0u, vtop);
+                const float k_old = vp.k;
+                if constexpr (VSCALE) vp.raise(cur.valid ? cur.vs : 0u);
                 {
                     const float ks = h2f(cur.ks), vs = h2f(cur.vs), re = PROD ? h2f(cur.re) : 0.0f;
                     const float kx = QSCALE ? 1.0f : ck, kr = QSCALE ? kAlphaK : cr;
@@ -1931,10 +1941,10 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                 }
                 // Online softmax with a lagging maximum: m_col moves (and the
                 // accumulators are rescaled) only when a logit passes it by more
-                // than 1, so the weights stay <= 2 (the PV operand is P * vs / 2).
+                // than 1, so the weights stay <= 2 (2^(k + 1)): the PV operand is
+                // P * vs / 2.
                 float mloc[NTA];
-                bool grow = VSCALE && vtop != vtop_old;
-                const float k_new = VSCALE ? v_power(vtop) : 0.0f;
+                bool grow = VSCALE && vp.k != k_old;
 #pragma unroll
                 for (int t = 0; t < NTA; ++t) {
                     // (IEEE maximum: no canonicalising of the lane-exchanged
@@ -1946,12 +1956,13 @@ __global__ __launch_bounds__(64 * kWaves) void attn_unit_split_kernel(
                     const auto mx = [](float x, float y) { return __builtin_elementwise_maximum(x, y); };
                     m = lane_xor_reduce<16>(m, mx);
                     mloc[t] = lane_xor_reduce<32>(m, mx) * (QSCALE ? qsc[t] : 1.0f);
-                    grow = grow || mloc[t] - k_new > m_col[t] + 1.0f;
+                    grow = grow || (VSCALE ? mloc[t] - vp.k : mloc[t]) > m_col[t] + 1.0f;
                 }
                 if (__any(grow)) {  // wave-uniform
 #pragma unroll
                     for (int t = 0; t < NTA; ++t) {
-                        const float m_new = fmaxf(m_col[t] + (VSCALE ? v_power(vtop_old) : 0.0f), mloc[t]) - k_new;
+                        const float m_new = VSCALE ? fmaxf(m_col[t] + k_old, mloc[t]) - vp.k
+                                                   : fmaxf(m_col[t], mloc[t]);
                         const float alpha = __builtin_amdgcn_exp2f(m_col[t] - m_new);
                         m_col[t] = m_new;
                         l_col[t] *= alpha;
@@ -2913,7 +2924,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         for (int v = 0; v < kNT; ++v) acl[v] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
     bool first = true;
-    uint32_t vtop = kVTop0;  // VSCALE: wave-uniform
+    VPower vp;  // VSCALE
 
     while (t0 < t_end) {  // wave-uniform
         {
@@ -2926,7 +2937,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if constexpr (VSCALE) v_raise(cur.valid ? cur.vs : 0u, vtop);
+        if constexpr (VSCALE) vp.raise(cur.valid ? cur.vs : 0u);
         Chunk nxt;
         const int t1 = t0 + kPass;
         if (t1 < t_end) {  // codes of the next chunk, slots of the one after
@@ -3035,7 +3046,7 @@ __global__ __launch_bounds__(64 * kWaves) void attn_decode_split_kernel(
         // v_exp_f32 without denormal handling: arguments are <= 0 and a weight
         // below 2^-126 of the running maximum is negligible.
         m_run = fmaxf(m_run, QSCALE ? mloc * qsc : mloc);
-        const float ref = VSCALE ? m_run - v_power(vtop) : m_run;
+        const float ref = VSCALE ? m_run - vp.k : m_run;
         const float alpha = first ? 0.0f : __builtin_amdgcn_exp2f(r_run - ref);
         r_run = ref;
         float lsum = 0.0f;

@@ -424,9 +424,13 @@ void* workspace(hipStream_t stream, size_t bytes, size_t want) {
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) throw Error("hipGetDevice failed");
     std::lock_guard<std::mutex> lock(g_ws_mu);
+    auto it = g_ws.find({dev, stream});
+    if (bytes == 0 && it != g_ws.end() && it->second.n >= want) {  // nothing to hand out or make
+        it->second.last_use = ++g_ws_tick;
+        return it->second.p;
+    }
     const bool cap = capturing(stream);
     const size_t need = cap ? bytes : std::max(bytes, want);
-    auto it = g_ws.find({dev, stream});
     if (need == 0 || (it != g_ws.end() && it->second.n >= need && it->second.p)) {
         if (it == g_ws.end()) return nullptr;
         it->second.captured = it->second.captured || (cap && bytes > 0);
